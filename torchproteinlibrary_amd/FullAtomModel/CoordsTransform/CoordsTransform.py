@@ -41,23 +41,20 @@ __all__ = ["CoordsTranslate", "CoordsTranslateFunction", "CoordsRotate", "Coords
            "Coords2Center", "Coords2CenterFunction", "getRotation", "getRandomRotation",
            "getBBox", "getRandomTranslation"]
 
-_STATUS_COUNT = 2
+_STATUS_COUNT, _STATUS_RANGE = 2, 4
 
 
 def _checks_enabled() -> bool:
     return os.environ.get("TPL_A2B_CHECKS", "1") != "0" and not torch.cuda.is_current_stream_capturing()
 
 
-def _status_word(device):
-    return torch.zeros(1, dtype=torch.int32, device=device) if _checks_enabled() else None
-
-
-def _check(out, status, name, where):
-    if status is not None:
-        if int(status.item()) & _STATUS_COUNT:
-            raise ValueError(f"{name}: num_atoms outside [0, coords.size(1)/3] (clamped on the device)")
-        if math.isnan(out.sum()):
-            raise Exception(f"{name}: {where} Nan")
+def _check(bits, out, name, where):
+    """Raises on the status bits of a checked call.  The kernels flag outputs
+    that are NaN, infinite or huge (1e26); only then is the output summed."""
+    if bits & _STATUS_COUNT:
+        raise ValueError(f"{name}: num_atoms outside [0, coords.size(1)/3] (clamped on the device)")
+    if bits & _STATUS_RANGE and math.isnan(out.sum()):
+        raise Exception(f"{name}: {where} Nan")
 
 
 def _rank2(t, name):
@@ -75,9 +72,11 @@ class CoordsTranslateFunction(Function):
         _rank2(input_coords, "CoordsTranslateFunction")
         ctx.save_for_backward(T, num_atoms)
         out = torch.empty_like(input_coords)
-        status = _status_word(input_coords.device)
-        ext.CoordsTranslateGPU_forward(input_coords, out, T.contiguous(), num_atoms, status)
-        _check(out, status, "CoordsTranslateFunction", "forward")
+        if _checks_enabled():
+            _check(ext.CoordsTranslateGPU_forward_checked(input_coords, out, T.contiguous(), num_atoms), out,
+                   "CoordsTranslateFunction", "forward")
+        else:
+            ext.CoordsTranslateGPU_forward(input_coords, out, T.contiguous(), num_atoms)
         return out
 
     @staticmethod
@@ -104,9 +103,11 @@ class CoordsRotateFunction(Function):
         R = R.contiguous()
         ctx.save_for_backward(R, num_atoms)
         out = torch.empty_like(input_coords)
-        status = _status_word(input_coords.device)
-        ext.CoordsRotateGPU_forward(input_coords, out, R, num_atoms, status)
-        _check(out, status, "CoordsRotateFunction", "forward")
+        if _checks_enabled():
+            _check(ext.CoordsRotateGPU_forward_checked(input_coords, out, R, num_atoms), out,
+                   "CoordsRotateFunction", "forward")
+        else:
+            ext.CoordsRotateGPU_forward(input_coords, out, R, num_atoms)
         return out
 
     @staticmethod
@@ -115,9 +116,11 @@ class CoordsRotateFunction(Function):
         R, num_atoms = ctx.saved_tensors
         grad_output_coords = grad_output_coords.contiguous()
         grad_input = torch.empty_like(grad_output_coords)
-        status = _status_word(grad_output_coords.device)
-        ext.CoordsRotateGPU_backward(grad_output_coords, grad_input, R, num_atoms, status)
-        _check(grad_input, status, "CoordsRotateFunction", "backward")
+        if _checks_enabled():
+            _check(ext.CoordsRotateGPU_backward_checked(grad_output_coords, grad_input, R, num_atoms), grad_input,
+                   "CoordsRotateFunction", "backward")
+        else:
+            ext.CoordsRotateGPU_backward(grad_output_coords, grad_input, R, num_atoms)
         return grad_input, None, None
 
 
@@ -134,9 +137,11 @@ class Coords2CenterFunction(Function):
         _rank2(input_coords, "Coords2CenterFunction")
         ctx.save_for_backward(input_coords, num_atoms)
         center = torch.empty(input_coords.size(0), 3, dtype=input_coords.dtype, device=input_coords.device)
-        status = _status_word(input_coords.device)
-        ext.Coords2CenterGPU_forward(input_coords, center, num_atoms, status)
-        _check(center, status, "Coords2CenterFunction", "forward")
+        if _checks_enabled():
+            _check(ext.Coords2CenterGPU_forward_checked(input_coords, center, num_atoms), center,
+                   "Coords2CenterFunction", "forward")
+        else:
+            ext.Coords2CenterGPU_forward(input_coords, center, num_atoms)
         return center
 
     @staticmethod
@@ -145,9 +150,11 @@ class Coords2CenterFunction(Function):
         input_coords, num_atoms = ctx.saved_tensors
         grad_output_center = grad_output_center.contiguous()
         grad_input = torch.empty_like(input_coords)
-        status = _status_word(input_coords.device)
-        ext.Coords2CenterGPU_backward(grad_output_center, grad_input, num_atoms, status)
-        _check(grad_input, status, "Coords2CenterFunction", "backward")
+        if _checks_enabled():
+            _check(ext.Coords2CenterGPU_backward_checked(grad_output_center, grad_input, num_atoms), grad_input,
+                   "Coords2CenterFunction", "backward")
+        else:
+            ext.Coords2CenterGPU_backward(grad_output_center, grad_input, num_atoms)
         return grad_input, None
 
 

@@ -14,17 +14,17 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "report.h"
 #include "tpl_xform.h"
+#include "xform_flagged.h"
 
 namespace {
 
 constexpr int kThreads = 256;
 
-__device__ __forceinline__ int clamp_count(int n, int A, uint32_t* status, bool report_it) {
+__device__ __forceinline__ int clamp_count(int n, int A, const Report& rep, bool report_it) {
     if (n < 0 || n > A) {
-        if (report_it && status)
-            __hip_atomic_fetch_or(status, TPL_XFORM_STATUS_COUNT, __ATOMIC_RELAXED,
-                                  __HIP_MEMORY_SCOPE_AGENT);
+        if (report_it) report_bits(rep, TPL_XFORM_STATUS_COUNT);
         return n < 0 ? 0 : A;
     }
     return n;
@@ -47,11 +47,11 @@ template <typename T>
 __global__ void __launch_bounds__(kThreads) xform_shift(T* out, const T* __restrict__ in,
                                                         const T* __restrict__ tv, int per_n,
                                                         const int32_t* __restrict__ num_atoms,
-                                                        uint32_t* status, int A, int nblk) {
+                                                        Report rep, int A, int nblk) {
     constexpr int E = 16 / (int)sizeof(T);  // values per 16-byte block
     const int b = blockIdx.x / nblk;
     const int64_t blk0 = (int64_t)(blockIdx.x - b * nblk) * kThreads * kBlocksPerThread;
-    const int n = clamp_count(num_atoms[b], A, status, blk0 == 0 && threadIdx.x == 0);
+    const int n = clamp_count(num_atoms[b], A, rep, blk0 == 0 && threadIdx.x == 0);
     const int64_t vals = 3 * (int64_t)A, valid = 3 * (int64_t)n;
     T* o = out + (size_t)b * vals;
     const T* p = in ? in + (size_t)b * vals : nullptr;
@@ -62,6 +62,7 @@ __global__ void __launch_bounds__(kThreads) xform_shift(T* out, const T* __restr
         for (int c = 0; c < 3; ++c) t[c] = tv[3 * (size_t)b + c] * sc;
     }
     const bool vec = aligned16(o) && (!p || aligned16(p));
+    bool range = false;
 #pragma unroll
     for (int r = 0; r < kBlocksPerThread; ++r) {
         const int64_t v0 = ((int64_t)blk0 + r * kThreads + threadIdx.x) * E;
@@ -81,6 +82,7 @@ __global__ void __launch_bounds__(kThreads) xform_shift(T* out, const T* __restr
 #pragma unroll
             for (int e = 0; e < E; ++e) {
                 v[e] = v0 + e < valid ? v[e] + t[c] : (T)0;
+                range |= out_of_range(v[e]);
                 c = c == 2 ? 0 : c + 1;
             }
             uint4 u;
@@ -89,10 +91,13 @@ __global__ void __launch_bounds__(kThreads) xform_shift(T* out, const T* __restr
         } else {
             for (int e = 0; e < E && v0 + e < vals; ++e) {
                 const int64_t i = v0 + e;
-                o[i] = i < valid ? (p ? p[i] : (T)0) + t[(uint32_t)i % 3u] : (T)0;
+                const T v1 = i < valid ? (p ? p[i] : (T)0) + t[(uint32_t)i % 3u] : (T)0;
+                range |= out_of_range(v1);
+                o[i] = v1;
             }
         }
     }
+    if (range) report_flag(rep, TPLX_XFORM_RANGE);
 }
 
 // out_i = M in_i + t for the atoms of the structure (M = R, R^T with
@@ -127,7 +132,7 @@ __global__ void __launch_bounds__(kThreads) xform_waves(T* out, const T* __restr
                                                         const T* __restrict__ R, int transpose,
                                                         const T* __restrict__ tv,
                                                         const int32_t* __restrict__ num_atoms,
-                                                        uint32_t* status, int A, int nblk) {
+                                                        Report rep, int A, int nblk) {
     constexpr int E = 16 / (int)sizeof(T);  // values per 16-byte access
     constexpr int V = 3 * kWaveAtoms;       // values per chunk
     constexpr int kPerLane = kWaveAtoms / 64;
@@ -136,7 +141,7 @@ __global__ void __launch_bounds__(kThreads) xform_waves(T* out, const T* __restr
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int a0 = ((blockIdx.x - b * nblk) * (kThreads / 64) + wave) * kWaveAtoms;
     if (a0 >= A) return;  // the whole wave: no workgroup barrier follows
-    const int n = clamp_count(num_atoms[b], A, status, a0 == 0 && lane == 0);
+    const int n = clamp_count(num_atoms[b], A, rep, a0 == 0 && lane == 0);
     T* o = out + (size_t)b * 3 * A;
     const T* p = in + (size_t)b * 3 * A;
     T m[9], t[3] = {(T)0, (T)0, (T)0};
@@ -157,6 +162,7 @@ __global__ void __launch_bounds__(kThreads) xform_waves(T* out, const T* __restr
             }
         }
         wave_lds_sync();
+        bool range = false;
 #pragma unroll
         for (int k = 0; k < kPerLane; ++k) {
             const int q = kPerLane * lane + k;
@@ -165,7 +171,10 @@ __global__ void __launch_bounds__(kThreads) xform_waves(T* out, const T* __restr
                 if (R) rotate_atom(m, transpose, v, w);
                 else w[0] = v[0], w[1] = v[1], w[2] = v[2];
 #pragma unroll
-                for (int c = 0; c < 3; ++c) w[c] += t[c];
+                for (int c = 0; c < 3; ++c) {
+                    w[c] += t[c];
+                    range |= out_of_range(w[c]);
+                }
             }
             buf[3 * q] = w[0];
             buf[3 * q + 1] = w[1];
@@ -177,8 +186,10 @@ __global__ void __launch_bounds__(kThreads) xform_waves(T* out, const T* __restr
             const int idx = (j * 64 + lane) * E;
             *reinterpret_cast<uint4*>(o + 3 * (size_t)a0 + idx) = *reinterpret_cast<const uint4*>(buf + idx);
         }
+        if (range) report_flag(rep, TPLX_XFORM_RANGE);
         return;
     }
+    bool range = false;
 #pragma unroll
     for (int k = 0; k < kPerLane; ++k) {
         const int i = a0 + kPerLane * lane + k;
@@ -191,12 +202,16 @@ __global__ void __launch_bounds__(kThreads) xform_waves(T* out, const T* __restr
             if (R) rotate_atom(m, transpose, v, w);
             else w[0] = v[0], w[1] = v[1], w[2] = v[2];
 #pragma unroll
-            for (int c = 0; c < 3; ++c) w[c] += t[c];
+            for (int c = 0; c < 3; ++c) {
+                w[c] += t[c];
+                range |= out_of_range(w[c]);
+            }
         }
         o[3 * (size_t)i] = w[0];
         o[3 * (size_t)i + 1] = w[1];
         o[3 * (size_t)i + 2] = w[2];
     }
+    if (range) report_flag(rep, TPLX_XFORM_RANGE);
 }
 
 // center[b] = (sum of the first n atoms) / n, summed in FP64: each thread over
@@ -205,12 +220,12 @@ __global__ void __launch_bounds__(kThreads) xform_waves(T* out, const T* __restr
 template <typename T>
 __global__ void __launch_bounds__(kThreads) xform_center(T* center, const T* __restrict__ in,
                                                          const int32_t* __restrict__ num_atoms,
-                                                         uint32_t* status, int A) {
+                                                         Report rep, int A) {
     constexpr int kParts = 16;
     __shared__ double s_m[3 * kThreads];
     __shared__ double s_p[3 * kParts];
     const int b = blockIdx.x, tid = threadIdx.x;
-    const int n = clamp_count(num_atoms[b], A, status, tid == 0);
+    const int n = clamp_count(num_atoms[b], A, rep, tid == 0);
     const T* p = in + (size_t)b * 3 * A;
     constexpr int kPer16 = 16 / (int)sizeof(T);
     double acc[3] = {0.0, 0.0, 0.0};
@@ -246,7 +261,9 @@ __global__ void __launch_bounds__(kThreads) xform_center(T* center, const T* __r
         double s = 0.0;
 #pragma unroll
         for (int part = 0; part < kParts; ++part) s += s_p[tid * kParts + part];
-        center[3 * (size_t)b + tid] = (T)(s / (double)n);
+        const T c = (T)(s / (double)n);
+        if (out_of_range(c)) report_flag(rep, TPLX_XFORM_RANGE);
+        center[3 * (size_t)b + tid] = c;
     }
 }
 
@@ -258,7 +275,7 @@ int check(int dtype, int B, int A) {
 }
 
 int launch_affine(int dtype, void* out, const void* in, const void* R, int transpose,
-                  const void* tv, int per_n, const int32_t* num_atoms, uint32_t* status, int B,
+                  const void* tv, int per_n, const int32_t* num_atoms, const Report& rep, int B,
                   int A, tpl_xform_stream_t stream) {
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (in && !per_n) {
@@ -270,12 +287,12 @@ int launch_affine(int dtype, void* out, const void* in, const void* R, int trans
             hipLaunchKernelGGL(xform_waves<float>, dim3(nblk * B), dim3(kThreads), 0, s,
                                static_cast<float*>(out), static_cast<const float*>(in),
                                static_cast<const float*>(R), transpose, static_cast<const float*>(tv),
-                               num_atoms, status, A, nblk);
+                               num_atoms, rep, A, nblk);
         else
             hipLaunchKernelGGL(xform_waves<double>, dim3(nblk * B), dim3(kThreads), 0, s,
                                static_cast<double*>(out), static_cast<const double*>(in),
                                static_cast<const double*>(R), transpose, static_cast<const double*>(tv),
-                               num_atoms, status, A, nblk);
+                               num_atoms, rep, A, nblk);
         return hipGetLastError() == hipSuccess ? TPL_XFORM_OK : TPL_XFORM_ERR_LAUNCH;
     }
     if (!R) {
@@ -286,14 +303,60 @@ int launch_affine(int dtype, void* out, const void* in, const void* R, int trans
         if (dtype == TPL_XFORM_F32)
             hipLaunchKernelGGL(xform_shift<float>, dim3(nblk * B), dim3(kThreads), 0, s,
                                static_cast<float*>(out), static_cast<const float*>(in),
-                               static_cast<const float*>(tv), per_n, num_atoms, status, A, nblk);
+                               static_cast<const float*>(tv), per_n, num_atoms, rep, A, nblk);
         else
             hipLaunchKernelGGL(xform_shift<double>, dim3(nblk * B), dim3(kThreads), 0, s,
                                static_cast<double*>(out), static_cast<const double*>(in),
-                               static_cast<const double*>(tv), per_n, num_atoms, status, A, nblk);
+                               static_cast<const double*>(tv), per_n, num_atoms, rep, A, nblk);
         return hipGetLastError() == hipSuccess ? TPL_XFORM_OK : TPL_XFORM_ERR_LAUNCH;
     }
     return TPL_XFORM_ERR_ARG;  // a rotation needs an input
+}
+
+// The entry points, reporting as `rep` says.
+int translate(int dtype, void* out, const void* in, const void* T, const int32_t* num_atoms, const Report& rep,
+              int batch, int atoms_stride, tpl_xform_stream_t stream) {
+    const int rc = check(dtype, batch, atoms_stride);
+    if (rc != TPL_XFORM_OK) return rc;
+    if (batch == 0 || atoms_stride == 0) return TPL_XFORM_OK;
+    if (!out || !in || !T || !num_atoms) return TPL_XFORM_ERR_ARG;
+    return launch_affine(dtype, out, in, nullptr, 0, T, 0, num_atoms, rep, batch, atoms_stride, stream);
+}
+
+int rotate(int dtype, void* out, const void* in, const void* R, int transpose, const int32_t* num_atoms,
+           const Report& rep, int batch, int atoms_stride, tpl_xform_stream_t stream) {
+    const int rc = check(dtype, batch, atoms_stride);
+    if (rc != TPL_XFORM_OK) return rc;
+    if (batch == 0 || atoms_stride == 0) return TPL_XFORM_OK;
+    if (!out || !in || !R || !num_atoms) return TPL_XFORM_ERR_ARG;
+    return launch_affine(dtype, out, in, R, transpose ? 1 : 0, nullptr, 0, num_atoms, rep, batch, atoms_stride,
+                         stream);
+}
+
+int center_of(int dtype, void* center, const void* in, const int32_t* num_atoms, const Report& rep, int batch,
+              int atoms_stride, tpl_xform_stream_t stream) {
+    const int rc = check(dtype, batch, atoms_stride);
+    if (rc != TPL_XFORM_OK) return rc;
+    if (batch == 0) return TPL_XFORM_OK;
+    if (!center || !num_atoms || (atoms_stride > 0 && !in)) return TPL_XFORM_ERR_ARG;
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    if (dtype == TPL_XFORM_F32)
+        hipLaunchKernelGGL(xform_center<float>, dim3(batch), dim3(kThreads), 0, s, static_cast<float*>(center),
+                           static_cast<const float*>(in), num_atoms, rep, atoms_stride);
+    else
+        hipLaunchKernelGGL(xform_center<double>, dim3(batch), dim3(kThreads), 0, s, static_cast<double*>(center),
+                           static_cast<const double*>(in), num_atoms, rep, atoms_stride);
+    return hipGetLastError() == hipSuccess ? TPL_XFORM_OK : TPL_XFORM_ERR_LAUNCH;
+}
+
+int center_backward(int dtype, void* grad_in, const void* grad_center, const int32_t* num_atoms,
+                    const Report& rep, int batch, int atoms_stride, tpl_xform_stream_t stream) {
+    const int rc = check(dtype, batch, atoms_stride);
+    if (rc != TPL_XFORM_OK) return rc;
+    if (batch == 0 || atoms_stride == 0) return TPL_XFORM_OK;
+    if (!grad_in || !grad_center || !num_atoms) return TPL_XFORM_ERR_ARG;
+    return launch_affine(dtype, grad_in, nullptr, nullptr, 0, grad_center, 1, num_atoms, rep, batch,
+                         atoms_stride, stream);
 }
 
 }  // namespace
@@ -313,12 +376,7 @@ const char* tpl_xform_strerror(int code) {
 int tpl_xform_translate(int dtype, void* out, const void* in, const void* T,
                         const int32_t* num_atoms, uint32_t* status, int batch, int atoms_stride,
                         tpl_xform_stream_t stream) {
-    const int rc = check(dtype, batch, atoms_stride);
-    if (rc != TPL_XFORM_OK) return rc;
-    if (batch == 0 || atoms_stride == 0) return TPL_XFORM_OK;
-    if (!out || !in || !T || !num_atoms) return TPL_XFORM_ERR_ARG;
-    return launch_affine(dtype, out, in, nullptr, 0, T, 0, num_atoms, status, batch, atoms_stride,
-                         stream);
+    return translate(dtype, out, in, T, num_atoms, Report{status, nullptr}, batch, atoms_stride, stream);
 }
 
 int tpl_xform_translate_backward(int dtype, void* grad_in, const void* grad_out,
@@ -328,48 +386,48 @@ int tpl_xform_translate_backward(int dtype, void* grad_in, const void* grad_out,
     if (rc != TPL_XFORM_OK) return rc;
     if (batch == 0 || atoms_stride == 0) return TPL_XFORM_OK;
     if (!grad_in || !grad_out || !num_atoms) return TPL_XFORM_ERR_ARG;
-    return launch_affine(dtype, grad_in, grad_out, nullptr, 0, nullptr, 0, num_atoms, status, batch,
-                         atoms_stride, stream);
+    return launch_affine(dtype, grad_in, grad_out, nullptr, 0, nullptr, 0, num_atoms, Report{status, nullptr},
+                         batch, atoms_stride, stream);
 }
 
 int tpl_xform_rotate(int dtype, void* out, const void* in, const void* R, int transpose,
                      const int32_t* num_atoms, uint32_t* status, int batch, int atoms_stride,
                      tpl_xform_stream_t stream) {
-    const int rc = check(dtype, batch, atoms_stride);
-    if (rc != TPL_XFORM_OK) return rc;
-    if (batch == 0 || atoms_stride == 0) return TPL_XFORM_OK;
-    if (!out || !in || !R || !num_atoms) return TPL_XFORM_ERR_ARG;
-    return launch_affine(dtype, out, in, R, transpose ? 1 : 0, nullptr, 0, num_atoms, status, batch,
-                         atoms_stride, stream);
+    return rotate(dtype, out, in, R, transpose, num_atoms, Report{status, nullptr}, batch, atoms_stride, stream);
 }
 
 int tpl_xform_center(int dtype, void* center, const void* in, const int32_t* num_atoms,
                      uint32_t* status, int batch, int atoms_stride, tpl_xform_stream_t stream) {
-    const int rc = check(dtype, batch, atoms_stride);
-    if (rc != TPL_XFORM_OK) return rc;
-    if (batch == 0) return TPL_XFORM_OK;
-    if (!center || !num_atoms || (atoms_stride > 0 && !in)) return TPL_XFORM_ERR_ARG;
-    hipStream_t s = static_cast<hipStream_t>(stream);
-    if (dtype == TPL_XFORM_F32)
-        hipLaunchKernelGGL(xform_center<float>, dim3(batch), dim3(kThreads), 0, s,
-                           static_cast<float*>(center), static_cast<const float*>(in), num_atoms,
-                           status, atoms_stride);
-    else
-        hipLaunchKernelGGL(xform_center<double>, dim3(batch), dim3(kThreads), 0, s,
-                           static_cast<double*>(center), static_cast<const double*>(in), num_atoms,
-                           status, atoms_stride);
-    return hipGetLastError() == hipSuccess ? TPL_XFORM_OK : TPL_XFORM_ERR_LAUNCH;
+    return center_of(dtype, center, in, num_atoms, Report{status, nullptr}, batch, atoms_stride, stream);
 }
 
 int tpl_xform_center_backward(int dtype, void* grad_in, const void* grad_center,
                               const int32_t* num_atoms, uint32_t* status, int batch,
                               int atoms_stride, tpl_xform_stream_t stream) {
-    const int rc = check(dtype, batch, atoms_stride);
-    if (rc != TPL_XFORM_OK) return rc;
-    if (batch == 0 || atoms_stride == 0) return TPL_XFORM_OK;
-    if (!grad_in || !grad_center || !num_atoms) return TPL_XFORM_ERR_ARG;
-    return launch_affine(dtype, grad_in, nullptr, nullptr, 0, grad_center, 1, num_atoms, status,
-                         batch, atoms_stride, stream);
+    return center_backward(dtype, grad_in, grad_center, num_atoms, Report{status, nullptr}, batch, atoms_stride,
+                           stream);
+}
+
+int tplx_xform_translate(int dtype, void* out, const void* in, const void* T, const int32_t* num_atoms,
+                         uint32_t* flags, int batch, int atoms_stride, tpl_xform_stream_t stream) {
+    return translate(dtype, out, in, T, num_atoms, Report{nullptr, flags}, batch, atoms_stride, stream);
+}
+
+int tplx_xform_rotate(int dtype, void* out, const void* in, const void* R, int transpose,
+                      const int32_t* num_atoms, uint32_t* flags, int batch, int atoms_stride,
+                      tpl_xform_stream_t stream) {
+    return rotate(dtype, out, in, R, transpose, num_atoms, Report{nullptr, flags}, batch, atoms_stride, stream);
+}
+
+int tplx_xform_center(int dtype, void* center, const void* in, const int32_t* num_atoms, uint32_t* flags,
+                      int batch, int atoms_stride, tpl_xform_stream_t stream) {
+    return center_of(dtype, center, in, num_atoms, Report{nullptr, flags}, batch, atoms_stride, stream);
+}
+
+int tplx_xform_center_backward(int dtype, void* grad_in, const void* grad_center, const int32_t* num_atoms,
+                               uint32_t* flags, int batch, int atoms_stride, tpl_xform_stream_t stream) {
+    return center_backward(dtype, grad_in, grad_center, num_atoms, Report{nullptr, flags}, batch, atoms_stride,
+                           stream);
 }
 
 }  // extern "C"

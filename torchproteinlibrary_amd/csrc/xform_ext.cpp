@@ -13,7 +13,9 @@
 #include <tuple>
 #include <vector>
 
+#include "host_flags.h"
 #include "tpl_xform.h"
+#include "xform_flagged.h"
 
 namespace {
 
@@ -137,6 +139,73 @@ void center_backward(torch::Tensor grad_output_center, torch::Tensor grad_input_
              "Coords2CenterGPU_backward");
 }
 
+// The checked forms: as the entry points above without a status, and they wait
+// for the work and return its status bits (xform_flagged.h).
+int64_t translate_forward_checked(torch::Tensor input_coords, torch::Tensor output_coords, torch::Tensor T,
+                                  torch::Tensor num_atoms) {
+    auto [B, A] = check_coords(input_coords, num_atoms);
+    check_like(output_coords, input_coords, {B, 3 * (int64_t)A}, "output_coords");
+    check_like(T, input_coords, {B, 3}, "T");
+    c10::DeviceGuard guard(input_coords.device());
+    hipStream_t s = stream_of(input_coords);
+    return host_flags::run(s, [&, B = B, A = A](uint32_t* flags) {
+        check_rc(tplx_xform_translate(dtype_code(input_coords), output_coords.data_ptr(), input_coords.data_ptr(),
+                                      T.data_ptr(), num_atoms.data_ptr<int32_t>(), flags, B, A, s),
+                 "CoordsTranslateGPU_forward");
+    });
+}
+
+int64_t rotate_checked(const torch::Tensor& in, const torch::Tensor& out, const torch::Tensor& R,
+                       const torch::Tensor& num_atoms, int transpose, const char* what) {
+    auto [B, A] = check_coords(in, num_atoms);
+    check_like(out, in, {B, 3 * (int64_t)A}, "output");
+    check_like(R, in, {B, 3, 3}, "R");
+    c10::DeviceGuard guard(in.device());
+    hipStream_t s = stream_of(in);
+    return host_flags::run(s, [&, B = B, A = A](uint32_t* flags) {
+        check_rc(tplx_xform_rotate(dtype_code(in), out.data_ptr(), in.data_ptr(), R.data_ptr(), transpose,
+                                   num_atoms.data_ptr<int32_t>(), flags, B, A, s),
+                 what);
+    });
+}
+
+int64_t rotate_forward_checked(torch::Tensor input_coords, torch::Tensor output_coords, torch::Tensor R,
+                               torch::Tensor num_atoms) {
+    return rotate_checked(input_coords, output_coords, R, num_atoms, 0, "CoordsRotateGPU_forward");
+}
+
+int64_t rotate_backward_checked(torch::Tensor grad_output_coords, torch::Tensor grad_input_coords,
+                                torch::Tensor R, torch::Tensor num_atoms) {
+    return rotate_checked(grad_output_coords, grad_input_coords, R, num_atoms, 1, "CoordsRotateGPU_backward");
+}
+
+int64_t center_forward_checked(torch::Tensor input_coords, torch::Tensor output_center,
+                               torch::Tensor num_atoms) {
+    auto [B, A] = check_coords(input_coords, num_atoms);
+    check_like(output_center, input_coords, {B, 3}, "output_center");
+    c10::DeviceGuard guard(input_coords.device());
+    hipStream_t s = stream_of(input_coords);
+    return host_flags::run(s, [&, B = B, A = A](uint32_t* flags) {
+        check_rc(tplx_xform_center(dtype_code(input_coords), output_center.data_ptr(), input_coords.data_ptr(),
+                                   num_atoms.data_ptr<int32_t>(), flags, B, A, s),
+                 "Coords2CenterGPU_forward");
+    });
+}
+
+int64_t center_backward_checked(torch::Tensor grad_output_center, torch::Tensor grad_input_coords,
+                                torch::Tensor num_atoms) {
+    auto [B, A] = check_coords(grad_input_coords, num_atoms);
+    check_like(grad_output_center, grad_input_coords, {B, 3}, "grad_output_center");
+    c10::DeviceGuard guard(grad_input_coords.device());
+    hipStream_t s = stream_of(grad_input_coords);
+    return host_flags::run(s, [&, B = B, A = A](uint32_t* flags) {
+        check_rc(tplx_xform_center_backward(dtype_code(grad_input_coords), grad_input_coords.data_ptr(),
+                                            grad_output_center.data_ptr(), num_atoms.data_ptr<int32_t>(), flags,
+                                            B, A, s),
+                 "Coords2CenterGPU_backward");
+    });
+}
+
 // Timing loop for bench.py: sets of [coords, out, T, R, center, num_atoms],
 // rotated per launch.  Returns the average HIP-event ms of one launch of
 // translate, rotate, centre and centre-backward, each run `reps` times.
@@ -216,6 +285,12 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
           py::arg("input_coords"), py::arg("output_center"), py::arg("num_atoms"), st);
     m.def("Coords2CenterGPU_backward", &center_backward, "Backward of coordinates center on GPU",
           py::arg("grad_output_center"), py::arg("grad_input_coords"), py::arg("num_atoms"), st);
+    auto nogil = py::call_guard<py::gil_scoped_release>();
+    m.def("CoordsTranslateGPU_forward_checked", &translate_forward_checked, "Status bits of the forward", nogil);
+    m.def("CoordsRotateGPU_forward_checked", &rotate_forward_checked, "Status bits of the forward", nogil);
+    m.def("CoordsRotateGPU_backward_checked", &rotate_backward_checked, "Status bits of the backward", nogil);
+    m.def("Coords2CenterGPU_forward_checked", &center_forward_checked, "Status bits of the forward", nogil);
+    m.def("Coords2CenterGPU_backward_checked", &center_backward_checked, "Status bits of the backward", nogil);
     m.def("bench", &bench, "average event ms of translate, rotate, centre, centre-backward");
     register_a2c(m);
     register_pdb(m);
