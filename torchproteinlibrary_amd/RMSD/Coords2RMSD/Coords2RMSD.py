@@ -54,14 +54,7 @@ def _checks_enabled() -> bool:
     return os.environ.get("TPL_A2B_CHECKS", "1") != "0" and not torch.cuda.is_current_stream_capturing()
 
 
-def _status_word(device):
-    return torch.zeros(1, dtype=torch.int32, device=device) if _checks_enabled() else None
-
-
-def _raise_on_status(status, where: str) -> None:
-    if status is None:
-        return
-    bits = int(status.item())
+def _raise_on_bits(bits: int, where: str) -> None:
     if bits & _STATUS_COUNT:
         raise ValueError("Coords2RMSDFunction: num_atoms outside [0, input.size(1)/3] "
                          "(clamped on the device)")
@@ -88,10 +81,11 @@ class Coords2RMSDFunction(Function):
         UT = torch.empty(B, 3, 3, dtype=dt, device=dev)
         state = (torch.empty(max(ext.state_bytes(B), 1), dtype=torch.uint8, device=dev)
                  if ctx.needs_input_grad[0] else None)
-        status = _status_word(dev)
-        ext.Coords2RMSDGPU_forward(centered_input, centered_target, output, num_atoms, UT, state,
-                                   status)
-        _raise_on_status(status, "forward")
+        if _checks_enabled():
+            _raise_on_bits(ext.Coords2RMSDGPU_forward_checked(centered_input, centered_target, output, num_atoms,
+                                                              UT, state), "forward")
+        else:
+            ext.Coords2RMSDGPU_forward(centered_input, centered_target, output, num_atoms, UT, state, None)
         ctx.mark_non_differentiable(UT)
         if state is not None:
             ctx.save_for_backward(centered_input, centered_target, num_atoms, state)
@@ -105,10 +99,12 @@ class Coords2RMSDFunction(Function):
         if gradRMSD.dtype != centered_input.dtype:
             gradRMSD = gradRMSD.to(centered_input.dtype)
         grad_input = torch.empty_like(centered_input)
-        status = _status_word(centered_input.device)
-        ext.Coords2RMSDGPU_backward(grad_input, gradRMSD, centered_input, centered_target,
-                                    num_atoms, state, status)
-        _raise_on_status(status, "backward")
+        if _checks_enabled():
+            _raise_on_bits(ext.Coords2RMSDGPU_backward_checked(grad_input, gradRMSD, centered_input,
+                                                               centered_target, num_atoms, state), "backward")
+        else:
+            ext.Coords2RMSDGPU_backward(grad_input, gradRMSD, centered_input, centered_target,
+                                        num_atoms, state, None)
         return grad_input, None, None
 
 

@@ -27,8 +27,8 @@ What differs, by design:
   frames past the chain there);
 * lengths outside [0, L_max] are clamped on the device and reported (the
   reference writes out of bounds);
-* the NaN / length checks read one status word written by the kernels (one
-  host sync, like the reference's ``output.sum()``); they are skipped while a
+* the NaN / length checks read status flags that the kernels write into host
+  memory (one host sync, like the reference's ``output.sum()``); they are skipped while a
   stream is being captured, and ``TPL_A2B_CHECKS=0`` turns them off;
 * the look-back words of the kernels live in one zero-initialised buffer per
   (device, stream), whose tickets, counters and flags every call returns to
@@ -66,25 +66,21 @@ def _status_word(device):
     return torch.zeros(1, dtype=torch.int32, device=device) if _checks_enabled() else None
 
 
-def _run_checked(launch, status, where: str, sync) -> None:
-    """Runs launch(status) and raises on the status bits.  A look-back
-    timeout or unclean look-back words make the result invalid: the words are
-    cleared and the call is run once more, with a RuntimeWarning, and only a
-    second failure raises.  The kernels' waits are bounded (a wave that never
-    sees its record gives up and reports TIMEOUT instead of hanging), so this
-    is the recovery path for a call that ran out of wait time."""
-    launch(status)
-    if status is None:
-        return
-    bits = int(status.item())
+def _run_checked(checked, where: str, sync) -> None:
+    """Runs checked(), which returns the call's status bits, and raises on
+    them.  A look-back timeout or unclean look-back words make the result
+    invalid: the words are cleared and the call is run once more, with a
+    RuntimeWarning, and only a second failure raises.  The kernels' waits are
+    bounded (a wave that never sees its record gives up and reports TIMEOUT
+    instead of hanging), so this is the recovery path for a call that ran out
+    of wait time."""
+    bits = checked()
     if bits & (_STATUS_TIMEOUT | _STATUS_SYNC):
         ext.sync_clear(sync)  # look-back words may be left set
         what = "look-back wait timed out" if bits & _STATUS_TIMEOUT else "look-back words were not clean"
         warnings.warn("Angles2BackboneFunction: %s %s; cleared and repeated" % (where, what),
                       RuntimeWarning)
-        status.zero_()
-        launch(status)
-        bits = int(status.item())
+        bits = checked()
         if bits & (_STATUS_TIMEOUT | _STATUS_SYNC):
             ext.sync_clear(sync)
             what = "look-back wait timed out" if bits & _STATUS_TIMEOUT else "look-back words were not clean"
@@ -155,10 +151,12 @@ class Angles2BackboneGPUFunction(Function):
                                                  list(cfg))
         state = _empty_bytes(st_bytes, dev) if ctx.needs_input_grad[0] else None
         sync = _sync_buffer(dev, sy_bytes)
-        status = _status_word(dev)
-        _run_checked(lambda st: ext.Angles2BackboneGPU_forward(input_angles, coords, angles_length,
-                                                               state, sync, st, list(cfg)),
-                     status, "forward", sync)
+        if _checks_enabled():
+            _run_checked(lambda: ext.Angles2BackboneGPU_forward_checked(input_angles, coords, angles_length,
+                                                                        state, sync, cfg),
+                         "forward", sync)
+        else:
+            ext.Angles2BackboneGPU_forward(input_angles, coords, angles_length, state, sync, None, cfg)
         if state is not None:
             ctx.save_for_backward(input_angles, angles_length, state)
         ctx.cfg = cfg
@@ -176,11 +174,13 @@ class Angles2BackboneGPUFunction(Function):
         gradInput = torch.empty(B, 3, L, dtype=input_angles.dtype, device=dev)
         _, sy_bytes = ext.workspace_bytes(input_angles.dtype == torch.float64, B, L, list(ctx.cfg))
         sync = _sync_buffer(dev, sy_bytes)
-        status = _status_word(dev)
-        _run_checked(lambda st: ext.Angles2BackboneGPU_backward(gradInput, gradOutput, input_angles,
-                                                                angles_length, state, sync, st,
-                                                                list(ctx.cfg)),
-                     status, "backward", sync)
+        if _checks_enabled():
+            _run_checked(lambda: ext.Angles2BackboneGPU_backward_checked(gradInput, gradOutput, input_angles,
+                                                                         angles_length, state, sync, ctx.cfg),
+                         "backward", sync)
+        else:
+            ext.Angles2BackboneGPU_backward(gradInput, gradOutput, input_angles, angles_length, state, sync,
+                                            None, ctx.cfg)
         return gradInput, None
 
 

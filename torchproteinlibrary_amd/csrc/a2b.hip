@@ -47,6 +47,8 @@
 #include <vector>
 
 #include "sincos_tab.h"
+#include "a2b_flagged.h"
+#include "report.h"
 #include "tpl_a2b.h"
 
 namespace {
@@ -507,7 +509,7 @@ struct ChunkArgs {
     const void* grad;        // backward input [B][9L]
     void* grad_angles;       // backward output [B][3][L]
     const int32_t* lengths;  // [B]
-    uint32_t* status;
+    Report rep;              // where status bits go
     double* ckpt;            // [B][nk][kF]: entry k is the frame of atom 3kK (N of
                              // residue kK), written for 0 < kK < n; null: none
     uint32_t* tickets;       // [8][sbx]: chain b at (b mod 8) * sbx + b / 8
@@ -705,7 +707,7 @@ __device__ __forceinline__ uint32_t ticket_issue(const ChunkArgs& a, int b) {
 __device__ __forceinline__ int ticket_read(const ChunkArgs& a, uint32_t v, int nreal) {
     const int t = (int)__builtin_amdgcn_readfirstlane(v);
     if (t < 0 || t >= nreal) {
-        if (threadIdx.x == 0) set_status(a.status, TPL_A2B_STATUS_SYNC);
+        if (threadIdx.x == 0) report_bits(a.rep, TPL_A2B_STATUS_SYNC);
         return -1;
     }
     return t;
@@ -745,7 +747,7 @@ constexpr int kSpinLimit = 1 << 20;
 constexpr int kMaxNap = 32;
 template <int N>
 __device__ __forceinline__ bool wait_record(const uint64_t* p, bool valid, double (&v)[N],
-                                            uint32_t* status) {
+                                            const Report& rep) {
     bool ok = !valid;
     int nap = 1;
     for (int spins = 0; spins < kSpinLimit; ++spins) {
@@ -760,7 +762,7 @@ __device__ __forceinline__ bool wait_record(const uint64_t* p, bool valid, doubl
         for (int z = 0; z < nap; ++z) __builtin_amdgcn_s_sleep(1);
         nap = nap < kMaxNap ? 2 * nap : kMaxNap;
     }
-    if (threadIdx.x == 0) set_status(status, TPL_A2B_STATUS_TIMEOUT);
+    if (threadIdx.x == 0) report_bits(rep, TPL_A2B_STATUS_TIMEOUT);
     return false;
 }
 
@@ -791,7 +793,7 @@ __device__ void fwd_lookback(const ChunkArgs& a, int b, int c, double P[kF]) {
     const int lo = c & ~63;
     if (lo > 0) {  // the previous group's inclusive prefix, read by lane 0
         double I[kF] = {};
-        if (!wait_record<kF>(pay + (size_t)(lo - 1) * kFwdPay, lane == 0, I, a.status)) return;
+        if (!wait_record<kF>(pay + (size_t)(lo - 1) * kFwdPay, lane == 0, I, a.rep)) return;
 #pragma unroll
         for (int e = 0; e < kF; ++e) P[e] = read_lane(I[e], 0);
     }
@@ -799,7 +801,7 @@ __device__ void fwd_lookback(const ChunkArgs& a, int b, int c, double P[kF]) {
     const int j = lo + lane;
     const bool valid = j < c;
     double v[kF] = {};
-    if (!wait_record<kF>(pay + (size_t)(valid ? j : lo) * kFwdPay, valid, v, a.status)) return;
+    if (!wait_record<kF>(pay + (size_t)(valid ? j : lo) * kFwdPay, valid, v, a.rep)) return;
     if (!valid) {
 #pragma unroll
         for (int e = 0; e < kF; ++e) v[e] = ident(e);
@@ -823,14 +825,14 @@ __device__ void bwd_lookback(const ChunkArgs& a, int b, int c, int nreal, double
     const int j = c + 1 + lane;  // lane k reads chunk c + 1 + k
     const bool valid = j < hi;
     double v[6] = {};  // zero in unused lanes
-    if (!wait_record<6>(pay + (size_t)(valid ? j : c) * kBwdPay, valid, v, a.status)) return;
+    if (!wait_record<6>(pay + (size_t)(valid ? j : c) * kBwdPay, valid, v, a.rep)) return;
     if (hi - c - 1 > 1) wave_scan_sum<6>(v);  // lane 63: the window's sum
     const int src = hi - c - 1 > 1 ? 63 : 0;   // a window of one chunk: lane 0
 #pragma unroll
     for (int e = 0; e < 6; ++e) carry[e] = read_lane(v[e], src);
     if (hi < nreal) {  // the next group's inclusive suffix, read by lane 0
         double in[6] = {};
-        if (!wait_record<6>(pay + (size_t)hi * kBwdPay, lane == 0, in, a.status)) return;
+        if (!wait_record<6>(pay + (size_t)hi * kBwdPay, lane == 0, in, a.rep)) return;
 #pragma unroll
         for (int e = 0; e < 6; ++e) carry[e] += read_lane(in[e], 0);
     }
@@ -860,7 +862,7 @@ __device__ __forceinline__ void fwd_slot(const ChunkArgs& a, const Slot& sl, T* 
     T* s_l = s_x + threadIdx.x * E9;
     const int lane = threadIdx.x;
     const int L = a.L, b = sl.b, n = sl.n, nreal = sl.nreal, s = sl.r;
-    if (sl.bad && s == 0 && lane == 0) set_status(a.status, TPL_A2B_STATUS_LENGTH);
+    if (sl.bad && s == 0 && lane == 0) report_bits(a.rep, TPL_A2B_STATUS_LENGTH);
     T* xrow = static_cast<T*>(a.coords) + (size_t)b * 9 * L;
     if (!sl.real) {  // past the chain: the first such slot writes all its zeros
         if (s == nreal) {
@@ -966,7 +968,7 @@ __device__ __forceinline__ void fwd_slot(const ChunkArgs& a, const Slot& sl, T* 
                 chk += (float)o;
             }
         }
-        if (!__builtin_isfinite(chk)) set_status(a.status, TPL_A2B_STATUS_NAN);
+        if (!__builtin_isfinite(chk)) report_bits(a.rep, TPL_A2B_STATUS_NAN);
     }
     const uint32_t done_old = nreal > 1 ? chain_done_issue(a, b) : 0u;
     wave_lds_sync();
@@ -1015,7 +1017,7 @@ __global__ void __launch_bounds__(64 * W) a2b_fwd_chain(ChunkArgs a) {
     const int nreal = (n + C - 1) / C;
     const int c = (wave + b) % W;  // this wave's chunk slot
     const bool real = c < nreal;
-    if (raw != n && threadIdx.x == 0) set_status(a.status, TPL_A2B_STATUS_LENGTH);
+    if (raw != n && threadIdx.x == 0) report_bits(a.rep, TPL_A2B_STATUS_LENGTH);
     for (int i = (int)threadIdx.x; i < 128; i += 64 * W) s_tab[i] = kTabCS[i];
     T* s_x = reinterpret_cast<T*>(s_dyn) + (size_t)wave * 9 * C;
     T* s_l = s_x + lane * E9;
@@ -1106,7 +1108,7 @@ __global__ void __launch_bounds__(64 * W) a2b_fwd_chain(ChunkArgs a) {
                 chk += (float)o;
             }
         }
-        if (!__builtin_isfinite(chk)) set_status(a.status, TPL_A2B_STATUS_NAN);
+        if (!__builtin_isfinite(chk)) report_bits(a.rep, TPL_A2B_STATUS_NAN);
     }
     wave_lds_sync();
     const int g0 = 9 * r0;
@@ -1145,7 +1147,7 @@ __device__ __forceinline__ void bwd_slot(const ChunkArgs& a, const Slot& sl, dou
     constexpr int C = 64 * R;
     const int lane = threadIdx.x;
     const int L = a.L, b = sl.b, n = sl.n, nreal = sl.nreal, s = sl.r;
-    if (sl.bad && s == 0 && lane == 0) set_status(a.status, TPL_A2B_STATUS_LENGTH);
+    if (sl.bad && s == 0 && lane == 0) report_bits(a.rep, TPL_A2B_STATUS_LENGTH);
     T* grow = static_cast<T*>(a.grad_angles) + (size_t)b * 3 * L;
     if (!sl.real) {  // past the chain: the first such slot writes all its zeros
         if (s == nreal) {
@@ -1348,7 +1350,7 @@ __device__ __forceinline__ void bwd_slot(const ChunkArgs& a, const Slot& sl, dou
             for (int q = 0; q < R; ++q) bad |= (out[k][q] != out[k][q]);
             lane_store<T, R>(grow + (size_t)k * L + rl, crow, out[k]);
         }
-        if (bad) set_status(a.status, TPL_A2B_STATUS_NAN);
+        if (bad) report_bits(a.rep, TPL_A2B_STATUS_NAN);
     } else {
         const int crow = min(max(L - rl, 0), R);
         if (crow > 0) {
@@ -1390,7 +1392,7 @@ __global__ void __launch_bounds__(64 * W) a2b_bwd_chain(ChunkArgs a) {
     const int nreal = (n + C - 1) / C;
     const int c = (wave + b) % W;  // this wave's chunk slot
     const bool real = c < nreal;
-    if (raw != n && threadIdx.x == 0) set_status(a.status, TPL_A2B_STATUS_LENGTH);
+    if (raw != n && threadIdx.x == 0) report_bits(a.rep, TPL_A2B_STATUS_LENGTH);
     for (int i = (int)threadIdx.x; i < 128; i += 64 * W) s_tab[i] = kTabCS[i];
     double* s_cs = s_dynd + (size_t)wave * 6 * R * 64;
     T* grow = static_cast<T*>(a.grad_angles) + (size_t)b * 3 * L;
@@ -1546,7 +1548,7 @@ __global__ void __launch_bounds__(64 * W) a2b_bwd_chain(ChunkArgs a) {
             for (int q = 0; q < R; ++q) bad |= (out[k][q] != out[k][q]);
             lane_store<T, R>(grow + (size_t)k * L + rl, crow, out[k]);
         }
-        if (bad) set_status(a.status, TPL_A2B_STATUS_NAN);
+        if (bad) report_bits(a.rep, TPL_A2B_STATUS_NAN);
     } else {
         const int crow = min(max(L - rl, 0), R);
         if (crow > 0) {
@@ -1942,6 +1944,64 @@ int launch_chain(KernelFn k, const ChunkArgs& a, size_t lds, hipStream_t stream)
     return hipGetLastError() == hipSuccess ? TPL_A2B_OK : TPL_A2B_ERR_LAUNCH;
 }
 
+// The two directions, reporting as `rep` says.
+int forward_on(int dtype, const void* angles, void* coords, const int32_t* lengths,
+                    void* state, void* sync, const Report& rep, int batch, int angles_stride,
+                    const tpl_a2b_config* cfg, tpl_stream_t stream) {
+    int rc = check_common(dtype, batch, angles_stride);
+    if (rc) return rc;
+    if (!valid_config(cfg) || !fits_dtype(dtype, cfg)) return TPL_A2B_ERR_CONFIG;
+    if (batch == 0 || angles_stride == 0) return TPL_A2B_OK;
+    if (!angles || !coords || !lengths || !sync) return TPL_A2B_ERR_ARG;
+    if (misaligned(state) || misaligned(sync)) return TPL_A2B_ERR_ARG;
+    const int R = cfg->fwd_res_per_lane;
+    ChunkArgs a = base_args(batch, angles_stride, 64 * R, cfg);
+    a.angles = angles;
+    a.coords = coords;
+    a.lengths = lengths;
+    a.rep = rep;
+    a.ckpt = static_cast<double*>(state);
+    bind_sync(a, sync, sync_layout(batch, angles_stride, cfg).fwd);
+    const bool f32 = dtype == TPL_A2B_F32;
+    const size_t lds = (size_t)9 * 64 * R * (f32 ? 4 : 8);
+    if (a.nc <= kChainMax) {
+        const KernelFn kc = f32 ? fwd_chain_kernel<float>(R, a.nc) : fwd_chain_kernel<double>(R, a.nc);
+        if (chain_fits(kc, a, lds)) return launch_chain(kc, a, lds, static_cast<hipStream_t>(stream));
+    }
+    return launch(f32 ? fwd_kernel<float>(R) : fwd_kernel<double>(R), a, lds,
+                  static_cast<hipStream_t>(stream));
+}
+
+int backward_on(int dtype, void* grad_angles, const void* grad_coords, const void* angles,
+                     const int32_t* lengths, const void* state, void* sync, const Report& rep,
+                     int batch, int angles_stride, const tpl_a2b_config* cfg,
+                     tpl_stream_t stream) {
+    int rc = check_common(dtype, batch, angles_stride);
+    if (rc) return rc;
+    if (!valid_config(cfg) || !fits_dtype(dtype, cfg)) return TPL_A2B_ERR_CONFIG;
+    if (batch == 0 || angles_stride == 0) return TPL_A2B_OK;
+    if (!grad_angles || !grad_coords || !angles || !lengths || !state || !sync)
+        return TPL_A2B_ERR_ARG;
+    if (misaligned(state) || misaligned(sync)) return TPL_A2B_ERR_ARG;
+    const int R = cfg->bwd_res_per_lane;
+    ChunkArgs a = base_args(batch, angles_stride, 64 * R, cfg);
+    a.angles = angles;
+    a.grad = grad_coords;
+    a.grad_angles = grad_angles;
+    a.lengths = lengths;
+    a.rep = rep;
+    a.ckpt = const_cast<double*>(static_cast<const double*>(state));
+    bind_sync(a, sync, sync_layout(batch, angles_stride, cfg).bwd);
+    const bool f32 = dtype == TPL_A2B_F32;
+    const size_t lds = (size_t)6 * R * 64 * sizeof(double);
+    if (a.nc <= kChainMax) {
+        const KernelFn kc = f32 ? bwd_chain_kernel<float>(R, a.nc) : bwd_chain_kernel<double>(R, a.nc);
+        if (chain_fits(kc, a, lds)) return launch_chain(kc, a, lds, static_cast<hipStream_t>(stream));
+    }
+    return launch(f32 ? bwd_kernel<float>(R) : bwd_kernel<double>(R), a, lds,
+                  static_cast<hipStream_t>(stream));
+}
+
 }  // namespace
 
 // =================================================================== C ABI
@@ -2001,58 +2061,30 @@ int tpl_a2b_sync_clear(void* sync, size_t bytes, tpl_stream_t stream) {
 int tpl_a2b_forward(int dtype, const void* angles, void* coords, const int32_t* lengths,
                     void* state, void* sync, uint32_t* status, int batch, int angles_stride,
                     const tpl_a2b_config* cfg, tpl_stream_t stream) {
-    int rc = check_common(dtype, batch, angles_stride);
-    if (rc) return rc;
-    if (!valid_config(cfg) || !fits_dtype(dtype, cfg)) return TPL_A2B_ERR_CONFIG;
-    if (batch == 0 || angles_stride == 0) return TPL_A2B_OK;
-    if (!angles || !coords || !lengths || !sync) return TPL_A2B_ERR_ARG;
-    if (misaligned(state) || misaligned(sync)) return TPL_A2B_ERR_ARG;
-    const int R = cfg->fwd_res_per_lane;
-    ChunkArgs a = base_args(batch, angles_stride, 64 * R, cfg);
-    a.angles = angles;
-    a.coords = coords;
-    a.lengths = lengths;
-    a.status = status;
-    a.ckpt = static_cast<double*>(state);
-    bind_sync(a, sync, sync_layout(batch, angles_stride, cfg).fwd);
-    const bool f32 = dtype == TPL_A2B_F32;
-    const size_t lds = (size_t)9 * 64 * R * (f32 ? 4 : 8);
-    if (a.nc <= kChainMax) {
-        const KernelFn kc = f32 ? fwd_chain_kernel<float>(R, a.nc) : fwd_chain_kernel<double>(R, a.nc);
-        if (chain_fits(kc, a, lds)) return launch_chain(kc, a, lds, static_cast<hipStream_t>(stream));
-    }
-    return launch(f32 ? fwd_kernel<float>(R) : fwd_kernel<double>(R), a, lds,
-                  static_cast<hipStream_t>(stream));
+    return forward_on(dtype, angles, coords, lengths, state, sync, Report{status, nullptr}, batch, angles_stride,
+                      cfg, stream);
 }
 
 int tpl_a2b_backward(int dtype, void* grad_angles, const void* grad_coords, const void* angles,
                      const int32_t* lengths, const void* state, void* sync, uint32_t* status,
                      int batch, int angles_stride, const tpl_a2b_config* cfg,
                      tpl_stream_t stream) {
-    int rc = check_common(dtype, batch, angles_stride);
-    if (rc) return rc;
-    if (!valid_config(cfg) || !fits_dtype(dtype, cfg)) return TPL_A2B_ERR_CONFIG;
-    if (batch == 0 || angles_stride == 0) return TPL_A2B_OK;
-    if (!grad_angles || !grad_coords || !angles || !lengths || !state || !sync)
-        return TPL_A2B_ERR_ARG;
-    if (misaligned(state) || misaligned(sync)) return TPL_A2B_ERR_ARG;
-    const int R = cfg->bwd_res_per_lane;
-    ChunkArgs a = base_args(batch, angles_stride, 64 * R, cfg);
-    a.angles = angles;
-    a.grad = grad_coords;
-    a.grad_angles = grad_angles;
-    a.lengths = lengths;
-    a.status = status;
-    a.ckpt = const_cast<double*>(static_cast<const double*>(state));
-    bind_sync(a, sync, sync_layout(batch, angles_stride, cfg).bwd);
-    const bool f32 = dtype == TPL_A2B_F32;
-    const size_t lds = (size_t)6 * R * 64 * sizeof(double);
-    if (a.nc <= kChainMax) {
-        const KernelFn kc = f32 ? bwd_chain_kernel<float>(R, a.nc) : bwd_chain_kernel<double>(R, a.nc);
-        if (chain_fits(kc, a, lds)) return launch_chain(kc, a, lds, static_cast<hipStream_t>(stream));
-    }
-    return launch(f32 ? bwd_kernel<float>(R) : bwd_kernel<double>(R), a, lds,
-                  static_cast<hipStream_t>(stream));
+    return backward_on(dtype, grad_angles, grad_coords, angles, lengths, state, sync, Report{status, nullptr},
+                       batch, angles_stride, cfg, stream);
+}
+
+int tplx_a2b_forward(int dtype, const void* angles, void* coords, const int32_t* lengths, void* state,
+                     void* sync, uint32_t* flags, int batch, int angles_stride, const tpl_a2b_config* cfg,
+                     tpl_stream_t stream) {
+    return forward_on(dtype, angles, coords, lengths, state, sync, Report{nullptr, flags}, batch, angles_stride,
+                      cfg, stream);
+}
+
+int tplx_a2b_backward(int dtype, void* grad_angles, const void* grad_coords, const void* angles,
+                      const int32_t* lengths, const void* state, void* sync, uint32_t* flags, int batch,
+                      int angles_stride, const tpl_a2b_config* cfg, tpl_stream_t stream) {
+    return backward_on(dtype, grad_angles, grad_coords, angles, lengths, state, sync, Report{nullptr, flags},
+                       batch, angles_stride, cfg, stream);
 }
 
 size_t tpl_a2b_noalloc_max_bytes(void) { return kScratchBytes; }
@@ -2072,7 +2104,7 @@ int tpl_a2b_forward_noalloc(int dtype, const void* angles, void* coords, const i
     a.angles = angles;
     a.coords = coords;
     a.lengths = lengths;
-    a.status = status;
+    a.rep = Report{status, nullptr};
     a.ckpt = nullptr;
     const bool f32 = dtype == TPL_A2B_F32;
     const size_t lds = (size_t)9 * 64 * R * (f32 ? 4 : 8);

@@ -15,6 +15,8 @@
 #include <tuple>
 #include <vector>
 
+#include "a2b_flagged.h"
+#include "host_flags.h"
 #include "tpl_a2b.h"
 #include "tpl_a2b_cpu.h"
 
@@ -162,6 +164,46 @@ void backward(torch::Tensor grad_input, torch::Tensor grad_output, torch::Tensor
                               status_ptr(status, input_angles), B, L, &cfg,
                               stream_of(input_angles)),
              "Angles2BackboneGPU_backward");
+}
+
+// The checked forms: as the two above without a status, and they wait for the
+// work and return its status bits (host_flags.h).
+int64_t forward_checked(torch::Tensor input_angles, torch::Tensor output_coords, torch::Tensor angles_length,
+                        c10::optional<torch::Tensor> state, torch::Tensor sync, std::vector<int64_t> config) {
+    auto [B, L] = check_inputs(input_angles, angles_length);
+    check_out(output_coords, input_angles, {B, 9 * (int64_t)L}, "output_coords");
+    const tpl_a2b_config cfg = to_config(config);
+    const int dt = dtype_code(input_angles);
+    c10::DeviceGuard guard(input_angles.device());
+    void* st = nullptr;
+    if (state.has_value() && state->defined())
+        st = opt_ptr(*state, tpl_a2b_state_bytes(dt, B, L, &cfg), "state", input_angles);
+    void* sy = opt_ptr(sync, tpl_a2b_sync_bytes(dt, B, L, &cfg), "sync", input_angles);
+    hipStream_t s = stream_of(input_angles);
+    return host_flags::run(s, [&, B = B, L = L](uint32_t* flags) {
+        check_rc(tplx_a2b_forward(dt, input_angles.data_ptr(), output_coords.data_ptr(),
+                                  angles_length.data_ptr<int32_t>(), st, sy, flags, B, L, &cfg, s),
+                 "Angles2BackboneGPU_forward");
+    });
+}
+
+int64_t backward_checked(torch::Tensor grad_input, torch::Tensor grad_output, torch::Tensor input_angles,
+                         torch::Tensor angles_length, torch::Tensor state, torch::Tensor sync,
+                         std::vector<int64_t> config) {
+    auto [B, L] = check_inputs(input_angles, angles_length);
+    check_out(grad_input, input_angles, {B, 3, L}, "gradInput");
+    check_out(grad_output, input_angles, {B, 9 * (int64_t)L}, "gradOutput");
+    const tpl_a2b_config cfg = to_config(config);
+    const int dt = dtype_code(input_angles);
+    c10::DeviceGuard guard(input_angles.device());
+    void* st = opt_ptr(state, tpl_a2b_state_bytes(dt, B, L, &cfg), "state", input_angles);
+    void* sy = opt_ptr(sync, tpl_a2b_sync_bytes(dt, B, L, &cfg), "sync", input_angles);
+    hipStream_t s = stream_of(input_angles);
+    return host_flags::run(s, [&, B = B, L = L](uint32_t* flags) {
+        check_rc(tplx_a2b_backward(dt, grad_input.data_ptr(), grad_output.data_ptr(), input_angles.data_ptr(),
+                                   angles_length.data_ptr<int32_t>(), st, sy, flags, B, L, &cfg, s),
+                 "Angles2BackboneGPU_backward");
+    });
 }
 
 void sync_clear(torch::Tensor sync) {
@@ -511,6 +553,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.doc() = "Angles2Backbone for MI355X: tensor glue over the tpl_a2b C ABI";
     m.def("Angles2BackboneGPU_forward", &forward, "Angles2Backbone gpu forward (chunk scan)");
     m.def("Angles2BackboneGPU_backward", &backward, "Angles2Backbone gpu backward (O(L) adjoint)");
+    m.def("Angles2BackboneGPU_forward_checked", &forward_checked, "status bits of the forward, once it has run",
+          pybind11::call_guard<pybind11::gil_scoped_release>());
+    m.def("Angles2BackboneGPU_backward_checked", &backward_checked, "status bits of the backward, once it has run",
+          pybind11::call_guard<pybind11::gil_scoped_release>());
     m.def("Angles2BackboneCPU_forward", &cpu_forward, "Angles2Backbone cpu forward (float64)");
     m.def("Angles2BackboneCPU_backward", &cpu_backward, "Angles2Backbone cpu backward (float64, O(L) adjoint)");
     m.def("Angles2BackboneGPU_forward_plain", &forward_plain, "plain serial forward");

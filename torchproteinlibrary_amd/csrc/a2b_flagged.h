@@ -1,0 +1,15 @@
+// a2b_flagged.h -- the entry points of libtpl_a2b.so that this package's own
+// extension calls: those of include/tpl_a2b.h with `flags` (report.h,
+// host_flags.h; null: no reports) in place of the status word.
+#pragma once
+
+#include "tpl_a2b.h"
+
+extern "C" {
+int tplx_a2b_forward(int dtype, const void* angles, void* coords, const int32_t* lengths, void* state,
+                     void* sync, uint32_t* flags, int batch, int angles_stride, const tpl_a2b_config* cfg,
+                     tpl_stream_t stream);
+int tplx_a2b_backward(int dtype, void* grad_angles, const void* grad_coords, const void* angles,
+                      const int32_t* lengths, const void* state, void* sync, uint32_t* flags, int batch,
+                      int angles_stride, const tpl_a2b_config* cfg, tpl_stream_t stream);
+}

@@ -25,6 +25,8 @@
 
 #include <algorithm>
 
+#include "report.h"
+#include "rmsd_flagged.h"
 #include "rmsd_math.h"
 #include "tpl_rmsd.h"
 
@@ -61,13 +63,9 @@ __device__ __forceinline__ bool aligned16(const void* p) {
     return (reinterpret_cast<uintptr_t>(p) & 15) == 0;
 }
 
-__device__ __forceinline__ void report(uint32_t* status, uint32_t bit) {
-    if (status) __hip_atomic_fetch_or(status, bit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-__device__ __forceinline__ int clamp_count(int n, int A, uint32_t* status, bool report_it) {
+__device__ __forceinline__ int clamp_count(int n, int A, const Report& rep, bool report_it) {
     if (n < 0 || n > A) {
-        if (report_it) report(status, TPL_RMSD_STATUS_COUNT);
+        if (report_it) report_bits(rep, TPL_RMSD_STATUS_COUNT);
         return n < 0 ? 0 : A;
     }
     return n;
@@ -77,7 +75,7 @@ template <typename T>
 __global__ void __launch_bounds__(kThreads) rmsd_fwd(const T* __restrict__ x, const T* __restrict__ y,
                                                      const int32_t* __restrict__ num_atoms,
                                                      T* rmsd_out, T* ut_out, double* state,
-                                                     uint32_t* status, int A) {
+                                                     Report rep, int A) {
     // Moment sums over the workgroup: every thread's 17 partial sums (laid
     // out [moment][thread]), then kParts partial sums per moment, then the
     // totals.  A cross-lane butterfly over 17 doubles measured 5 us per
@@ -88,7 +86,7 @@ __global__ void __launch_bounds__(kThreads) rmsd_fwd(const T* __restrict__ x, co
     __shared__ double s_p[kMoments * kParts];
     __shared__ double s_tot[kMoments];
     const int b = blockIdx.x, tid = threadIdx.x;
-    const int n = clamp_count(num_atoms[b], A, status, tid == 0);
+    const int n = clamp_count(num_atoms[b], A, rep, tid == 0);
     const T* xb = x + (size_t)b * 3 * A;
     const T* yb = y + (size_t)b * 3 * A;
     double x0[3] = {0.0, 0.0, 0.0}, y0[3] = {0.0, 0.0, 0.0};
@@ -193,7 +191,7 @@ __global__ void __launch_bounds__(kThreads) rmsd_fwd(const T* __restrict__ x, co
         for (int k = 0; k < 9; ++k) s[6 + k] = U[k];
         s[15] = rmsd;
     }
-    if (rmsd != rmsd) report(status, TPL_RMSD_STATUS_NAN);
+    if (rmsd != rmsd) report_bits(rep, TPL_RMSD_STATUS_NAN);
 }
 
 // One thread per atom slot; the grid covers nblk blocks per structure.
@@ -203,11 +201,11 @@ __global__ void __launch_bounds__(kBwdThreads) rmsd_bwd(T* gx, const T* __restri
                                                         const T* __restrict__ y,
                                                         const int32_t* __restrict__ num_atoms,
                                                         const double* __restrict__ state,
-                                                        uint32_t* status, int A, int nblk) {
+                                                        Report rep, int A, int nblk) {
     const int b = blockIdx.x / nblk;
     const int i = (blockIdx.x - b * nblk) * kBwdThreads + threadIdx.x;
     if (i >= A) return;
-    const int n = clamp_count(num_atoms[b], A, status, false);
+    const int n = clamp_count(num_atoms[b], A, rep, false);
     T* g = gx + (size_t)b * 3 * A + 3 * (size_t)i;
     if (i >= n) {
         g[0] = (T)0;
@@ -233,7 +231,7 @@ __global__ void __launch_bounds__(kBwdThreads) rmsd_bwd(T* gx, const T* __restri
         bad |= (v != v);
         g[c] = v;
     }
-    if (bad) report(status, TPL_RMSD_STATUS_NAN);
+    if (bad) report_bits(rep, TPL_RMSD_STATUS_NAN);
 }
 
 size_t align256(size_t v) { return (v + 255) & ~size_t(255); }
@@ -243,6 +241,56 @@ int check(int dtype, int B, int A) {
     if (B < 0 || A < 0) return TPL_RMSD_ERR_ARG;
     if ((int64_t)3 * A > INT32_MAX || (int64_t)9 * B > INT32_MAX) return TPL_RMSD_ERR_SIZE;
     return TPL_RMSD_OK;
+}
+
+// The two directions, reporting as `rep` says.
+int forward_on(int dtype, const void* input, const void* target, const int32_t* num_atoms,
+                     void* rmsd, void* ut, void* state, const Report& rep, int batch,
+                     int atoms_stride, tpl_rmsd_stream_t stream) {
+    const int rc = check(dtype, batch, atoms_stride);
+    if (rc != TPL_RMSD_OK) return rc;
+    if (batch == 0) return TPL_RMSD_OK;
+    if (!num_atoms || !rmsd || !ut || (atoms_stride > 0 && (!input || !target)))
+        return TPL_RMSD_ERR_ARG;
+    if (state && (reinterpret_cast<uintptr_t>(state) & 255)) return TPL_RMSD_ERR_ARG;
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    if (dtype == TPL_RMSD_F32)
+        hipLaunchKernelGGL(rmsd_fwd<float>, dim3(batch), dim3(kThreads), 0, s,
+                           static_cast<const float*>(input), static_cast<const float*>(target),
+                           num_atoms, static_cast<float*>(rmsd), static_cast<float*>(ut),
+                           static_cast<double*>(state), rep, atoms_stride);
+    else
+        hipLaunchKernelGGL(rmsd_fwd<double>, dim3(batch), dim3(kThreads), 0, s,
+                           static_cast<const double*>(input), static_cast<const double*>(target),
+                           num_atoms, static_cast<double*>(rmsd), static_cast<double*>(ut),
+                           static_cast<double*>(state), rep, atoms_stride);
+    return hipGetLastError() == hipSuccess ? TPL_RMSD_OK : TPL_RMSD_ERR_LAUNCH;
+}
+
+int backward_on(int dtype, void* grad_input, const void* grad_rmsd, const void* input,
+                      const void* target, const int32_t* num_atoms, const void* state,
+                      const Report& rep, int batch, int atoms_stride, tpl_rmsd_stream_t stream) {
+    const int rc = check(dtype, batch, atoms_stride);
+    if (rc != TPL_RMSD_OK) return rc;
+    if (batch == 0 || atoms_stride == 0) return TPL_RMSD_OK;
+    if (!grad_input || !grad_rmsd || !input || !target || !num_atoms || !state)
+        return TPL_RMSD_ERR_ARG;
+    if (reinterpret_cast<uintptr_t>(state) & 255) return TPL_RMSD_ERR_ARG;
+    const int nblk = (atoms_stride + kBwdThreads - 1) / kBwdThreads;
+    if ((int64_t)nblk * batch > INT32_MAX) return TPL_RMSD_ERR_SIZE;
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    const dim3 grid(nblk * batch);
+    if (dtype == TPL_RMSD_F32)
+        hipLaunchKernelGGL(rmsd_bwd<float>, grid, dim3(kBwdThreads), 0, s,
+                           static_cast<float*>(grad_input), static_cast<const float*>(grad_rmsd),
+                           static_cast<const float*>(input), static_cast<const float*>(target),
+                           num_atoms, static_cast<const double*>(state), rep, atoms_stride, nblk);
+    else
+        hipLaunchKernelGGL(rmsd_bwd<double>, grid, dim3(kBwdThreads), 0, s,
+                           static_cast<double*>(grad_input), static_cast<const double*>(grad_rmsd),
+                           static_cast<const double*>(input), static_cast<const double*>(target),
+                           num_atoms, static_cast<const double*>(state), rep, atoms_stride, nblk);
+    return hipGetLastError() == hipSuccess ? TPL_RMSD_OK : TPL_RMSD_ERR_LAUNCH;
 }
 
 }  // namespace
@@ -266,50 +314,29 @@ size_t tpl_rmsd_state_bytes(int batch) {
 int tpl_rmsd_forward(int dtype, const void* input, const void* target, const int32_t* num_atoms,
                      void* rmsd, void* ut, void* state, uint32_t* status, int batch,
                      int atoms_stride, tpl_rmsd_stream_t stream) {
-    const int rc = check(dtype, batch, atoms_stride);
-    if (rc != TPL_RMSD_OK) return rc;
-    if (batch == 0) return TPL_RMSD_OK;
-    if (!num_atoms || !rmsd || !ut || (atoms_stride > 0 && (!input || !target)))
-        return TPL_RMSD_ERR_ARG;
-    if (state && (reinterpret_cast<uintptr_t>(state) & 255)) return TPL_RMSD_ERR_ARG;
-    hipStream_t s = static_cast<hipStream_t>(stream);
-    if (dtype == TPL_RMSD_F32)
-        hipLaunchKernelGGL(rmsd_fwd<float>, dim3(batch), dim3(kThreads), 0, s,
-                           static_cast<const float*>(input), static_cast<const float*>(target),
-                           num_atoms, static_cast<float*>(rmsd), static_cast<float*>(ut),
-                           static_cast<double*>(state), status, atoms_stride);
-    else
-        hipLaunchKernelGGL(rmsd_fwd<double>, dim3(batch), dim3(kThreads), 0, s,
-                           static_cast<const double*>(input), static_cast<const double*>(target),
-                           num_atoms, static_cast<double*>(rmsd), static_cast<double*>(ut),
-                           static_cast<double*>(state), status, atoms_stride);
-    return hipGetLastError() == hipSuccess ? TPL_RMSD_OK : TPL_RMSD_ERR_LAUNCH;
+    return forward_on(dtype, input, target, num_atoms, rmsd, ut, state, Report{status, nullptr}, batch,
+                      atoms_stride, stream);
 }
 
 int tpl_rmsd_backward(int dtype, void* grad_input, const void* grad_rmsd, const void* input,
                       const void* target, const int32_t* num_atoms, const void* state,
                       uint32_t* status, int batch, int atoms_stride, tpl_rmsd_stream_t stream) {
-    const int rc = check(dtype, batch, atoms_stride);
-    if (rc != TPL_RMSD_OK) return rc;
-    if (batch == 0 || atoms_stride == 0) return TPL_RMSD_OK;
-    if (!grad_input || !grad_rmsd || !input || !target || !num_atoms || !state)
-        return TPL_RMSD_ERR_ARG;
-    if (reinterpret_cast<uintptr_t>(state) & 255) return TPL_RMSD_ERR_ARG;
-    const int nblk = (atoms_stride + kBwdThreads - 1) / kBwdThreads;
-    if ((int64_t)nblk * batch > INT32_MAX) return TPL_RMSD_ERR_SIZE;
-    hipStream_t s = static_cast<hipStream_t>(stream);
-    const dim3 grid(nblk * batch);
-    if (dtype == TPL_RMSD_F32)
-        hipLaunchKernelGGL(rmsd_bwd<float>, grid, dim3(kBwdThreads), 0, s,
-                           static_cast<float*>(grad_input), static_cast<const float*>(grad_rmsd),
-                           static_cast<const float*>(input), static_cast<const float*>(target),
-                           num_atoms, static_cast<const double*>(state), status, atoms_stride, nblk);
-    else
-        hipLaunchKernelGGL(rmsd_bwd<double>, grid, dim3(kBwdThreads), 0, s,
-                           static_cast<double*>(grad_input), static_cast<const double*>(grad_rmsd),
-                           static_cast<const double*>(input), static_cast<const double*>(target),
-                           num_atoms, static_cast<const double*>(state), status, atoms_stride, nblk);
-    return hipGetLastError() == hipSuccess ? TPL_RMSD_OK : TPL_RMSD_ERR_LAUNCH;
+    return backward_on(dtype, grad_input, grad_rmsd, input, target, num_atoms, state, Report{status, nullptr},
+                       batch, atoms_stride, stream);
+}
+
+int tplx_rmsd_forward(int dtype, const void* input, const void* target, const int32_t* num_atoms, void* rmsd,
+                      void* ut, void* state, uint32_t* flags, int batch, int atoms_stride,
+                      tpl_rmsd_stream_t stream) {
+    return forward_on(dtype, input, target, num_atoms, rmsd, ut, state, Report{nullptr, flags}, batch,
+                      atoms_stride, stream);
+}
+
+int tplx_rmsd_backward(int dtype, void* grad_input, const void* grad_rmsd, const void* input, const void* target,
+                       const int32_t* num_atoms, const void* state, uint32_t* flags, int batch, int atoms_stride,
+                       tpl_rmsd_stream_t stream) {
+    return backward_on(dtype, grad_input, grad_rmsd, input, target, num_atoms, state, Report{nullptr, flags},
+                       batch, atoms_stride, stream);
 }
 
 }  // extern "C"

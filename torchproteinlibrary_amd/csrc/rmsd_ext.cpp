@@ -12,6 +12,8 @@
 #include <tuple>
 #include <vector>
 
+#include "host_flags.h"
+#include "rmsd_flagged.h"
 #include "tpl_rmsd.h"
 
 namespace {
@@ -114,6 +116,40 @@ void backward(torch::Tensor grad_input, torch::Tensor grad_rmsd, torch::Tensor i
              "Coords2RMSDGPU_backward");
 }
 
+// The checked forms: as the two above without a status, and they wait for the
+// work and return its status bits (host_flags.h).
+int64_t forward_checked(torch::Tensor input, torch::Tensor target, torch::Tensor output,
+                        torch::Tensor num_atoms, torch::Tensor UT, c10::optional<torch::Tensor> state) {
+    auto [B, A] = check_inputs(input, target, num_atoms);
+    check_like(output, input, {B}, "output");
+    check_like(UT, input, {B, 3, 3}, "UT");
+    c10::DeviceGuard guard(input.device());
+    void* st = (state.has_value() && state->defined()) ? state_ptr(*state, B, input) : nullptr;
+    hipStream_t s = stream_of(input);
+    return host_flags::run(s, [&, B = B, A = A](uint32_t* flags) {
+        check_rc(tplx_rmsd_forward(dtype_code(input), input.data_ptr(), target.data_ptr(),
+                                   num_atoms.data_ptr<int32_t>(), output.data_ptr(), UT.data_ptr(), st, flags, B,
+                                   A, s),
+                 "Coords2RMSDGPU_forward");
+    });
+}
+
+int64_t backward_checked(torch::Tensor grad_input, torch::Tensor grad_rmsd, torch::Tensor input,
+                         torch::Tensor target, torch::Tensor num_atoms, torch::Tensor state) {
+    auto [B, A] = check_inputs(input, target, num_atoms);
+    check_like(grad_input, input, {B, 3 * (int64_t)A}, "gradInput");
+    check_like(grad_rmsd, input, {B}, "gradRMSD");
+    c10::DeviceGuard guard(input.device());
+    const void* st = state_ptr(state, B, input);
+    hipStream_t s = stream_of(input);
+    return host_flags::run(s, [&, B = B, A = A](uint32_t* flags) {
+        check_rc(tplx_rmsd_backward(dtype_code(input), grad_input.data_ptr(), grad_rmsd.data_ptr(),
+                                    input.data_ptr(), target.data_ptr(), num_atoms.data_ptr<int32_t>(), st, flags,
+                                    B, A, s),
+                 "Coords2RMSDGPU_backward");
+    });
+}
+
 // Timing loop for bench.py: sets of [input, target, num_atoms, rmsd, UT,
 // state, grad_rmsd, grad_input], rotated per step.  Returns HIP-event ms for
 // `steps` back-to-back forward+backward steps, and the average ms of one
@@ -186,6 +222,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.doc() = "Coords2RMSD for MI355X: tensor glue over the tpl_rmsd C ABI";
     m.def("Coords2RMSDGPU_forward", &forward, "Coords2RMSD forward on GPU (centring, moments, eigenproblem)");
     m.def("Coords2RMSDGPU_backward", &backward, "Coords2RMSD backward on GPU");
+    m.def("Coords2RMSDGPU_forward_checked", &forward_checked, "status bits of the forward, once it has run",
+          pybind11::call_guard<pybind11::gil_scoped_release>());
+    m.def("Coords2RMSDGPU_backward_checked", &backward_checked, "status bits of the backward, once it has run",
+          pybind11::call_guard<pybind11::gil_scoped_release>());
     m.def("state_bytes", &state_bytes, "forward->backward state bytes for a batch");
     m.def("bench", &bench, "time fwd+bwd steps and each kernel alone (event ms)");
 }
