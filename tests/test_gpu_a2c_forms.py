@@ -1,0 +1,156 @@
+"""The forms of the Angles2Coords kernels agree: one workgroup per structure,
+and the group kernels with a workspace, over the sizes where their blocks (64
+residues), groups (256), rounds and staging end, for odd strides, empty and
+flagged structures and scheduling orders."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import a2c_oracle as O
+from torchproteinlibrary_amd import _build
+from torchproteinlibrary_amd.FullAtomModel.Angles2Coords import convertStringList
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda:0")
+FUSED, GROUPS = 1, 2
+
+
+def _lib():
+    lib = ctypes.CDLL(_build.lib_path("libtpl_a2c.so"))
+    lib.tplx_a2c_workspace_bytes.restype = ctypes.c_size_t
+    return lib
+
+
+def _batch(lengths, L, seed, dtype, letters=O.AA20):
+    rng = np.random.default_rng(seed)
+    seqs = ["".join(rng.choice(list(letters), size=n)) for n in lengths]
+    ang = np.zeros((len(lengths), 8, L))
+    for b, n in enumerate(lengths):
+        ang[b, 0, :n] = rng.normal(-1.1, 0.3, n)
+        ang[b, 1, :n] = rng.normal(2.3, 0.4, n)
+        ang[b, 2, :n] = np.pi + rng.normal(0, 0.05, n)
+        ang[b, 3:, :n] = rng.uniform(-np.pi, np.pi, (5, n))
+    return seqs, torch.tensor(ang, dtype=dtype, device=DEV)
+
+
+def _p(t):
+    return None if t is None else ctypes.c_void_p(t.data_ptr())
+
+
+def _forward(form, seqs, X, A, order=None, offset=0):
+    """(coords, res_names, atom_names, status) of one form; outputs start full
+    of other values, `offset` values into their buffers."""
+    lib, B, L = _lib(), X.shape[0], X.shape[2]
+    S = convertStringList(seqs).to(DEV)
+    buf = torch.full((B * 3 * A + offset,), 7.0, dtype=X.dtype, device=DEV)
+    coords = buf[offset:].view(B, 3 * A)
+    rn = torch.full((B, A, 4), 255, dtype=torch.uint8, device=DEV)
+    an = torch.full((B, A, 4), 255, dtype=torch.uint8, device=DEV)
+    st = torch.zeros(1, dtype=torch.int32, device=DEV)
+    ws = torch.empty(max(lib.tplx_a2c_workspace_bytes(B, L), 1), dtype=torch.uint8, device=DEV)
+    torch.cuda.synchronize()
+    assert lib.tplx_a2c_forward(form, _p(order), 0 if X.dtype == torch.float32 else 1, _p(S), S.shape[1], _p(X), L,
+                                _p(coords), _p(rn), _p(an), A, _p(ws), _p(st), None, B, None) == 0
+    torch.cuda.synchronize()
+    assert offset == 0 or bool((buf[:offset] == 7.0).all())
+    return coords, rn, an, int(st.item())
+
+
+def _tolerance(X, scale):
+    """Two products of up to 3L rotations in float64 (8 roundings each), and
+    one rounding to float32."""
+    return scale * (3 * X.shape[2] * 8 * 2.0 ** -53 + (2.0 ** -23 if X.dtype == torch.float32 else 0.0))
+
+
+SHAPES = [([1, 64, 65, 63], 65), ([65, 128, 127, 0, 3], 129), ([255, 256, 257, 64, 1], 257),
+          ([513, 512, 30, 300], 515), ([1024, 1025, 1, 700], 1025), ([2100, 64, 1500], 2100), ([70] * 2050, 71)]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("shape", range(len(SHAPES)))
+def test_forward_forms_agree(shape, dtype):
+    lengths, L = SHAPES[shape]
+    seqs, X = _batch(lengths, L, 100 + shape, dtype)
+    natoms = [O.num_atoms(s) for s in seqs]
+    A = max(natoms) + (5, 2, 0, 3, 1, 4, 7)[shape]
+    print(f"a2c forward forms: {len(lengths)} structures, stride {L}, {dtype}", flush=True)
+    outs = [_forward(f, seqs, X, A, offset=shape % 3) for f in (FUSED, GROUPS)]
+    assert outs[0][3] == outs[1][3] == 0
+    scale = float(outs[0][0].abs().max())
+    assert float((outs[0][0] - outs[1][0]).abs().max()) <= _tolerance(X, scale)
+    for k in (1, 2):
+        assert torch.equal(outs[0][k], outs[1][k])
+    for c, rn, an, _ in outs:
+        for b in range(0, len(lengths), max(1, len(lengths) // 8)):
+            n = natoms[b]
+            assert not c[b, 3 * n:].any() and not rn[b, n:].any() and not an[b, n:].any()
+            res, atoms = O.names_one(seqs[b])
+            assert [bytes(v).rstrip(b"\0").decode() for v in an[b, :n].cpu().numpy()] == atoms
+            assert [bytes(v).rstrip(b"\0").decode() for v in rn[b, :n].cpu().numpy()] == res
+    b = int(np.argmin([abs(n - 300) for n in lengths]))  # the oracle on one structure
+    want = O.forward_one(seqs[b], X[b].double().cpu().numpy())[0]
+    for c, *_ in outs:
+        assert np.abs(c[b, :3 * natoms[b]].double().cpu().numpy() - want).max() <= _tolerance(X, scale)
+
+
+@pytest.mark.parametrize("letters", ["W", "G", "P"])
+def test_forward_forms_at_the_largest_and_smallest_residues(letters):
+    seqs, X = _batch([64, 130, 300, 1], 300, 7, torch.float32, letters)
+    A = max(O.num_atoms(s) for s in seqs)
+    a, b = _forward(FUSED, seqs, X, A), _forward(GROUPS, seqs, X, A)
+    assert float((a[0] - b[0]).abs().max()) <= _tolerance(X, float(a[0].abs().max()))
+    assert torch.equal(a[1], b[1]) and torch.equal(a[2], b[2])
+    one = _batch([64, 64, 3, 20, 33], 64, 8, torch.float64, letters)  # one block per structure
+    n = [O.num_atoms(s) for s in one[0]]
+    c = _forward(FUSED, one[0], one[1], max(n))[0]
+    for k in range(5):
+        want = O.forward_one(one[0][k], one[1][k].cpu().numpy())[0]
+        assert np.abs(c[k, :3 * n[k]].cpu().numpy() - want).max() <= 1e-10
+
+
+@pytest.mark.parametrize("L", [40, 200, 700])
+def test_forward_forms_flag_alike(L):
+    """A bad letter (in the last block), too many residues, too many atoms: the
+    structure is zeros, its bit is set, the others are built."""
+    good = "ACDEFGHIKLMNPQRSTVWY" * (L // 20)
+    A = O.num_atoms(good)
+    for bad, bit in ((good[:-1] + "X", 1), (good + "G", 2), ("W" * L, 4)):
+        seqs = [good, bad, "G" * L, good[:30]]
+        _, X = _batch([L] * 4, L, 3, torch.float32)
+        outs = [_forward(f, seqs, X, A) for f in (FUSED, GROUPS)]
+        for c, rn, an, st in outs:
+            assert st == bit
+            assert not c[1].any() and not rn[1].any() and not an[1].any()
+            assert c[0].any() and c[2].any() and c[3].any()
+        assert float((outs[0][0] - outs[1][0]).abs().max()) <= _tolerance(X, float(outs[0][0].abs().max()))
+
+
+def test_forward_forms_take_an_order():
+    seqs, X = _batch([300, 20, 500, 64, 257], 500, 11, torch.float32)
+    A = max(O.num_atoms(s) for s in seqs)
+    for form in (FUSED, GROUPS):
+        plain = _forward(form, seqs, X, A)
+        turned = _forward(form, seqs, X, A, torch.tensor([2, 0, 4, 3, 1], dtype=torch.int32, device=DEV))
+        for k in range(3):
+            assert torch.equal(plain[k], turned[k])
+        c, rn, an, st = _forward(form, seqs, X, A, torch.tensor([2, 0, 5, 3, 1], dtype=torch.int32, device=DEV))
+        assert st == 8
+        assert bool((c[4] == 7.0).all()) and bool((rn[4] == 255).all())  # displaced: unwritten
+        assert torch.equal(c[:4], plain[0][:4])
+
+
+@pytest.mark.parametrize("lengths,L", [([21], 21), ([300, 40], 300), ([600] * 300, 600)])
+def test_layer_raises_where_the_coordinate_sum_is_nan(lengths, L):
+    from torchproteinlibrary_amd.FullAtomModel import Angles2Coords
+    seqs, X = _batch(lengths, L, 5, torch.float32)
+    Angles2Coords()(X, seqs)
+    for value in (float("nan"), float("inf")):
+        Y = X.clone()
+        Y[-1, 0, lengths[-1] // 2] = value
+        with pytest.raises(Exception, match="forward Nan"):
+            Angles2Coords()(Y, seqs)
+    Y = X.clone()
+    Y[0, 7, :] = 1e9  # large, finite: no error
+    Angles2Coords()(Y, seqs)

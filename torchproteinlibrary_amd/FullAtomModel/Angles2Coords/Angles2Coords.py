@@ -41,7 +41,7 @@ from ..._native_xform import ext
 
 __all__ = ["Angles2Coords", "Angles2CoordsFunction", "convertStringList", "convertString"]
 
-_STATUS_SEQ, _STATUS_LENGTH, _STATUS_ATOMS, _STATUS_ORDER = 1, 2, 4, 8
+_STATUS_SEQ, _STATUS_LENGTH, _STATUS_ATOMS, _STATUS_ORDER, _STATUS_RANGE = 1, 2, 4, 8, 16
 _LETTERS = set("ACDEFGHIKLMNPQRSTVWY")
 
 
@@ -79,19 +79,19 @@ def _checks_enabled() -> bool:
     return os.environ.get("TPL_A2B_CHECKS", "1") != "0" and not torch.cuda.is_current_stream_capturing()
 
 
-def _check(out, status, where):
-    if status is not None:
-        s = int(status.item())
-        if s & _STATUS_SEQ:
-            raise ValueError("Angles2CoordsFunction: a sequence holds a letter outside the 20 amino acids")
-        if s & _STATUS_LENGTH:
-            raise ValueError("Angles2CoordsFunction: a sequence is longer than input_angles.size(2)")
-        if s & _STATUS_ATOMS:
-            raise ValueError("Angles2CoordsFunction: a structure has more atoms than the output holds")
-        if s & _STATUS_ORDER:
-            raise RuntimeError("Angles2CoordsFunction: the scheduling order holds an index outside the batch")
-        if math.isnan(out.sum()):
-            raise Exception(f"Angles2CoordsFunction: {where} Nan")
+def _check(s, out, where):
+    """Raises on the status bits of a checked call.  The kernels flag outputs
+    that are NaN, infinite or huge (1e26); only then is the output summed."""
+    if s & _STATUS_SEQ:
+        raise ValueError("Angles2CoordsFunction: a sequence holds a letter outside the 20 amino acids")
+    if s & _STATUS_LENGTH:
+        raise ValueError("Angles2CoordsFunction: a sequence is longer than input_angles.size(2)")
+    if s & _STATUS_ATOMS:
+        raise ValueError("Angles2CoordsFunction: a structure has more atoms than the output holds")
+    if s & _STATUS_ORDER:
+        raise RuntimeError("Angles2CoordsFunction: the scheduling order holds an index outside the batch")
+    if s & _STATUS_RANGE and math.isnan(out.sum()):
+        raise Exception(f"Angles2CoordsFunction: {where} Nan")
 
 
 class Angles2CoordsFunction(Function):
@@ -119,11 +119,13 @@ class Angles2CoordsFunction(Function):
         coords = torch.empty(B, 3 * max_atoms, dtype=input_angles.dtype, device=dev)
         res_names = torch.empty(B, max_atoms, 4, dtype=torch.uint8, device=dev)
         atom_names = torch.empty(B, max_atoms, 4, dtype=torch.uint8, device=dev)
-        status = torch.zeros(1, dtype=torch.int32, device=dev) if _checks_enabled() else None
         if order is not None:
             order = order.to(dev).contiguous()
-        ext.Angles2Coords_forward(seqs, input_angles, coords, res_names, atom_names, status, order)
-        _check(coords, status, "forward")
+        if _checks_enabled():
+            _check(ext.Angles2Coords_forward_checked(seqs, input_angles, coords, res_names, atom_names, order),
+                   coords, "forward")
+        else:
+            ext.Angles2Coords_forward(seqs, input_angles, coords, res_names, atom_names, None, order)
         ctx.save_for_backward(seqs, coords)
         ctx.order = order
         ctx.mark_non_differentiable(res_names, atom_names, num_atoms)
@@ -137,7 +139,8 @@ class Angles2CoordsFunction(Function):
         grad_angles = torch.empty(ctx.angles_shape, dtype=coords.dtype, device=coords.device)
         status = torch.zeros(1, dtype=torch.int32, device=coords.device) if _checks_enabled() else None
         ext.Angles2Coords_backward_coords(grad_atoms, grad_angles, seqs, coords, status, ctx.order)
-        _check(grad_angles, status, "backward")
+        if status is not None:
+            _check(int(status.item()) | _STATUS_RANGE, grad_angles, "backward")
         return grad_angles, None, None, None
 
 

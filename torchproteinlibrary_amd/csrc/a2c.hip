@@ -5,15 +5,16 @@
 // on the CPU and walks it recursively (Layers/FullAtomModel/cConformation.cpp:
 // 29-158); its backward visits, for every angle, every atom below it
 // (:160-195), O(atoms x tree depth) with a chain's depth growing with its
-// length.  Here one workgroup takes one structure:
+// length.  Here one wave takes 64 consecutive residues of a structure, one per
+// lane:
 //
-//   1. each thread takes a contiguous run of residues and multiplies their
-//      residue steps S_i = T_CA(phi_i) T_C(psi_i) T_N(omega_i) (FP64 3x4), the
-//      transform from residue i's N frame to residue i+1's;
-//   2. a workgroup scan of those products (DPP within each wave, the waves'
-//      totals through LDS) gives each thread the N frame of its first
-//      residue, and a scan of the atom counts gives its first atom;
-//   3. each thread walks its residues: N, CA, the side chain, C, writing atoms.
+//   1. each lane multiplies out its residue's step S_i = T_CA(phi_i) T_C(psi_i)
+//      T_N(omega_i) (FP64 3x4), the transform from residue i's N frame to
+//      residue i+1's;
+//   2. a wave scan of those products (DPP), folded with the products of the
+//      blocks before, gives each residue its N frame, and a scan of the atom
+//      counts its first atom;
+//   3. each lane walks its residue: N, CA, the side chain, C, writing atoms.
 //
 // The backward uses dL/dalpha = u . (sum_{x in subtree} x cross g
 // - p cross sum_{x in subtree} g) for a node with x axis u and origin p (the
@@ -32,7 +33,9 @@
 #include <mutex>
 #include <vector>
 
+#include "a2c_flagged.h"
 #include "a2c_table.h"
+#include "report.h"
 #include "sincos_tab.h"
 #include "tpl_a2c.h"
 
@@ -40,25 +43,30 @@ namespace {
 
 using namespace a2c;
 
-// Workgroup sizes: 256 threads, or 512 for long structures (see use_large_fwd
-// and use_large_bwd), where a thread then walks half as many residues.  LDS:
-// forward 13.6 / 14.0 KB (the tables), run backward 0.8 / 1.0 KB.
+// Workgroup sizes of the run backward: 256 threads, or 512 for long structures
+// (see use_large_bwd), where a thread then walks half as many residues.
 constexpr int kThreadsSmall = 256, kThreadsLarge = 512;
 
 __constant__ Residue kRes[kTypes] = A2C_RESIDUES;
 __constant__ Side kSide[kTypes][kMaxSide] = A2C_SIDES;
 __constant__ Atom kAtom[kTypes][kMaxAtoms] = A2C_ATOMS;
 
-// Workgroup-shared tables, filled once per workgroup from the constant ones:
-// local atom positions, and per side-chain node cos/sin of beta and of a
-// constant alpha, d, and the packed (row, first atom, count).
-struct Tables {
+// Workgroup-shared tables.  StepTables: what the residue steps and the atom
+// counts need.  Tables: also local atom positions, per side-chain node cos/sin
+// of beta and of a constant alpha, d, and the packed (row, first atom, count),
+// and the names as words.
+struct alignas(16) StepTables {
+    double tab[128];       // the sincos table of sincos_tab.h
+    double bb[3][2];       // cos/sin of beta for the CA, C and N transforms
+    int res_i[kTypes];     // natoms | nca << 8 | nside << 16
+    uint8_t type[256];     // residue type of a letter, 0xff: none
+    uint8_t atoms[256];    // its atoms, 0: none
+};
+struct alignas(16) Tables : StepTables {
     double loc[kTypes * kMaxAtoms][3];
     double side[kTypes * kMaxSide][5];
     int side_i[kTypes * kMaxSide];
-    int res_i[kTypes];  // natoms | nca << 8 | nside << 16
-    double bb[3][2];    // cos/sin of beta for the CA, C and N transforms
-    double tab[128];    // the sincos table of sincos_tab.h
+    uint2 name[kTypes * kMaxAtoms];  // the residue's, the atom's
 };
 
 // The table sincos (sincos_tab.h) over the workgroup's LDS copy of its table.
@@ -88,6 +96,14 @@ __device__ void fill_tables(Tables& tb) {
         tb.side[k][4] = s.d;
         tb.side_i[k] = (s.row & 0xff) | (s.first << 8) | (s.count << 16);
     }
+    for (int k = threadIdx.x; k < kTypes * kMaxAtoms; k += NT)
+        tb.name[k] = make_uint2(*reinterpret_cast<const uint32_t*>(kRes[k / kMaxAtoms].name3),
+                                *reinterpret_cast<const uint32_t*>(kAtom[k / kMaxAtoms][k % kMaxAtoms].name));
+    for (int k = threadIdx.x; k < 256; k += NT) {
+        const int t = residue_type((uint8_t)k);
+        tb.type[k] = (uint8_t)t;
+        tb.atoms[k] = t < 0 ? (uint8_t)0 : (uint8_t)kRes[t].natoms;
+    }
     if (threadIdx.x < kTypes) {
         const Residue r = kRes[threadIdx.x];
         tb.res_i[threadIdx.x] = r.natoms | (r.nca << 8) | (r.nside << 16);
@@ -113,11 +129,11 @@ __global__ void __launch_bounds__(256) a2c_init_tables() {
     for (int k = threadIdx.x; k < (int)(sizeof(Tables) / 8); k += 256) dst[k] = src[k];
 }
 
-template <int NT>
-__device__ __forceinline__ void copy_tables(Tables& tb) {
-    const double* src = reinterpret_cast<const double*>(&g_tab);
-    double* dst = reinterpret_cast<double*>(&tb);
-    for (int k = threadIdx.x; k < (int)(sizeof(Tables) / 8); k += NT) dst[k] = src[k];
+template <typename TB>
+__device__ __forceinline__ void copy_tables(TB& tb, int nt) {
+    const uint4* src = reinterpret_cast<const uint4*>(&static_cast<const TB&>(g_tab));
+    uint4* dst = reinterpret_cast<uint4*>(&tb);
+    for (int k = threadIdx.x; k < (int)(sizeof(TB) / 16); k += nt) dst[k] = src[k];
 }
 
 // m (3x4, row-major) <- m * Ry(beta) Tx(d) Rx(alpha), with cb/sb of beta and
@@ -255,23 +271,6 @@ __device__ __forceinline__ void find_length(const uint8_t* seq, int seq_stride, 
     }
 }
 
-template <typename T>
-__device__ __forceinline__ double angle(const T* ang, int row, int stride, int i) {
-    return (double)ang[(size_t)row * stride + i];
-}
-
-// The 8 angles of residue i, loaded together at the top of the residue so
-// that their latencies overlap (one global-load latency per residue walk
-// instead of one per transform).
-template <typename T>
-struct ResAngles {
-    T v[8];
-    __device__ __forceinline__ void load(const T* ang, int stride, int i) {
-#pragma unroll
-        for (int r = 0; r < 8; ++r) v[r] = ang[(size_t)r * stride + i];
-    }
-};
-
 // The side-chain angles xi1..xi5 of a residue in the order its side-chain
 // nodes bind them: every template binds rows 3, 4, ... consecutively (the
 // table test checks this), so each bound node takes the next one.  Shifting
@@ -279,9 +278,9 @@ struct ResAngles {
 template <typename T>
 struct SideRows {
     T v[5];
-    __device__ __forceinline__ explicit SideRows(const ResAngles<T>& a) {
+    __device__ __forceinline__ explicit SideRows(const T (&a)[8]) {
 #pragma unroll
-        for (int k = 0; k < 5; ++k) v[k] = a.v[3 + k];
+        for (int k = 0; k < 5; ++k) v[k] = a[3 + k];
     }
     __device__ __forceinline__ double pop() {
         const T x = v[0];
@@ -290,21 +289,6 @@ struct SideRows {
         return (double)x;
     }
 };
-
-// The residue step S_i applied to m: m <- m T_CA(phi) T_C(psi) T_N(omega).
-template <typename T>
-__device__ __forceinline__ void residue_step(double m[12], const Tables& tb, const T* ang, int stride,
-                                             int i) {
-    const double phi = angle(ang, 0, stride, i), psi = angle(ang, 1, stride, i),
-                 omega = angle(ang, 2, stride, i);
-    double s, c;
-    sincos_tab(phi, tb.tab, &s, &c);
-    step(m, tb.bb[0][0], tb.bb[0][1], c, s, geo::R_N_CA);
-    sincos_tab(psi, tb.tab, &s, &c);
-    step(m, tb.bb[1][0], tb.bb[1][1], c, s, geo::R_CA_C);
-    sincos_tab(omega, tb.tab, &s, &c);
-    step(m, tb.bb[2][0], tb.bb[2][1], c, s, geo::R_C_N);
-}
 
 // The structure this workgroup builds: order[blockIdx.x], or blockIdx.x
 // without an order.  An index outside the batch is reported
@@ -318,196 +302,763 @@ __device__ __forceinline__ int structure_of(const int* order, uint32_t* status) 
     return -1;
 }
 
-// Per structure: the sequence length (first 0 byte), the residues' validity,
-// this thread's run [r0, r1), and the workgroup scans giving the N frame of
-// residue r0 (frame) and its first atom (atom0).  Returns false (for every
-// thread of the workgroup) if the structure is flagged.
+// A thread's run of residues [r0, r1) of a structure of L, its first atom and
+// the structure's atoms.
 struct Run {
     int L, r0, r1, atom0, total;
 };
 
-template <int NT, typename T>
-__device__ bool prepare(const uint8_t* seq, int seq_stride, const T* ang, int ang_stride,
-                        int atoms_stride, uint32_t* status, const Tables& tb, double (*s_m)[NT / 64],
-                        int* s_c, int* s_flag, Run& run, double frame[12], ResAngles<T>& av0,
-                        uint8_t& code0) {
-    const int tid = threadIdx.x;
-    if (tid == 0) {
-        s_flag[0] = seq_stride;  // length
-        s_flag[1] = 0;           // status bits
-    }
-    __syncthreads();
-    find_length<NT>(seq, seq_stride, &s_flag[0]);
-    __syncthreads();
-    int L = s_flag[0];
-    if (L > ang_stride) {
-        if (tid == 0) atomicOr(&s_flag[1], (int)TPL_A2C_STATUS_LENGTH);
-        L = 0;
-    }
-    const int chunk = (L + NT - 1) / NT;
-    const int r0 = min(L, tid * chunk), r1 = min(L, r0 + chunk);
-    // The walk's first residue: its angles and letter are loaded now, so
-    // that they arrive while the workgroup scans.
-    if (r0 < r1) {
-        av0.load(ang, ang_stride, r0);
-        code0 = seq[r0];
-    }
-    double P[12];
-    identity(P);
-    int cnt = 0;
-    bool bad = false;
-    for (int i = r0; i < r1; ++i) {
-        const int t = residue_type(seq[i]);
-        if (t < 0) {
-            bad = true;
-            continue;
-        }
-        cnt += tb.res_i[t] & 0xff;
-        residue_step(P, tb, ang, ang_stride, i);
-    }
-    if (bad) atomicOr(&s_flag[1], (int)TPL_A2C_STATUS_SEQ);
-    // Ordered product of the runs' steps and sum of their atom counts over
-    // the workgroup: inclusive within each wave by DPP, then across waves
-    // through LDS (the waves' totals; each wave composes those before it).
-    // frame = product of the earlier runs' steps, atom0 = their atoms.
-    constexpr int NW = NT / 64;
-    const int wv = tid >> 6;
-    int cinc = cnt;
-    if ((tid & ~63) * chunk < L) {  // a wave whose runs are all past the structure holds identities and zeros
-        cinc = wave_scan_int(cnt);
-        wave_scan_frames(P);
-    }
-    if ((tid & 63) == 63) {
-#pragma unroll
-        for (int k = 0; k < 12; ++k) s_m[k][wv] = P[k];
-        s_c[wv] = cinc;
-    }
-    double E[12];
-#pragma unroll
-    for (int k = 0; k < 12; ++k) E[k] = dpp_double<kWaveShr1, 0xf>(P[k], ident12(k));
-    __syncthreads();
-    double W[12];
-    identity(W);
-    int before = 0, total = 0;
-#pragma unroll
-    for (int w = 0; w < NW; ++w) {
-        if (w < wv) {
-            double Tw[12], R2[12];
-#pragma unroll
-            for (int k = 0; k < 12; ++k) Tw[k] = s_m[k][w];
-            compose(W, Tw, R2);
-#pragma unroll
-            for (int k = 0; k < 12; ++k) W[k] = R2[k];
-            before += s_c[w];
-        }
-        total += s_c[w];
-    }
-    compose(W, E, frame);
-    run.atom0 = before + cinc - cnt;
-    run.total = total;
-    if (run.total > atoms_stride && tid == 0) atomicOr(&s_flag[1], (int)TPL_A2C_STATUS_ATOMS);
-    __syncthreads();
-    const int flags = s_flag[1];
-    if (flags && tid == 0 && status) __hip_atomic_fetch_or(status, (uint32_t)flags, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    run.L = L;
-    run.r0 = r0;
-    run.r1 = r1;
-    if (flags) {
-        run.L = run.r0 = run.r1 = run.total = 0;
-        return false;
-    }
-    return true;
+// ---- forward: one wave per block of 64 residues ----
+// A structure is cut into blocks of kBlock consecutive residues; a wave builds
+// one block's atoms, each lane one residue's, so the lanes' angles and letters
+// are consecutive in memory and every wave has the same work, whatever the mix
+// of lengths.  A residue needs its N frame (the product of the residue steps
+// before it) and its first atom:
+//   * a2c_fwd_steps + a2c_fwd_walk: the first kernel multiplies out groups of
+//     256 residues, four per lane, and leaves every residue's frame within its
+//     group, the groups' products and the atom counts in the caller's
+//     workspace; the second puts the groups before in front.  Both wait on
+//     latencies (of memory, LDS and dependent FP64) more than half of their
+//     waves' time; so the first also writes the zeros past the structures
+//     (three quarters of all bytes at mixed lengths), and the frames go through
+//     memory (72 bytes per residue) rather than being multiplied out again;
+//   * a2c_fwd_single where a structure is one block (angles_stride <= 64): the
+//     wave scans its 64 steps;
+//   * a2c_fwd_fused: one workgroup per structure, whose waves' scans meet in
+//     LDS.  It needs no workspace and one launch, and serves calls without a
+//     workspace and small batches.
+// Waves whose residues would lie past the structure write its padding's zeros.
+// Against one workgroup of 256 or 512 threads per structure whose threads
+// walked runs of up to four residues and wrote their atoms and names one by one
+// (names included, us): lengths 30-1000 at B=1024 118 -> 62, in float64
+// 159 -> 93; 256 x 1000 60 -> 38; 32 x 350 18.2 -> 13.6; 1024 x 30 16.1 -> 11.2;
+// one peptide of 21 in float64 12.8 -> 9.0.
+//
+// Workgroups go to the 8 XCDs in turn, those of one XCD to its 32 CUs in turn,
+// and a workgroup's waves to the CU's SIMDs.  What only some structures have
+// (their later groups and blocks) must not always meet the same of these: the
+// grids run over the structures first and their groups second, and the waves
+// of a workgroup take its shares rotated as the workgroups come round to a CU
+// (turned_wave).  With the groups of a structure side by side the XCDs of the
+// even workgroups had the first groups: 1024 structures of lengths 30-1000 took
+// 55 us in the walk, against 38.
+constexpr int kBlock = 64;                   // residues per wave of the walk: one per lane
+constexpr int kQuad = 4;                     // residues per lane of the steps
+constexpr int kGroup = kBlock * kQuad;       // residues per wave of the steps
+constexpr int kGroupWaves = kGroup / kBlock; // blocks per group; waves per workgroup of the steps
+
+// The share of wave `wave` of W in workgroup `wg`.
+__device__ __forceinline__ int turned_wave(int wave, int W, int wg) {
+    return (int)((uint32_t)(wave + (wg >> 3) + (wg >> 8)) % (uint32_t)W);
 }
 
-// At 256 threads the forward is held to four waves per SIMD (<= 128 VGPRs,
-// a few dwords spilled) so that four workgroups fit on a CU, as LDS allows:
-// 85 -> 71 us at mixed lengths 30-1000, B=1024, against three workgroups.
-template <int NT, typename T>
-__global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT == 256 ? 4 : 1, 8))) a2c_fwd(const uint8_t* __restrict__ seqs, int seq_stride,
-                                                    const T* __restrict__ angles, int ang_stride,
-                                                    T* __restrict__ coords, uint32_t* __restrict__ res_names,
-                                                    uint32_t* __restrict__ atom_names, int atoms_stride,
-                                                    uint32_t* status, const int* __restrict__ order) {
+// A group's products and counts.
+struct alignas(16) GroupRec {
+    double f[12];             // the product of its residue steps
+    int before[kGroupWaves];  // the structure's atoms before each of its blocks
+};
+// The frames of a group's residues within it: their x and y axes and origins
+// (z = x cross y).  Component k of residue 4q + e is at v[k][64e + q], so that
+// the steps' stores and the walk's loads are of consecutive doubles.
+struct alignas(16) GroupFrames {
+    double v[9][kGroup];
+};
+
+// The structure of slot b of the batch: order[b], or b without an order; -1
+// for an entry outside the batch, which is reported (TPL_A2C_STATUS_ORDER)
+// and builds nothing.
+__device__ __forceinline__ int structure_at(const int* order, int b, int batch, const Report& rep) {
+    if (!order) return b;
+    const int o = __builtin_amdgcn_readfirstlane(order[b]);
+    if (o >= 0 && o < batch) return o;
+    report_bits(rep, TPL_A2C_STATUS_ORDER);
+    return -1;
+}
+
+// A sequence row read by one wave, 16 loads of 64 consecutive bytes at a time;
+// the first 1024 bytes are loaded by load(), so that the caller can do other
+// work before it needs them.
+struct RowScan {
+    static constexpr int kAtOnce = 16;
+    uint8_t c[kAtOnce];
+
+    __device__ __forceinline__ void load(const uint8_t* seq, int stride, int lane, int base = 0) {
+#pragma unroll
+        for (int e = 0; e < kAtOnce; ++e) {
+            const int i = base + 64 * e + lane;
+            c[e] = i < stride ? seq[i] : (uint8_t)0;
+        }
+    }
+    // The row's length: its first 0 byte, or its stride.  With `atoms`, also
+    // the atoms of its letters, those before residue `upto`, and whether one
+    // of them is not a residue's.
+    template <bool ATOMS>
+    __device__ __forceinline__ int finish(const uint8_t* seq, int stride, int lane, const StepTables* tb, int upto,
+                                          int& atoms, int& before, bool& bad) {
+        int n = -1, cnt = 0, bef = 0;
+        bool odd = false;
+        for (int base = 0; n < 0; base += 64 * kAtOnce) {
+            if (base > 0) load(seq, stride, lane, base);
+#pragma unroll
+            for (int e = 0; e < kAtOnce; ++e) {
+                if (n >= 0) continue;
+                const uint64_t zero = __builtin_amdgcn_ballot_w64(c[e] == 0);
+                const int i = base + 64 * e + lane;
+                if (zero) n = base + 64 * e + (int)__builtin_ctzll(zero);
+                if (ATOMS && (n < 0 || i < n)) {
+                    const int k = tb->atoms[c[e]];
+                    odd |= k == 0;
+                    cnt += k;
+                    if (i < upto) bef += k;
+                }
+            }
+        }
+        if (ATOMS) {
+            atoms = __builtin_amdgcn_readlane(wave_scan_int(cnt), 63);
+            before = __builtin_amdgcn_readlane(wave_scan_int(bef), 63);
+            bad = __builtin_amdgcn_ballot_w64(odd) != 0;
+        }
+        return n;
+    }
+};
+
+__device__ __forceinline__ int wave_length(const uint8_t* seq, int stride, int lane) {
+    RowScan row;
+    row.load(seq, stride, lane);
+    int atoms, before;
+    bool bad;
+    return row.finish<false>(seq, stride, lane, nullptr, 0, atoms, before, bad);
+}
+
+// Cosines and sines of a residue's phi and psi, for its steps and its walk.
+struct Turns {
+    double c[2], s[2];
+};
+
+// m <- the step of a residue with the angles phi, psi, omega.
+__device__ __forceinline__ void first_step(double m[12], const StepTables& tb, double phi, double psi, double omega,
+                                           Turns& tu) {
+    double s, c;
+    sincos_tab(phi, tb.tab, &tu.s[0], &tu.c[0]);
+    sincos_tab(psi, tb.tab, &tu.s[1], &tu.c[1]);
+    sincos_tab(omega, tb.tab, &s, &c);
+    identity(m);
+    step(m, tb.bb[0][0], tb.bb[0][1], tu.c[0], tu.s[0], geo::R_N_CA);
+    step(m, tb.bb[1][0], tb.bb[1][1], tu.c[1], tu.s[1], geo::R_CA_C);
+    step(m, tb.bb[2][0], tb.bb[2][1], c, s, geo::R_C_N);
+}
+
+// The lane's residue i: its letter (0 past the structure's length n) and its
+// angles.
+template <typename T>
+__device__ __forceinline__ uint8_t lane_residue(const uint8_t* seq, int n, const T* ang, int stride, int i,
+                                                T (&av)[8]) {
+    uint8_t code = 0;
+#pragma unroll
+    for (int r = 0; r < 8; ++r) av[r] = (T)0;
+    if (i < n) {
+        code = seq[i];
+#pragma unroll
+        for (int r = 0; r < 8; ++r) av[r] = ang[(size_t)r * stride + i];
+    }
+    return code;
+}
+
+// The type of a letter (-1: none), and its residue's step (the identity for
+// -1).
+template <typename T>
+__device__ __forceinline__ int lane_step(uint8_t code, const StepTables& tb, const T (&av)[8], double m[12],
+                                         Turns& tu) {
+    const int t = (int)(int8_t)tb.type[code];
+    if (t >= 0)
+        first_step(m, tb, (double)av[0], (double)av[1], (double)av[2], tu);
+    else
+        identity(m);
+    return t;
+}
+
+// P <- P * the products of `count` records, in order (wave-uniform).
+template <typename R>
+__device__ __forceinline__ void fold(double P[12], const R* rec, int count) {
+    for (int k = 0; k < count; ++k) {
+        double A[12], Q[12];
+#pragma unroll
+        for (int e = 0; e < 12; ++e) A[e] = rec[k].f[e];
+        compose(P, A, Q);
+#pragma unroll
+        for (int e = 0; e < 12; ++e) P[e] = Q[e];
+    }
+}
+
+// An angle that may give coordinates that are NaN, infinite or huge: bounded
+// angles give rotations, and positions within 14 A per residue.
+template <typename T>
+__device__ __forceinline__ bool wild(T a) {
+    return !(a < (T)1e8 && a > (T)-1e8);
+}
+
+// The atoms of the lane's residue of type t with N frame F, at atom `at` of
+// out (wave-uniform).  A group's first atom is its frame's origin.  C and O come
+// before the side chain, so that one frame is live in its loop.  The side
+// chain's first node is fixed and has no atoms and no length: a turn about x.
+template <typename T>
+__device__ __forceinline__ void walk_residue(const Tables& tb, int t, const T (&av)[8], const Turns& tu, double F[12],
+                                             T* out, uint32_t at) {
+    const int ri = tb.res_i[t];
+    const int natoms = ri & 0xff, nca = (ri >> 8) & 0xff, nside = ri >> 16;
+    const double* loc = tb.loc[t * kMaxAtoms];
+    const uint32_t bytes = (uint32_t)(3 * sizeof(T));
+    const uint32_t o = bytes * at;  // byte offsets within a block fit 32 bits
+    auto origin = [&](int slot, const double m[12]) {
+        T* q = reinterpret_cast<T*>(reinterpret_cast<char*>(out) + (o + bytes * (uint32_t)slot));
+        q[0] = (T)m[3];
+        q[1] = (T)m[7];
+        q[2] = (T)m[11];
+    };
+    auto put = [&](int slot, const double m[12]) {
+        double x[3];
+        apply(m, loc + 3 * slot, x);
+        T* q = reinterpret_cast<T*>(reinterpret_cast<char*>(out) + (o + bytes * (uint32_t)slot));
+        q[0] = (T)x[0];
+        q[1] = (T)x[1];
+        q[2] = (T)x[2];
+    };
+    origin(0, F);
+    step(F, tb.bb[0][0], tb.bb[0][1], tu.c[0], tu.s[0], geo::R_N_CA);  // F: CA
+    origin(1, F);
+    {
+        double C[12];
+#pragma unroll
+        for (int k = 0; k < 12; ++k) C[k] = F[k];
+        step(C, tb.bb[1][0], tb.bb[1][1], tu.c[1], tu.s[1], geo::R_CA_C);
+        origin(natoms - 2, C);
+        put(natoms - 1, C);
+    }
+    for (int k = 2; k <= nca; ++k) put(k, F);
+    {
+        const double c = tb.side[t * kMaxSide][2], s = tb.side[t * kMaxSide][3];
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            const double y = F[4 * i + 1], z = F[4 * i + 2];
+            F[4 * i + 1] = y * c + z * s;
+            F[4 * i + 2] = z * c - y * s;
+        }
+    }
+    SideRows<T> rows(av);
+    for (int n = 1; n < nside; ++n) {
+        const int q = t * kMaxSide + n;
+        const int si = tb.side_i[q];
+        const int row = (int)(int8_t)(si & 0xff), first = (si >> 8) & 0xff, count = si >> 16;
+        double c = tb.side[q][2], s = tb.side[q][3];
+        if (row >= 0) sincos_tab(rows.pop(), tb.tab, &s, &c);
+        step(F, tb.side[q][0], tb.side[q][1], c, s, tb.side[q][4]);
+        origin(first, F);
+        for (int k = first + 1; k < first + count; ++k) put(k, F);
+    }
+}
+
+// Wave-scope LDS ordering (the wave's writes before its reads).
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// The names of a block's `count` atoms at rn, an: each lane notes its
+// residue's (type, slot) per atom in the wave's LDS, and the wave writes the
+// words of 64 consecutive atoms at a time.  (A lane writing its own residue's
+// names, each from a dependent table load, took as long as the coordinates.)
+__device__ __forceinline__ void write_names(const Tables& tb, int t, int natoms, int at, int count, uint32_t* rn,
+                                            uint32_t* an, uint16_t* s_role, int lane) {
+    for (int s = 0; s < natoms; ++s) s_role[at + s] = (uint16_t)(t * kMaxAtoms + s);
+    wave_lds_sync();
+    for (int k = lane; k < count; k += 64) {
+        const uint2 names = tb.name[s_role[k]];
+        rn[(uint32_t)k] = names.x;
+        an[(uint32_t)k] = names.y;
+    }
+}
+
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+
+// The walk's coordinates go through the wave's LDS: a lane writing its own
+// residue's atoms to memory makes every store instruction touch 64 lines.  A
+// block's atoms are staged at most kStage at a time (64 residues have 525 on
+// average, 896 at most; at 576 two workgroups of a2c_fwd_walk fit on a CU).
+constexpr int kStage = 576;
+template <typename T>
+constexpr int stage_values() {
+    return 3 * kStage + 16 / (int)sizeof(T);
+}
+
+// Values [0, count) from the wave's LDS to dst, as 16-byte stores where dst is
+// aligned; s_w[0] holds the value of dst rounded down to 16 bytes, so that both
+// sides are aligned together.
+template <typename T>
+__device__ __forceinline__ void flush_stage(T* dst, int count, const T* s_w, int lane) {
+    constexpr int V = 16 / (int)sizeof(T);
+    const int mis = (int)((reinterpret_cast<uintptr_t>(dst) & 15) / sizeof(T));
+    T* d0 = dst - mis;
+    const int end = mis + count, first = mis ? V : 0, last = end / V * V;
+    if (mis && lane >= mis && lane < V && lane < end) d0[lane] = s_w[lane];
+    for (int k = first + V * lane; k < last; k += V * 64)
+        *reinterpret_cast<uint4*>(d0 + k) = *reinterpret_cast<const uint4*>(s_w + k);
+    const int tail = last > first ? last : first;
+    if (tail + lane < end) d0[tail + lane] = s_w[tail + lane];
+}
+
+// Share f of F of the zeros over words [0, count) of p, by one wave: the waves
+// take 1 KB pieces (16-byte streaming stores, whole 128-byte lines) in turn, so
+// that they write one stretch of memory together; share 0 also takes the words
+// before the first whole line and after the last 16 bytes.
+__device__ __forceinline__ void zero_words(uint32_t* p, int64_t count, int f, int F, int lane) {
+    if (count <= 0) return;
+    const int mis = (int)((128 - (reinterpret_cast<uintptr_t>(p) & 127)) & 127) / 4;
+    const int head = (int)(mis < count ? mis : count);
+    const int64_t nvec = (count - head) / 4, tail = head + 4 * nvec;
+    const u32x4 z = {0u, 0u, 0u, 0u};
+    u32x4* q = reinterpret_cast<u32x4*>(p + head);
+    for (int64_t v = 64 * f + lane; v < nvec; v += 64 * F) __builtin_nontemporal_store(z, q + v);
+    if (f == 0) {
+        if (lane < head) p[lane] = 0u;
+        if (tail + lane < count) p[tail + lane] = 0u;
+    }
+}
+
+// Share f of F of the zeros past a structure's `total` atoms, by one wave.
+template <typename T>
+__device__ __forceinline__ void zero_share(T* out, uint32_t* rn, uint32_t* an, int total, int atoms_stride, int f,
+                                           int F, int lane) {
+    const int64_t rest = atoms_stride - total;
+    constexpr int W = (int)(sizeof(T) / 4);
+    zero_words(reinterpret_cast<uint32_t*>(out + 3 * (size_t)total), 3 * W * rest, f, F, lane);
+    if (rn) {
+        zero_words(rn + total, rest, f, F, lane);
+        zero_words(an + total, rest, f, F, lane);
+    }
+}
+
+// The frames within each group, its product and its atom counts, one wave per
+// (structure, group) and four residues per lane; and the zeros past the
+// structure.  Every wave reads the whole row of letters (one round of loads)
+// and so knows the structure's length, atoms and flags by itself.
+template <typename T>
+__global__ void __launch_bounds__(64 * kGroupWaves) a2c_fwd_steps(
+    const uint8_t* __restrict__ seqs, int seq_stride, const T* __restrict__ angles, int ang_stride,
+    int* __restrict__ lens, GroupRec* __restrict__ rec, GroupFrames* __restrict__ frames, T* __restrict__ coords,
+    uint32_t* __restrict__ res_names, uint32_t* __restrict__ atom_names, int atoms_stride, Report rep,
+    const int* __restrict__ order, int batch, int ng) {
+    __shared__ StepTables tb;
+    const int wave = turned_wave((int)(threadIdx.x >> 6), kGroupWaves, (int)blockIdx.x);
+    const int lane = (int)(threadIdx.x & 63);
+    const int w = (int)blockIdx.x * kGroupWaves + wave;
+    const int g = w / batch, slot = w - g * batch;
+    const int b = g < ng ? structure_at(order, slot, batch, g == 0 ? rep : Report{nullptr, nullptr}) : -1;
+    const uint8_t* seq = seqs + (size_t)(b < 0 ? 0 : b) * seq_stride;
+    const T* ang = angles + (size_t)(b < 0 ? 0 : b) * 8 * ang_stride;
+    // All loads go out before the first wait: the row, and this lane's letters
+    // and angles (zeros where the strides end; unused past the structure).
+    RowScan row;
+    row.load(seq, seq_stride, lane);
+    const int i0 = kGroup * g + kQuad * lane;
+    uint8_t code[kQuad];
+    T a[3][kQuad];
+#pragma unroll
+    for (int e = 0; e < kQuad; ++e) {
+        const bool in = i0 + e < ang_stride;
+        code[e] = in && i0 + e < seq_stride ? seq[i0 + e] : (uint8_t)0;
+#pragma unroll
+        for (int r = 0; r < 3; ++r) a[r][e] = in ? ang[(size_t)r * ang_stride + i0 + e] : (T)0;
+    }
+    copy_tables(tb, 64 * kGroupWaves);
+    __syncthreads();
+    if (b < 0) {
+        if (g == 0 && lane == 0) lens[slot] = 0;
+        return;
+    }
+    int total = 0, before = 0, flags = 0;
+    bool bad = false;
+    int n = row.finish<true>(seq, seq_stride, lane, &tb, kGroup * g, total, before, bad);
+    if (n > ang_stride) {
+        flags = TPL_A2C_STATUS_LENGTH;
+    } else {
+        if (bad) flags |= TPL_A2C_STATUS_SEQ;
+        if (total > atoms_stride) flags |= TPL_A2C_STATUS_ATOMS;
+    }
+    if (flags) {  // a flagged structure is all zeros
+        if (g == 0 && lane == 0) report_bits(rep, (uint32_t)flags);
+        n = total = 0;
+    }
+    T* out = coords + (size_t)b * 3 * atoms_stride;
+    uint32_t* rn = res_names ? res_names + (size_t)b * atoms_stride : nullptr;
+    uint32_t* an = atom_names ? atom_names + (size_t)b * atoms_stride : nullptr;
+    const int here = (n + kGroup - 1) / kGroup;  // groups that hold residues
+    GroupRec* r = rec + (size_t)b * ng + g;
+    if (g == 0 && lane == 0) lens[slot] = n;
+    if (g < here) {
+        double m[12], turn[kQuad - 1][3][2];  // the first residues' (cos, sin), for their frames
+        identity(m);
+        int cnt = 0;
+#pragma unroll
+        for (int e = 0; e < kQuad; ++e) {
+            const bool in = i0 + e < n;
+            cnt += in ? tb.atoms[code[e]] : 0;
+            double v[3][2];
+#pragma unroll
+            for (int r = 0; r < 3; ++r) sincos_tab((double)a[r][e], tb.tab, &v[r][1], &v[r][0]);
+            if (in) {
+                step(m, tb.bb[0][0], tb.bb[0][1], v[0][0], v[0][1], geo::R_N_CA);
+                step(m, tb.bb[1][0], tb.bb[1][1], v[1][0], v[1][1], geo::R_CA_C);
+                step(m, tb.bb[2][0], tb.bb[2][1], v[2][0], v[2][1], geo::R_C_N);
+            }
+            if (e < kQuad - 1) {
+#pragma unroll
+                for (int r = 0; r < 3; ++r) turn[e][r][0] = v[r][0], turn[e][r][1] = v[r][1];
+            }
+        }
+        const int cinc = wave_scan_int(cnt);
+        wave_scan_frames(m);
+        if ((lane & 15) == 0) r->before[lane >> 4] = before + cinc - cnt;
+        if (lane == 63) {
+#pragma unroll
+            for (int k = 0; k < 12; ++k) r->f[k] = m[k];
+        }
+#pragma unroll
+        for (int k = 0; k < 12; ++k) m[k] = dpp_double<kWaveShr1, 0xf>(m[k], ident12(k));
+        GroupFrames* gf = frames + ((size_t)b * ng + g);
+#pragma unroll
+        for (int e = 0; e < kQuad; ++e) {
+            if (i0 + e < n) {
+#pragma unroll
+                for (int i = 0; i < 3; ++i) {
+                    gf->v[i][64 * e + lane] = m[4 * i];
+                    gf->v[3 + i][64 * e + lane] = m[4 * i + 1];
+                    gf->v[6 + i][64 * e + lane] = m[4 * i + 3];
+                }
+            }
+            if (e < kQuad - 1) {
+                step(m, tb.bb[0][0], tb.bb[0][1], turn[e][0][0], turn[e][0][1], geo::R_N_CA);
+                step(m, tb.bb[1][0], tb.bb[1][1], turn[e][1][0], turn[e][1][1], geo::R_CA_C);
+                step(m, tb.bb[2][0], tb.bb[2][1], turn[e][2][0], turn[e][2][1], geo::R_C_N);
+            }
+        }
+    }
+    // the padding: by the groups past the structure, or by all where none is
+    if (here == ng)
+        zero_share(out, rn, an, total, atoms_stride, g, ng, lane);
+    else if (g >= here)
+        zero_share(out, rn, an, total, atoms_stride, g - here, ng - here, lane);
+}
+
+// The atoms (and names) of a block of `total` atoms, by one wave: the lane's
+// residue has the type t, the N frame F and `cnt` atoms from `at` on; out, rn
+// and an are the block's.
+template <typename T>
+__device__ __forceinline__ void build_block(const Tables& tb, int t, const T (&av)[8], const Turns& tu, double F[12],
+                                            int at, int cnt, int total, T* out, uint32_t* rn, uint32_t* an, T* s_w,
+                                            int lane) {
+    for (int base = 0; base < total;) {  // once, unless the block has more than kStage atoms
+        const uint64_t later = __builtin_amdgcn_ballot_w64(at + cnt > base + kStage);
+        const int end = later ? __builtin_amdgcn_readlane(at, (int)__builtin_ctzll(later)) : total;
+        T* dst = out + 3 * (size_t)base;
+        const int mis = (int)((reinterpret_cast<uintptr_t>(dst) & 15) / sizeof(T));
+        if (t >= 0 && at >= base && at < end) walk_residue(tb, t, av, tu, F, s_w + mis, (uint32_t)(at - base));
+        wave_lds_sync();
+        flush_stage(dst, 3 * (end - base), s_w, lane);
+        wave_lds_sync();
+        base = end;
+    }
+    if (rn) {
+        write_names(tb, t, cnt, at, total, rn, an, reinterpret_cast<uint16_t*>(s_w), lane);
+        wave_lds_sync();
+    }
+}
+
+// Whether an angle may give coordinates out of range.
+template <typename T>
+__device__ __forceinline__ bool any_wild(const T (&av)[8]) {
+    bool suspect = false;
+#pragma unroll
+    for (int r = 0; r < 8; ++r) suspect |= wild(av[r]);
+    return suspect;
+}
+
+// The atoms of structures of one block (ang_stride <= kBlock), one wave each.
+template <typename T>
+__global__ void __launch_bounds__(64 * kGroupWaves) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 3 : 2, 8)))
+a2c_fwd_single(const uint8_t* __restrict__ seqs, int seq_stride, const T* __restrict__ angles, int ang_stride,
+               T* __restrict__ coords, uint32_t* __restrict__ res_names, uint32_t* __restrict__ atom_names,
+               int atoms_stride, Report rep, const int* __restrict__ order, int batch) {
     __shared__ Tables tb;
-    __shared__ double s_m[12][NT / 64];  // the waves' products
-    __shared__ int s_c[NT / 64];          // the waves' atom counts
-    __shared__ int s_flag[2];
-    const int b = structure_of(order, status);
+    __shared__ __align__(16) T s_stage[kGroupWaves][stage_values<T>()];
+    const int wave = (int)(threadIdx.x >> 6), lane = (int)(threadIdx.x & 63);
+    const int slot = (int)blockIdx.x * kGroupWaves + wave;
+    const int b = slot < batch ? structure_at(order, slot, batch, rep) : -1;
+    const uint8_t* seq = seqs + (size_t)(b < 0 ? 0 : b) * seq_stride;
+    int n = b < 0 ? 0 : wave_length(seq, seq_stride, lane), flags = 0;
+    if (n > ang_stride) {
+        flags = TPL_A2C_STATUS_LENGTH;
+        n = 0;
+    }
+    T av[8];
+    const uint8_t code =
+        lane_residue(seq, n, angles + (size_t)(b < 0 ? 0 : b) * 8 * ang_stride, ang_stride, lane, av);
+    copy_tables(tb, 64 * kGroupWaves);
+    __syncthreads();
+    if (b < 0) return;
+    T* out = coords + (size_t)b * 3 * atoms_stride;
+    uint32_t* rn = res_names ? res_names + (size_t)b * atoms_stride : nullptr;
+    uint32_t* an = atom_names ? atom_names + (size_t)b * atoms_stride : nullptr;
+    double m[12];
+    Turns tu;
+    const int t = lane_step(code, tb, av, m, tu);
+    const int cnt = t >= 0 ? tb.res_i[t] & 0xff : 0;
+    const int cinc = wave_scan_int(cnt);
+    const int total = __builtin_amdgcn_readlane(cinc, 63);
+    if (__builtin_amdgcn_ballot_w64(lane < n && t < 0)) flags |= TPL_A2C_STATUS_SEQ;
+    if (total > atoms_stride) flags |= TPL_A2C_STATUS_ATOMS;
+    if (flags) {  // a flagged structure is all zeros
+        if (lane == 0) report_bits(rep, (uint32_t)flags);
+        zero_share(out, rn, an, 0, atoms_stride, 0, 1, lane);
+        return;
+    }
+    if (any_wild(av)) report_flag(rep, TPLX_A2C_RANGE);
+    wave_scan_frames(m);
+#pragma unroll
+    for (int k = 0; k < 12; ++k) m[k] = dpp_double<kWaveShr1, 0xf>(m[k], ident12(k));
+    build_block(tb, t, av, tu, m, cinc - cnt, cnt, total, out, rn, an, s_stage[wave], lane);
+    zero_share(out, rn, an, total, atoms_stride, 0, 1, lane);
+}
+
+// The atoms after a2c_fwd_steps, which also took care of the flags and the
+// padding.  The waves of a grid that stays resident share the blocks that hold
+// residues: every workgroup sums up the structures' block counts (a segment of
+// the batch at a time), and wave w of W takes blocks w, w + W, ... of that
+// list.  One block per wave in a grid over all blocks left a CU's slots to
+// waves that found their block past the structure and to workgroups with one
+// wave at work, each copying the tables anew: lengths 30-1000 at B=1024 took
+// 38 us, against 31.
+constexpr int kWalkWaves = 8;
+constexpr int kSegment = 2048;  // structures per segment: their block counts' sums live in LDS
+template <typename T>
+__global__ void __launch_bounds__(64 * kWalkWaves) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 4 : 2, 8)))
+a2c_fwd_walk(const uint8_t* __restrict__ seqs, int seq_stride, const T* __restrict__ angles, int ang_stride,
+             const int* __restrict__ lens, const GroupRec* __restrict__ rec, const GroupFrames* __restrict__ frames,
+             T* __restrict__ coords, uint32_t* __restrict__ res_names, uint32_t* __restrict__ atom_names,
+             int atoms_stride, Report rep, const int* __restrict__ order, int batch, int ng) {
+    constexpr int NT = 64 * kWalkWaves, kPer = kSegment / NT;
+    __shared__ Tables tb;
+    __shared__ __align__(16) T s_stage[kWalkWaves][stage_values<T>()];
+    __shared__ int s_first[kSegment + 1];  // blocks before a structure of the segment
+    __shared__ uint8_t s_last[kSegment];   // residues of its last block, less one
+    __shared__ int s_sum[kWalkWaves];
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = (int)(threadIdx.x & 63);
+    const int step = (int)gridDim.x * kWalkWaves;
+    bool suspect = false;
+    for (int base = 0; base < batch; base += kSegment) {
+        const int m = batch - base < kSegment ? batch - base : kSegment;
+        int nb[kPer], sum = 0, last[kPer];
+#pragma unroll
+        for (int e = 0; e < kPer; ++e) {
+            const int k = kPer * (int)threadIdx.x + e;
+            last[e] = k < m ? lens[base + k] : 0;
+        }
+        if (base == 0) copy_tables(tb, NT);
+#pragma unroll
+        for (int e = 0; e < kPer; ++e) {
+            nb[e] = (last[e] + kBlock - 1) / kBlock;
+            last[e] = (last[e] - 1) & (kBlock - 1);
+            sum += nb[e];
+        }
+        const int inc = wave_scan_int(sum);
+        if (base > 0) __syncthreads();  // the segment before is done
+        if (lane == 63) s_sum[wave] = inc;
+        __syncthreads();
+        int at = inc - sum, items = 0;
+#pragma unroll
+        for (int k = 0; k < kWalkWaves; ++k) {
+            at += k < wave ? s_sum[k] : 0;
+            items += s_sum[k];
+        }
+#pragma unroll
+        for (int e = 0; e < kPer; ++e) {
+            s_first[kPer * (int)threadIdx.x + e] = at;
+            s_last[kPer * (int)threadIdx.x + e] = (uint8_t)last[e];
+            at += nb[e];
+        }
+        if (threadIdx.x == NT - 1) s_first[kSegment] = at;
+        __syncthreads();
+        for (int it = (int)blockIdx.x * kWalkWaves + wave; it < items; it += step) {
+            // the last structure that starts at or before block `it` and has one:
+            // first among every 32nd, then among the 32 (empty ones share the
+            // start of the next, so the last is the one)
+            static_assert(kSegment == 64 * 32, "two rounds of comparisons");
+            const int hi = 32 * (__builtin_popcountll(__builtin_amdgcn_ballot_w64(s_first[32 * lane] <= it)) - 1);
+            const uint64_t le = __builtin_amdgcn_ballot_w64(lane < 32 && s_first[hi + (lane & 31)] <= it);
+            const int k = hi + __builtin_popcountll(le) - 1;
+            const int first = __builtin_amdgcn_readfirstlane(s_first[k]);
+            const int j = it - first;
+            const int bn = kBlock * (__builtin_amdgcn_readfirstlane(s_first[k + 1]) - first - 1) +
+                           __builtin_amdgcn_readfirstlane((int)s_last[k]) + 1;
+            const int b = structure_at(order, base + k, batch, Report{nullptr, nullptr});
+            const int g = j / kGroupWaves, part = j % kGroupWaves;
+            const int i = kBlock * j + lane;
+            const GroupRec* rb = rec + (size_t)b * ng;
+            const GroupFrames* gf = frames + ((size_t)b * ng + g);
+            T av[8];
+            const uint8_t code = lane_residue(seqs + (size_t)b * seq_stride, bn,
+                                              angles + (size_t)b * 8 * ang_stride, ang_stride, i, av);
+            const int before = __builtin_amdgcn_readfirstlane(rb[g].before[part]);
+            double G[12];
+            {
+                const uint32_t r = kBlock * part + lane, at4 = 64 * (r & 3) + (r >> 2);
+#pragma unroll
+                for (int c = 0; c < 3; ++c) {
+                    G[4 * c] = i < bn ? gf->v[c][at4] : 0.0;
+                    G[4 * c + 1] = i < bn ? gf->v[3 + c][at4] : 0.0;
+                    G[4 * c + 3] = i < bn ? gf->v[6 + c][at4] : 0.0;
+                }
+            }
+            const int t = (int)(int8_t)tb.type[code];
+            const int cnt = t >= 0 ? tb.res_i[t] & 0xff : 0;
+            const int cinc = wave_scan_int(cnt);
+            suspect |= any_wild(av);
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {  // z = x cross y
+                const int p = (c + 1) % 3, q = (c + 2) % 3;
+                G[4 * c + 2] = G[4 * p] * G[4 * q + 1] - G[4 * q] * G[4 * p + 1];
+            }
+            for (int h = g - 1; h >= 0; --h) {  // the groups before
+                double M[12];
+#pragma unroll
+                for (int c = 0; c < 12; ++c) M[c] = G[c];
+                compose(rb[h].f, M, G);
+            }
+            Turns tu;
+            sincos_tab((double)av[0], tb.tab, &tu.s[0], &tu.c[0]);
+            sincos_tab((double)av[1], tb.tab, &tu.s[1], &tu.c[1]);
+            const size_t row = (size_t)b * atoms_stride + before;
+            build_block(tb, t, av, tu, G, cinc - cnt, cnt, __builtin_amdgcn_readlane(cinc, 63), coords + 3 * row,
+                        res_names ? res_names + row : nullptr, atom_names ? atom_names + row : nullptr,
+                        s_stage[wave], lane);
+        }
+    }
+    if (suspect) report_flag(rep, TPLX_A2C_RANGE);
+}
+
+// One workgroup per structure, of at most MAXW waves (blockDim / 64, one per
+// block of the stride where that fits): the waves take their blocks together,
+// whose products meet in LDS.  EU: the waves per SIMD it is held to.
+struct BlockRec {
+    double f[12];  // the product of its residue steps
+    int atoms, flags;
+};
+template <int MAXW, int EU, typename T>
+__global__ void __launch_bounds__(64 * MAXW) __attribute__((amdgpu_waves_per_eu(EU, 8))) a2c_fwd_fused(
+    const uint8_t* __restrict__ seqs, int seq_stride, const T* __restrict__ angles, int ang_stride,
+    T* __restrict__ coords, uint32_t* __restrict__ res_names, uint32_t* __restrict__ atom_names, int atoms_stride,
+    Report rep, const int* __restrict__ order, int batch) {
+    __shared__ Tables tb;
+    __shared__ uint16_t s_role[MAXW][kBlock * kMaxAtoms];
+    __shared__ BlockRec s_rec[MAXW];
+    __shared__ int s_sum[2];  // atoms and flags of a structure of more than NW blocks
+    const int NW = (int)(blockDim.x >> 6);
+    const int wave = turned_wave((int)(threadIdx.x >> 6), NW, (int)blockIdx.x), lane = (int)(threadIdx.x & 63);
+    const int b = structure_at(order, (int)blockIdx.x, batch, rep);
     if (b < 0) return;
     const uint8_t* seq = seqs + (size_t)b * seq_stride;
     const T* ang = angles + (size_t)b * 8 * ang_stride;
-    T* out = coords + (size_t)b * 3 * atoms_stride;
-    copy_tables<NT>(tb);
+    copy_tables(tb, 64 * NW);
+    if (threadIdx.x < 2) s_sum[threadIdx.x] = 0;
+    int n = wave_length(seq, seq_stride, lane), flags = 0;  // every wave alike
+    if (n > ang_stride) {
+        flags = TPL_A2C_STATUS_LENGTH;
+        n = 0;
+    }
+    const int nb = (n + kBlock - 1) / kBlock;
     __syncthreads();
-    Run run;
-    double G[12];
-    ResAngles<T> av;
-    uint8_t code = 0;
-    prepare<NT>(seq, seq_stride, ang, ang_stride, atoms_stride, status, tb, s_m, s_c, s_flag, run, G, av, code);
-    int a = run.atom0;
+    int total = 0;
+    if (nb > NW) {  // the whole structure's atoms and flags before its first block is written
+        int cnt = 0;
+        bool bad = false;
+        for (int i = (int)threadIdx.x; i < n; i += 64 * NW) {
+            const int t = (int)(int8_t)tb.type[seq[i]];
+            bad |= t < 0;
+            if (t >= 0) cnt += tb.res_i[t] & 0xff;
+        }
+        atomicAdd(&s_sum[0], cnt);
+        if (bad) atomicOr(&s_sum[1], (int)TPL_A2C_STATUS_SEQ);
+        __syncthreads();
+        total = s_sum[0];
+        flags |= s_sum[1];
+    }
+    T* out = coords + (size_t)b * 3 * atoms_stride;
     uint32_t* rn = res_names ? res_names + (size_t)b * atoms_stride : nullptr;
     uint32_t* an = atom_names ? atom_names + (size_t)b * atoms_stride : nullptr;
-    for (int i = run.r0; i < run.r1; ++i) {
-        // the next residue's angles and letter go out before this one's work
-        ResAngles<T> nav;
-        uint8_t ncode = 0;
-        if (i + 1 < run.r1) {
-            nav.load(ang, ang_stride, i + 1);
-            ncode = seq[i + 1];
-        }
-        const int t = residue_type(code);
-        const int ri = tb.res_i[t];
-        const int natoms = ri & 0xff, nca = (ri >> 8) & 0xff, nside = ri >> 16;
-        const double* loc = tb.loc[t * kMaxAtoms];
-        double x[3];
-        auto put = [&](int slot, const double m[12]) {
-            apply(m, loc + 3 * slot, x);
-            T* o = out + 3 * (size_t)(a + slot);
-            o[0] = (T)x[0];
-            o[1] = (T)x[1];
-            o[2] = (T)x[2];
-        };
-        put(0, G);
-        double s, c, F[12], CA[12];
+    double P[12];
+    identity(P);
+    int before = 0;
+    bool suspect = false;
+    if (total > atoms_stride) flags |= TPL_A2C_STATUS_ATOMS;
+    for (int k0 = 0; k0 < nb && !flags; k0 += NW) {
+        const int j = k0 + wave, i = kBlock * j + lane;
+        T av[8];
+        double m[12];
+        Turns tu;
+        int t = -1, cnt = 0, cinc = 0;
+        if (j < nb) {
+            t = lane_step(lane_residue(seq, n, ang, ang_stride, i, av), tb, av, m, tu);
+            cnt = t >= 0 ? tb.res_i[t] & 0xff : 0;
+            const bool bad = __builtin_amdgcn_ballot_w64(i < n && t < 0) != 0;
+            cinc = wave_scan_int(cnt);
+            wave_scan_frames(m);
+            if (lane == 63) {
 #pragma unroll
-        for (int k = 0; k < 12; ++k) CA[k] = G[k];
-        sincos_tab((double)av.v[0], tb.tab, &s, &c);
-        step(CA, tb.bb[0][0], tb.bb[0][1], c, s, geo::R_N_CA);
-        for (int k = 1; k <= nca; ++k) put(k, CA);
-#pragma unroll
-        for (int k = 0; k < 12; ++k) F[k] = CA[k];
-        SideRows<T> rows(av);
-        for (int n = 0; n < nside; ++n) {
-            const int q = t * kMaxSide + n;
-            const int si = tb.side_i[q];
-            const int row = (int)(int8_t)(si & 0xff), first = (si >> 8) & 0xff, count = si >> 16;
-            double ca = tb.side[q][2], sa = tb.side[q][3];
-            if (row >= 0) sincos_tab(rows.pop(), tb.tab, &sa, &ca);
-            step(F, tb.side[q][0], tb.side[q][1], ca, sa, tb.side[q][4]);
-            for (int k = first; k < first + count; ++k) put(k, F);
-        }
-        sincos_tab((double)av.v[1], tb.tab, &s, &c);
-        step(CA, tb.bb[1][0], tb.bb[1][1], c, s, geo::R_CA_C);  // CA now holds the C frame
-        put(natoms - 2, CA);
-        put(natoms - 1, CA);
-        if (rn) {
-            const uint32_t r3 = *reinterpret_cast<const uint32_t*>(kRes[t].name3);
-            for (int k = 0; k < natoms; ++k) {
-                rn[a + k] = r3;
-                an[a + k] = *reinterpret_cast<const uint32_t*>(kAtom[t][k].name);
+                for (int k = 0; k < 12; ++k) s_rec[wave].f[k] = m[k];
+                s_rec[wave].atoms = cinc;
+                s_rec[wave].flags = bad ? (int)TPL_A2C_STATUS_SEQ : 0;
             }
         }
-        sincos_tab((double)av.v[2], tb.tab, &s, &c);
-        step(CA, tb.bb[2][0], tb.bb[2][1], c, s, geo::R_C_N);
+        __syncthreads();
+        const int here = nb - k0 < NW ? nb - k0 : NW;
+        int mine = before;
+        for (int k = 0; k < here; ++k) {
+            if (k < wave) mine += s_rec[k].atoms;
+            before += s_rec[k].atoms;
+            if (nb <= NW) flags |= s_rec[k].flags;
+        }
+        if (nb <= NW) {
+            total = before;
+            if (total > atoms_stride) flags |= TPL_A2C_STATUS_ATOMS;
+        }
+        if (!flags) {
+            fold(P, s_rec, wave < here ? wave : here);
+            if (j < nb) {
+                double E[12], G[12];
 #pragma unroll
-        for (int k = 0; k < 12; ++k) G[k] = CA[k];
-        a += natoms;
-        av = nav;
-        code = ncode;
+                for (int k = 0; k < 12; ++k) E[k] = dpp_double<kWaveShr1, 0xf>(m[k], ident12(k));
+                compose(P, E, G);
+#pragma unroll
+                for (int r = 0; r < 8; ++r) suspect |= wild(av[r]);
+                const int at = cinc - cnt;
+                if (t >= 0) walk_residue(tb, t, av, tu, G, out + 3 * (size_t)mine, (uint32_t)at);
+                if (rn)
+                    write_names(tb, t, cnt, at, __builtin_amdgcn_readlane(cinc, 63), rn + mine, an + mine,
+                                s_role[wave], lane);
+            }
+            if (k0 + NW < nb) fold(P, s_rec + wave, here - wave);  // here is NW: P for the next NW blocks
+        }
+        __syncthreads();
     }
-    for (int k = 3 * run.total + threadIdx.x; k < 3 * atoms_stride; k += NT) out[k] = (T)0;
-    if (rn)
-        for (int k = run.total + threadIdx.x; k < atoms_stride; k += NT) rn[k] = an[k] = 0u;
+    if (suspect) report_flag(rep, TPLX_A2C_RANGE);
+    if (flags) {
+        if (threadIdx.x == 0) report_bits(rep, (uint32_t)flags);
+        zero_share(out, rn, an, 0, atoms_stride, wave, NW, lane);
+    } else if (nb < NW) {  // the waves without a block
+        if (wave >= nb) zero_share(out, rn, an, total, atoms_stride, wave - nb, NW - nb, lane);
+    } else {
+        zero_share(out, rn, an, total, atoms_stride, wave, NW, lane);
+    }
 }
 
 struct Sums {
@@ -1088,16 +1639,8 @@ __global__ void __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_
         if (k % ang_stride >= L) ga[k] = (T)0;
 }
 
-// 512-thread workgroups when some structure may be longer than 256 residues:
-// always for the run backward (mixed lengths 30-1000 at B=1024: 155 -> 129
-// us), and for the forward only up to twice as many structures as CUs (B=256
-// of 1000 residues: 33.7 -> 28.6 us; B=512 of 300: 23.8 -> 21.8 us; at
-// B=1024 512 threads measured slower, with fewer workgroups per CU: mixed
-// lengths 30-1000 48.4 -> 55.7 us, 1024 x 270 32.0 -> 39.6 us).
-bool use_large_fwd(int batch, int ang_stride) {
-    return batch <= 512 && ang_stride > kThreadsSmall;
-}
-
+// Run backward: 512-thread workgroups when some structure may be longer than
+// 256 residues (mixed lengths 30-1000 at B=1024: 155 -> 129 us).
 bool use_large_bwd(int ang_stride) {
     return ang_stride > kThreadsSmall;
 }
@@ -1139,6 +1682,114 @@ int check(int dtype, int B, int seq_stride, int ang_stride, int atoms_stride) {
     return TPL_A2C_OK;
 }
 
+int blocks_of(int residues) { return residues <= kBlock ? 1 : (residues + kBlock - 1) / kBlock; }
+int groups_of(int residues) { return (residues + kGroup - 1) / kGroup; }
+
+// The workspace: the structures' lengths by slot of the batch (0 for flagged
+// ones), the groups' records, the residues' frames.
+size_t lens_bytes(int batch) { return ((size_t)batch * sizeof(int) + 15) / 16 * 16; }
+size_t recs_bytes(int batch, int angles_stride) {
+    return (size_t)batch * groups_of(angles_stride) * sizeof(GroupRec);
+}
+size_t frames_bytes(int batch, int angles_stride) {
+    return (size_t)batch * groups_of(angles_stride) * sizeof(GroupFrames);
+}
+
+// CUs of the current device (256 where it cannot be asked).
+int compute_units() {
+    static std::mutex mu;
+    static std::vector<int> cus;
+    int dev = 0, n = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0) return 256;
+    std::lock_guard<std::mutex> lock(mu);
+    if ((int)cus.size() <= dev) cus.resize(dev + 1, 0);
+    if (cus[dev] == 0)
+        cus[dev] = hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0 ? n : 256;
+    return cus[dev];
+}
+
+// The group kernels (two launches) or one workgroup per structure.  The group
+// kernels share the blocks evenly over the GPU and win where the structures
+// need more than one round of workgroups (fused -> groups, us, float32 with
+// names: lengths 30-1000 at B=1024 85 -> 62, 1024 x 300 55 -> 46, 300 x 600
+// 44 -> 38, 300 x 1000 57 -> 48; not yet 512 x 300 25 -> 35 and 1024 x 128
+// 22 -> 25), and where a structure has more blocks than a workgroup waves (8 x
+// 3000 82 -> 30, 100 x 1400 48 -> 38) or needs sixteen, which hold few
+// registers, while CUs stay idle (1 x 1000 26 -> 22, 64 x 1000 28 -> 27; 256 x
+// 1000 38 -> 42).
+bool use_groups(int batch, int angles_stride) {
+    const int nb = blocks_of(angles_stride), cus = compute_units();
+    if (nb > 16) return true;
+    return batch > cus ? (int64_t)batch * nb >= 3000 : nb > 8 && batch <= cus / 4;
+}
+
+template <typename T>
+void launch_forward(int form, hipStream_t s, const uint8_t* sequences, int seq_stride, const T* a, int angles_stride,
+                    T* c, uint32_t* rn, uint32_t* an, int atoms_stride, void* workspace, const Report& rep,
+                    const int32_t* order, int batch) {
+    const int nslot = blocks_of(angles_stride), ng = groups_of(angles_stride);
+    const dim3 block(64 * kGroupWaves);
+    if (nslot == 1) {
+        hipLaunchKernelGGL((a2c_fwd_single<T>), dim3((batch + kGroupWaves - 1) / kGroupWaves), block, 0, s, sequences,
+                           seq_stride, a, angles_stride, c, rn, an, atoms_stride, rep, order, batch);
+        return;
+    }
+    if (form == TPLX_A2C_FWD_GROUPS) {
+        char* ws = static_cast<char*>(workspace);
+        int* lens = reinterpret_cast<int*>(ws);
+        GroupRec* rec = reinterpret_cast<GroupRec*>(ws + lens_bytes(batch));
+        GroupFrames* frames =
+            reinterpret_cast<GroupFrames*>(ws + lens_bytes(batch) + recs_bytes(batch, angles_stride));
+        hipLaunchKernelGGL((a2c_fwd_steps<T>), dim3((batch * ng + kGroupWaves - 1) / kGroupWaves), block, 0, s,
+                           sequences, seq_stride, a, angles_stride, lens, rec, frames, c, rn, an, atoms_stride, rep,
+                           order, batch, ng);
+        // what stays resident: two workgroups per CU (one in float64), as their LDS allows
+        const int fill = (sizeof(T) == 4 ? 2 : 1) * compute_units();
+        const int wgs = (batch * nslot + kWalkWaves - 1) / kWalkWaves;
+        hipLaunchKernelGGL((a2c_fwd_walk<T>), dim3(wgs < fill ? wgs : fill), dim3(64 * kWalkWaves), 0, s, sequences,
+                           seq_stride, a, angles_stride, lens, rec, frames, c, rn, an, atoms_stride, rep, order,
+                           batch, ng);
+        return;
+    }
+    // One wave per block up to 8, or up to 16 where every structure can have a
+    // CU; above that the waves go round.  Beyond one structure per CU the
+    // kernel is held to 128 VGPRs, so that two workgroups of 8 waves fit (512 x
+    // 300: 30 -> 25 us).
+    const bool few = batch <= compute_units();
+    const int most = few ? 16 : 8, rounds = (nslot + most - 1) / most, nw = (nslot + rounds - 1) / rounds;
+    const auto kernel = nw > 8 ? a2c_fwd_fused<16, 4, T> : few ? a2c_fwd_fused<8, 2, T> : a2c_fwd_fused<8, 4, T>;
+    hipLaunchKernelGGL(kernel, dim3(batch), dim3(64 * nw), 0, s, sequences, seq_stride, a, angles_stride, c, rn, an,
+                       atoms_stride, rep, order, batch);
+}
+
+// form: TPLX_A2C_FWD_*; GROUPS needs the workspace (where a structure is more
+// than one block), AUTO uses it if there is one.
+int forward_on(int form, const int32_t* order, int dtype, const uint8_t* sequences, int seq_stride,
+               const void* angles, int angles_stride, void* coords, uint8_t* res_names, uint8_t* atom_names,
+               int atoms_stride, void* workspace, const Report& rep, int batch, tpl_a2c_stream_t stream) {
+    const int rc = check(dtype, batch, seq_stride, angles_stride, atoms_stride);
+    if (rc != TPL_A2C_OK) return rc;
+    if (batch == 0) return TPL_A2C_OK;
+    if (!sequences || (angles_stride > 0 && !angles) || (atoms_stride > 0 && !coords) ||
+        (!res_names) != (!atom_names))
+        return TPL_A2C_ERR_ARG;
+    const bool groups_fit = workspace && (int64_t)batch * groups_of(angles_stride) <= INT32_MAX / kGroup;
+    if (form == TPLX_A2C_FWD_AUTO)
+        form = groups_fit && use_groups(batch, angles_stride) ? TPLX_A2C_FWD_GROUPS : TPLX_A2C_FWD_FUSED;
+    if (form == TPLX_A2C_FWD_GROUPS && blocks_of(angles_stride) > 1 && !groups_fit) return TPL_A2C_ERR_ARG;
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    if (!tables_ready(s)) return TPL_A2C_ERR_LAUNCH;
+    uint32_t* rn = reinterpret_cast<uint32_t*>(res_names);
+    uint32_t* an = reinterpret_cast<uint32_t*>(atom_names);
+    if (dtype == TPL_A2C_F32)
+        launch_forward<float>(form, s, sequences, seq_stride, static_cast<const float*>(angles), angles_stride,
+                              static_cast<float*>(coords), rn, an, atoms_stride, workspace, rep, order, batch);
+    else
+        launch_forward<double>(form, s, sequences, seq_stride, static_cast<const double*>(angles), angles_stride,
+                               static_cast<double*>(coords), rn, an, atoms_stride, workspace, rep, order, batch);
+    return hipGetLastError() == hipSuccess ? TPL_A2C_OK : TPL_A2C_ERR_LAUNCH;
+}
+
 }  // namespace
 
 extern "C" {
@@ -1169,37 +1820,21 @@ int tpl_a2c_forward_ordered(const int32_t* order, int dtype, const uint8_t* sequ
                             const void* angles, int angles_stride, void* coords, uint8_t* res_names,
                             uint8_t* atom_names, int atoms_stride, uint32_t* status, int batch,
                             tpl_a2c_stream_t stream) {
-    const int rc = check(dtype, batch, seq_stride, angles_stride, atoms_stride);
-    if (rc != TPL_A2C_OK) return rc;
-    if (batch == 0) return TPL_A2C_OK;
-    if (!sequences || (angles_stride > 0 && !angles) || (atoms_stride > 0 && !coords) ||
-        (!res_names) != (!atom_names))
-        return TPL_A2C_ERR_ARG;
-    hipStream_t s = static_cast<hipStream_t>(stream);
-    if (!tables_ready(s)) return TPL_A2C_ERR_LAUNCH;
-    uint32_t* rn = reinterpret_cast<uint32_t*>(res_names);
-    uint32_t* an = reinterpret_cast<uint32_t*>(atom_names);
-    const bool large = use_large_fwd(batch, angles_stride);
-    if (dtype == TPL_A2C_F32) {
-        const float* a = static_cast<const float*>(angles);
-        float* c = static_cast<float*>(coords);
-        if (large)
-            hipLaunchKernelGGL((a2c_fwd<kThreadsLarge, float>), dim3(batch), dim3(kThreadsLarge), 0, s,
-                               sequences, seq_stride, a, angles_stride, c, rn, an, atoms_stride, status, order);
-        else
-            hipLaunchKernelGGL((a2c_fwd<kThreadsSmall, float>), dim3(batch), dim3(kThreadsSmall), 0, s,
-                               sequences, seq_stride, a, angles_stride, c, rn, an, atoms_stride, status, order);
-    } else {
-        const double* a = static_cast<const double*>(angles);
-        double* c = static_cast<double*>(coords);
-        if (large)
-            hipLaunchKernelGGL((a2c_fwd<kThreadsLarge, double>), dim3(batch), dim3(kThreadsLarge), 0, s,
-                               sequences, seq_stride, a, angles_stride, c, rn, an, atoms_stride, status, order);
-        else
-            hipLaunchKernelGGL((a2c_fwd<kThreadsSmall, double>), dim3(batch), dim3(kThreadsSmall), 0, s,
-                               sequences, seq_stride, a, angles_stride, c, rn, an, atoms_stride, status, order);
-    }
-    return hipGetLastError() == hipSuccess ? TPL_A2C_OK : TPL_A2C_ERR_LAUNCH;
+    return forward_on(TPLX_A2C_FWD_AUTO, order, dtype, sequences, seq_stride, angles, angles_stride, coords,
+                      res_names, atom_names, atoms_stride, nullptr, Report{status, nullptr}, batch, stream);
+}
+
+int tplx_a2c_forward(int form, const int32_t* order, int dtype, const uint8_t* sequences, int seq_stride,
+                     const void* angles, int angles_stride, void* coords, uint8_t* res_names, uint8_t* atom_names,
+                     int atoms_stride, void* workspace, uint32_t* status, uint32_t* flags, int batch,
+                     tpl_a2c_stream_t stream) {
+    return forward_on(form, order, dtype, sequences, seq_stride, angles, angles_stride, coords, res_names,
+                      atom_names, atoms_stride, workspace, Report{status, flags}, batch, stream);
+}
+
+size_t tplx_a2c_workspace_bytes(int batch, int angles_stride) {
+    if (batch <= 0 || blocks_of(angles_stride) == 1) return 0;
+    return lens_bytes(batch) + recs_bytes(batch, angles_stride) + frames_bytes(batch, angles_stride);
 }
 
 int tpl_a2c_forward(int dtype, const uint8_t* sequences, int seq_stride, const void* angles,

@@ -12,6 +12,8 @@
 #include <tuple>
 #include <vector>
 
+#include "a2c_flagged.h"
+#include "host_flags.h"
 #include "tpl_a2c.h"
 
 namespace {
@@ -65,9 +67,16 @@ hipStream_t stream_of(const torch::Tensor& t) {
     return c10::hip::getCurrentHIPStream(t.device().index()).stream();
 }
 
-void forward(torch::Tensor sequences, torch::Tensor input_angles, torch::Tensor output_coords,
-             torch::Tensor res_names, torch::Tensor atom_names, c10::optional<torch::Tensor> status,
-             c10::optional<torch::Tensor> order) {
+// The forward's workspace (none where it needs none), from torch's allocator.
+torch::Tensor workspace_for(const torch::Tensor& angles) {
+    const size_t need = tplx_a2c_workspace_bytes((int)angles.size(0), (int)angles.size(2));
+    if (need == 0) return torch::Tensor();
+    return torch::empty({(int64_t)need}, angles.options().dtype(torch::kByte));
+}
+
+void forward_on(const torch::Tensor& sequences, const torch::Tensor& input_angles,
+                const torch::Tensor& output_coords, const torch::Tensor& res_names, const torch::Tensor& atom_names,
+                uint32_t* status, uint32_t* flags, const c10::optional<torch::Tensor>& order, hipStream_t stream) {
     check_common(sequences, input_angles);
     A2C_CHECK_GPU(output_coords);
     A2C_CHECK_GPU(res_names);
@@ -85,13 +94,34 @@ void forward(torch::Tensor sequences, torch::Tensor input_angles, torch::Tensor 
         TORCH_CHECK(n->device() == input_angles.device(), "names must be on the device of the angles");
     }
     TORCH_CHECK(output_coords.device() == input_angles.device(), "coordinates must be on the device of the angles");
-    c10::DeviceGuard guard(input_angles.device());
-    check_rc(tpl_a2c_forward_ordered(order_ptr(order, input_angles), dtype_code(input_angles),
-                                     sequences.data_ptr<uint8_t>(), (int)sequences.size(1), input_angles.data_ptr(),
-                                     (int)input_angles.size(2), output_coords.data_ptr(),
-                                     res_names.data_ptr<uint8_t>(), atom_names.data_ptr<uint8_t>(), (int)A,
-                                     status_ptr(status, input_angles), (int)B, stream_of(input_angles)),
+    const torch::Tensor ws = workspace_for(input_angles);
+    check_rc(tplx_a2c_forward(TPLX_A2C_FWD_AUTO, order_ptr(order, input_angles), dtype_code(input_angles),
+                              sequences.data_ptr<uint8_t>(), (int)sequences.size(1), input_angles.data_ptr(),
+                              (int)input_angles.size(2), output_coords.data_ptr(), res_names.data_ptr<uint8_t>(),
+                              atom_names.data_ptr<uint8_t>(), (int)A, ws.defined() ? ws.data_ptr() : nullptr, status,
+                              flags, (int)B, stream),
              "Angles2Coords_forward");
+}
+
+void forward(torch::Tensor sequences, torch::Tensor input_angles, torch::Tensor output_coords,
+             torch::Tensor res_names, torch::Tensor atom_names, c10::optional<torch::Tensor> status,
+             c10::optional<torch::Tensor> order) {
+    check_common(sequences, input_angles);
+    c10::DeviceGuard guard(input_angles.device());
+    forward_on(sequences, input_angles, output_coords, res_names, atom_names, status_ptr(status, input_angles),
+               nullptr, order, stream_of(input_angles));
+}
+
+// As forward without a status; waits for the work and returns its status bits
+// (a2c_flagged.h).
+int64_t forward_checked(torch::Tensor sequences, torch::Tensor input_angles, torch::Tensor output_coords,
+                        torch::Tensor res_names, torch::Tensor atom_names, c10::optional<torch::Tensor> order) {
+    check_common(sequences, input_angles);
+    c10::DeviceGuard guard(input_angles.device());
+    hipStream_t stream = stream_of(input_angles);
+    return host_flags::run(stream, [&](uint32_t* flags) {
+        forward_on(sequences, input_angles, output_coords, res_names, atom_names, nullptr, flags, order, stream);
+    });
 }
 
 // From the forward's coordinates (what the Python layer saves).
@@ -168,11 +198,14 @@ std::tuple<double, double, double> bench(std::vector<std::vector<torch::Tensor>>
     c10::DeviceGuard guard(sets[0][1].device());
     hipStream_t stream = stream_of(sets[0][1]);
     const int dt = dtype_code(sets[0][1]);
+    const torch::Tensor ws = workspace_for(sets[0][1]);
+    for (auto& t : sets) TORCH_CHECK(t[1].sizes() == sets[0][1].sizes(), "bench: sets differ in shape");
     auto fwd = [&](std::vector<torch::Tensor>& t) {
         const int32_t* order = t.size() == 6 ? t[5].data_ptr<int32_t>() : nullptr;
-        check_rc(tpl_a2c_forward_ordered(order, dt, t[0].data_ptr<uint8_t>(), (int)t[0].size(1), t[1].data_ptr(),
-                                         (int)t[1].size(2), t[2].data_ptr(), nullptr, nullptr,
-                                         (int)(t[2].size(1) / 3), nullptr, (int)t[1].size(0), stream),
+        check_rc(tplx_a2c_forward(TPLX_A2C_FWD_AUTO, order, dt, t[0].data_ptr<uint8_t>(), (int)t[0].size(1),
+                                  t[1].data_ptr(), (int)t[1].size(2), t[2].data_ptr(), nullptr, nullptr,
+                                  (int)(t[2].size(1) / 3), ws.defined() ? ws.data_ptr() : nullptr, nullptr, nullptr,
+                                  (int)t[1].size(0), stream),
                  "forward");
     };
     auto bwd = [&](std::vector<torch::Tensor>& t) {
@@ -213,6 +246,9 @@ void register_a2c(pybind11::module& m) {
     m.def("Angles2Coords_forward", &forward, "full-atom coordinates and names from angles (GPU)",
           py::arg("sequences"), py::arg("input_angles"), py::arg("output_coords"), py::arg("res_names"),
           py::arg("atom_names"), st, od);
+    m.def("Angles2Coords_forward_checked", &forward_checked, "status bits of the forward, once it has run",
+          py::arg("sequences"), py::arg("input_angles"), py::arg("output_coords"), py::arg("res_names"),
+          py::arg("atom_names"), od, py::call_guard<py::gil_scoped_release>());
     m.def("Angles2Coords_backward", &backward, "gradient of the coordinates with respect to the angles (GPU)",
           py::arg("grad_atoms"), py::arg("grad_angles"), py::arg("sequences"), py::arg("input_angles"), st);
     m.def("Angles2Coords_backward_coords", &backward_coords,

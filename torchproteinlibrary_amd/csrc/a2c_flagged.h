@@ -1,0 +1,27 @@
+// a2c_flagged.h -- the entry points of libtpl_a2c.so that this package's own
+// extension calls: those of include/tpl_a2c.h with a workspace, and with
+// `flags` (report.h, host_flags.h) beside the status word; either may be null.
+// The flags also report TPLX_A2C_RANGE.
+#pragma once
+
+#include "tpl_a2c.h"
+
+// Some output value is NaN, infinite or at least 1e26 in magnitude (report.h).
+#define TPLX_A2C_RANGE 16u
+
+// Forward kernels: one workgroup per structure, or one per group of 256
+// residues (needs the workspace); AUTO picks by the batch and the stride.
+#define TPLX_A2C_FWD_AUTO 0
+#define TPLX_A2C_FWD_FUSED 1
+#define TPLX_A2C_FWD_GROUPS 2
+
+extern "C" {
+// Bytes of the workspace (16-byte aligned; 0: none is used).  A call writes
+// what it reads there.
+size_t tplx_a2c_workspace_bytes(int batch, int angles_stride);
+
+int tplx_a2c_forward(int form, const int32_t* order, int dtype, const uint8_t* sequences, int seq_stride,
+                     const void* angles, int angles_stride, void* coords, uint8_t* res_names, uint8_t* atom_names,
+                     int atoms_stride, void* workspace, uint32_t* status, uint32_t* flags, int batch,
+                     tpl_a2c_stream_t stream);
+}
