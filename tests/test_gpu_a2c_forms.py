@@ -154,3 +154,93 @@ def test_layer_raises_where_the_coordinate_sum_is_nan(lengths, L):
     Y = X.clone()
     Y[0, 7, :] = 1e9  # large, finite: no error
     Angles2Coords()(Y, seqs)
+
+
+def _backward(form, seqs, coords, g, L, order=None):
+    """(grad_angles, status) of one form; the output starts full of others."""
+    lib, B, A = _lib(), coords.shape[0], coords.shape[1] // 3
+    lib.tplx_a2c_backward_workspace_bytes.restype = ctypes.c_size_t
+    S = convertStringList(seqs).to(DEV)
+    ga = torch.full((B, 8, L), 7.0, dtype=coords.dtype, device=DEV)
+    st = torch.zeros(1, dtype=torch.int32, device=DEV)
+    ws = torch.empty(lib.tplx_a2c_backward_workspace_bytes(B, L), dtype=torch.uint8, device=DEV)
+    torch.cuda.synchronize()
+    assert lib.tplx_a2c_backward(form, _p(order), 0 if coords.dtype == torch.float32 else 1, _p(S), S.shape[1],
+                                 _p(coords), _p(g), A, _p(ga), L, _p(ws), _p(st), None, B, None) == 0
+    torch.cuda.synchronize()
+    return ga, int(st.item())
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("shape", range(len(SHAPES)))
+def test_backward_forms_agree(shape, dtype):
+    """Both forms sum the same float64 terms in other orders: up to 14L terms,
+    each bounded by the largest gradient's terms, and one rounding."""
+    lengths, L = SHAPES[shape]
+    seqs, X = _batch(lengths, L, 200 + shape, dtype)
+    natoms = [O.num_atoms(s) for s in seqs]
+    coords = _forward(FUSED, seqs, X, max(natoms) + shape % 3)[0]
+    g = torch.randn(coords.shape, dtype=dtype, device=DEV, generator=torch.Generator(DEV).manual_seed(shape))
+    print(f"a2c backward forms: {len(lengths)} structures, stride {L}, {dtype}", flush=True)
+    outs = [_backward(f, seqs, coords, g, L) for f in (FUSED, GROUPS)]
+    assert outs[0][1] == outs[1][1] == 0
+    tol = 14 * L * 2.0 ** -53 * 8 + (2.0 ** -23 if dtype == torch.float32 else 0.0)
+    for b in range(len(lengths)):
+        scale = float(outs[0][0][b].abs().max())
+        assert float((outs[0][0][b] - outs[1][0][b]).abs().max()) <= tol * scale, b
+        for ga, _ in outs:
+            assert not ga[b, :, lengths[b]:].any()
+    b = int(np.argmin([abs(n - 300) for n in lengths]))  # the oracle on one structure
+    want = O.backward_fast(seqs[b], X[b].double().cpu().numpy(), g[b, :3 * natoms[b]].double().cpu().numpy())
+    for ga, _ in outs:
+        rel = np.abs(ga[b].double().cpu().numpy() - want).max() / np.abs(want).max()
+        assert rel <= (1e-9 if dtype == torch.float64 else 1e-4), rel
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("letters", ["W", "G", "P"])
+def test_backward_forms_at_the_largest_and_smallest_residues(letters, dtype):
+    seqs, X = _batch([64, 130, 300, 1, 0], 301, 17, dtype, letters)
+    coords = _forward(FUSED, seqs, X, max(O.num_atoms(s) for s in seqs))[0]
+    g = torch.randn(coords.shape, dtype=dtype, device=DEV, generator=torch.Generator(DEV).manual_seed(1))
+    for form in (FUSED, GROUPS):
+        ga, st = _backward(form, seqs, coords, g, 301)
+        assert st == 0 and not ga[4].any()
+        for b in (0, 1, 3):
+            n = O.num_atoms(seqs[b])
+            want = O.backward_fast(seqs[b], X[b].double().cpu().numpy(), g[b, :3 * n].double().cpu().numpy())
+            rel = np.abs(ga[b].double().cpu().numpy() - want).max() / max(np.abs(want).max(), 1e-12)
+            assert rel <= (1e-9 if dtype == torch.float64 else 1e-4), (form, b, rel)
+
+
+def test_backward_forms_flag_and_order_alike():
+    L = 200
+    good = O.AA20 * (L // 20)
+    A = O.num_atoms(good)
+    _, X = _batch([L] * 4, L, 3, torch.float32)
+    g = torch.randn(4, 3 * A, device=DEV)
+    for bad, bit in ((good[:-1] + "X", 1), (good + "G", 2), ("W" * L, 4)):
+        seqs = [good, bad, "G" * L, good[:30]]
+        coords = _forward(FUSED, seqs, X, A)[0]
+        outs = [_backward(f, seqs, coords, g, L) for f in (FUSED, GROUPS)]
+        for ga, st in outs:
+            assert st == bit and not ga[1].any() and ga[0].any() and ga[2].any()
+    seqs = [good, good[:70], "G" * L, good[:30]]
+    coords = _forward(FUSED, seqs, X, A)[0]
+    for form in (FUSED, GROUPS):
+        plain = _backward(form, seqs, coords, g, L)[0]
+        turned = _backward(form, seqs, coords, g, L, torch.tensor([2, 0, 3, 1], dtype=torch.int32, device=DEV))[0]
+        assert torch.equal(plain, turned)
+        ga, st = _backward(form, seqs, coords, g, L, torch.tensor([2, 0, -1, 1], dtype=torch.int32, device=DEV))
+        assert st == 8 and bool((ga[3] == 7.0).all()) and torch.equal(ga[:3], plain[:3])
+
+
+@pytest.mark.parametrize("lengths,L", [([21], 21), ([300, 40], 300), ([600] * 300, 600)])
+def test_layer_raises_where_the_gradient_sum_is_nan(lengths, L):
+    from torchproteinlibrary_amd.FullAtomModel import Angles2Coords
+    seqs, X = _batch(lengths, L, 5, torch.float32)
+    coords = Angles2Coords()(X.requires_grad_(True), seqs)[0]
+    g = torch.zeros_like(coords)
+    g[-1, 3 * (O.num_atoms(seqs[-1]) - 1)] = float("nan")
+    with pytest.raises(Exception, match="backward Nan"):
+        coords.backward(g)

@@ -137,10 +137,11 @@ class Angles2CoordsFunction(Function):
         seqs, coords = ctx.saved_tensors
         grad_atoms = grad_atoms.contiguous()
         grad_angles = torch.empty(ctx.angles_shape, dtype=coords.dtype, device=coords.device)
-        status = torch.zeros(1, dtype=torch.int32, device=coords.device) if _checks_enabled() else None
-        ext.Angles2Coords_backward_coords(grad_atoms, grad_angles, seqs, coords, status, ctx.order)
-        if status is not None:
-            _check(int(status.item()) | _STATUS_RANGE, grad_angles, "backward")
+        if _checks_enabled():
+            _check(ext.Angles2Coords_backward_checked(grad_atoms, grad_angles, seqs, coords, ctx.order), grad_angles,
+                   "backward")
+        else:
+            ext.Angles2Coords_backward_coords(grad_atoms, grad_angles, seqs, coords, None, ctx.order)
         return grad_angles, None, None, None
 
 

@@ -31,6 +31,8 @@
 #include <stdint.h>
 
 #include <mutex>
+#include <set>
+#include <utility>
 #include <vector>
 
 #include "a2c_flagged.h"
@@ -393,8 +395,8 @@ struct RowScan {
     // the atoms of its letters, those before residue `upto`, and whether one
     // of them is not a residue's.
     template <bool ATOMS>
-    __device__ __forceinline__ int finish(const uint8_t* seq, int stride, int lane, const StepTables* tb, int upto,
-                                          int& atoms, int& before, bool& bad) {
+    __device__ __forceinline__ int finish(const uint8_t* seq, int stride, int lane, const uint8_t* letter_atoms,
+                                          int upto, int& atoms, int& before, bool& bad) {
         int n = -1, cnt = 0, bef = 0;
         bool odd = false;
         for (int base = 0; n < 0; base += 64 * kAtOnce) {
@@ -406,7 +408,7 @@ struct RowScan {
                 const int i = base + 64 * e + lane;
                 if (zero) n = base + 64 * e + (int)__builtin_ctzll(zero);
                 if (ATOMS && (n < 0 || i < n)) {
-                    const int k = tb->atoms[c[e]];
+                    const int k = letter_atoms[c[e]];
                     odd |= k == 0;
                     cnt += k;
                     if (i < upto) bef += k;
@@ -678,7 +680,7 @@ __global__ void __launch_bounds__(64 * kGroupWaves) a2c_fwd_steps(
     }
     int total = 0, before = 0, flags = 0;
     bool bad = false;
-    int n = row.finish<true>(seq, seq_stride, lane, &tb, kGroup * g, total, before, bad);
+    int n = row.finish<true>(seq, seq_stride, lane, tb.atoms, kGroup * g, total, before, bad);
     if (n > ang_stride) {
         flags = TPL_A2C_STATUS_LENGTH;
     } else {
@@ -830,76 +832,96 @@ a2c_fwd_single(const uint8_t* __restrict__ seqs, int seq_stride, const T* __rest
     zero_share(out, rn, an, total, atoms_stride, 0, 1, lane);
 }
 
-// The atoms after a2c_fwd_steps, which also took care of the flags and the
-// padding.  The waves of a grid that stays resident share the blocks that hold
-// residues: every workgroup sums up the structures' block counts (a segment of
-// the batch at a time), and wave w of W takes blocks w, w + W, ... of that
-// list.  One block per wave in a grid over all blocks left a CU's slots to
-// waves that found their block past the structure and to workgroups with one
-// wave at work, each copying the tables anew: lengths 30-1000 at B=1024 took
-// 38 us, against 31.
+// The blocks that hold residues, as a list that a resident grid's waves share:
+// structure by structure, a segment of the batch at a time.  Every workgroup
+// sums up the structures' block counts from their lengths, and wave w of W
+// takes blocks w, w + W, ... of the list.  One block per wave in a grid over all
+// blocks left a CU's slots to waves that found their block past the structure
+// and to workgroups with one wave at work, each copying the tables anew: the
+// walk of lengths 30-1000 at B=1024 took 38 us, against 31.
 constexpr int kWalkWaves = 8;
 constexpr int kSegment = 2048;  // structures per segment: their block counts' sums live in LDS
+struct BlockList {
+    int first[kSegment + 1];  // blocks before a structure of the segment
+    uint8_t last[kSegment];   // residues of its last block, less one
+    int sum[kWalkWaves];
+};
+
+// Fills the list for m structures from their lengths; returns its blocks.
+// meanwhile() runs while the lengths are loaded.  Ends with a barrier.
+template <typename Meanwhile>
+__device__ __forceinline__ int list_blocks(BlockList& l, const int* lens, int m, int wave, int lane,
+                                           Meanwhile meanwhile) {
+    constexpr int NT = 64 * kWalkWaves, kPer = kSegment / NT;
+    int nb[kPer], last[kPer], sum = 0;
+#pragma unroll
+    for (int e = 0; e < kPer; ++e) {
+        const int k = kPer * (int)threadIdx.x + e;
+        last[e] = k < m ? lens[k] : 0;
+    }
+    meanwhile();
+#pragma unroll
+    for (int e = 0; e < kPer; ++e) {
+        nb[e] = (last[e] + kBlock - 1) / kBlock;
+        last[e] = (last[e] - 1) & (kBlock - 1);
+        sum += nb[e];
+    }
+    const int inc = wave_scan_int(sum);
+    __syncthreads();  // a list before this one is done with
+    if (lane == 63) l.sum[wave] = inc;
+    __syncthreads();
+    int at = inc - sum, blocks = 0;
+#pragma unroll
+    for (int k = 0; k < kWalkWaves; ++k) {
+        at += k < wave ? l.sum[k] : 0;
+        blocks += l.sum[k];
+    }
+#pragma unroll
+    for (int e = 0; e < kPer; ++e) {
+        l.first[kPer * (int)threadIdx.x + e] = at;
+        l.last[kPer * (int)threadIdx.x + e] = (uint8_t)last[e];
+        at += nb[e];
+    }
+    if (threadIdx.x == NT - 1) l.first[kSegment] = at;
+    __syncthreads();
+    return blocks;
+}
+
+// Block `it` of the list: its structure k of the segment (the last one that
+// starts at or before it: empty ones share the start of the next), which block
+// j of it, and that structure's length n.  All wave-uniform.
+__device__ __forceinline__ void find_block(const BlockList& l, int it, int lane, int& k, int& j, int& n) {
+    static_assert(kSegment == 64 * 32, "two rounds of comparisons: every 32nd, then 32");
+    const int hi = 32 * (__builtin_popcountll(__builtin_amdgcn_ballot_w64(l.first[32 * lane] <= it)) - 1);
+    k = hi + __builtin_popcountll(__builtin_amdgcn_ballot_w64(lane < 32 && l.first[hi + (lane & 31)] <= it)) - 1;
+    const int first = __builtin_amdgcn_readfirstlane(l.first[k]);
+    j = it - first;
+    n = kBlock * (__builtin_amdgcn_readfirstlane(l.first[k + 1]) - first - 1) +
+        __builtin_amdgcn_readfirstlane((int)l.last[k]) + 1;
+}
+
+// The atoms after a2c_fwd_steps, which also took care of the flags and the
+// padding: the blocks of the list above.
 template <typename T>
 __global__ void __launch_bounds__(64 * kWalkWaves) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 4 : 2, 8)))
 a2c_fwd_walk(const uint8_t* __restrict__ seqs, int seq_stride, const T* __restrict__ angles, int ang_stride,
              const int* __restrict__ lens, const GroupRec* __restrict__ rec, const GroupFrames* __restrict__ frames,
              T* __restrict__ coords, uint32_t* __restrict__ res_names, uint32_t* __restrict__ atom_names,
              int atoms_stride, Report rep, const int* __restrict__ order, int batch, int ng) {
-    constexpr int NT = 64 * kWalkWaves, kPer = kSegment / NT;
     __shared__ Tables tb;
     __shared__ __align__(16) T s_stage[kWalkWaves][stage_values<T>()];
-    __shared__ int s_first[kSegment + 1];  // blocks before a structure of the segment
-    __shared__ uint8_t s_last[kSegment];   // residues of its last block, less one
-    __shared__ int s_sum[kWalkWaves];
+    __shared__ BlockList s_list;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = (int)(threadIdx.x & 63);
     const int step = (int)gridDim.x * kWalkWaves;
     bool suspect = false;
     for (int base = 0; base < batch; base += kSegment) {
-        const int m = batch - base < kSegment ? batch - base : kSegment;
-        int nb[kPer], sum = 0, last[kPer];
-#pragma unroll
-        for (int e = 0; e < kPer; ++e) {
-            const int k = kPer * (int)threadIdx.x + e;
-            last[e] = k < m ? lens[base + k] : 0;
-        }
-        if (base == 0) copy_tables(tb, NT);
-#pragma unroll
-        for (int e = 0; e < kPer; ++e) {
-            nb[e] = (last[e] + kBlock - 1) / kBlock;
-            last[e] = (last[e] - 1) & (kBlock - 1);
-            sum += nb[e];
-        }
-        const int inc = wave_scan_int(sum);
-        if (base > 0) __syncthreads();  // the segment before is done
-        if (lane == 63) s_sum[wave] = inc;
-        __syncthreads();
-        int at = inc - sum, items = 0;
-#pragma unroll
-        for (int k = 0; k < kWalkWaves; ++k) {
-            at += k < wave ? s_sum[k] : 0;
-            items += s_sum[k];
-        }
-#pragma unroll
-        for (int e = 0; e < kPer; ++e) {
-            s_first[kPer * (int)threadIdx.x + e] = at;
-            s_last[kPer * (int)threadIdx.x + e] = (uint8_t)last[e];
-            at += nb[e];
-        }
-        if (threadIdx.x == NT - 1) s_first[kSegment] = at;
-        __syncthreads();
-        for (int it = (int)blockIdx.x * kWalkWaves + wave; it < items; it += step) {
-            // the last structure that starts at or before block `it` and has one:
-            // first among every 32nd, then among the 32 (empty ones share the
-            // start of the next, so the last is the one)
-            static_assert(kSegment == 64 * 32, "two rounds of comparisons");
-            const int hi = 32 * (__builtin_popcountll(__builtin_amdgcn_ballot_w64(s_first[32 * lane] <= it)) - 1);
-            const uint64_t le = __builtin_amdgcn_ballot_w64(lane < 32 && s_first[hi + (lane & 31)] <= it);
-            const int k = hi + __builtin_popcountll(le) - 1;
-            const int first = __builtin_amdgcn_readfirstlane(s_first[k]);
-            const int j = it - first;
-            const int bn = kBlock * (__builtin_amdgcn_readfirstlane(s_first[k + 1]) - first - 1) +
-                           __builtin_amdgcn_readfirstlane((int)s_last[k]) + 1;
+        const int blocks =
+            list_blocks(s_list, lens + base, batch - base < kSegment ? batch - base : kSegment, wave, lane, [&] {
+                if (base == 0) copy_tables(tb, 64 * kWalkWaves);
+            });
+        for (int it = (int)blockIdx.x * kWalkWaves + wave; it < blocks; it += step) {
+            int k, j, bn;
+            find_block(s_list, it, lane, k, j, bn);
             const int b = structure_at(order, base + k, batch, Report{nullptr, nullptr});
             const int g = j / kGroupWaves, part = j % kGroupWaves;
             const int i = kBlock * j + lane;
@@ -1639,22 +1661,555 @@ __global__ void __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_
         if (k % ang_stride >= L) ga[k] = (T)0;
 }
 
+// ---- backward: one lane per residue ----
+// As in the forward, a wave takes a block of 64 consecutive residues, one per
+// lane, the last residue first: sums over a residue's subtree run over the
+// later residues, so they are prefixes over the lanes.  The block's atoms and
+// their gradients come through the wave's LDS (coalesced loads, each read
+// once), and a lane sums its residue's groups from the end: C and O, then the
+// side chain, whose angles' gradients follow at once (their subtrees end
+// with the residue), CA, N.  A scan of the residues' sums over the lanes and
+// the sums of the later blocks give the backbone angles' subtrees.
+//   * a2c_bwd_sums + a2c_bwd_walk: the first kernel leaves each block's sums in
+//     the caller's workspace (and writes the zeros past the structures), the
+//     second takes the blocks of the list (list_blocks);
+//   * a2c_bwd_fused: one workgroup per structure, whose waves' sums meet in
+//     LDS.  One launch, no workspace.
+// Against runs of residues per thread, or atom tiles walked by one workgroup per
+// structure (kept for callers that pin them), us: lengths 30-1000 at B=1024
+// 94 -> 60 (60 -> 60 with the structures ordered by size), in float64 168 -> 95;
+// 256 x 1000 50 -> 36, 1 x 1000 34 -> 18, 32 x 350 17.1 -> 14.2, 1024 x 128
+// 34 -> 17, 1024 x 30 14.3 -> 9.8, one peptide of 21 in float64 12.0 -> 8.3; 512 x
+// 300 26 -> 29.  What bounds it: the LDS that a block's atoms take holds eight
+// waves on a CU, and those wait on latencies two thirds of their time.
+struct alignas(16) BackTables {
+    int res_i[kTypes];              // natoms | nca << 8 | nside << 16
+    int side_i[kTypes * kMaxSide];  // row & 0xff | first << 8 | count << 16
+    uint8_t type[256];              // residue type of a letter, 0xff: none
+    uint8_t atoms[256];             // its atoms, 0: none
+};
+
+constexpr BackTables make_back_tables() {
+    constexpr Residue res[kTypes] = A2C_RESIDUES;
+    constexpr Side side[kTypes][kMaxSide] = A2C_SIDES;
+    BackTables t{};
+    for (int c = 0; c < 256; ++c) t.type[c] = 0xff;
+    for (int k = 0; k < kTypes; ++k) {
+        t.res_i[k] = res[k].natoms | (res[k].nca << 8) | (res[k].nside << 16);
+        for (int n = 0; n < kMaxSide; ++n)
+            t.side_i[k * kMaxSide + n] = (side[k][n].row & 0xff) | (side[k][n].first << 8) | (side[k][n].count << 16);
+        t.type[(uint8_t)kCodes[k]] = (uint8_t)k;
+        t.atoms[(uint8_t)kCodes[k]] = (uint8_t)res[k].natoms;
+    }
+    return t;
+}
+__constant__ BackTables kBack = make_back_tables();
+
+__device__ __forceinline__ void copy_back_tables(BackTables& tb, int nt) {
+    const uint4* src = reinterpret_cast<const uint4*>(&kBack);
+    uint4* dst = reinterpret_cast<uint4*>(&tb);
+    for (int k = threadIdx.x; k < (int)(sizeof(BackTables) / 16); k += nt) dst[k] = src[k];
+}
+
+// Atoms staged at a time (in float64 a block takes two rounds, so that eight
+// waves fit on a CU), and the values per array: those atoms', two more atoms
+// before them (the C and O of the residue before), and the offset that aligns
+// both sides.
+template <typename T>
+constexpr int back_stage() {
+    return sizeof(T) == 4 ? 576 : 288;
+}
+template <typename T>
+constexpr int back_values() {
+    return 3 * (back_stage<T>() + 2) + 16 / (int)sizeof(T);
+}
+
+// A run of values on its way from memory to the wave's LDS: fetch() issues the
+// loads (16 bytes per lane where src is aligned), commit() writes them to LDS,
+// whose s_w[0] holds the value of src rounded down to 16 bytes (flush_stage's
+// layout).  The two stand apart, so that other work hides the loads.
+template <typename T>
+struct Fetch {
+    static constexpr int V = 16 / (int)sizeof(T);
+    static constexpr int kBody = (back_values<T>() + 64 * V - 1) / (64 * V);
+    uint4 body[kBody];
+    T head, tail;
+
+    __device__ __forceinline__ static int offset(const T* src) {
+        return (int)((reinterpret_cast<uintptr_t>(src) & 15) / sizeof(T));
+    }
+    __device__ __forceinline__ void fetch(const T* src, int count, int lane) {
+        const int mis = offset(src), end = mis + count, first = mis ? V : 0, last = end / V * V;
+        const T* d0 = src - mis;
+        head = tail = (T)0;
+        if (mis && lane >= mis && lane < V && lane < end) head = d0[lane];
+#pragma unroll
+        for (int e = 0; e < kBody; ++e) {
+            const int k = first + V * (64 * e + lane);
+            body[e] = make_uint4(0, 0, 0, 0);
+            if (k < last) body[e] = *reinterpret_cast<const uint4*>(d0 + k);
+        }
+        const int t = (last > first ? last : first) + lane;
+        if (t < end) tail = d0[t];
+    }
+    __device__ __forceinline__ void commit(const T* src, int count, T* s_w, int lane) const {
+        const int mis = offset(src), end = mis + count, first = mis ? V : 0, last = end / V * V;
+        if (mis && lane >= mis && lane < V && lane < end) s_w[lane] = head;
+#pragma unroll
+        for (int e = 0; e < kBody; ++e) {
+            const int k = first + V * (64 * e + lane);
+            if (k < last) *reinterpret_cast<uint4*>(s_w + k) = body[e];
+        }
+        const int t = (last > first ? last : first) + lane;
+        if (t < end) s_w[t] = tail;
+    }
+};
+
+// s += the sums (g, x cross g) of atoms [k0, k1) of the staged x and g.
+template <typename T>
+__device__ __forceinline__ void staged_sums(const T* x, const T* g, int k0, int k1, double s[6]) {
+    for (int k = k0; k < k1; ++k) {
+        double p[3], h[3];
+        load3(x + 3 * k, p);
+        load3(g + 3 * k, h);
+        s[0] += h[0];
+        s[1] += h[1];
+        s[2] += h[2];
+        s[3] += p[1] * h[2] - p[2] * h[1];
+        s[4] += p[2] * h[0] - p[0] * h[2];
+        s[5] += p[0] * h[1] - p[1] * h[0];
+    }
+}
+
+// What a lane keeps of its residue for the backbone angles.
+template <typename T>
+struct BackResidue {
+    double sc[6];  // sums over C and O
+    double sa[6];  // over the side chain and CA's group
+    double sn[6];  // over N
+    T n[3], ca[3], c[3], prev[3];  // origins, prev: the C before
+};
+
+// The lane's residue of type t from its staged atoms x and g: its sums and
+// origins, and its side chain's gradients (0 for the rows it does not bind).
+// Returns whether a gradient is out of range.
+template <typename T>
+__device__ __forceinline__ bool back_residue(const BackTables& tb, int t, bool first, const T* x, const T* g,
+                                             BackResidue<T>& r, T* ga, uint32_t stride, uint32_t i) {
+    const int ri = tb.res_i[t];
+    const int natoms = ri & 0xff, nca = (ri >> 8) & 0xff, nside = ri >> 16;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        r.n[c] = x[c];
+        r.ca[c] = x[3 + c];
+        r.c[c] = x[3 * (natoms - 2) + c];
+        r.prev[c] = first ? (T)0 : x[c - 6];
+    }
+#pragma unroll
+    for (int k = 0; k < 6; ++k) r.sc[k] = r.sa[k] = r.sn[k] = 0.0;
+    staged_sums(x, g, natoms - 2, natoms, r.sc);
+    bool range = false;
+    int bound = 0;
+    int si = nside > 0 ? tb.side_i[t * kMaxSide + nside - 1] : 0;
+    for (int n = nside - 1; n > 0; --n) {  // node 0 is fixed and has no atoms
+        const int sp = tb.side_i[t * kMaxSide + n - 1];
+        const int row = (int)(int8_t)(si & 0xff), first_atom = (si >> 8) & 0xff, count = si >> 16;
+        staged_sums(x, g, first_atom, first_atom + count, r.sa);
+        if (row >= 0) {
+            // the parent's origin: the node before, or CA for the first
+            const int parent = (sp >> 16) > 0 ? (sp >> 8) & 0xff : 1;
+            double p[3], q[3];
+            load3(x + 3 * first_atom, p);
+            load3(x + 3 * parent, q);
+            const T v = (T)bond_torque_rsq(p, q, r.sa);
+            range |= out_of_range(v);
+            ga[(uint32_t)row * stride + i] = v;
+            bound |= 1 << row;
+        }
+        si = sp;
+    }
+#pragma unroll
+    for (int row = 3; row < 8; ++row)
+        if (!((bound >> row) & 1)) ga[(uint32_t)row * stride + i] = (T)0;
+    staged_sums(x, g, 1, 1 + nca, r.sa);
+    staged_sums(x, g, 0, 1, r.sn);
+    return range;
+}
+
+// The backbone angles of the lane's residue i of n, whose later residues'
+// atoms sum to `after`: psi turns C and what follows, phi CA's group and the
+// side chain too, omega of the residue before everything from N on.
+template <typename T>
+__device__ __forceinline__ bool back_backbone(const BackResidue<T>& r, const double after[6], T* ga, uint32_t stride,
+                                              uint32_t i, uint32_t n) {
+    double s[6], p[3], q[3], a[3], c[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) p[k] = (double)r.n[k], a[k] = (double)r.ca[k], c[k] = (double)r.c[k], q[k] = (double)r.prev[k];
+#pragma unroll
+    for (int k = 0; k < 6; ++k) s[k] = after[k] + r.sc[k];
+    const T psi = (T)bond_torque_rsq(c, a, s);
+#pragma unroll
+    for (int k = 0; k < 6; ++k) s[k] += r.sa[k];
+    const T phi = (T)bond_torque_rsq(a, p, s);
+    ga[i] = phi;
+    ga[stride + i] = psi;
+    bool range = out_of_range(phi) || out_of_range(psi);
+    if (i > 0) {
+#pragma unroll
+        for (int k = 0; k < 6; ++k) s[k] += r.sn[k];
+        const T omega = (T)bond_torque_rsq(p, q, s);
+        range |= out_of_range(omega);
+        ga[2 * stride + i - 1] = omega;
+    }
+    if (i == n - 1) ga[2 * stride + i] = (T)0;
+    return range;
+}
+
+// v <- the sum over the lanes before (exclusive prefix); all: the wave's sum.
+__device__ __forceinline__ void lanes_before(double v[6], double all[6]) {
+#pragma unroll
+    for (int k = 0; k < 6; ++k) {
+        const double inc = wave_scan_double(v[k]);
+        all[k] = readlane_double(inc, 63);
+        v[k] = dpp_double<kWaveShr1, 0xf>(inc, 0.0);
+    }
+}
+
+// The atoms of a block that starts at atom a0 and has `total`, on their way to
+// LDS: at first as many as are staged at a time, with the C and O before them.
+template <typename T>
+struct BackFetch {
+    Fetch<T> x, g;
+
+    __device__ __forceinline__ static int lead(int a0) { return a0 >= 2 ? 2 : 0; }
+    __device__ __forceinline__ static int values(int a0, int total) {
+        return 3 * ((total < back_stage<T>() ? total : back_stage<T>()) + lead(a0));
+    }
+    __device__ __forceinline__ void fetch(const T* xs, const T* gs, int a0, int total, int lane) {
+        const size_t from = 3 * (size_t)(a0 - lead(a0));
+        x.fetch(xs + from, values(a0, total), lane);
+        g.fetch(gs + from, values(a0, total), lane);
+    }
+    __device__ __forceinline__ void commit(const T* xs, const T* gs, int a0, int total, T* s_x, T* s_g, int lane) const {
+        const size_t from = 3 * (size_t)(a0 - lead(a0));
+        x.commit(xs + from, values(a0, total), s_x, lane);
+        g.commit(gs + from, values(a0, total), s_g, lane);
+    }
+};
+
+// A block's residues, by one wave: lane l holds residue i0 + 63 - l, of type t
+// (-1: none) with cnt atoms from `at` on; f holds the block's first atoms.
+// Fills r; returns whether a gradient is out of range.
+template <typename T>
+__device__ __forceinline__ bool back_block(const BackTables& tb, int t, int at, int cnt, int total, int a0, const T* xs,
+                                           const T* gs, BackFetch<T>& f, BackResidue<T>& r, T* ga, uint32_t stride,
+                                           uint32_t i, T* s_x, T* s_g, int lane) {
+    bool range = false;
+    for (int base = 0; base < total;) {
+        // residues go down the lanes: the first one that does not fit is in the highest of those lanes
+        const uint64_t later = __builtin_amdgcn_ballot_w64(t >= 0 && at + cnt > base + back_stage<T>());
+        const int end = later ? __builtin_amdgcn_readlane(at, 63 - (int)__builtin_clzll(later)) : total;
+        const int from = a0 + base, lead = BackFetch<T>::lead(from);
+        if (base > 0) f.fetch(xs, gs, from, total - base, lane);
+        f.commit(xs, gs, from, total - base, s_x, s_g, lane);
+        wave_lds_sync();
+        if (t >= 0 && at >= base && at < end) {
+            const size_t first = 3 * (size_t)(from - lead);
+            const int o = 3 * (at - base + lead);
+            range |= back_residue(tb, t, a0 + at == 0, s_x + Fetch<T>::offset(xs + first) + o,
+                                  s_g + Fetch<T>::offset(gs + first) + o, r, ga, stride, i);
+        }
+        wave_lds_sync();
+        base = end;
+    }
+    return range;
+}
+
+// A block's sums, for the blocks before it.
+struct alignas(16) BackRec {
+    double s[6];
+    int a0, total;  // its first atom and its atoms
+    int pad[2];
+};
+
+// Zeros for residues [r0, r1) of a structure's 8 rows, by one wave.
+template <typename T>
+__device__ __forceinline__ void zero_rows(T* ga, uint32_t stride, int r0, int r1, int lane) {
+    for (int row = 0; row < 8; ++row)
+        for (int i = r0 + lane; i < r1; i += 64) ga[(size_t)row * stride + i] = (T)0;
+}
+
+// Each block's sums, one wave per (structure, block), structures first; and the
+// zeros of the blocks past the structure.  Every wave reads the whole row of
+// letters and so knows the structure's length, atoms and flags by itself.
+constexpr int kSumWaves = 4;
+template <typename T>
+__global__ void __launch_bounds__(64 * kSumWaves) a2c_bwd_sums(
+    const uint8_t* __restrict__ seqs, int seq_stride, const T* __restrict__ coords, const T* __restrict__ grads,
+    int atoms_stride, int* __restrict__ lens, BackRec* __restrict__ rec, T* __restrict__ grad_angles, int ang_stride,
+    Report rep, const int* __restrict__ order, int batch, int nslot) {
+    __shared__ BackTables tb;
+    const int wave = (int)(threadIdx.x >> 6), lane = (int)(threadIdx.x & 63);
+    const int w = __builtin_amdgcn_readfirstlane((int)blockIdx.x * kSumWaves + wave);
+    const int j = w / batch, slot = w - j * batch;
+    const int b = j < nslot ? structure_at(order, slot, batch, j == 0 ? rep : Report{nullptr, nullptr}) : -1;
+    const uint8_t* seq = seqs + (size_t)(b < 0 ? 0 : b) * seq_stride;
+    RowScan row;
+    row.load(seq, seq_stride, lane);
+    const int i = kBlock * j + lane;
+    const uint8_t code = b >= 0 && i < ang_stride && i < seq_stride ? seq[i] : (uint8_t)0;
+    copy_back_tables(tb, 64 * kSumWaves);
+    __syncthreads();
+    if (b < 0) {
+        if (j == 0 && slot < batch && lane == 0) lens[slot] = 0;
+        return;
+    }
+    int total = 0, before = 0, flags = 0;
+    bool bad = false;
+    int n = row.finish<true>(seq, seq_stride, lane, tb.atoms, kBlock * j, total, before, bad);
+    if (n > ang_stride) {
+        flags = TPL_A2C_STATUS_LENGTH;
+    } else {
+        if (bad) flags |= TPL_A2C_STATUS_SEQ;
+        if (total > atoms_stride) flags |= TPL_A2C_STATUS_ATOMS;
+    }
+    if (flags) {  // a flagged structure's gradients are zeros
+        if (j == 0 && lane == 0) report_bits(rep, (uint32_t)flags);
+        n = 0;
+    }
+    if (j == 0 && lane == 0) lens[slot] = n;
+    T* ga = grad_angles + (size_t)b * 8 * ang_stride;
+    if (kBlock * j >= n) {
+        const int r1 = kBlock * (j + 1) < ang_stride ? kBlock * (j + 1) : ang_stride;
+        zero_rows(ga, (uint32_t)ang_stride, kBlock * j, r1, lane);
+        return;
+    }
+    const int here = __builtin_amdgcn_readlane(wave_scan_int(i < n ? (int)tb.atoms[code] : 0), 63);
+    const T* xs = coords + 3 * ((size_t)b * atoms_stride + before);
+    const T* gs = grads + 3 * ((size_t)b * atoms_stride + before);
+    double s[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    constexpr int kAtOnce = 3;  // atoms per lane in flight
+    for (int k0 = lane; k0 < here; k0 += 64 * kAtOnce) {
+        T p[kAtOnce][3], h[kAtOnce][3];
+#pragma unroll
+        for (int e = 0; e < kAtOnce; ++e) {
+            const int k = k0 + 64 * e < here ? k0 + 64 * e : k0;
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                p[e][c] = xs[3 * k + c];
+                h[e][c] = gs[3 * k + c];
+            }
+        }
+#pragma unroll
+        for (int e = 0; e < kAtOnce; ++e)
+            if (k0 + 64 * e < here) staged_sums(p[e], h[e], 0, 1, s);
+    }
+    double all[6];
+    lanes_before(s, all);
+    if (lane == 0) {
+        BackRec* r = rec + (size_t)b * nslot + j;
+#pragma unroll
+        for (int k = 0; k < 6; ++k) r->s[k] = all[k];
+        r->a0 = before;
+        r->total = here;
+    }
+}
+
+// The gradients after a2c_bwd_sums: the blocks of the list.
+template <typename T>
+__global__ void __launch_bounds__(64 * kWalkWaves) a2c_bwd_walk(
+    const uint8_t* __restrict__ seqs, int seq_stride, const T* __restrict__ coords, const T* __restrict__ grads,
+    int atoms_stride, const int* __restrict__ lens, const BackRec* __restrict__ rec, T* __restrict__ grad_angles,
+    int ang_stride, Report rep, const int* __restrict__ order, int batch, int nslot) {
+    __shared__ BackTables tb;
+    __shared__ BlockList s_list;
+    extern __shared__ __align__(16) unsigned char s_dyn[];
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = (int)(threadIdx.x & 63);
+    T* s_x = reinterpret_cast<T*>(s_dyn) + (size_t)wave * 2 * back_values<T>();
+    T* s_g = s_x + back_values<T>();
+    const int step = (int)gridDim.x * kWalkWaves;
+    const uint32_t stride = (uint32_t)ang_stride;
+    bool range = false;
+    for (int base = 0; base < batch; base += kSegment) {
+        const int blocks =
+            list_blocks(s_list, lens + base, batch - base < kSegment ? batch - base : kSegment, wave, lane, [&] {
+                if (base == 0) copy_back_tables(tb, 64 * kWalkWaves);
+            });
+        // A block's letters and record are loaded while the one before it is
+        // walked, and its atoms while that one's backbone is.
+        int it = (int)blockIdx.x * kWalkWaves + wave, b = 0, j = 0, n = 0, a0 = 0, total = 0;
+        uint8_t code = 0;
+        BackFetch<T> f;
+        const auto find = [&](int at) {
+            int k;
+            find_block(s_list, at, lane, k, j, n);
+            b = structure_at(order, base + k, batch, Report{nullptr, nullptr});
+            const int i = kBlock * j + 63 - lane;
+            code = i < n ? seqs[(size_t)b * seq_stride + i] : (uint8_t)0;
+            const BackRec* rb = rec + (size_t)b * nslot + j;
+            a0 = rb->a0;
+            total = rb->total;
+        };
+        const auto fetch = [&]() {
+            a0 = __builtin_amdgcn_readfirstlane(a0);
+            total = __builtin_amdgcn_readfirstlane(total);
+            f.fetch(coords + 3 * (size_t)b * atoms_stride, grads + 3 * (size_t)b * atoms_stride, a0, total, lane);
+        };
+        if (it < blocks) {
+            find(it);
+            fetch();
+        }
+        for (; it < blocks; it += step) {
+            const int cb = b, cj = j, cn = n, ca0 = a0, ctotal = total;
+            const int i = kBlock * cj + 63 - lane;
+            const int t = (int)(int8_t)tb.type[code];
+            const int cnt = t >= 0 ? tb.res_i[t] & 0xff : 0;
+            // the lanes up to this one hold its residue's atoms and the later ones'
+            const int at = ctotal - wave_scan_int(cnt);
+            // the later blocks' sums, one block per lane
+            const BackRec* rb = rec + (size_t)cb * nslot + cj;
+            double carry[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+            const int nb = (cn + kBlock - 1) / kBlock;
+            for (int h = cj + 1 + lane; h < nb + lane; h += 64) {
+#pragma unroll
+                for (int c = 0; c < 6; ++c) carry[c] += h < nb ? rb[h - cj].s[c] : 0.0;
+            }
+            const T* xs = coords + 3 * (size_t)cb * atoms_stride;
+            const T* gs = grads + 3 * (size_t)cb * atoms_stride;
+            T* ga = grad_angles + (size_t)cb * 8 * ang_stride;
+            const bool more = it + step < blocks;
+            if (more) find(it + step);
+            BackResidue<T> r;
+            range |= back_block(tb, t, at, cnt, ctotal, ca0, xs, gs, f, r, ga, stride, (uint32_t)i, s_x, s_g, lane);
+            if (more) fetch();
+            double after[6], all[6];
+            if (nb > cj + 1) {
+                double later[6];
+                lanes_before(carry, later);
+#pragma unroll
+                for (int c = 0; c < 6; ++c) carry[c] = later[c];
+            }
+#pragma unroll
+            for (int c = 0; c < 6; ++c) after[c] = t >= 0 ? r.sc[c] + r.sa[c] + r.sn[c] : 0.0;
+            lanes_before(after, all);
+#pragma unroll
+            for (int c = 0; c < 6; ++c) after[c] += carry[c];
+            if (t >= 0)
+                range |= back_backbone(r, after, ga, stride, (uint32_t)i, (uint32_t)cn);
+            else if (i < ang_stride)
+                for (int row = 0; row < 8; ++row) ga[(uint32_t)row * stride + (uint32_t)i] = (T)0;
+        }
+    }
+    if (range) report_flag(rep, TPLX_A2C_RANGE);
+}
+
+// One workgroup per structure, of blockDim / 64 waves: the waves take their
+// blocks together, from the structure's end, as many at a time as there are
+// waves.
+constexpr int kBackWaves = 8;
+template <typename T>
+__global__ void __launch_bounds__(64 * kBackWaves) a2c_bwd_fused(
+    const uint8_t* __restrict__ seqs, int seq_stride, const T* __restrict__ coords, const T* __restrict__ grads,
+    int atoms_stride, T* __restrict__ grad_angles, int ang_stride, Report rep, const int* __restrict__ order,
+    int batch) {
+    __shared__ BackTables tb;
+    __shared__ double s_sum[kBackWaves][6];
+    __shared__ int s_cnt[kBackWaves];
+    extern __shared__ __align__(16) unsigned char s_dyn[];
+    const int NW = (int)(blockDim.x >> 6);
+    const int wave = turned_wave(__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), NW, (int)blockIdx.x);
+    const int lane = (int)(threadIdx.x & 63);
+    T* s_x = reinterpret_cast<T*>(s_dyn) + (size_t)wave * 2 * back_values<T>();
+    T* s_g = s_x + back_values<T>();
+    const int b = structure_at(order, (int)blockIdx.x, batch, rep);
+    if (b < 0) return;
+    const uint8_t* seq = seqs + (size_t)b * seq_stride;
+    RowScan row;
+    row.load(seq, seq_stride, lane);
+    copy_back_tables(tb, 64 * NW);
+    __syncthreads();
+    // every wave alike
+    int atoms = 0, unused = 0, flags = 0;
+    bool bad = false;
+    int n = row.finish<true>(seq, seq_stride, lane, tb.atoms, 0, atoms, unused, bad);
+    if (n > ang_stride) {
+        flags = TPL_A2C_STATUS_LENGTH;
+    } else {
+        if (bad) flags |= TPL_A2C_STATUS_SEQ;
+        if (atoms > atoms_stride) flags |= TPL_A2C_STATUS_ATOMS;
+    }
+    if (flags) {
+        if (threadIdx.x == 0) report_bits(rep, (uint32_t)flags);
+        n = 0;
+    }
+    const T* xs = coords + 3 * (size_t)b * atoms_stride;
+    const T* gs = grads + 3 * (size_t)b * atoms_stride;
+    T* ga = grad_angles + (size_t)b * 8 * ang_stride;
+    const uint32_t stride = (uint32_t)ang_stride;
+    const int nb = (n + kBlock - 1) / kBlock;
+    double carry[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};  // sums past the blocks at hand
+    bool range = false;
+    for (int hi = nb; hi > 0; hi -= NW) {
+        const int lo = hi > NW ? hi - NW : 0, j = hi - 1 - wave;  // wave 0 takes the last block
+        const int i = kBlock * j + 63 - lane;
+        const bool real = j >= lo;
+        const uint8_t code = real && i < n ? seq[i] : (uint8_t)0;
+        const int t = (int)(int8_t)tb.type[code];
+        const int cnt = t >= 0 ? tb.res_i[t] & 0xff : 0;
+        const int inc = wave_scan_int(cnt);
+        const int total = __builtin_amdgcn_readlane(inc, 63);
+        // this block's first atom, from the later blocks' counts
+        if (lane == 0) s_cnt[wave] = total;
+        __syncthreads();
+        const int here = hi - lo;
+        int a0 = atoms - total;
+        for (int k = 0; k < here; ++k) {
+            if (k < wave) a0 -= s_cnt[k];
+            atoms -= s_cnt[k];
+        }
+        BackResidue<T> r;
+        double after[6], all[6];
+        if (real) {
+            BackFetch<T> f;
+            f.fetch(xs, gs, a0, total, lane);
+            range |= back_block(tb, t, total - inc, cnt, total, a0, xs, gs, f, r, ga, stride, (uint32_t)i, s_x, s_g,
+                                lane);
+#pragma unroll
+            for (int c = 0; c < 6; ++c) after[c] = t >= 0 ? r.sc[c] + r.sa[c] + r.sn[c] : 0.0;
+            lanes_before(after, all);
+            if (lane == 0) {
+#pragma unroll
+                for (int c = 0; c < 6; ++c) s_sum[wave][c] = all[c];
+            }
+        }
+        __syncthreads();
+        double past[6];
+#pragma unroll
+        for (int c = 0; c < 6; ++c) past[c] = carry[c];
+        for (int k = 0; k < here; ++k) {
+#pragma unroll
+            for (int c = 0; c < 6; ++c) {
+                if (k < wave) past[c] += s_sum[k][c];
+                carry[c] += s_sum[k][c];
+            }
+        }
+        if (t >= 0) {
+#pragma unroll
+            for (int c = 0; c < 6; ++c) after[c] += past[c];
+            range |= back_backbone(r, after, ga, stride, (uint32_t)i, (uint32_t)n);
+        }
+        __syncthreads();  // the sums, before the next blocks'
+    }
+    if (range) report_flag(rep, TPLX_A2C_RANGE);
+    // angles past the sequence (and every angle of a flagged structure)
+    for (int row8 = wave; row8 < 8; row8 += NW)
+        for (int i = n + lane; i < ang_stride; i += 64) ga[(uint32_t)row8 * stride + (uint32_t)i] = (T)0;
+}
+
 // Run backward: 512-thread workgroups when some structure may be longer than
 // 256 residues (mixed lengths 30-1000 at B=1024: 155 -> 129 us).
 bool use_large_bwd(int ang_stride) {
     return ang_stride > kThreadsSmall;
-}
-
-// The atom-tile backward where the batch fills the GPU: it moves the atoms
-// with coalesced loads and reads each once, but walks a structure's tiles
-// one after another, so a lone long structure takes longer than with
-// per-thread runs.  Measured (FP32, backward us, runs -> tiles): mixed
-// lengths 30-1000 at B=1024 108 -> 87, 256 x 1000 88 -> 49, 128 x 1000
-// 52 -> 48, 512 x 300 34 -> 25, 1024 x 270 56 -> 47; 64 x 1000 44 -> 47,
-// 128 x 300 17.5 -> 18.9, 32 x 350 17.8 -> 18.9, 1024 x 30 13.7 -> 21.4,
-// 1 x 1000 36 -> 45.
-bool use_tiles(int batch, int ang_stride) {
-    return ang_stride <= kTileMaxRes && (int64_t)batch * ang_stride >= 100000;
 }
 
 // g_tab of the current device, filled on the first forward there: the
@@ -1790,6 +2345,83 @@ int forward_on(int form, const int32_t* order, int dtype, const uint8_t* sequenc
     return hipGetLastError() == hipSuccess ? TPL_A2C_OK : TPL_A2C_ERR_LAUNCH;
 }
 
+// The backward's workspace: the structures' lengths by slot of the batch, the
+// blocks' sums.
+size_t back_recs_bytes(int batch, int angles_stride) {
+    return (size_t)batch * blocks_of(angles_stride) * sizeof(BackRec);
+}
+
+// Dynamic LDS beyond 64 KB has to be allowed per kernel and device, once.
+bool allow_lds(const void* kernel, size_t bytes) {
+    static std::mutex mu;
+    static std::set<std::pair<int, const void*>> allowed;
+    if (bytes <= 60u << 10) return true;
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return false;
+    std::lock_guard<std::mutex> lock(mu);
+    if (allowed.count({dev, kernel})) return true;
+    if (hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) != hipSuccess) return false;
+    allowed.insert({dev, kernel});
+    return true;
+}
+
+// The backward's block kernels where the forward's rule says so, but not for
+// structures of one or two blocks, which one workgroup each handles well however
+// many there are (fused -> blocks, us, float32: lengths 30-1000 at B=1024
+// 80 -> 60, 1024 x 300 53 -> 50, 300 x 600 47 -> 39, 8 x 3000 78 -> 27, 1 x 1000
+// 26 -> 18; not 1024 x 128 17 -> 24, 256 x 1000 36 -> 43, 512 x 300 29 -> 35).
+bool use_back_groups(int batch, int angles_stride) {
+    return blocks_of(angles_stride) > 2 && use_groups(batch, angles_stride);
+}
+
+template <typename T>
+int launch_backward(int form, hipStream_t s, const uint8_t* sequences, int seq_stride, const T* x, const T* g,
+                    int atoms_stride, T* ga, int angles_stride, void* workspace, const Report& rep,
+                    const int32_t* order, int batch) {
+    const int nslot = blocks_of(angles_stride);
+    constexpr size_t per_wave = 2 * back_values<T>() * sizeof(T);
+    if (form == TPLX_A2C_BWD_GROUPS) {
+        int* lens = static_cast<int*>(workspace);
+        BackRec* rec = reinterpret_cast<BackRec*>(static_cast<char*>(workspace) + lens_bytes(batch));
+        const int wgs = (batch * nslot + kWalkWaves - 1) / kWalkWaves, fill = compute_units();
+        const size_t lds = kWalkWaves * per_wave;
+        if (!allow_lds(reinterpret_cast<const void*>(a2c_bwd_walk<T>), lds)) return TPL_A2C_ERR_LAUNCH;
+        hipLaunchKernelGGL((a2c_bwd_sums<T>), dim3((batch * nslot + kSumWaves - 1) / kSumWaves), dim3(64 * kSumWaves),
+                           0, s, sequences, seq_stride, x, g, atoms_stride, lens, rec, ga, angles_stride, rep, order,
+                           batch, nslot);
+        hipLaunchKernelGGL((a2c_bwd_walk<T>), dim3(wgs < fill ? wgs : fill), dim3(64 * kWalkWaves), lds, s, sequences,
+                           seq_stride, x, g, atoms_stride, lens, rec, ga, angles_stride, rep, order, batch, nslot);
+    } else {
+        const int rounds = (nslot + kBackWaves - 1) / kBackWaves, nw = (nslot + rounds - 1) / rounds;
+        if (!allow_lds(reinterpret_cast<const void*>(a2c_bwd_fused<T>), kBackWaves * per_wave))
+            return TPL_A2C_ERR_LAUNCH;
+        hipLaunchKernelGGL((a2c_bwd_fused<T>), dim3(batch), dim3(64 * nw), nw * per_wave, s, sequences, seq_stride, x,
+                           g, atoms_stride, ga, angles_stride, rep, order, batch);
+    }
+    return hipGetLastError() == hipSuccess ? TPL_A2C_OK : TPL_A2C_ERR_LAUNCH;
+}
+
+int backward_on(int form, const int32_t* order, int dtype, const uint8_t* sequences, int seq_stride,
+                const void* coords, const void* grad_coords, int atoms_stride, void* grad_angles, int angles_stride,
+                void* workspace, const Report& rep, int batch, tpl_a2c_stream_t stream) {
+    const int rc = check(dtype, batch, seq_stride, angles_stride, atoms_stride);
+    if (rc != TPL_A2C_OK) return rc;
+    if (batch == 0 || angles_stride == 0) return TPL_A2C_OK;
+    if (!sequences || !grad_angles || (atoms_stride > 0 && (!coords || !grad_coords))) return TPL_A2C_ERR_ARG;
+    const bool groups_fit = workspace && (int64_t)batch * blocks_of(angles_stride) <= INT32_MAX / kBlock;
+    if (form == TPLX_A2C_BWD_AUTO)
+        form = groups_fit && use_back_groups(batch, angles_stride) ? TPLX_A2C_BWD_GROUPS : TPLX_A2C_BWD_FUSED;
+    if (form == TPLX_A2C_BWD_GROUPS && !groups_fit) return TPL_A2C_ERR_ARG;
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    if (dtype == TPL_A2C_F32)
+        return launch_backward<float>(form, s, sequences, seq_stride, static_cast<const float*>(coords),
+                                      static_cast<const float*>(grad_coords), atoms_stride,
+                                      static_cast<float*>(grad_angles), angles_stride, workspace, rep, order, batch);
+    return launch_backward<double>(form, s, sequences, seq_stride, static_cast<const double*>(coords),
+                                   static_cast<const double*>(grad_coords), atoms_stride,
+                                   static_cast<double*>(grad_angles), angles_stride, workspace, rep, order, batch);
+}
+
 }  // namespace
 
 extern "C" {
@@ -1837,6 +2469,18 @@ size_t tplx_a2c_workspace_bytes(int batch, int angles_stride) {
     return lens_bytes(batch) + recs_bytes(batch, angles_stride) + frames_bytes(batch, angles_stride);
 }
 
+size_t tplx_a2c_backward_workspace_bytes(int batch, int angles_stride) {
+    return batch <= 0 ? 0 : lens_bytes(batch) + back_recs_bytes(batch, angles_stride);
+}
+
+int tplx_a2c_backward(int form, const int32_t* order, int dtype, const uint8_t* sequences, int seq_stride,
+                      const void* coords, const void* grad_coords, int atoms_stride, void* grad_angles,
+                      int angles_stride, void* workspace, uint32_t* status, uint32_t* flags, int batch,
+                      tpl_a2c_stream_t stream) {
+    return backward_on(form, order, dtype, sequences, seq_stride, coords, grad_coords, atoms_stride, grad_angles,
+                       angles_stride, workspace, Report{status, flags}, batch, stream);
+}
+
 int tpl_a2c_forward(int dtype, const uint8_t* sequences, int seq_stride, const void* angles,
                     int angles_stride, void* coords, uint8_t* res_names, uint8_t* atom_names,
                     int atoms_stride, uint32_t* status, int batch, tpl_a2c_stream_t stream) {
@@ -1848,6 +2492,9 @@ int tpl_a2c_backward_form(int form, const int32_t* order, int dtype, const uint8
                           const void* coords, const void* grad_coords, int atoms_stride, void* grad_angles,
                           int angles_stride, uint32_t* status, int batch, tpl_a2c_stream_t stream) {
     if (form != TPL_A2C_BWD_AUTO && form != TPL_A2C_BWD_RUNS && form != TPL_A2C_BWD_TILES) return TPL_A2C_ERR_ARG;
+    if (form == TPL_A2C_BWD_AUTO)
+        return backward_on(TPLX_A2C_BWD_AUTO, order, dtype, sequences, seq_stride, coords, grad_coords, atoms_stride,
+                           grad_angles, angles_stride, nullptr, Report{status, nullptr}, batch, stream);
     const int rc = check(dtype, batch, seq_stride, angles_stride, atoms_stride);
     if (rc != TPL_A2C_OK) return rc;
     if (form == TPL_A2C_BWD_TILES && angles_stride > kTileMaxRes) return TPL_A2C_ERR_SIZE;
@@ -1855,7 +2502,6 @@ int tpl_a2c_backward_form(int form, const int32_t* order, int dtype, const uint8
     if (!sequences || !grad_angles || (atoms_stride > 0 && (!coords || !grad_coords)))
         return TPL_A2C_ERR_ARG;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    if (form == TPL_A2C_BWD_AUTO) form = use_tiles(batch, angles_stride) ? TPL_A2C_BWD_TILES : TPL_A2C_BWD_RUNS;
     if (form == TPL_A2C_BWD_TILES) {
         if (dtype == TPL_A2C_F32)
             hipLaunchKernelGGL((a2c_bwd_tiled<float>), dim3(batch), dim3(kTileThreads), 0, s, sequences,

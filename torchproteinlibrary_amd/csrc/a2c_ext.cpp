@@ -124,11 +124,9 @@ int64_t forward_checked(torch::Tensor sequences, torch::Tensor input_angles, tor
     });
 }
 
-// From the forward's coordinates (what the Python layer saves).
-void backward_coords(torch::Tensor grad_atoms, torch::Tensor grad_angles, torch::Tensor sequences,
-                     torch::Tensor coords, c10::optional<torch::Tensor> status,
-                     c10::optional<torch::Tensor> order) {
-    check_common(sequences, grad_angles);
+void backward_on(const torch::Tensor& grad_atoms, const torch::Tensor& grad_angles, const torch::Tensor& sequences,
+                 const torch::Tensor& coords, uint32_t* status, uint32_t* flags,
+                 const c10::optional<torch::Tensor>& order, hipStream_t stream) {
     A2C_CHECK_GPU(grad_atoms);
     A2C_CHECK_GPU(coords);
     const int64_t B = grad_angles.size(0);
@@ -142,12 +140,36 @@ void backward_coords(torch::Tensor grad_atoms, torch::Tensor grad_angles, torch:
                 "gradients and coordinates must be on one device");
     const int64_t A = grad_atoms.size(1) / 3;
     TORCH_CHECK(A <= INT32_MAX / 3, "grad_atoms too large");
-    c10::DeviceGuard guard(grad_angles.device());
-    check_rc(tpl_a2c_backward_form(TPL_A2C_BWD_AUTO, order_ptr(order, grad_angles), dtype_code(grad_angles),
-                                   sequences.data_ptr<uint8_t>(), (int)sequences.size(1), coords.data_ptr(),
-                                   grad_atoms.data_ptr(), (int)A, grad_angles.data_ptr(), (int)grad_angles.size(2),
-                                   status_ptr(status, grad_angles), (int)B, stream_of(grad_angles)),
+    const size_t need = tplx_a2c_backward_workspace_bytes((int)B, (int)grad_angles.size(2));
+    torch::Tensor ws;
+    if (need) ws = torch::empty({(int64_t)need}, grad_angles.options().dtype(torch::kByte));
+    check_rc(tplx_a2c_backward(TPLX_A2C_BWD_AUTO, order_ptr(order, grad_angles), dtype_code(grad_angles),
+                               sequences.data_ptr<uint8_t>(), (int)sequences.size(1), coords.data_ptr(),
+                               grad_atoms.data_ptr(), (int)A, grad_angles.data_ptr(), (int)grad_angles.size(2),
+                               ws.defined() ? ws.data_ptr() : nullptr, status, flags, (int)B, stream),
              "Angles2Coords_backward");
+}
+
+// From the forward's coordinates (what the Python layer saves).
+void backward_coords(torch::Tensor grad_atoms, torch::Tensor grad_angles, torch::Tensor sequences,
+                     torch::Tensor coords, c10::optional<torch::Tensor> status,
+                     c10::optional<torch::Tensor> order) {
+    check_common(sequences, grad_angles);
+    c10::DeviceGuard guard(grad_angles.device());
+    backward_on(grad_atoms, grad_angles, sequences, coords, status_ptr(status, grad_angles), nullptr, order,
+                stream_of(grad_angles));
+}
+
+// As backward_coords without a status; waits for the work and returns its
+// status bits (a2c_flagged.h).
+int64_t backward_checked(torch::Tensor grad_atoms, torch::Tensor grad_angles, torch::Tensor sequences,
+                         torch::Tensor coords, c10::optional<torch::Tensor> order) {
+    check_common(sequences, grad_angles);
+    c10::DeviceGuard guard(grad_angles.device());
+    hipStream_t stream = stream_of(grad_angles);
+    return host_flags::run(stream, [&](uint32_t* flags) {
+        backward_on(grad_atoms, grad_angles, sequences, coords, nullptr, flags, order, stream);
+    });
 }
 
 // The reference's signature (angles, not coordinates): the coordinates are
@@ -199,6 +221,9 @@ std::tuple<double, double, double> bench(std::vector<std::vector<torch::Tensor>>
     hipStream_t stream = stream_of(sets[0][1]);
     const int dt = dtype_code(sets[0][1]);
     const torch::Tensor ws = workspace_for(sets[0][1]);
+    const torch::Tensor bws =
+        torch::empty({(int64_t)tplx_a2c_backward_workspace_bytes((int)sets[0][1].size(0), (int)sets[0][1].size(2)) + 16},
+                     sets[0][1].options().dtype(torch::kByte));
     for (auto& t : sets) TORCH_CHECK(t[1].sizes() == sets[0][1].sizes(), "bench: sets differ in shape");
     auto fwd = [&](std::vector<torch::Tensor>& t) {
         const int32_t* order = t.size() == 6 ? t[5].data_ptr<int32_t>() : nullptr;
@@ -210,9 +235,9 @@ std::tuple<double, double, double> bench(std::vector<std::vector<torch::Tensor>>
     };
     auto bwd = [&](std::vector<torch::Tensor>& t) {
         const int32_t* order = t.size() == 6 ? t[5].data_ptr<int32_t>() : nullptr;
-        check_rc(tpl_a2c_backward_form(TPL_A2C_BWD_AUTO, order, dt, t[0].data_ptr<uint8_t>(), (int)t[0].size(1),
-                                       t[2].data_ptr(), t[3].data_ptr(), (int)(t[3].size(1) / 3), t[4].data_ptr(),
-                                       (int)t[4].size(2), nullptr, (int)t[1].size(0), stream),
+        check_rc(tplx_a2c_backward(TPLX_A2C_BWD_AUTO, order, dt, t[0].data_ptr<uint8_t>(), (int)t[0].size(1),
+                                   t[2].data_ptr(), t[3].data_ptr(), (int)(t[3].size(1) / 3), t[4].data_ptr(),
+                                   (int)t[4].size(2), bws.data_ptr(), nullptr, nullptr, (int)t[1].size(0), stream),
                  "backward");
     };
     hipEvent_t e0, e1;
@@ -254,6 +279,9 @@ void register_a2c(pybind11::module& m) {
     m.def("Angles2Coords_backward_coords", &backward_coords,
           "the same from the forward's coordinates (GPU)", py::arg("grad_atoms"), py::arg("grad_angles"),
           py::arg("sequences"), py::arg("coords"), st, od);
+    m.def("Angles2Coords_backward_checked", &backward_checked, "status bits of the backward, once it has run",
+          py::arg("grad_atoms"), py::arg("grad_angles"), py::arg("sequences"), py::arg("coords"), od,
+          py::call_guard<py::gil_scoped_release>());
     m.def("getSeqNumAtoms", &num_atoms, "atoms of a sequence", py::arg("sequence"));
     m.def("a2c_bench", &bench, "average event ms of Angles2Coords (step, fwd, bwd)");
 }

@@ -15,6 +15,12 @@
 #define TPLX_A2C_FWD_FUSED 1
 #define TPLX_A2C_FWD_GROUPS 2
 
+// Backward kernels, likewise: one workgroup per structure, or the blocks shared
+// over the GPU (needs the workspace).
+#define TPLX_A2C_BWD_AUTO 0
+#define TPLX_A2C_BWD_FUSED 1
+#define TPLX_A2C_BWD_GROUPS 2
+
 extern "C" {
 // Bytes of the workspace (16-byte aligned; 0: none is used).  A call writes
 // what it reads there.
@@ -24,4 +30,11 @@ int tplx_a2c_forward(int form, const int32_t* order, int dtype, const uint8_t* s
                      const void* angles, int angles_stride, void* coords, uint8_t* res_names, uint8_t* atom_names,
                      int atoms_stride, void* workspace, uint32_t* status, uint32_t* flags, int batch,
                      tpl_a2c_stream_t stream);
+
+size_t tplx_a2c_backward_workspace_bytes(int batch, int angles_stride);
+
+int tplx_a2c_backward(int form, const int32_t* order, int dtype, const uint8_t* sequences, int seq_stride,
+                      const void* coords, const void* grad_coords, int atoms_stride, void* grad_angles,
+                      int angles_stride, void* workspace, uint32_t* status, uint32_t* flags, int batch,
+                      tpl_a2c_stream_t stream);
 }
