@@ -1,0 +1,106 @@
+"""The one-kernel step (Angles2BackboneStep with equal chunk sizes in both
+directions) against the float64 host path, at the sizes where it can go wrong:
+empty and one-residue chains, chunk edges (64 R), chains of 1 to 8 chunks,
+batches that fit on the GPU at once and batches packed by length, strides with
+every alignment and padding past the chains.  Several runs on changed inputs,
+under a capture too."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _case(B, L, lens, dtype, seed):
+    rng = np.random.default_rng(seed)
+    a = torch.from_numpy(rng.uniform(-np.pi, np.pi, (B, 3, L)))
+    a[:, 2] = np.pi + 0.05 * a[:, 2]  # omega
+    a = a.to(dtype).cuda()
+    g = torch.from_numpy(rng.standard_normal((B, 9 * L))).to(dtype).cuda()
+    return a, torch.tensor(lens, dtype=torch.int32, device="cuda"), g
+
+
+def _oracle(a, lens, g):
+    from torchproteinlibrary_amd import ReducedModel
+    ac = a.double().cpu().requires_grad_()
+    c = ReducedModel.Angles2Backbone()(ac, lens.cpu())
+    # the step's gradients past the chain are not used
+    c.backward(g.double().cpu())
+    return c.detach(), ac.grad
+
+
+def _check(step, a, lens, g, dtype):
+    c, ga = _oracle(a, lens, g)
+    L = a.size(2)
+    nmax = max(1, int(lens.max()))
+    eps = torch.finfo(dtype).eps
+    # The frames are FP64; positions reach 3.8 A a residue, rounded once to the
+    # dtype.  The step and the oracle differ by their order of products: 3 n
+    # steps of a few units of 2^-53 each, on coordinates and on a gradient that
+    # sums 3 n torques of up to 3.8 n times |g| < 6.
+    acc = 64 * 3 * nmax * 2.0 ** -53
+    tol_c = 3.8 * nmax * (eps + acc)
+    scale = ga.abs().amax(dim=(1, 2), keepdim=True)
+    tol_g = scale * eps + 3 * nmax * 3.8 * nmax * 6 * acc
+    assert (step.coords.double().cpu() - c).abs().max() <= tol_c
+    assert ((step.grad_angles.double().cpu() - ga).abs() <= tol_g).all()
+    for b, n in enumerate(lens.tolist()):
+        assert not step.coords[b, 9 * n:].any()
+        assert not step.grad_angles[b, :, n:].any()
+
+
+def _lengths(B, L, kind, C, rng):
+    if kind == "equal":
+        return [L] * B
+    edges = [0, 1, 2, C - 1, C, C + 1, 2 * C - 1, 2 * C, 2 * C + 1, 3 * C, 4 * C, 4 * C + 1, L - 1, L]
+    lens = [min(e, L) for e in edges]
+    lens += [int(v) for v in np.exp(rng.uniform(np.log(2), np.log(L), max(0, B - len(lens))))]
+    rng.shuffle(lens)
+    return lens[:B]
+
+
+@pytest.mark.parametrize("dtype,R", [(torch.float32, 1), (torch.float32, 2), (torch.float32, 4),
+                                     (torch.float64, 1), (torch.float64, 2)])
+@pytest.mark.parametrize("B,L,kind", [
+    (1, 1, "equal"), (3, 5, "equal"), (2, 127, "equal"), (2, 129, "equal"), (5, 512, "equal"),
+    (17, 515, "mixed"), (14, 1023, "mixed"), (16, 1024, "mixed"), (18, 2048, "mixed"), (600, 333, "mixed"), (1100, 770, "mixed"),
+    (1537, 514, "mixed"), (2050, 101, "mixed"), (4095, 259, "mixed"),
+])
+def test_step_matches_oracle(dtype, R, B, L, kind):
+    from torchproteinlibrary_amd.ReducedModel.Angles2Backbone.Angles2Backbone import Angles2BackboneStep
+    rng = np.random.default_rng(B * 10007 + L)
+    lens = _lengths(B, L, kind, 64 * R, rng)
+    a, ln, g = _case(B, L, lens, dtype, B + L)
+    step = Angles2BackboneStep(a, ln, config=(R, R))
+    step.coords.fill_(float("nan"))
+    step.grad_angles.fill_(float("nan"))
+    step.grad_coords.copy_(g)
+    step.replay()
+    _check(step, a, ln, g, dtype)
+    # new angles and lengths in the same memory
+    a.copy_(a.flip(0))
+    ln.copy_(ln.flip(0))
+    step.replay()
+    _check(step, a, ln, g, dtype)
+
+
+@pytest.mark.parametrize("B", [5, 1500])
+def test_step_under_capture(B):
+    from torchproteinlibrary_amd.ReducedModel.Angles2Backbone.Angles2Backbone import Angles2BackboneStep
+    L = 300
+    a, ln, g = _case(B, L, _lengths(B, L, "mixed", 128, np.random.default_rng(1)), torch.float32, 1)
+    step = Angles2BackboneStep(a, ln, config=(2, 2))
+    step.grad_coords.copy_(g)
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        step.replay()
+    for _ in range(3):
+        a.copy_(a.flip(0))
+        step.coords.zero_()
+        step.grad_angles.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        got = step.coords.clone(), step.grad_angles.clone()
+        step.replay()
+        assert torch.equal(got[0], step.coords) and torch.equal(got[1], step.grad_angles)

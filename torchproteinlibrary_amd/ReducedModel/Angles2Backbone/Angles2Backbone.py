@@ -276,17 +276,22 @@ class Angles2Backbone(Module):
 
 
 class Angles2BackboneStep:
-    """Angles2Backbone forward and backward for fixed shapes, captured once
-    into one HIP graph and replayed.
+    """Angles2Backbone forward and backward for fixed shapes, laid out once
+    and replayed.
 
     For loops that run the same shapes many times (fitting, serving): one
     ``replay()`` runs the forward (``angles`` -> ``coords``) and the backward
     (``grad_coords`` -> ``grad_angles``) on the current stream, with nothing
-    allocated, no host synchronisation and one launch per step.  The graph
-    reads ``angles``, ``angles_length`` and ``grad_coords`` from their memory
-    at every replay, so a loop updates them in place between replays; it
-    writes ``coords`` and ``grad_angles``.  The chunk sizes are the tuned ones
-    for these inputs, or ``config`` (forward, backward residues per lane).
+    allocated, no host synchronisation and one launch per step, or two: chains
+    of at most 8 chunks run in one kernel when both directions have the same
+    chunk size (in float64 always), other shapes in the layer's two.  In one
+    kernel the coordinates are those the gradients are computed from, rounded
+    once from float64; they can differ from the layer's in the last digits.
+    A step reads ``angles``, ``angles_length`` and ``grad_coords`` from their
+    memory at every replay, so a loop updates them in place between replays;
+    it writes ``coords`` and ``grad_angles``.  A replay under a capture is
+    captured.  The chunk sizes are the tuned ones for these inputs, or
+    ``config`` (forward, backward residues per lane).
 
     Replays do not check for NaN or out-of-range lengths (the checks of the
     layer read a status word on the host); lengths must stay within
@@ -314,9 +319,9 @@ class Angles2BackboneStep:
         st_bytes, sy_bytes = ext.workspace_bytes(dt == torch.float64, B, L, list(cfg))
         self._state = _empty_bytes(max(int(st_bytes), 256), dev)
         self._sync = torch.zeros(max(int(sy_bytes), 256), dtype=torch.uint8, device=dev)
-        self._graph = ext.StepGraph(angles, angles_length, self.grad_coords, self.coords,
-                                    self.grad_angles, self._state, self._sync, list(cfg))
+        self._step = ext.Step(angles, angles_length, self.grad_coords, self.coords,
+                              self.grad_angles, self._state, self._sync, list(cfg))
 
     def replay(self):
         """Runs one forward+backward step on the current stream."""
-        self._graph.replay()
+        self._step.run()

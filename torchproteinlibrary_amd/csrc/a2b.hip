@@ -42,6 +42,7 @@
 #include <cstdint>
 #include <cstring>
 #include <map>
+#include <set>
 #include <mutex>
 #include <tuple>
 #include <vector>
@@ -1015,7 +1016,7 @@ __global__ void __launch_bounds__(64 * W) a2b_fwd_chain(ChunkArgs a) {
     const int raw = a.lengths[b];
     const int n = raw < 0 ? 0 : (raw > L ? L : raw);
     const int nreal = (n + C - 1) / C;
-    const int c = (wave + b) % W;  // this wave's chunk slot
+    const int c = (wave + (b >> 3) + (b >> 8)) % W;  // this wave's chunk slot
     const bool real = c < nreal;
     if (raw != n && threadIdx.x == 0) report_bits(a.rep, TPL_A2B_STATUS_LENGTH);
     for (int i = (int)threadIdx.x; i < 128; i += 64 * W) s_tab[i] = kTabCS[i];
@@ -1390,7 +1391,7 @@ __global__ void __launch_bounds__(64 * W) a2b_bwd_chain(ChunkArgs a) {
     const int raw = a.lengths[b];
     const int n = raw < 0 ? 0 : (raw > L ? L : raw);
     const int nreal = (n + C - 1) / C;
-    const int c = (wave + b) % W;  // this wave's chunk slot
+    const int c = (wave + (b >> 3) + (b >> 8)) % W;  // this wave's chunk slot
     const bool real = c < nreal;
     if (raw != n && threadIdx.x == 0) report_bits(a.rep, TPL_A2B_STATUS_LENGTH);
     for (int i = (int)threadIdx.x; i < 128; i += 64 * W) s_tab[i] = kTabCS[i];
@@ -1556,6 +1557,411 @@ __global__ void __launch_bounds__(64 * W) a2b_bwd_chain(ChunkArgs a) {
             for (int k = 0; k < 3; ++k) lane_store_zero<T, R>(grow + (size_t)k * L + rl, crow);
         }
     }
+}
+
+// ------------------------------------------------------------------- step
+// Forward and backward of chains of at most W chunks in one kernel, for callers
+// that have the coordinate gradients beforehand (tplx_a2b_step): the angles are
+// loaded, their sincos taken and the lane frames scanned once for both, no
+// checkpoints go through memory, and the coordinates are the positions that
+// pass B steps through anyway (from E in FP64, where the forward rounds the
+// lane's own positions to FP32 in between).  One workgroup of W waves takes
+// W waves' worth of chunks; what its chunks of one chain need of each other
+// meets in LDS, the frames across one barrier and the sums across a second.
+//
+// BINS: a chain of nreal chunks takes a slot of nreal waves rounded up to a
+// power of two, and the workgroups take W / slot chains of one slot size each,
+// the longest chains first; with mixed lengths nearly every wave has a chunk
+// (B=1024 of lengths 30..1000, W = 4: 455 workgroups of work instead of 1024).
+// Each workgroup finds its chains from the lengths.  Without BINS workgroup b
+// takes chain b (fewer chains than fit on the GPU).
+//
+// A lane's LDS: its (cos, sin) pairs element-major as in the backward, and, in
+// the same memory as they are used up, its coordinates value-major at a stride
+// of 65 values (so that neither the lanes' writes nor the transposing reads
+// meet in a bank): the wave's run starts kStepLead values before the pairs, and
+// at step s, which has used pairs 0..s, atom s + 1 ends at 195 (s + 2) values.
+//
+// What bounds it: the two passes of FP64 frame products (some 2700 vector
+// instructions a wave at R = 4, two waves to a SIMD) where all chains fit at
+// once, and with padding the stores.  Forward and backward against the two
+// kernels (run to run within 0.2 us), launches back to back:
+//   B = 256, L = 700, float32, (4,4):                 16.4 -> 10.4 us
+//   B = 32,  L = 200, float32, (1,1):                  9.6 ->  6.2
+//   B = 512, L = 500, lengths 50..500, float32, (2,2): 18.3 -> 10.5
+//   B = 1024, L = 1000, lengths 30..1000, float32, (4,4): 31.0 -> 19.1
+//   the same in float64, (4,2):                       43.3 -> 29.0
+// Each workgroup writing the zeros of its own chains took 22.0 us in the fourth
+// (the short chains' workgroups have nearly all of them) and 33.6 in the fifth.
+template <typename T, int R>
+constexpr int step_lead_doubles() {
+    // f32: 195 (s + 2) <= lead + 256 (s + 1) and 195 <= lead: lead = 196 values.
+    // f64: 195 (s + 2) <= lead + 128 (s + 1) up to s = 3R - 2.
+    return sizeof(T) == 4 ? 98 : 195 * 3 * R - 128 * (3 * R - 1);
+}
+template <typename T, int R>
+constexpr int step_wave_doubles() {
+    return step_lead_doubles<T, R>() + 6 * R * 64;
+}
+constexpr int kStepStride = 65;
+constexpr int kStepMaxBatch = 4096;  // BINS: every workgroup reads all lengths
+
+// The wave's chunk run dst[0, count) from its value-major coordinates: elements
+// at or past nsrc are 0.  Element p is value p % N of lane p / N.
+template <typename T, int N>
+__device__ __forceinline__ void store_transposed(T* dst, int count, int nsrc, const T* s_v, int lane) {
+    constexpr int V = 16 / (int)sizeof(T);
+    const auto value = [&](int p) {
+        const int l = p / N, v = p - l * N;
+        return p < nsrc ? s_v[v * kStepStride + l] : (T)0;
+    };
+    const int mis = (int)((reinterpret_cast<uintptr_t>(dst) / sizeof(T)) % V);
+    const int head = min((V - mis) % V, count);
+    const int nvec = (count - head) / V;
+    const int tail0 = head + nvec * V;
+    if (lane < head) dst[lane] = value(lane);
+    for (int k = lane; k < nvec; k += 64) {
+        const int p0 = head + k * V;
+        T w[V];
+        if (N % V == 0 && head == 0) {  // uniform: the run lies in one lane
+            const int l = p0 / N, v = p0 - l * N;
+#pragma unroll
+            for (int e = 0; e < V; ++e) w[e] = p0 + e < nsrc ? s_v[(v + e) * kStepStride + l] : (T)0;
+        } else {
+#pragma unroll
+            for (int e = 0; e < V; ++e) w[e] = value(p0 + e);
+        }
+        u32x4 u;
+        __builtin_memcpy(&u, w, sizeof(u));
+        __builtin_nontemporal_store(u, reinterpret_cast<u32x4*>(dst + p0));
+    }
+    if (tail0 + lane < count) dst[tail0 + lane] = value(tail0 + lane);
+}
+
+// Share f of F of the zeros of dst[0, count), by one wave.
+template <typename T>
+__device__ __forceinline__ void store_zeros(T* dst, int count, int f, int F, int lane) {
+    constexpr int V = 16 / (int)sizeof(T);
+    const int mis = (int)((reinterpret_cast<uintptr_t>(dst) / sizeof(T)) % V);
+    const int head = min((V - mis) % V, count);
+    const int nvec = (count - head) / V;
+    const int tail0 = head + nvec * V;
+    const u32x4 z = {0u, 0u, 0u, 0u};
+    for (int k = 64 * f + lane; k < nvec; k += 64 * F) __builtin_nontemporal_store(z, reinterpret_cast<u32x4*>(dst + head) + k);
+    if (f == 0) {
+        if (lane < head) dst[lane] = (T)0;
+        if (tail0 + lane < count) dst[tail0 + lane] = (T)0;
+    }
+}
+
+__device__ __forceinline__ int wave_scan_int(int v) {
+    v += __builtin_amdgcn_update_dpp(0, v, kRowShr1, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, kRowShr2, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, kRowShr4, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, kRowShr8, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, kRowBcast15, 0xa, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, kRowBcast31, 0xc, 0xf, false);
+    return v;
+}
+
+// The chains of this workgroup: s_chain[q], q < W / size, or -1; returns the
+// slot size (0: the workgroup has none).  Slot sizes are 2^k, k < 4; counts of
+// the four travel packed, 16 bits each, two to an int.
+template <int R, int W>
+__device__ __forceinline__ int find_chains(const ChunkArgs& a, int* s_chain, int (*s_count)[2], int& nwg) {
+    constexpr int C = 64 * R, NT = 64 * W;
+    const int tid = (int)threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int per = (a.B + NT - 1) / NT, b0 = tid * per;  // per <= 16
+    uint32_t logs = 0;  // of the thread's chains: log2 of the slot size, 2 bits each
+    int c[2] = {0, 0};
+    for (int e0 = 0; e0 < per; e0 += 4) {
+        int raw[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) raw[e] = e0 + e < per && b0 + e0 + e < a.B ? a.lengths[b0 + e0 + e] : -1;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int n = min(max(raw[e], 0), a.L);
+            const int k = (n > C) + (n > 2 * C) + (n > 4 * C);
+            if (e0 + e < per && b0 + e0 + e < a.B) {
+                logs |= (uint32_t)k << (2 * (e0 + e));
+                c[k >> 1] += 1 << (16 * (k & 1));
+            }
+        }
+    }
+    const int i0 = wave_scan_int(c[0]), i1 = wave_scan_int(c[1]);
+    if (lane == 63) {
+        s_count[wave][0] = i0;
+        s_count[wave][1] = i1;
+    }
+    if (tid < W) s_chain[tid] = -1;
+    __syncthreads();
+    int before[2] = {i0 - c[0], i1 - c[1]}, total[2] = {0, 0};
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            if (w < wave) before[h] += s_count[w][h];
+            total[h] += s_count[w][h];
+        }
+    }
+    int g = (int)blockIdx.x, size = 0, mine = -1;
+    nwg = 0;
+#pragma unroll
+    for (int k = 3; k >= 0; --k) {
+        const int n = (total[k >> 1] >> (16 * (k & 1))) & 0xffff, per_wg = W >> k;
+        const int wgs = per_wg > 0 ? (n + per_wg - 1) / per_wg : 0;
+        nwg += wgs;
+        if (size == 0) {
+            if (g < wgs) {
+                size = 1 << k;
+                mine = k;
+            } else {
+                g -= wgs;
+            }
+        }
+    }
+    if (size > 0) {
+        const int per_wg = W / size, r0 = g * per_wg;
+        int r = (before[mine >> 1] >> (16 * (mine & 1))) & 0xffff;
+        for (int e = 0; e < per && r < r0 + per_wg; ++e)
+            if (b0 + e < a.B && (int)(logs >> (2 * e) & 3u) == mine) {
+                if (r >= r0) s_chain[r - r0] = b0 + e;
+                ++r;
+            }
+    }
+    __syncthreads();
+    return size;
+}
+
+__device__ __forceinline__ int chunks_of(int n, int C) { return (n + C - 1) / C; }
+
+template <typename T, int R, int W, bool BINS>
+__global__ void __launch_bounds__(64 * W) a2b_step(ChunkArgs a) {
+    constexpr int C = 64 * R;
+    extern __shared__ double s_dynd[];  // [W][step_wave_doubles]
+    __shared__ double s_tab[128];
+    __shared__ double s_agg[W][kF];
+    __shared__ double s_tot[W][6];
+    __shared__ int s_chain[W];
+    __shared__ int s_count[W][2];
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = (int)(threadIdx.x & 63);
+    const int L = a.L;
+    for (int i = (int)threadIdx.x; i < 128; i += 64 * W) s_tab[i] = kTabCS[i];
+    int nwg = 0;
+    int b, c, size, first = 0;  // the chain, this wave's chunk of it, its slot: waves first .. first + size - 1
+    if (BINS) {
+        size = find_chains<R, W>(a, s_chain, s_count, nwg);
+        if (size == 0) return;
+        b = __builtin_amdgcn_readfirstlane(s_chain[wave / size]);
+        first = wave / size * size;
+        c = wave - first;
+    } else {
+        b = (int)blockIdx.x;
+        size = W;
+        // rotated as the workgroups come round to a CU (8 XCDs of 32 CUs)
+        c = (int)((uint32_t)(wave + (b >> 3) + (b >> 8)) % W);
+    }
+    int n = 0;
+    if (b >= 0) {
+        const int raw = a.lengths[b];
+        n = raw < 0 ? 0 : (raw > L ? L : raw);
+    }
+    const int nreal = (n + C - 1) / C;
+    const bool real = b >= 0 && c < nreal;
+    double* s_wave = s_dynd + (size_t)wave * step_wave_doubles<T, R>();
+    double* s_cs = s_wave + step_lead_doubles<T, R>();
+    T* s_v = reinterpret_cast<T*>(s_wave);
+    const size_t row = b >= 0 ? (size_t)b : 0;
+    T* grow = static_cast<T*>(a.grad_angles) + row * 3 * L;
+    T* xrow = static_cast<T*>(a.coords) + row * 9 * L;
+    const T* arow = static_cast<const T*>(a.angles) + row * 3 * L;
+    const T* gin = static_cast<const T*>(a.grad) + row * 9 * L;
+    const int r0 = c * C;
+    const int rl = r0 + lane * R;
+    const int cnt = min(max(n - rl, 0), R);
+    T ang[3][R];
+    T gr[9 * R];
+    if (real) {
+        if (cnt > 0) {  // a lane wholly past the chain reads nothing
+            lane_load_rows<T, R>(arow + rl, L, cnt, L - rl, ang);
+            lane_load<T, 9 * R>(gin + (size_t)9 * rl, 9 * cnt, gr, 9 * (L - rl));
+        } else {
+#pragma unroll
+            for (int kk = 0; kk < 3; ++kk)
+#pragma unroll
+                for (int i = 0; i < R; ++i) ang[kk][i] = (T)0;
+#pragma unroll
+            for (int i = 0; i < 9 * R; ++i) gr[i] = (T)0;
+        }
+    }
+    if (!BINS) __syncthreads();  // s_tab (find_chains ends with a barrier)
+
+    double f[kF], W6[6], S[6];
+    double M[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+    double F[3] = {0, 0, 0};
+    if (real) {
+        // Pass 1 in the lane's own frame.
+        frame_identity(f);
+        F[0] = (double)gr[0];
+        F[1] = (double)gr[1];
+        F[2] = (double)gr[2];
+#pragma unroll
+        for (int q = 0; q < R; ++q) {
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                double sn, cs;
+                sincos_tab((double)ang[k][q], s_tab, &sn, &cs);
+                s_cs[(6 * q + 2 * k) * 64 + lane] = cs;
+                s_cs[(6 * q + 2 * k + 1) * 64 + lane] = sn;
+                if (k == 0) frame_step<0>(f, cs, sn);
+                if (k == 1) frame_step<1>(f, cs, sn);
+                if (k == 2) frame_step<2>(f, cs, sn);
+                const int at = 3 * q + k + 1;
+                if (at < 3 * R) {
+                    const double g0 = (double)gr[3 * at], g1 = (double)gr[3 * at + 1],
+                                 g2 = (double)gr[3 * at + 2];
+#pragma unroll
+                    for (int m = 0; m < 3; ++m) {
+                        M[3 * m] = fma(f[9 + m], g0, M[3 * m]);
+                        M[3 * m + 1] = fma(f[9 + m], g1, M[3 * m + 1]);
+                        M[3 * m + 2] = fma(f[9 + m], g2, M[3 * m + 2]);
+                    }
+                    F[0] += g0;
+                    F[1] += g1;
+                    F[2] += g2;
+                }
+            }
+        }
+        wave_scan_frames(f);
+        if (lane == 63) {
+#pragma unroll
+            for (int e = 0; e < kF; ++e) s_agg[first + c][e] = f[e];
+        }
+        wave_shift_frames(f);
+    }
+    // The zeros past the chains' chunks: nothing is loaded from here on, so the
+    // stores drain behind the rest.
+    const auto zeros = [&](int zb, int f, int F) {
+        const int raw = a.lengths[zb];
+        const int p = min(chunks_of(raw < 0 ? 0 : (raw > L ? L : raw), C) * C, L);
+        store_zeros<T>(static_cast<T*>(a.coords) + (size_t)9 * zb * L + (size_t)9 * p, 9 * (L - p), f, F, lane);
+#pragma unroll
+        for (int k = 0; k < 3; ++k)
+            store_zeros<T>(static_cast<T*>(a.grad_angles) + ((size_t)3 * zb + k) * L + p, L - p, f, F, lane);
+    };
+    if (BINS) {
+        for (int u = (int)blockIdx.x * W + wave; u < 4 * a.B; u += nwg * W) zeros(u >> 2, u & 3, 4);
+    } else {
+        zeros(b, c, W);
+    }
+    __syncthreads();  // the aggregates
+    if (real) {
+        if (c > 0) {
+            double P[kF], Q[kF];
+#pragma unroll
+            for (int e = 0; e < kF; ++e) P[e] = s_agg[first][e];
+            for (int j = 1; j < c; ++j) {
+                frame_rmul_to(P, s_agg[first + j], Q);
+#pragma unroll
+                for (int e = 0; e < kF; ++e) P[e] = Q[e];
+            }
+            frame_lmul(P, f);
+        }  // f = E, the frame of the lane's first atom
+        auto rm = [&](int j, int k) {
+            return f[j] * M[k] + f[3 + j] * M[3 + k] + f[6 + j] * M[6 + k];
+        };
+        W6[0] = rm(1, 2) - rm(2, 1) + (f[10] * F[2] - f[11] * F[1]);
+        W6[1] = rm(2, 0) - rm(0, 2) + (f[11] * F[0] - f[9] * F[2]);
+        W6[2] = rm(0, 1) - rm(1, 0) + (f[9] * F[1] - f[10] * F[0]);
+        W6[3] = F[0];
+        W6[4] = F[1];
+        W6[5] = F[2];
+#pragma unroll
+        for (int e = 0; e < 6; ++e) S[e] = W6[e];
+        wave_scan_sum<6>(S);  // inclusive prefix over lanes
+        double tot[6];
+#pragma unroll
+        for (int e = 0; e < 6; ++e) {
+            tot[e] = read_lane(S[e], 63);
+            S[e] = tot[e] - S[e];
+        }
+        if (lane == 0) {
+#pragma unroll
+            for (int e = 0; e < 6; ++e) s_tot[first + c][e] = tot[e];
+        }
+    }
+    __syncthreads();  // the chunks' sums
+    if (!real) return;
+    for (int j = c + 1; j < nreal; ++j) {
+#pragma unroll
+        for (int e = 0; e < 6; ++e) S[e] += s_tot[first + j][e];
+    }
+    const int crow = min(max(L - rl, 0), R);
+    if (cnt > 0) {
+        // S becomes the suffix from the lane's atom 1: add the lane's own
+        // atoms, drop atom 0.
+        {
+            const double g0 = (double)gr[0], g1 = (double)gr[1], g2 = (double)gr[2];
+            S[0] += W6[0] - (f[10] * g2 - f[11] * g1);
+            S[1] += W6[1] - (f[11] * g0 - f[9] * g2);
+            S[2] += W6[2] - (f[9] * g1 - f[10] * g0);
+            S[3] += W6[3] - g0;
+            S[4] += W6[4] - g1;
+            S[5] += W6[5] - g2;
+        }
+        // The fence keeps the stores behind the loads of the pairs that other
+        // lanes had in their place (to one lane the two never look the same);
+        // the wave's LDS instructions run in order, so it costs nothing.
+        auto keep = [&](int at) {
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+            for (int m = 0; m < 3; ++m) s_v[(3 * at + m) * kStepStride + lane] = (T)f[9 + m];
+        };
+        double nc = s_cs[lane], ns = s_cs[64 + lane];  // the next pair, loaded a step ahead
+        keep(0);
+        T out[3][R];
+#pragma unroll
+        for (int q = 0; q < R; ++q) {
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                const double cs = nc, sn = ns;
+                if (3 * q + k + 1 < 3 * R) {
+                    nc = s_cs[(6 * q + 2 * k + 2) * 64 + lane];
+                    ns = s_cs[(6 * q + 2 * k + 3) * 64 + lane];
+                }
+                if (k == 0) frame_step<0>(f, cs, sn);
+                if (k == 1) frame_step<1>(f, cs, sn);
+                if (k == 2) frame_step<2>(f, cs, sn);
+                const int j = 3 * q + k + 1;
+                const double x0 = f[9], x1 = f[10], x2 = f[11];
+                const double v = f[0] * (S[0] - (x1 * S[5] - x2 * S[4])) +
+                                 f[1] * (S[1] - (x2 * S[3] - x0 * S[5])) +
+                                 f[2] * (S[2] - (x0 * S[4] - x1 * S[3]));
+                const int r = rl + q;
+                const bool zero = (r >= n) || (r == n - 1 && k > 0);
+                out[k][q] = zero ? (T)0 : (T)v;
+                if (j < 3 * R) {
+                    keep(j);
+                    const double g0 = (double)gr[3 * j], g1 = (double)gr[3 * j + 1],
+                                 g2 = (double)gr[3 * j + 2];
+                    S[0] -= x1 * g2 - x2 * g1;
+                    S[1] -= x2 * g0 - x0 * g2;
+                    S[2] -= x0 * g1 - x1 * g0;
+                    S[3] -= g0;
+                    S[4] -= g1;
+                    S[5] -= g2;
+                }
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < 3; ++k) lane_store<T, R>(grow + (size_t)k * L + rl, crow, out[k]);
+    } else if (crow > 0) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) lane_store_zero<T, R>(grow + (size_t)k * L + rl, crow);
+    }
+    wave_lds_sync();
+    const int g0 = 9 * r0, wcount = min(9 * C, 9 * L - g0);
+    store_transposed<T, 9 * R>(xrow + g0, wcount, min(max(9 * n - g0, 0), wcount), s_v, lane);
 }
 
 __global__ void a2b_zero_words(uint32_t* p, size_t n) {
@@ -1944,6 +2350,68 @@ int launch_chain(KernelFn k, const ChunkArgs& a, size_t lds, hipStream_t stream)
     return hipGetLastError() == hipSuccess ? TPL_A2B_OK : TPL_A2B_ERR_LAUNCH;
 }
 
+// The step kernel: R residues per lane, W waves per workgroup (4, or 8 where
+// the chains need it).
+template <typename T, int R>
+KernelFn step_kernel_w(int w, bool bins) {
+    if (w <= 4) return bins ? a2b_step<T, R, 4, true> : a2b_step<T, R, 4, false>;
+    if constexpr (R == 1)
+        return nullptr;  // step_form
+    else
+        return bins ? a2b_step<T, R, 8, true> : a2b_step<T, R, 8, false>;
+}
+template <typename T, int R>
+size_t step_lds(int w) {
+    return (size_t)(w <= 4 ? 4 : 8) * step_wave_doubles<T, R>() * sizeof(double);
+}
+struct StepForm {
+    KernelFn kernel;
+    int waves;
+    size_t lds;
+    bool bins;
+};
+
+// Dynamic LDS beyond 64 KB has to be allowed per kernel and device, once.
+bool allow_lds(KernelFn k, size_t bytes) {
+    static std::mutex mu;
+    static std::set<std::pair<int, const void*>> allowed;
+    if (bytes <= 60u << 10) return true;
+    int dev = -1;
+    const void* p = reinterpret_cast<const void*>(k);
+    if (hipGetDevice(&dev) != hipSuccess) return false;
+    std::lock_guard<std::mutex> lock(mu);
+    if (allowed.count({dev, p})) return true;
+    if (hipFuncSetAttribute(p, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) != hipSuccess) return false;
+    allowed.insert({dev, p});
+    return true;
+}
+
+// The form for a shape with R residues per lane; false where the chains have
+// more chunks than a workgroup has waves (8; with one residue per lane 4: 8
+// waves of so little work each spend it at the barriers, 13.3 us for B = 512,
+// L = 500 against 10.5 with two residues per lane), or the batch does not fit
+// at once and is too large for its lengths to be read by every workgroup.
+bool step_form(int dtype, int B, int L, int R, StepForm& s) {
+    const int nc = chunks(L, 64 * R);
+    if (nc > (R == 1 ? 4 : 8)) return false;
+    s.waves = nc <= 4 ? 4 : 8;
+    for (int bins = 0; bins < 2; ++bins) {
+        s.bins = bins;
+        if (dtype == TPL_A2B_F32) {
+            s.kernel = R == 1   ? step_kernel_w<float, 1>(s.waves, bins)
+                       : R == 2 ? step_kernel_w<float, 2>(s.waves, bins)
+                                : step_kernel_w<float, 4>(s.waves, bins);
+            s.lds = R == 1 ? step_lds<float, 1>(s.waves) : R == 2 ? step_lds<float, 2>(s.waves) : step_lds<float, 4>(s.waves);
+        } else {
+            s.kernel = R == 1 ? step_kernel_w<double, 1>(s.waves, bins) : step_kernel_w<double, 2>(s.waves, bins);
+            s.lds = R == 1 ? step_lds<double, 1>(s.waves) : step_lds<double, 2>(s.waves);
+        }
+        if (!allow_lds(s.kernel, s.lds)) return false;
+        if (!bins && B <= resident_workgroups(s.kernel, 64 * s.waves, s.lds)) return true;
+    }
+    return B <= kStepMaxBatch;
+}
+
 // The two directions, reporting as `rep` says.
 int forward_on(int dtype, const void* angles, void* coords, const int32_t* lengths,
                     void* state, void* sync, const Report& rep, int batch, int angles_stride,
@@ -2085,6 +2553,35 @@ int tplx_a2b_backward(int dtype, void* grad_angles, const void* grad_coords, con
                       int angles_stride, const tpl_a2b_config* cfg, tpl_stream_t stream) {
     return backward_on(dtype, grad_angles, grad_coords, angles, lengths, state, sync, Report{nullptr, flags},
                        batch, angles_stride, cfg, stream);
+}
+
+int tplx_a2b_step_fits(int dtype, int batch, int angles_stride, const tpl_a2b_config* cfg) {
+    if (check_common(dtype, batch, angles_stride) || !valid_config(cfg) || !fits_dtype(dtype, cfg)) return 0;
+    if (dtype == TPL_A2B_F32 && cfg->fwd_res_per_lane != cfg->bwd_res_per_lane) return 0;
+    if (batch == 0 || angles_stride == 0) return 0;
+    StepForm form;
+    return step_form(dtype, batch, angles_stride, cfg->bwd_res_per_lane, form) ? 1 : 0;
+}
+
+int tplx_a2b_step(int dtype, const void* angles, const int32_t* lengths, const void* grad_coords, void* coords,
+                  void* grad_angles, int batch, int angles_stride, const tpl_a2b_config* cfg, tpl_stream_t stream) {
+    int rc = check_common(dtype, batch, angles_stride);
+    if (rc) return rc;
+    if (!valid_config(cfg) || !fits_dtype(dtype, cfg)) return TPL_A2B_ERR_CONFIG;
+    if (batch == 0 || angles_stride == 0) return TPL_A2B_OK;
+    if (!angles || !lengths || !grad_coords || !coords || !grad_angles) return TPL_A2B_ERR_ARG;
+    StepForm form;
+    const int R = cfg->bwd_res_per_lane;
+    if (!step_form(dtype, batch, angles_stride, R, form)) return TPL_A2B_ERR_CONFIG;
+    ChunkArgs a = base_args(batch, angles_stride, 64 * R, cfg);
+    a.angles = angles;
+    a.lengths = lengths;
+    a.grad = grad_coords;
+    a.coords = coords;
+    a.grad_angles = grad_angles;
+    hipLaunchKernelGGL(form.kernel, dim3((unsigned)batch), dim3(64 * form.waves), form.lds,
+                       static_cast<hipStream_t>(stream), a);
+    return hipGetLastError() == hipSuccess ? TPL_A2B_OK : TPL_A2B_ERR_LAUNCH;
 }
 
 size_t tpl_a2b_noalloc_max_bytes(void) { return kScratchBytes; }

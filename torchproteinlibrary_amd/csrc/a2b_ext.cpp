@@ -480,76 +480,67 @@ std::tuple<double, double, int64_t> bench_graph(std::vector<std::vector<torch::T
     return {(double)ms, std::chrono::duration<double, std::milli>(t1 - t0).count(), reps * per};
 }
 
-// One forward+backward step over fixed buffers, captured once into a HIP
-// graph (on a private stream, thread-local capture mode) and replayed on the
-// current stream.  Each replay reads angles, lengths and grad_output from
-// their memory and writes output_coords and grad_input; the look-back words
-// (sync) must be zero before the first replay, and every replay leaves them
-// zero.  The tensors are held for the graph's lifetime.
-class StepGraph {
+// One forward+backward step over fixed buffers: everything is checked once,
+// and run() only launches, on the current stream (or into the capture that is
+// open on it).  Each run reads angles, lengths and grad_output from their
+// memory and writes output_coords and grad_input; the look-back words (sync)
+// must be zero before the first run, and every run leaves them zero.  The
+// memory is held for the step's lifetime, through detached tensors, whose
+// sizes and data no later set_() or .data of the caller's tensors changes.
+//
+// The kernels are launched directly: a launch of a two-kernel HIP graph holds
+// the host for 14 to 20 us, two kernel launches for 6 (B = 32, L = 200).
+class Step {
   public:
-    StepGraph(torch::Tensor angles, torch::Tensor lengths, torch::Tensor grad_output,
-              torch::Tensor output_coords, torch::Tensor grad_input, torch::Tensor state,
-              torch::Tensor sync, std::vector<int64_t> config)
-        : held_{angles, lengths, grad_output, output_coords, grad_input, state, sync} {
-        const tpl_a2b_config cfg = to_config(config);
-        auto [B, L] = check_inputs(angles, lengths);
-        const int dt = dtype_code(angles);
+    Step(torch::Tensor angles, torch::Tensor lengths, torch::Tensor grad_output, torch::Tensor output_coords,
+         torch::Tensor grad_input, torch::Tensor state, torch::Tensor sync, std::vector<int64_t> config)
+        : angles_(angles.detach()), lengths_(lengths.detach()), grad_output_(grad_output.detach()),
+          coords_(output_coords.detach()), grad_input_(grad_input.detach()), state_(state.detach()),
+          sync_(sync.detach()), cfg_(to_config(config)) {
+        std::tie(B_, L_) = check_inputs(angles, lengths);
+        dt_ = dtype_code(angles);
         c10::DeviceGuard guard(angles.device());
-        device_ = angles.device().index();
-        check_out(grad_output, angles, {B, 9 * (int64_t)L}, "gradOutput");
-        check_out(output_coords, angles, {B, 9 * (int64_t)L}, "output_coords");
-        check_out(grad_input, angles, {B, 3, L}, "gradInput");
-        void* st = opt_ptr(state, tpl_a2b_state_bytes(dt, B, L, &cfg), "state", angles);
-        void* sy = opt_ptr(sync, tpl_a2b_sync_bytes(dt, B, L, &cfg), "sync", angles);
-        hipStream_t cs;
-        TORCH_CHECK(hipStreamCreateWithFlags(&cs, hipStreamNonBlocking) == hipSuccess,
-                    "StepGraph: hipStreamCreateWithFlags failed");
-        std::string err;
-        if (hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal) != hipSuccess) {
-            err = "hipStreamBeginCapture failed";
+        check_out(grad_output, angles, {B_, 9 * (int64_t)L_}, "gradOutput");
+        check_out(output_coords, angles, {B_, 9 * (int64_t)L_}, "output_coords");
+        check_out(grad_input, angles, {B_, 3, L_}, "gradInput");
+        st_ = opt_ptr(state, tpl_a2b_state_bytes(dt_, B_, L_, &cfg_), "state", angles);
+        sy_ = opt_ptr(sync, tpl_a2b_sync_bytes(dt_, B_, L_, &cfg_), "sync", angles);
+        fused_ = tplx_a2b_step_fits(dt_, B_, L_, &cfg_);
+    }
+    void run() {
+        const c10::Device dev = angles_.device();
+        c10::DeviceGuard guard(dev);
+        const hipStream_t s = c10::hip::getCurrentHIPStream(dev.index()).stream();
+        const int32_t* len = lengths_.data_ptr<int32_t>();
+        int rc;
+        if (fused_) {
+            rc = tplx_a2b_step(dt_, angles_.data_ptr(), len, grad_output_.data_ptr(), coords_.data_ptr(),
+                               grad_input_.data_ptr(), B_, L_, &cfg_, s);
         } else {
-            int rc = tpl_a2b_forward(dt, angles.data_ptr(), output_coords.data_ptr(),
-                                     lengths.data_ptr<int32_t>(), st, sy, nullptr, B, L, &cfg, cs);
+            rc = tpl_a2b_forward(dt_, angles_.data_ptr(), coords_.data_ptr(), len, st_, sy_, nullptr, B_, L_, &cfg_, s);
             if (rc == TPL_A2B_OK)
-                rc = tpl_a2b_backward(dt, grad_input.data_ptr(), grad_output.data_ptr(), angles.data_ptr(),
-                                      lengths.data_ptr<int32_t>(), st, sy, nullptr, B, L, &cfg, cs);
-            hipGraph_t g = nullptr;
-            const hipError_t ec = hipStreamEndCapture(cs, &g);
-            if (rc != TPL_A2B_OK || ec != hipSuccess || !g)
-                err = rc != TPL_A2B_OK ? tpl_a2b_strerror(rc) : "hipStreamEndCapture failed";
-            else if (hipGraphInstantiate(&exec_, g, nullptr, nullptr, 0) != hipSuccess)
-                err = "hipGraphInstantiate failed";
-            if (g) (void)hipGraphDestroy(g);
+                rc = tpl_a2b_backward(dt_, grad_input_.data_ptr(), grad_output_.data_ptr(), angles_.data_ptr(), len,
+                                      st_, sy_, nullptr, B_, L_, &cfg_, s);
         }
-        (void)hipStreamDestroy(cs);
-        TORCH_CHECK(err.empty(), "StepGraph: ", err);
-    }
-    StepGraph(const StepGraph&) = delete;
-    StepGraph& operator=(const StepGraph&) = delete;
-    ~StepGraph() {
-        if (exec_) (void)hipGraphExecDestroy(exec_);
-    }
-    void replay() {
-        c10::DeviceGuard guard(held_[0].device());
-        hipStream_t s = c10::hip::getCurrentHIPStream(device_).stream();
-        TORCH_CHECK(hipGraphLaunch(exec_, s) == hipSuccess, "StepGraph: hipGraphLaunch failed");
+        TORCH_CHECK(rc == TPL_A2B_OK, "Angles2BackboneStep: ", tpl_a2b_strerror(rc));
     }
 
   private:
-    std::vector<torch::Tensor> held_;
-    hipGraphExec_t exec_ = nullptr;
-    int device_ = 0;
+    torch::Tensor angles_, lengths_, grad_output_, coords_, grad_input_, state_, sync_;
+    tpl_a2b_config cfg_;
+    int B_ = 0, L_ = 0, dt_ = 0;
+    void *st_ = nullptr, *sy_ = nullptr;
+    bool fused_ = false;
 };
 
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
-    pybind11::class_<StepGraph>(m, "StepGraph")
+    pybind11::class_<Step>(m, "Step")
         .def(pybind11::init<torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor, torch::Tensor,
                             torch::Tensor, torch::Tensor, std::vector<int64_t>>(),
-             "capture one fwd+bwd step into a HIP graph")
-        .def("replay", &StepGraph::replay, "launch the step on the current stream");
+             "one fwd+bwd step on fixed buffers")
+        .def("run", &Step::run, "launch the step on the current stream");
     m.doc() = "Angles2Backbone for MI355X: tensor glue over the tpl_a2b C ABI";
     m.def("Angles2BackboneGPU_forward", &forward, "Angles2Backbone gpu forward (chunk scan)");
     m.def("Angles2BackboneGPU_backward", &backward, "Angles2Backbone gpu backward (O(L) adjoint)");

@@ -12,4 +12,13 @@ int tplx_a2b_forward(int dtype, const void* angles, void* coords, const int32_t*
 int tplx_a2b_backward(int dtype, void* grad_angles, const void* grad_coords, const void* angles,
                       const int32_t* lengths, const void* state, void* sync, uint32_t* flags, int batch,
                       int angles_stride, const tpl_a2b_config* cfg, tpl_stream_t stream);
+
+// Forward and backward of one step in one kernel, for gradients that are there
+// beforehand, with cfg->bwd_res_per_lane residues per lane; no state and no
+// look-back words.  tplx_a2b_step_fits: whether the shape has such a kernel and
+// the configuration asks for one (float32: the same chunk in both directions;
+// float64, where the backward has at most 2 residues per lane, any).
+int tplx_a2b_step_fits(int dtype, int batch, int angles_stride, const tpl_a2b_config* cfg);
+int tplx_a2b_step(int dtype, const void* angles, const int32_t* lengths, const void* grad_coords, void* coords,
+                  void* grad_angles, int batch, int angles_stride, const tpl_a2b_config* cfg, tpl_stream_t stream);
 }
