@@ -1,6 +1,7 @@
-"""The one-kernel step (Angles2BackboneStep with equal chunk sizes in both
-directions) against the float64 host path, at the sizes where it can go wrong:
-empty and one-residue chains, chunk edges (64 R), chains of 1 to 8 chunks,
+"""The step's own kernels (Angles2BackboneStep with equal chunk sizes in both
+directions, and with long chains) against the float64 host path, at the sizes where it can go wrong:
+empty and one-residue chains, chunk edges (64 R), chains of 1 to 8 chunks
+and of up to 256 in groups of 64 (and one more, which takes the layer's kernels),
 batches that fit on the GPU at once and batches packed by length, strides with
 every alignment and padding past the chains.  Several runs on changed inputs,
 under a capture too."""
@@ -52,6 +53,9 @@ def _check(step, a, lens, g, dtype):
 def _lengths(B, L, kind, C, rng):
     if kind == "equal":
         return [L] * B
+    if kind == "long":  # groups of 64 chunks
+        lens = [min(v, L) for v in (64 * C, 64 * C + 1, 64 * C - 1, 65 * C, 128 * C + 1, 192 * C, L, 0, 5 * C)]
+        return lens[:B]
     edges = [0, 1, 2, C - 1, C, C + 1, 2 * C - 1, 2 * C, 2 * C + 1, 3 * C, 4 * C, 4 * C + 1, L - 1, L]
     lens = [min(e, L) for e in edges]
     lens += [int(v) for v in np.exp(rng.uniform(np.log(2), np.log(L), max(0, B - len(lens))))]
@@ -65,6 +69,7 @@ def _lengths(B, L, kind, C, rng):
     (1, 1, "equal"), (3, 5, "equal"), (2, 127, "equal"), (2, 129, "equal"), (5, 512, "equal"),
     (17, 515, "mixed"), (14, 1023, "mixed"), (16, 1024, "mixed"), (18, 2048, "mixed"), (600, 333, "mixed"), (1100, 770, "mixed"),
     (1537, 514, "mixed"), (2050, 101, "mixed"), (4095, 259, "mixed"),
+    (3, 2049, "equal"), (19, 4100, "mixed"), (9, 8400, "long"), (9, 16500, "long"),
 ])
 def test_step_matches_oracle(dtype, R, B, L, kind):
     from torchproteinlibrary_amd.ReducedModel.Angles2Backbone.Angles2Backbone import Angles2BackboneStep

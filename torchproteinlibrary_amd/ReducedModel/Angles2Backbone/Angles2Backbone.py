@@ -284,9 +284,10 @@ class Angles2BackboneStep:
     (``grad_coords`` -> ``grad_angles``) on the current stream, with nothing
     allocated, no host synchronisation and one launch per step, or two: chains
     of at most 8 chunks run in one kernel when both directions have the same
-    chunk size (in float64 always), other shapes in the layer's two.  In one
-    kernel the coordinates are those the gradients are computed from, rounded
-    once from float64; they can differ from the layer's in the last digits.
+    chunk size (in float64 always), chains of up to 256 chunks in two, other
+    shapes in the layer's two.  In the step's own kernels the coordinates are
+    those the gradients are computed from, rounded once from float64; they can
+    differ from the layer's in the last digits.
     A step reads ``angles``, ``angles_length`` and ``grad_coords`` from their
     memory at every replay, so a loop updates them in place between replays;
     it writes ``coords`` and ``grad_angles``.  A replay under a capture is

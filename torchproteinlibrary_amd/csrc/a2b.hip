@@ -1584,13 +1584,13 @@ __global__ void __launch_bounds__(64 * W) a2b_bwd_chain(ChunkArgs a) {
 //
 // What bounds it: the two passes of FP64 frame products (some 2700 vector
 // instructions a wave at R = 4, two waves to a SIMD) where all chains fit at
-// once, and with padding the stores.  Forward and backward against the two
-// kernels (run to run within 0.2 us), launches back to back:
-//   B = 256, L = 700, float32, (4,4):                 16.4 -> 10.4 us
-//   B = 32,  L = 200, float32, (1,1):                  9.6 ->  6.2
-//   B = 512, L = 500, lengths 50..500, float32, (2,2): 18.3 -> 10.5
-//   B = 1024, L = 1000, lengths 30..1000, float32, (4,4): 31.0 -> 19.1
-//   the same in float64, (4,2):                       43.3 -> 29.0
+// once, and with padding the stores.  Against the forward and the backward
+// kernel replayed from a graph (runs of one side within 0.2 us), back to back:
+//   B = 256, L = 700, float32, (4,4):                     20.2 -> 10.4 us
+//   B = 32,  L = 200, float32, (1,1):                     14.3 ->  6.2
+//   B = 512, L = 500, lengths 50..500, float32, (2,2):    21.1 -> 10.5
+//   B = 1024, L = 1000, lengths 30..1000, float32, (4,4): 35.8 -> 19.1
+//   the same in float64, (4,2):                           48.0 -> 29.0
 // Each workgroup writing the zeros of its own chains took 22.0 us in the fourth
 // (the short chains' workgroups have nearly all of them) and 33.6 in the fifth.
 template <typename T, int R>
@@ -1735,21 +1735,197 @@ __device__ __forceinline__ int find_chains(const ChunkArgs& a, int* s_chain, int
 
 __device__ __forceinline__ int chunks_of(int n, int C) { return (n + C - 1) / C; }
 
-template <typename T, int R, int W, bool BINS>
+// Long chains (WALK): one wave per chunk, W chunks of a chain to a workgroup,
+// in two kernels.  a2b_step_sums takes each chunk's frame and its sums (M, F)
+// in the chunk's own frame; then in a2b_step each wave reads the records of
+// its whole chain (64 chunks at a time, one to a lane), scans the frames and
+// sums the torques of the later chunks, and does the rest as above.  The
+// angles and gradients are read twice and their sincos taken twice, but no
+// workgroup waits for another.
+//
+// Against the forward and backward kernels, whose waves take tickets and poll
+// for the records of earlier chunks, replayed from a graph, back to back:
+//   B = 64, L = 16384, lengths 4096..16384, float32: 74.0 -> 46.8 us (15.6 + 31;
+//                                                    67.9 launched directly)
+//   B = 20, L = 5000, float32:                       29.1 -> 18.8
+//   B = 1,  L = 16384, float32:                      33.5 -> 18.3
+//   B = 32, L = 16384, lengths 4096..16384, float64: 80.7 -> 39.5
+// What bounds it: FP64 issue and the latency of one wave (14 us from its loads
+// to its stores): the first has 2.7 waves to a SIMD, and 2 fit at 235 VGPRs.
+// Held to 168 VGPRs so that 3 fit it spills (56.8 us).
+//
+// Workgroup g takes block g / B of chain (g + g / B) mod B: first blocks first,
+// so that the padding comes last, and the blocks of one chain on all XCDs.
+constexpr int kStepRec = kF + 12;  // doubles per chunk: frame, M, F; record value e of chunk c of
+                                   // chain b at (b * kStepRec + e) * nc + c
+constexpr int kWalkMaxChunks = 256;
+
+template <int W>
+__device__ __forceinline__ void walk_slot(const ChunkArgs& a, int wave, int& b, int& c) {
+    const int blk = (int)blockIdx.x / a.B;
+    b = (int)(((unsigned)blockIdx.x + (unsigned)blk) % (unsigned)a.B);
+    c = blk * W + wave;
+}
+
+// The frame P before chunk c of chain b and the sums S over the chunks after it.
+// What is uniform goes back to scalar registers (248 -> 168 VGPRs at R = 2, and
+// so 3 waves to a SIMD: 42.5 -> 39.5 us in the last line above).  EARLY loads
+// the sums before the scan (R = 4, where 2 waves fit either way: 47.6 -> 46.8).
+template <bool EARLY>
+__device__ __forceinline__ void walk_chain(const ChunkArgs& a, int b, int c, int nreal, int lane, double P[kF],
+                                           double S[6]) {
+    const double* rec = a.ckpt + (size_t)b * kStepRec * a.nc;
+    double I[kF];  // the frame before the group
+    frame_identity(I);
+    frame_identity(P);
+#pragma unroll
+    for (int e = 0; e < 6; ++e) S[e] = 0.0;
+    for (int lo = 0; lo < nreal; lo += 64) {
+        const int j = lo + lane;
+        const bool valid = j < nreal;
+        double v[kF];
+#pragma unroll
+        for (int e = 0; e < kF; ++e) v[e] = valid ? rec[(size_t)e * a.nc + j] : ident(e);
+        double m[12];
+        const auto load_sums = [&] {
+#pragma unroll
+            for (int e = 0; e < 12; ++e) m[e] = valid && j > c ? rec[(size_t)(kF + e) * a.nc + j] : 0.0;
+        };
+        if (EARLY) load_sums();
+        wave_scan_frames(v);
+        if (lo > 0) frame_lmul(I, v);
+        double next[kF];
+#pragma unroll
+        for (int e = 0; e < kF; ++e) next[e] = read_lane(v[e], 63);
+        wave_shift_frames(v);  // the frame before chunk j
+        if (lo > 0 && lane == 0) {
+#pragma unroll
+            for (int e = 0; e < kF; ++e) v[e] = I[e];
+        }
+        if (lo <= c && c < lo + 64) {
+#pragma unroll
+            for (int e = 0; e < kF; ++e) P[e] = read_lane(v[e], c - lo);
+        }
+        if (min(lo + 64, nreal) > c + 1) {
+            if (!EARLY) load_sums();
+            auto rm = [&](int i, int k) { return v[i] * m[k] + v[3 + i] * m[3 + k] + v[6 + i] * m[6 + k]; };
+            double w[6];
+            w[0] = rm(1, 2) - rm(2, 1) + (v[10] * m[11] - v[11] * m[10]);
+            w[1] = rm(2, 0) - rm(0, 2) + (v[11] * m[9] - v[9] * m[11]);
+            w[2] = rm(0, 1) - rm(1, 0) + (v[9] * m[10] - v[10] * m[9]);
+            w[3] = m[9];
+            w[4] = m[10];
+            w[5] = m[11];
+            wave_scan_sum<6>(w);
+#pragma unroll
+            for (int e = 0; e < 6; ++e) S[e] = read_lane(S[e] + w[e], 63);
+        }
+#pragma unroll
+        for (int e = 0; e < kF; ++e) I[e] = next[e];
+    }
+}
+
+template <typename T, int R, int W>
+__global__ void __launch_bounds__(64 * W) a2b_step_sums(ChunkArgs a) {
+    constexpr int C = 64 * R;
+    __shared__ double s_tab[128];
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = (int)(threadIdx.x & 63);
+    const int L = a.L;
+    int b, c;
+    walk_slot<W>(a, wave, b, c);
+    const int raw = a.lengths[b], n = raw < 0 ? 0 : (raw > L ? L : raw);
+    if (c - wave >= chunks_of(n, C)) return;  // the whole workgroup
+    for (int i = (int)threadIdx.x; i < 128; i += 64 * W) s_tab[i] = kTabCS[i];
+    const int rl = c * C + lane * R;
+    const int cnt = min(max(n - rl, 0), R);
+    T ang[3][R];
+    T gr[9 * R];
+    if (cnt > 0) {
+        lane_load_rows<T, R>(static_cast<const T*>(a.angles) + (size_t)3 * b * L + rl, L, cnt, L - rl, ang);
+        lane_load<T, 9 * R>(static_cast<const T*>(a.grad) + (size_t)9 * b * L + (size_t)9 * rl, 9 * cnt, gr,
+                            9 * (L - rl));
+    } else {
+#pragma unroll
+        for (int kk = 0; kk < 3; ++kk)
+#pragma unroll
+            for (int i = 0; i < R; ++i) ang[kk][i] = (T)0;
+#pragma unroll
+        for (int i = 0; i < 9 * R; ++i) gr[i] = (T)0;
+    }
+    __syncthreads();  // s_tab
+    if (c >= chunks_of(n, C)) return;
+    double f[kF];
+    double M[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+    double F[3] = {(double)gr[0], (double)gr[1], (double)gr[2]};
+    frame_identity(f);
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            double sn, cs;
+            sincos_tab((double)ang[k][q], s_tab, &sn, &cs);
+            if (k == 0) frame_step<0>(f, cs, sn);
+            if (k == 1) frame_step<1>(f, cs, sn);
+            if (k == 2) frame_step<2>(f, cs, sn);
+            const int at = 3 * q + k + 1;
+            if (at < 3 * R) {
+                const double g0 = (double)gr[3 * at], g1 = (double)gr[3 * at + 1], g2 = (double)gr[3 * at + 2];
+#pragma unroll
+                for (int m = 0; m < 3; ++m) {
+                    M[3 * m] = fma(f[9 + m], g0, M[3 * m]);
+                    M[3 * m + 1] = fma(f[9 + m], g1, M[3 * m + 1]);
+                    M[3 * m + 2] = fma(f[9 + m], g2, M[3 * m + 2]);
+                }
+                F[0] += g0;
+                F[1] += g1;
+                F[2] += g2;
+            }
+        }
+    }
+    wave_scan_frames(f);
+    double* rec = a.ckpt + (size_t)b * kStepRec * a.nc + c;
+    if (lane == 63) {
+#pragma unroll
+        for (int e = 0; e < kF; ++e) rec[(size_t)e * a.nc] = f[e];
+    }
+    wave_shift_frames(f);
+    double m[12];  // the lane's sums in the chunk's frame
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+        for (int k = 0; k < 3; ++k)
+            m[3 * i + k] = f[i] * M[k] + f[3 + i] * M[3 + k] + f[6 + i] * M[6 + k] + f[9 + i] * F[k];
+    m[9] = F[0];
+    m[10] = F[1];
+    m[11] = F[2];
+    wave_scan_sum<12>(m);
+    if (lane == 63) {
+#pragma unroll
+        for (int e = 0; e < 12; ++e) rec[(size_t)(kF + e) * a.nc] = m[e];
+    }
+}
+
+enum StepMode { CHAIN, BINS, WALK };
+
+template <typename T, int R, int W, StepMode MODE>
 __global__ void __launch_bounds__(64 * W) a2b_step(ChunkArgs a) {
     constexpr int C = 64 * R;
     extern __shared__ double s_dynd[];  // [W][step_wave_doubles]
     __shared__ double s_tab[128];
-    __shared__ double s_agg[W][kF];
-    __shared__ double s_tot[W][6];
-    __shared__ int s_chain[W];
-    __shared__ int s_count[W][2];
+    constexpr int WS = MODE == WALK ? 1 : W;
+    __shared__ double s_agg[WS][kF];
+    __shared__ double s_tot[WS][6];
+    __shared__ int s_chain[WS];
+    __shared__ int s_count[WS][2];
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = (int)(threadIdx.x & 63);
     const int L = a.L;
     for (int i = (int)threadIdx.x; i < 128; i += 64 * W) s_tab[i] = kTabCS[i];
     int nwg = 0;
     int b, c, size, first = 0;  // the chain, this wave's chunk of it, its slot: waves first .. first + size - 1
-    if (BINS) {
+    if constexpr (MODE == WALK) {
+        size = 1;
+        walk_slot<W>(a, wave, b, c);
+    } else if constexpr (MODE == BINS) {
         size = find_chains<R, W>(a, s_chain, s_count, nwg);
         if (size == 0) return;
         b = __builtin_amdgcn_readfirstlane(s_chain[wave / size]);
@@ -1794,7 +1970,18 @@ __global__ void __launch_bounds__(64 * W) a2b_step(ChunkArgs a) {
             for (int i = 0; i < 9 * R; ++i) gr[i] = (T)0;
         }
     }
-    if (!BINS) __syncthreads();  // s_tab (find_chains ends with a barrier)
+    if (MODE != BINS) __syncthreads();  // s_tab (find_chains ends with a barrier)
+    double P[kF], later[6];  // WALK
+    if constexpr (MODE == WALK) {
+        if (!real) {  // the zeros of a chunk past the chain
+            const int p = min(c * C, L), cnt0 = min(C, L - p);
+            store_zeros<T>(xrow + (size_t)9 * p, 9 * cnt0, 0, 1, lane);
+#pragma unroll
+            for (int k = 0; k < 3; ++k) store_zeros<T>(grow + (size_t)k * L + p, cnt0, 0, 1, lane);
+            return;
+        }
+        walk_chain<R == 4>(a, b, c, nreal, lane, P, later);
+    }
 
     double f[kF], W6[6], S[6];
     double M[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
@@ -1833,7 +2020,7 @@ __global__ void __launch_bounds__(64 * W) a2b_step(ChunkArgs a) {
             }
         }
         wave_scan_frames(f);
-        if (lane == 63) {
+        if (MODE != WALK && lane == 63) {
 #pragma unroll
             for (int e = 0; e < kF; ++e) s_agg[first + c][e] = f[e];
         }
@@ -1849,15 +2036,17 @@ __global__ void __launch_bounds__(64 * W) a2b_step(ChunkArgs a) {
         for (int k = 0; k < 3; ++k)
             store_zeros<T>(static_cast<T*>(a.grad_angles) + ((size_t)3 * zb + k) * L + p, L - p, f, F, lane);
     };
-    if (BINS) {
+    if constexpr (MODE == BINS) {
         for (int u = (int)blockIdx.x * W + wave; u < 4 * a.B; u += nwg * W) zeros(u >> 2, u & 3, 4);
-    } else {
+    } else if constexpr (MODE == CHAIN) {
         zeros(b, c, W);
     }
-    __syncthreads();  // the aggregates
+    if (MODE != WALK) __syncthreads();  // the aggregates
     if (real) {
-        if (c > 0) {
-            double P[kF], Q[kF];
+        if constexpr (MODE == WALK) {
+            frame_lmul(P, f);
+        } else if (c > 0) {
+            double Q[kF];
 #pragma unroll
             for (int e = 0; e < kF; ++e) P[e] = s_agg[first][e];
             for (int j = 1; j < c; ++j) {
@@ -1885,16 +2074,21 @@ __global__ void __launch_bounds__(64 * W) a2b_step(ChunkArgs a) {
             tot[e] = read_lane(S[e], 63);
             S[e] = tot[e] - S[e];
         }
-        if (lane == 0) {
+        if (MODE != WALK && lane == 0) {
 #pragma unroll
             for (int e = 0; e < 6; ++e) s_tot[first + c][e] = tot[e];
         }
     }
-    __syncthreads();  // the chunks' sums
-    if (!real) return;
-    for (int j = c + 1; j < nreal; ++j) {
+    if constexpr (MODE == WALK) {
 #pragma unroll
-        for (int e = 0; e < 6; ++e) S[e] += s_tot[first + j][e];
+        for (int e = 0; e < 6; ++e) S[e] += later[e];
+    } else {
+        __syncthreads();  // the chunks' sums
+        if (!real) return;
+        for (int j = c + 1; j < nreal; ++j) {
+#pragma unroll
+            for (int e = 0; e < 6; ++e) S[e] += s_tot[first + j][e];
+        }
     }
     const int crow = min(max(L - rl, 0), R);
     if (cnt > 0) {
@@ -2350,25 +2544,13 @@ int launch_chain(KernelFn k, const ChunkArgs& a, size_t lds, hipStream_t stream)
     return hipGetLastError() == hipSuccess ? TPL_A2B_OK : TPL_A2B_ERR_LAUNCH;
 }
 
-// The step kernel: R residues per lane, W waves per workgroup (4, or 8 where
-// the chains need it).
-template <typename T, int R>
-KernelFn step_kernel_w(int w, bool bins) {
-    if (w <= 4) return bins ? a2b_step<T, R, 4, true> : a2b_step<T, R, 4, false>;
-    if constexpr (R == 1)
-        return nullptr;  // step_form
-    else
-        return bins ? a2b_step<T, R, 8, true> : a2b_step<T, R, 8, false>;
-}
-template <typename T, int R>
-size_t step_lds(int w) {
-    return (size_t)(w <= 4 ? 4 : 8) * step_wave_doubles<T, R>() * sizeof(double);
-}
+// The step's kernels for a shape with R residues per lane.
 struct StepForm {
-    KernelFn kernel;
+    KernelFn kernel, sums;  // sums: WALK
     int waves;
     size_t lds;
-    bool bins;
+    unsigned grid;
+    size_t rec_bytes;  // WALK: the records
 };
 
 // Dynamic LDS beyond 64 KB has to be allowed per kernel and device, once.
@@ -2386,30 +2568,52 @@ bool allow_lds(KernelFn k, size_t bytes) {
     return true;
 }
 
-// The form for a shape with R residues per lane; false where the chains have
-// more chunks than a workgroup has waves (8; with one residue per lane 4: 8
-// waves of so little work each spend it at the barriers, 13.3 us for B = 512,
-// L = 500 against 10.5 with two residues per lane), or the batch does not fit
-// at once and is too large for its lengths to be read by every workgroup.
-bool step_form(int dtype, int B, int L, int R, StepForm& s) {
-    const int nc = chunks(L, 64 * R);
-    if (nc > (R == 1 ? 4 : 8)) return false;
-    s.waves = nc <= 4 ? 4 : 8;
-    for (int bins = 0; bins < 2; ++bins) {
-        s.bins = bins;
-        if (dtype == TPL_A2B_F32) {
-            s.kernel = R == 1   ? step_kernel_w<float, 1>(s.waves, bins)
-                       : R == 2 ? step_kernel_w<float, 2>(s.waves, bins)
-                                : step_kernel_w<float, 4>(s.waves, bins);
-            s.lds = R == 1 ? step_lds<float, 1>(s.waves) : R == 2 ? step_lds<float, 2>(s.waves) : step_lds<float, 4>(s.waves);
-        } else {
-            s.kernel = R == 1 ? step_kernel_w<double, 1>(s.waves, bins) : step_kernel_w<double, 2>(s.waves, bins);
-            s.lds = R == 1 ? step_lds<double, 1>(s.waves) : step_lds<double, 2>(s.waves);
-        }
-        if (!allow_lds(s.kernel, s.lds)) return false;
-        if (!bins && B <= resident_workgroups(s.kernel, 64 * s.waves, s.lds)) return true;
+template <typename T, int R>
+void step_kernel(StepForm& s, StepMode mode) {
+    s.sums = nullptr;
+    if (mode == WALK) {
+        s.kernel = a2b_step<T, R, 4, WALK>;
+        s.sums = a2b_step_sums<T, R, 4>;
+    } else if (s.waves == 4) {
+        s.kernel = mode == BINS ? a2b_step<T, R, 4, BINS> : a2b_step<T, R, 4, CHAIN>;
+    } else if constexpr (R > 1) {
+        s.kernel = mode == BINS ? a2b_step<T, R, 8, BINS> : a2b_step<T, R, 8, CHAIN>;
     }
-    return B <= kStepMaxBatch;
+    s.lds = s.waves * step_wave_doubles<T, R>() * sizeof(double);
+}
+
+// Chains of at most 8 chunks run in one kernel, if both directions have the
+// same chunk (in float64, where the backward has at most 2 residues per lane,
+// always): CHAIN where all chains fit on the GPU at once, else BINS, if there
+// are few enough that every workgroup can read their lengths.  With one residue
+// per lane only up to 4 chunks: 8 waves of so little work each spend it at the
+// barriers, 13.3 us for B = 512, L = 500 against 10.5 with two residues per
+// lane.  Longer chains of up to kWalkMaxChunks chunks: WALK.  The rest (false)
+// goes through the forward and the backward kernel.
+bool step_form(int dtype, int B, int L, const tpl_a2b_config* cfg, StepForm& s) {
+    const int R = cfg->bwd_res_per_lane;
+    const int nc = chunks(L, 64 * R);
+    s.waves = nc > 4 && nc <= 8 ? 8 : 4;
+    s.rec_bytes = 0;
+    const auto pick = [&](StepMode mode) {
+        s.grid = (unsigned)(mode == WALK ? B * chunks(nc, s.waves) : B);
+        if (dtype == TPL_A2B_F32) {
+            R == 1 ? step_kernel<float, 1>(s, mode) : R == 2 ? step_kernel<float, 2>(s, mode) : step_kernel<float, 4>(s, mode);
+        } else {
+            R == 1 ? step_kernel<double, 1>(s, mode) : step_kernel<double, 2>(s, mode);
+        }
+        return allow_lds(s.kernel, s.lds);
+    };
+    if (nc > 8) {
+        if (nc > kWalkMaxChunks || !pick(WALK)) return false;
+        s.rec_bytes = (size_t)B * kStepRec * nc * sizeof(double);
+        return true;
+    }
+    if (dtype == TPL_A2B_F32 && cfg->fwd_res_per_lane != R) return false;
+    if (R == 1 && nc > 4) return false;
+    if (!pick(CHAIN)) return false;
+    if (B <= resident_workgroups(s.kernel, 64 * s.waves, s.lds)) return true;
+    return B <= kStepMaxBatch && pick(BINS);
 }
 
 // The two directions, reporting as `rep` says.
@@ -2555,32 +2759,36 @@ int tplx_a2b_backward(int dtype, void* grad_angles, const void* grad_coords, con
                        batch, angles_stride, cfg, stream);
 }
 
-int tplx_a2b_step_fits(int dtype, int batch, int angles_stride, const tpl_a2b_config* cfg) {
+int tplx_a2b_step_fits(int dtype, int batch, int angles_stride, const tpl_a2b_config* cfg, size_t* workspace) {
     if (check_common(dtype, batch, angles_stride) || !valid_config(cfg) || !fits_dtype(dtype, cfg)) return 0;
-    if (dtype == TPL_A2B_F32 && cfg->fwd_res_per_lane != cfg->bwd_res_per_lane) return 0;
     if (batch == 0 || angles_stride == 0) return 0;
     StepForm form;
-    return step_form(dtype, batch, angles_stride, cfg->bwd_res_per_lane, form) ? 1 : 0;
+    if (!step_form(dtype, batch, angles_stride, cfg, form)) return 0;
+    *workspace = form.rec_bytes;
+    return 1;
 }
 
 int tplx_a2b_step(int dtype, const void* angles, const int32_t* lengths, const void* grad_coords, void* coords,
-                  void* grad_angles, int batch, int angles_stride, const tpl_a2b_config* cfg, tpl_stream_t stream) {
+                  void* grad_angles, void* workspace, int batch, int angles_stride, const tpl_a2b_config* cfg,
+                  tpl_stream_t stream) {
     int rc = check_common(dtype, batch, angles_stride);
     if (rc) return rc;
     if (!valid_config(cfg) || !fits_dtype(dtype, cfg)) return TPL_A2B_ERR_CONFIG;
     if (batch == 0 || angles_stride == 0) return TPL_A2B_OK;
     if (!angles || !lengths || !grad_coords || !coords || !grad_angles) return TPL_A2B_ERR_ARG;
     StepForm form;
-    const int R = cfg->bwd_res_per_lane;
-    if (!step_form(dtype, batch, angles_stride, R, form)) return TPL_A2B_ERR_CONFIG;
-    ChunkArgs a = base_args(batch, angles_stride, 64 * R, cfg);
+    if (!step_form(dtype, batch, angles_stride, cfg, form)) return TPL_A2B_ERR_CONFIG;
+    if (form.rec_bytes && (!workspace || misaligned(workspace))) return TPL_A2B_ERR_ARG;
+    ChunkArgs a = base_args(batch, angles_stride, 64 * cfg->bwd_res_per_lane, cfg);
     a.angles = angles;
     a.lengths = lengths;
     a.grad = grad_coords;
     a.coords = coords;
     a.grad_angles = grad_angles;
-    hipLaunchKernelGGL(form.kernel, dim3((unsigned)batch), dim3(64 * form.waves), form.lds,
-                       static_cast<hipStream_t>(stream), a);
+    a.ckpt = static_cast<double*>(workspace);
+    const hipStream_t s = static_cast<hipStream_t>(stream);
+    if (form.sums) hipLaunchKernelGGL(form.sums, dim3(form.grid), dim3(64 * form.waves), 0, s, a);
+    hipLaunchKernelGGL(form.kernel, dim3(form.grid), dim3(64 * form.waves), form.lds, s, a);
     return hipGetLastError() == hipSuccess ? TPL_A2B_OK : TPL_A2B_ERR_LAUNCH;
 }
 

@@ -505,7 +505,9 @@ class Step {
         check_out(grad_input, angles, {B_, 3, L_}, "gradInput");
         st_ = opt_ptr(state, tpl_a2b_state_bytes(dt_, B_, L_, &cfg_), "state", angles);
         sy_ = opt_ptr(sync, tpl_a2b_sync_bytes(dt_, B_, L_, &cfg_), "sync", angles);
-        fused_ = tplx_a2b_step_fits(dt_, B_, L_, &cfg_);
+        size_t bytes = 0;
+        fused_ = tplx_a2b_step_fits(dt_, B_, L_, &cfg_, &bytes);
+        if (bytes) records_ = torch::empty({(int64_t)bytes}, angles.options().dtype(torch::kByte));
     }
     void run() {
         const c10::Device dev = angles_.device();
@@ -515,7 +517,8 @@ class Step {
         int rc;
         if (fused_) {
             rc = tplx_a2b_step(dt_, angles_.data_ptr(), len, grad_output_.data_ptr(), coords_.data_ptr(),
-                               grad_input_.data_ptr(), B_, L_, &cfg_, s);
+                               grad_input_.data_ptr(), records_.defined() ? records_.data_ptr() : nullptr, B_, L_,
+                               &cfg_, s);
         } else {
             rc = tpl_a2b_forward(dt_, angles_.data_ptr(), coords_.data_ptr(), len, st_, sy_, nullptr, B_, L_, &cfg_, s);
             if (rc == TPL_A2B_OK)
@@ -526,7 +529,7 @@ class Step {
     }
 
   private:
-    torch::Tensor angles_, lengths_, grad_output_, coords_, grad_input_, state_, sync_;
+    torch::Tensor angles_, lengths_, grad_output_, coords_, grad_input_, state_, sync_, records_;
     tpl_a2b_config cfg_;
     int B_ = 0, L_ = 0, dt_ = 0;
     void *st_ = nullptr, *sy_ = nullptr;

@@ -13,12 +13,13 @@ int tplx_a2b_backward(int dtype, void* grad_angles, const void* grad_coords, con
                       const int32_t* lengths, const void* state, void* sync, uint32_t* flags, int batch,
                       int angles_stride, const tpl_a2b_config* cfg, tpl_stream_t stream);
 
-// Forward and backward of one step in one kernel, for gradients that are there
+// Forward and backward of one step together, for gradients that are there
 // beforehand, with cfg->bwd_res_per_lane residues per lane; no state and no
-// look-back words.  tplx_a2b_step_fits: whether the shape has such a kernel and
-// the configuration asks for one (float32: the same chunk in both directions;
-// float64, where the backward has at most 2 residues per lane, any).
-int tplx_a2b_step_fits(int dtype, int batch, int angles_stride, const tpl_a2b_config* cfg);
+// look-back words.  tplx_a2b_step_fits: whether the shape and the configuration
+// have such a form, and the bytes of workspace it needs (256-byte aligned; its
+// contents do not matter).
+int tplx_a2b_step_fits(int dtype, int batch, int angles_stride, const tpl_a2b_config* cfg, size_t* workspace);
 int tplx_a2b_step(int dtype, const void* angles, const int32_t* lengths, const void* grad_coords, void* coords,
-                  void* grad_angles, int batch, int angles_stride, const tpl_a2b_config* cfg, tpl_stream_t stream);
+                  void* grad_angles, void* workspace, int batch, int angles_stride, const tpl_a2b_config* cfg,
+                  tpl_stream_t stream);
 }
