@@ -38,6 +38,7 @@ from torch.autograd.function import once_differentiable
 from torch.nn.modules.module import Module
 
 from ..._native_xform import ext
+from ..._plain import is_plain
 
 __all__ = ["Angles2Coords", "Angles2CoordsFunction", "convertStringList", "convertString"]
 
@@ -62,13 +63,11 @@ def convertString(string):
 
 
 def schedule(num_atoms):
-    """The order in which the GPU takes the structures: the most atoms first
+    """An order in which a GPU can take the structures, the most atoms first
     (ties in batch order), as an int32 CPU tensor, or None when every
-    structure has the same size (batch order is then as good).  One
-    workgroup builds one structure and workgroups start in index order, so
-    with mixed sizes this keeps the long structures from starting last:
-    mixed lengths 30-1000 at B=1024 measured 59 -> 50 us (forward) and
-    112 -> 77 us (backward)."""
+    structure has the same size.  For callers of the C entry points that take
+    one, whose kernels build one structure per workgroup; the layer needs
+    none, since its kernels spread mixed sizes over the GPU themselves."""
     n = np.asarray(num_atoms, dtype=np.int64)
     if n.size < 2 or (n == n[0]).all():
         return None
@@ -94,13 +93,30 @@ def _check(s, out, where):
         raise Exception(f"Angles2CoordsFunction: {where} Nan")
 
 
+def _native(input_angles, sequences, num_atoms, order=None, max_atoms=-1):
+    """A plain eager call of the function below, as the same function in native
+    code; None if the call is not a plain one."""
+    if not is_plain((input_angles, sequences, num_atoms) + (() if order is None else (order,))):
+        return None
+    out = ext.Angles2Coords_apply(input_angles, sequences, num_atoms, order, max_atoms)
+    return None if out is None else out + (num_atoms,)
+
+
 class Angles2CoordsFunction(Function):
     """Protein angles -> coordinates (reference Angles2Coords.py:34-71).
     ``sequenceTensor`` is the uint8 [B, S] tensor of ``convertStringList`` on
     the angles' device.  ``order`` (optional, int32 [B]) is the order in
     which the GPU takes the structures (a permutation of 0..B-1; the outputs
-    do not depend on it): ``Angles2Coords`` passes the structures from the
-    most atoms to the fewest when their sizes differ."""
+    do not depend on it).  A plain eager call runs as the same function in
+    native code."""
+
+    @classmethod
+    def apply(cls, *args, **kwargs):
+        if cls is Angles2CoordsFunction and 3 <= len(args) <= 4 and not kwargs:
+            out = _native(*args)
+            if out is not None:
+                return out
+        return super().apply(*args, **kwargs)
 
     @staticmethod
     def forward(ctx, input_angles, sequenceTensor, num_atoms, order=None):
@@ -154,6 +170,12 @@ class Angles2Coords(Module):
         self.num_atoms = None
 
     def forward(self, input_angles, sequences):
+        if is_plain((input_angles,)) and type(sequences) in (list, tuple):
+            prepared = ext.Angles2Coords_prepare(list(sequences), input_angles)
+            if prepared is not None:
+                self.num_atoms, seqs, num_atoms = prepared
+                out = _native(input_angles, seqs, num_atoms, None, max(self.num_atoms))
+                return Angles2CoordsFunction.apply(input_angles, seqs, num_atoms) if out is None else out
         for s in sequences:
             if not set(s) <= _LETTERS:
                 raise ValueError("Angles2Coords: a sequence holds a letter outside the 20 amino acids: "
@@ -161,4 +183,4 @@ class Angles2Coords(Module):
         self.num_atoms = [ext.getSeqNumAtoms(s) if s else 0 for s in sequences]
         num_atoms = torch.tensor(self.num_atoms, dtype=torch.int32, device=input_angles.device)
         stringListTensor = convertStringList(sequences)
-        return Angles2CoordsFunction.apply(input_angles, stringListTensor, num_atoms, schedule(self.num_atoms))
+        return Angles2CoordsFunction.apply(input_angles, stringListTensor, num_atoms)

@@ -36,6 +36,7 @@ from torch.autograd.function import once_differentiable
 from torch.nn.modules.module import Module
 
 from ..._native_xform import ext
+from ..._plain import is_plain
 
 __all__ = ["CoordsTranslate", "CoordsTranslateFunction", "CoordsRotate", "CoordsRotateFunction",
            "Coords2Center", "Coords2CenterFunction", "getRotation", "getRandomRotation",
@@ -64,8 +65,21 @@ def _rank2(t, name):
         raise RuntimeError(f"{name}: this build runs on the GPU only; input must be a GPU tensor")
 
 
+def _native(own, apply, count, args, kwargs):
+    """A plain eager call of a function below, as the same function in native
+    code; None if the call is not a plain one."""
+    if own and len(args) == count and not kwargs and is_plain(args) and args[0].dim() == 2:
+        return apply(*args)
+    return None
+
+
 class CoordsTranslateFunction(Function):
     """Coordinates translation (reference CoordsTransform.py:46-91)."""
+
+    @classmethod
+    def apply(cls, *args, **kwargs):
+        out = _native(cls is CoordsTranslateFunction, ext.CoordsTranslate_apply, 3, args, kwargs)
+        return super().apply(*args, **kwargs) if out is None else out
 
     @staticmethod
     def forward(ctx, input_coords, T, num_atoms):
@@ -96,6 +110,11 @@ class CoordsTranslate(Module):
 
 class CoordsRotateFunction(Function):
     """Coordinates rotation, R x per atom (reference CoordsTransform.py:101-149)."""
+
+    @classmethod
+    def apply(cls, *args, **kwargs):
+        out = _native(cls is CoordsRotateFunction, ext.CoordsRotate_apply, 3, args, kwargs)
+        return super().apply(*args, **kwargs) if out is None else out
 
     @staticmethod
     def forward(ctx, input_coords, R, num_atoms):
@@ -131,6 +150,11 @@ class CoordsRotate(Module):
 
 class Coords2CenterFunction(Function):
     """Geometric centre of each structure (reference CoordsTransform.py:158-206)."""
+
+    @classmethod
+    def apply(cls, *args, **kwargs):
+        out = _native(cls is Coords2CenterFunction, ext.Coords2Center_apply, 2, args, kwargs)
+        return super().apply(*args, **kwargs) if out is None else out
 
     @staticmethod
     def forward(ctx, input_coords, num_atoms):

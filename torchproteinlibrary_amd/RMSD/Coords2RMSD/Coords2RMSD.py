@@ -45,6 +45,7 @@ from torch.autograd.function import once_differentiable
 from torch.nn.modules.module import Module
 
 from ..._native_rmsd import ext
+from ..._plain import is_plain
 
 _STATUS_NAN = 1
 _STATUS_COUNT = 2
@@ -66,7 +67,16 @@ class Coords2RMSDFunction(Function):
     """Protein coords, target coords -> (rmsd, UT).
 
     Reference: TorchProteinLibrary/RMSD/Coords2RMSD/Coords2RMSD.py:12-62.
+    A plain eager call runs as the same function in native code.
     """
+
+    @classmethod
+    def apply(cls, *args, **kwargs):
+        if cls is Coords2RMSDFunction and len(args) == 3 and not kwargs and is_plain(args) and args[0].dim() == 2:
+            out = ext.Coords2RMSD_apply(*args)
+            if out is not None:
+                return out
+        return super().apply(*args, **kwargs)
 
     @staticmethod
     def forward(ctx, centered_input, centered_target, num_atoms):

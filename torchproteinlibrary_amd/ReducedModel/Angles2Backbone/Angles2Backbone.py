@@ -41,7 +41,6 @@ What differs, by design:
 from __future__ import annotations
 
 import os
-import threading
 import warnings
 
 import torch
@@ -51,6 +50,7 @@ from torch.nn.modules.module import Module
 
 from ... import _tuning
 from ..._native import ext
+from ..._plain import is_plain
 
 _STATUS_NAN = 1
 _STATUS_LENGTH = 2
@@ -77,15 +77,19 @@ def _run_checked(checked, where: str, sync) -> None:
     bits = checked()
     if bits & (_STATUS_TIMEOUT | _STATUS_SYNC):
         ext.sync_clear(sync)  # look-back words may be left set
-        what = "look-back wait timed out" if bits & _STATUS_TIMEOUT else "look-back words were not clean"
-        warnings.warn("Angles2BackboneFunction: %s %s; cleared and repeated" % (where, what),
-                      RuntimeWarning)
+        _report_lost(bits, where, True)
         bits = checked()
         if bits & (_STATUS_TIMEOUT | _STATUS_SYNC):
             ext.sync_clear(sync)
-            what = "look-back wait timed out" if bits & _STATUS_TIMEOUT else "look-back words were not clean"
-            raise RuntimeError("Angles2BackboneFunction: %s %s (result invalid)" % (where, what))
+            _report_lost(bits, where, False)
     _raise_on_bits(bits, where)
+
+
+def _report_lost(bits: int, where: str, repeated: bool) -> None:
+    what = "look-back wait timed out" if bits & _STATUS_TIMEOUT else "look-back words were not clean"
+    if not repeated:
+        raise RuntimeError("Angles2BackboneFunction: %s %s (result invalid)" % (where, what))
+    warnings.warn("Angles2BackboneFunction: %s %s; cleared and repeated" % (where, what), RuntimeWarning)
 
 
 def _raise_on_status(status, where: str) -> None:
@@ -114,31 +118,20 @@ def _empty_bytes(n, device):
     return torch.empty(int(n), dtype=torch.uint8, device=device)
 
 
-_sync_lock = threading.Lock()
-_sync_bufs: dict = {}
-
-
-def _sync_buffer(device, nbytes: int):
-    """The look-back buffer of (device, current stream), zeroed when made;
-    every call returns its tickets, counters and flags to zero.  Grown (a new
-    zeroed buffer) when too small.  Calls on one stream are ordered, so they
-    can share it."""
-    stream = torch.cuda.current_stream(device)
-    key = (device.index, stream.cuda_stream)
-    with _sync_lock:
-        buf = _sync_bufs.get(key)
-        if buf is None or buf.numel() < nbytes:
-            buf = torch.zeros(max(int(nbytes), 256), dtype=torch.uint8, device=device)
-            _sync_bufs[key] = buf
-    return buf
-
-
 class Angles2BackboneGPUFunction(Function):
     """Backbone angles -> backbone coordinates (chunk scan forward, O(L)
     adjoint backward from checkpoints).
 
     Reference: TorchProteinLibrary/ReducedModel/Angles2Backbone/Angles2Backbone.py:8-52.
+    A plain eager call runs as the same function in native code.
     """
+
+    @classmethod
+    def apply(cls, *args, **kwargs):
+        if (cls is Angles2BackboneGPUFunction and len(args) == 2 and not kwargs and is_plain(args)
+                and args[0].dim() == 3 and ext.Angles2Backbone_plain(*args)):
+            return ext.Angles2Backbone_apply(*args, _tuning.config_for(*args))
+        return super().apply(*args, **kwargs)
 
     @staticmethod
     def forward(ctx, input_angles, angles_length):
@@ -150,7 +143,7 @@ class Angles2BackboneGPUFunction(Function):
         st_bytes, sy_bytes = ext.workspace_bytes(input_angles.dtype == torch.float64, B, L,
                                                  list(cfg))
         state = _empty_bytes(st_bytes, dev) if ctx.needs_input_grad[0] else None
-        sync = _sync_buffer(dev, sy_bytes)
+        sync = ext.sync_buffer(input_angles, sy_bytes)
         if _checks_enabled():
             _run_checked(lambda: ext.Angles2BackboneGPU_forward_checked(input_angles, coords, angles_length,
                                                                         state, sync, cfg),
@@ -173,7 +166,7 @@ class Angles2BackboneGPUFunction(Function):
         dev = input_angles.device
         gradInput = torch.empty(B, 3, L, dtype=input_angles.dtype, device=dev)
         _, sy_bytes = ext.workspace_bytes(input_angles.dtype == torch.float64, B, L, list(ctx.cfg))
-        sync = _sync_buffer(dev, sy_bytes)
+        sync = ext.sync_buffer(input_angles, sy_bytes)
         if _checks_enabled():
             _run_checked(lambda: ext.Angles2BackboneGPU_backward_checked(gradInput, gradOutput, input_angles,
                                                                          angles_length, state, sync, ctx.cfg),

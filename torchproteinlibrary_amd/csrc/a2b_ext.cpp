@@ -11,12 +11,15 @@
 #include <c10/hip/HIPStream.h>
 
 #include <chrono>
+#include <map>
+#include <mutex>
 #include <string>
 #include <tuple>
 #include <vector>
 
 #include "a2b_flagged.h"
 #include "host_flags.h"
+#include "native_fn.h"
 #include "tpl_a2b.h"
 #include "tpl_a2b_cpu.h"
 
@@ -480,6 +483,86 @@ std::tuple<double, double, int64_t> bench_graph(std::vector<std::vector<torch::T
     return {(double)ms, std::chrono::duration<double, std::milli>(t1 - t0).count(), reps * per};
 }
 
+// The look-back words of (device, current stream), zeroed when made; every call
+// returns its tickets, counters and flags to zero.  Grown (a new zeroed buffer)
+// when too small.  Calls on one stream are ordered, so they can share it.
+torch::Tensor sync_buffer(const torch::Device& device, int64_t bytes) {
+    static std::mutex mu;
+    static auto* buffers = new std::map<std::pair<int, hipStream_t>, torch::Tensor>;  // outlives the runtime's end
+    const std::pair<int, hipStream_t> key{device.index(), c10::hip::getCurrentHIPStream(device.index()).stream()};
+    std::lock_guard<std::mutex> lock(mu);
+    torch::Tensor& buf = (*buffers)[key];
+    if (!buf.defined() || buf.nbytes() < (size_t)bytes)
+        buf = torch::zeros({std::max<int64_t>(bytes, 256)}, torch::TensorOptions().dtype(torch::kByte).device(device));
+    return buf;
+}
+
+// The autograd function of a plain call (native_fn.h); what it does is written
+// at Angles2BackboneGPUFunction.
+struct Angles2Backbone : torch::autograd::Function<Angles2Backbone> {
+    // Runs call(flags, sync) with the checks and the one repeat of _run_checked.
+    template <typename Call>
+    static void run(const torch::Tensor& angles, const tpl_a2b_config& cfg, int dt, int B, int L, const char* where,
+                    Call call) {
+        constexpr const char* kLayer = "torchproteinlibrary_amd.ReducedModel.Angles2Backbone.Angles2Backbone";
+        constexpr uint32_t kLost = TPL_A2B_STATUS_TIMEOUT | TPL_A2B_STATUS_SYNC;
+        const hipStream_t s = stream_of(angles);
+        const torch::Tensor sync = sync_buffer(angles.device(), (int64_t)tpl_a2b_sync_bytes(dt, B, L, &cfg));
+        uint32_t bits = 0;
+        for (bool first = true;; first = false) {
+            bits = native_fn::run(s, [&](uint32_t* flags) {
+                check_rc(call(s, sync.data_ptr(), flags), where);
+            });
+            if (!(bits & kLost)) break;
+            sync_clear(sync);  // look-back words may be left set
+            native_fn::python(kLayer, "_report_lost", bits, where, first);  // warns, then raises
+        }
+        if (bits) native_fn::python(kLayer, "_raise_on_bits", bits, where);
+    }
+    static torch::Tensor forward(torch::autograd::AutogradContext* ctx, torch::Tensor angles, torch::Tensor lengths,
+                                 std::vector<int64_t> config, bool needs) {
+        auto [B, L] = check_inputs(angles, lengths);
+        const tpl_a2b_config cfg = to_config(config);
+        const int dt = dtype_code(angles);
+        c10::DeviceGuard guard(angles.device());
+        torch::Tensor coords = torch::empty({B, 9 * (int64_t)L}, angles.options()), state;
+        if (needs)
+            state = torch::empty({(int64_t)tpl_a2b_state_bytes(dt, B, L, &cfg)}, angles.options().dtype(torch::kByte));
+        run(angles, cfg, dt, B, L, "forward", [&, B = B, L = L](hipStream_t s, void* sync, uint32_t* flags) {
+            return tplx_a2b_forward(dt, angles.data_ptr(), coords.data_ptr(), lengths.data_ptr<int32_t>(),
+                                    needs && state.nbytes() ? state.data_ptr() : nullptr, sync, flags, B, L, &cfg, s);
+        });
+        if (needs) ctx->save_for_backward({angles, lengths, state});
+        ctx->saved_data["config"] = config;
+        return coords;
+    }
+    static native_fn::variable_list backward(torch::autograd::AutogradContext* ctx, native_fn::variable_list grads) {
+        const auto saved = ctx->get_saved_variables();
+        return native_fn::backward(grads, [&]() -> native_fn::variable_list {
+            const torch::Tensor &angles = saved[0], &lengths = saved[1], &state = saved[2];
+            auto [B, L] = check_inputs(angles, lengths);
+            const tpl_a2b_config cfg = to_config(ctx->saved_data["config"].toIntVector());
+            const int dt = dtype_code(angles);
+            c10::DeviceGuard guard(angles.device());
+            const torch::Tensor g = native_fn::like_dtype(grads[0], angles);
+            check_out(g, angles, {B, 9 * (int64_t)L}, "gradOutput");
+            torch::Tensor out = torch::empty({B, 3, L}, angles.options());
+            const void* st = opt_ptr(state, tpl_a2b_state_bytes(dt, B, L, &cfg), "state", angles);
+            run(angles, cfg, dt, B, L, "backward", [&, B = B, L = L](hipStream_t s, void* sync, uint32_t* flags) {
+                return tplx_a2b_backward(dt, out.data_ptr(), g.data_ptr(), angles.data_ptr(),
+                                         lengths.data_ptr<int32_t>(), st, sync, flags, B, L, &cfg, s);
+            });
+            return {out, torch::Tensor(), torch::Tensor(), torch::Tensor()};
+        });
+    }
+};
+
+bool plain(torch::Tensor angles, torch::Tensor lengths) { return native_fn::plain({&angles, &lengths}); }
+
+torch::Tensor apply(torch::Tensor angles, torch::Tensor lengths, std::vector<int64_t> config) {
+    return Angles2Backbone::apply(angles, lengths, config, native_fn::needs_grad(angles));
+}
+
 // One forward+backward step over fixed buffers: everything is checked once,
 // and run() only launches, on the current stream (or into the capture that is
 // open on it).  Each run reads angles, lengths and grad_output from their
@@ -551,6 +634,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
           pybind11::call_guard<pybind11::gil_scoped_release>());
     m.def("Angles2BackboneGPU_backward_checked", &backward_checked, "status bits of the backward, once it has run",
           pybind11::call_guard<pybind11::gil_scoped_release>());
+    m.def("Angles2Backbone_plain", &plain, "whether a call is a plain one");
+    m.def("Angles2Backbone_apply", &apply, "a plain differentiable call",
+          pybind11::call_guard<pybind11::gil_scoped_release>());
+    m.def("sync_buffer", [](const torch::Tensor& like, int64_t bytes) { return sync_buffer(like.device(), bytes); },
+          "the look-back buffer of the current stream");
     m.def("Angles2BackboneCPU_forward", &cpu_forward, "Angles2Backbone cpu forward (float64)");
     m.def("Angles2BackboneCPU_backward", &cpu_backward, "Angles2Backbone cpu backward (float64, O(L) adjoint)");
     m.def("Angles2BackboneGPU_forward_plain", &forward_plain, "plain serial forward");

@@ -9,11 +9,14 @@
 #include <torch/extension.h>
 #include <c10/hip/HIPStream.h>
 
+#include <algorithm>
+#include <string>
 #include <tuple>
 #include <vector>
 
 #include "a2c_flagged.h"
 #include "host_flags.h"
+#include "native_fn.h"
 #include "tpl_a2c.h"
 
 namespace {
@@ -193,6 +196,108 @@ void backward(torch::Tensor grad_atoms, torch::Tensor grad_angles, torch::Tensor
     backward_coords(grad_atoms, grad_angles, sequences, coords, status, c10::nullopt);
 }
 
+// The autograd function of a plain call (native_fn.h); what it does is written
+// at Angles2CoordsFunction.
+constexpr const char* kLayer = "torchproteinlibrary_amd.FullAtomModel.Angles2Coords.Angles2Coords";
+using native_fn::variable_list;
+using torch::Tensor;
+using torch::autograd::AutogradContext;
+
+struct Angles2Coords : torch::autograd::Function<Angles2Coords> {
+    static variable_list forward(AutogradContext* ctx, Tensor angles, Tensor sequences, int64_t max_atoms,
+                                 c10::optional<Tensor> order) {
+        angles = angles.contiguous();
+        const torch::Device dev = angles.device();
+        c10::DeviceGuard guard(dev);
+        const Tensor seqs = sequences.to(dev).contiguous();
+        check_common(seqs, angles);
+        if (order.has_value()) order = order->to(dev).contiguous();
+        const int64_t B = angles.size(0);
+        const auto bytes = angles.options().dtype(torch::kByte);
+        Tensor coords = torch::empty({B, 3 * max_atoms}, angles.options());
+        Tensor res_names = torch::empty({B, max_atoms, 4}, bytes), atom_names = torch::empty({B, max_atoms, 4}, bytes);
+        const hipStream_t s = stream_of(angles);
+        const uint32_t bits = native_fn::run(s, [&](uint32_t* flags) {
+            forward_on(seqs, angles, coords, res_names, atom_names, nullptr, flags, order, s);
+        });
+        if (bits) native_fn::python(kLayer, "_check", bits, coords, "forward");
+        ctx->save_for_backward({seqs, coords});
+        ctx->saved_data["length"] = angles.size(2);
+        ctx->saved_data["order"] = order;
+        ctx->mark_non_differentiable({res_names, atom_names});
+        return {coords, res_names, atom_names};
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list grads) {
+        const auto saved = ctx->get_saved_variables();
+        return native_fn::backward(grads, [&]() -> variable_list {
+            const Tensor &seqs = saved[0], &coords = saved[1], g = grads[0].contiguous();
+            c10::DeviceGuard guard(coords.device());
+            const hipStream_t s = stream_of(coords);
+            Tensor out = torch::empty({coords.size(0), 8, ctx->saved_data["length"].toInt()}, coords.options());
+            check_common(seqs, out);
+            const auto order = ctx->saved_data["order"].toOptional<Tensor>();
+            const uint32_t bits = native_fn::run(s, [&](uint32_t* flags) {
+                backward_on(g, out, seqs, coords, nullptr, flags, order, s);
+            });
+            if (bits) native_fn::python(kLayer, "_check", bits, out, "backward");
+            return {out, Tensor(), Tensor(), Tensor()};
+        });
+    }
+};
+
+// (coords, res_names, atom_names), or nothing if the call is not a plain one.
+// max_atoms < 0: the largest of num_atoms, read from wherever it is (B integers
+// straight to the host; the largest found by a kernel first takes longer).
+c10::optional<std::tuple<Tensor, Tensor, Tensor>> apply(Tensor angles, Tensor sequences, Tensor num_atoms,
+                                                        c10::optional<Tensor> order, int64_t max_atoms) {
+    if (!native_fn::plain({&angles}) || sequences.requires_grad() || num_atoms.requires_grad() ||
+        !torch::isIntegralType(num_atoms.scalar_type(), false) || angles.dim() != 3 || angles.size(1) != 8)
+        return c10::nullopt;
+    if (max_atoms < 0) {
+        const Tensor n = num_atoms.to(torch::kCPU).to(torch::kLong).contiguous();
+        const int64_t* p = n.data_ptr<int64_t>();
+        max_atoms = n.numel() ? *std::max_element(p, p + n.numel()) : 0;
+    }
+    auto out = Angles2Coords::apply(angles, sequences, max_atoms, order);
+    return std::make_tuple(out[0], out[1], out[2]);
+}
+
+// The sequences of a call as the device wants them: (atom counts, the uint8
+// [batch, longest + 1] tensor of convertStringList on the device, the counts as
+// int32 on the device), copied from pinned memory without a wait; None if
+// a sequence is not a string of the 20 letters, or a capture is open (the
+// copies would read their staging memory again on each replay).
+pybind11::object prepare(pybind11::list sequences, torch::Tensor angles) {
+    namespace py = pybind11;
+    const size_t B = sequences.size();
+    if (B == 0 || !angles.is_cuda()) return py::none();
+    c10::DeviceGuard guard(angles.device());
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream_of(angles), &capture) != hipSuccess || capture != hipStreamCaptureStatusNone)
+        return py::none();
+    std::vector<std::pair<const char*, size_t>> s(B);
+    size_t longest = 0;
+    std::vector<int32_t> counts(B);
+    for (size_t i = 0; i < B; ++i) {
+        PyObject* o = PyList_GET_ITEM(sequences.ptr(), (Py_ssize_t)i);
+        if (!PyUnicode_CheckExact(o) || !PyUnicode_IS_COMPACT_ASCII(o)) return py::none();
+        s[i] = {reinterpret_cast<const char*>(PyUnicode_1BYTE_DATA(o)), (size_t)PyUnicode_GET_LENGTH(o)};
+        counts[i] = tpl_a2c_num_atoms(s[i].first);
+        if (counts[i] < 0 || std::strlen(s[i].first) != s[i].second) return py::none();
+        longest = std::max(longest, s[i].second);
+    }
+    const auto pinned = torch::TensorOptions().pinned_memory(true);
+    const Tensor seqs = torch::empty({(int64_t)B, (int64_t)longest + 1}, pinned.dtype(torch::kByte));
+    const Tensor n = torch::empty({(int64_t)B}, pinned.dtype(torch::kInt));
+    std::memset(seqs.data_ptr(), 0, seqs.nbytes());
+    for (size_t i = 0; i < B; ++i)
+        std::memcpy(seqs.data_ptr<uint8_t>() + i * (longest + 1), s[i].first, s[i].second);
+    std::memcpy(n.data_ptr(), counts.data(), B * sizeof(int32_t));
+    const Tensor dseqs = seqs.to(angles.device(), /*non_blocking=*/true);
+    const Tensor dn = n.to(angles.device(), /*non_blocking=*/true);
+    return py::make_tuple(counts, dseqs, dn);
+}
+
 int num_atoms(const std::string& sequence) {
     const int n = tpl_a2c_num_atoms(sequence.c_str());
     TORCH_CHECK(n >= 0, "getSeqNumAtoms: sequence holds a letter outside the 20 amino acids: ", sequence);
@@ -282,6 +387,9 @@ void register_a2c(pybind11::module& m) {
     m.def("Angles2Coords_backward_checked", &backward_checked, "status bits of the backward, once it has run",
           py::arg("grad_atoms"), py::arg("grad_angles"), py::arg("sequences"), py::arg("coords"), od,
           py::call_guard<py::gil_scoped_release>());
+    m.def("Angles2Coords_apply", &apply, "a plain differentiable call: (coords, names, names), or None",
+          py::call_guard<py::gil_scoped_release>());
+    m.def("Angles2Coords_prepare", &prepare, "atom counts and device tensors of sequences, or None");
     m.def("getSeqNumAtoms", &num_atoms, "atoms of a sequence", py::arg("sequence"));
     m.def("a2c_bench", &bench, "average event ms of Angles2Coords (step, fwd, bwd)");
 }

@@ -13,6 +13,7 @@
 #include <vector>
 
 #include "host_flags.h"
+#include "native_fn.h"
 #include "rmsd_flagged.h"
 #include "tpl_rmsd.h"
 
@@ -150,6 +151,59 @@ int64_t backward_checked(torch::Tensor grad_input, torch::Tensor grad_rmsd, torc
     });
 }
 
+// The autograd function of a plain call (native_fn.h); what it does is written
+// at Coords2RMSDFunction.
+constexpr const char* kLayer = "torchproteinlibrary_amd.RMSD.Coords2RMSD.Coords2RMSD";
+
+struct Coords2RMSD : torch::autograd::Function<Coords2RMSD> {
+    static native_fn::variable_list forward(torch::autograd::AutogradContext* ctx, torch::Tensor x, torch::Tensor y,
+                                            torch::Tensor n, bool needs) {
+        auto [B, A] = check_inputs(x, y, n);
+        c10::DeviceGuard guard(x.device());
+        const hipStream_t s = stream_of(x);
+        const int dt = dtype_code(x);
+        torch::Tensor rmsd = torch::empty({B}, x.options()), UT = torch::empty({B, 3, 3}, x.options()), state;
+        if (needs)
+            state = torch::empty({std::max<int64_t>(1, (int64_t)tpl_rmsd_state_bytes(B))},
+                                 x.options().dtype(torch::kByte));
+        const uint32_t bits = native_fn::run(s, [&, B = B, A = A](uint32_t* flags) {
+            check_rc(tplx_rmsd_forward(dt, x.data_ptr(), y.data_ptr(), n.data_ptr<int32_t>(), rmsd.data_ptr(),
+                                       UT.data_ptr(), needs ? state_ptr(state, B, x) : nullptr, flags, B, A, s),
+                     "Coords2RMSDGPU_forward");
+        });
+        if (bits) native_fn::python(kLayer, "_raise_on_bits", bits, "forward");
+        ctx->mark_non_differentiable({UT});
+        if (needs) ctx->save_for_backward({x, y, n, state});
+        return {rmsd, UT};
+    }
+    static native_fn::variable_list backward(torch::autograd::AutogradContext* ctx, native_fn::variable_list grads) {
+        const auto saved = ctx->get_saved_variables();
+        return native_fn::backward(grads, [&]() -> native_fn::variable_list {
+            const torch::Tensor &x = saved[0], &y = saved[1], &n = saved[2];
+            auto [B, A] = check_inputs(x, y, n);
+            c10::DeviceGuard guard(x.device());
+            const hipStream_t s = stream_of(x);
+            const torch::Tensor g = native_fn::like_dtype(grads[0], x);
+            check_like(g, x, {B}, "gradRMSD");
+            torch::Tensor gx = torch::empty_like(x);
+            const uint32_t bits = native_fn::run(s, [&, B = B, A = A](uint32_t* flags) {
+                check_rc(tplx_rmsd_backward(dtype_code(x), gx.data_ptr(), g.data_ptr(), x.data_ptr(), y.data_ptr(),
+                                            n.data_ptr<int32_t>(), state_ptr(saved[3], B, x), flags, B, A, s),
+                         "Coords2RMSDGPU_backward");
+            });
+            if (bits) native_fn::python(kLayer, "_raise_on_bits", bits, "backward");
+            return {gx, torch::Tensor(), torch::Tensor(), torch::Tensor()};
+        });
+    }
+};
+
+// (rmsd, UT), or nothing if the call is not a plain one.
+c10::optional<std::tuple<torch::Tensor, torch::Tensor>> apply(torch::Tensor x, torch::Tensor y, torch::Tensor n) {
+    if (!native_fn::plain({&x, &y, &n})) return c10::nullopt;
+    auto out = Coords2RMSD::apply(x, y, n, native_fn::needs_grad(x));
+    return std::make_tuple(out[0], out[1]);
+}
+
 // Timing loop for bench.py: sets of [input, target, num_atoms, rmsd, UT,
 // state, grad_rmsd, grad_input], rotated per step.  Returns HIP-event ms for
 // `steps` back-to-back forward+backward steps, and the average ms of one
@@ -225,6 +279,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("Coords2RMSDGPU_forward_checked", &forward_checked, "status bits of the forward, once it has run",
           pybind11::call_guard<pybind11::gil_scoped_release>());
     m.def("Coords2RMSDGPU_backward_checked", &backward_checked, "status bits of the backward, once it has run",
+          pybind11::call_guard<pybind11::gil_scoped_release>());
+    m.def("Coords2RMSD_apply", &apply, "a plain differentiable call: (rmsd, UT), or None",
           pybind11::call_guard<pybind11::gil_scoped_release>());
     m.def("state_bytes", &state_bytes, "forward->backward state bytes for a batch");
     m.def("bench", &bench, "time fwd+bwd steps and each kernel alone (event ms)");

@@ -14,6 +14,7 @@
 #include <vector>
 
 #include "host_flags.h"
+#include "native_fn.h"
 #include "tpl_xform.h"
 #include "xform_flagged.h"
 
@@ -206,6 +207,124 @@ int64_t center_backward_checked(torch::Tensor grad_output_center, torch::Tensor 
     });
 }
 
+// The autograd functions of plain calls (native_fn.h); what they do is written
+// at the Python functions of the same names.
+using native_fn::variable_list;
+using torch::Tensor;
+using torch::autograd::AutogradContext;
+
+void report(uint32_t bits, const Tensor& out, const char* name, const char* where) {
+    if (bits)
+        native_fn::python("torchproteinlibrary_amd.FullAtomModel.CoordsTransform.CoordsTransform", "_check", bits, out,
+                          name, where);
+}
+
+Tensor rotated(const Tensor& in, const Tensor& R, const Tensor& n, int transpose, const char* where) {
+    auto [B, A] = check_coords(in, n);
+    check_like(R, in, {B, 3, 3}, "R");
+    c10::DeviceGuard guard(in.device());
+    const hipStream_t s = stream_of(in);
+    Tensor out = torch::empty_like(in);
+    const uint32_t bits = native_fn::run(s, [&, B = B, A = A](uint32_t* flags) {
+        check_rc(tplx_xform_rotate(dtype_code(in), out.data_ptr(), in.data_ptr(), R.data_ptr(), transpose,
+                                   n.data_ptr<int32_t>(), flags, B, A, s),
+                 transpose ? "CoordsRotateGPU_backward" : "CoordsRotateGPU_forward");
+    });
+    report(bits, out, "CoordsRotateFunction", where);
+    return out;
+}
+
+struct CoordsTranslate : torch::autograd::Function<CoordsTranslate> {
+    static Tensor forward(AutogradContext* ctx, Tensor x, Tensor T, Tensor n) {
+        ctx->save_for_backward({T, n});
+        T = T.contiguous();
+        auto [B, A] = check_coords(x, n);
+        check_like(T, x, {B, 3}, "T");
+        c10::DeviceGuard guard(x.device());
+        const hipStream_t s = stream_of(x);
+        Tensor out = torch::empty_like(x);
+        const uint32_t bits = native_fn::run(s, [&, B = B, A = A](uint32_t* flags) {
+            check_rc(tplx_xform_translate(dtype_code(x), out.data_ptr(), x.data_ptr(), T.data_ptr(),
+                                          n.data_ptr<int32_t>(), flags, B, A, s),
+                     "CoordsTranslateGPU_forward");
+        });
+        report(bits, out, "CoordsTranslateFunction", "forward");
+        return out;
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list grads) {
+        const auto saved = ctx->get_saved_variables();
+        return native_fn::backward(grads, [&]() -> variable_list {
+            const Tensor g = grads[0].contiguous();
+            Tensor gx = torch::empty_like(g);
+            translate_backward(g, gx, saved[0], saved[1], c10::nullopt);
+            return {gx, Tensor(), Tensor()};
+        });
+    }
+};
+
+struct CoordsRotate : torch::autograd::Function<CoordsRotate> {
+    static Tensor forward(AutogradContext* ctx, Tensor x, Tensor R, Tensor n) {
+        R = R.contiguous();
+        ctx->save_for_backward({R, n});
+        return rotated(x, R, n, 0, "forward");
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list grads) {
+        const auto saved = ctx->get_saved_variables();
+        return native_fn::backward(grads, [&]() -> variable_list {
+            return {rotated(grads[0].contiguous(), saved[0], saved[1], 1, "backward"), Tensor(), Tensor()};
+        });
+    }
+};
+
+struct Coords2Center : torch::autograd::Function<Coords2Center> {
+    static Tensor forward(AutogradContext* ctx, Tensor x, Tensor n) {
+        ctx->save_for_backward({x, n});
+        auto [B, A] = check_coords(x, n);
+        c10::DeviceGuard guard(x.device());
+        const hipStream_t s = stream_of(x);
+        Tensor center = torch::empty({B, 3}, x.options());
+        const uint32_t bits = native_fn::run(s, [&, B = B, A = A](uint32_t* flags) {
+            check_rc(tplx_xform_center(dtype_code(x), center.data_ptr(), x.data_ptr(), n.data_ptr<int32_t>(), flags,
+                                       B, A, s),
+                     "Coords2CenterGPU_forward");
+        });
+        report(bits, center, "Coords2CenterFunction", "forward");
+        return center;
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list grads) {
+        const auto saved = ctx->get_saved_variables();
+        return native_fn::backward(grads, [&]() -> variable_list {
+            const Tensor &x = saved[0], &n = saved[1], g = grads[0].contiguous();
+            auto [B, A] = check_coords(x, n);
+            check_like(g, x, {B, 3}, "output_center");
+            c10::DeviceGuard guard(x.device());
+            const hipStream_t s = stream_of(x);
+            Tensor gx = torch::empty_like(x);
+            const uint32_t bits = native_fn::run(s, [&, B = B, A = A](uint32_t* flags) {
+                check_rc(tplx_xform_center_backward(dtype_code(x), gx.data_ptr(), g.data_ptr(),
+                                                    n.data_ptr<int32_t>(), flags, B, A, s),
+                         "Coords2CenterGPU_backward");
+            });
+            report(bits, gx, "Coords2CenterFunction", "backward");
+            return {gx, Tensor()};
+        });
+    }
+};
+
+// The result, or nothing if the call is not a plain one.
+c10::optional<Tensor> translate_apply(Tensor x, Tensor T, Tensor n) {
+    if (!native_fn::plain({&x, &T, &n})) return c10::nullopt;
+    return CoordsTranslate::apply(x, T, n);
+}
+c10::optional<Tensor> rotate_apply(Tensor x, Tensor R, Tensor n) {
+    if (!native_fn::plain({&x, &R, &n})) return c10::nullopt;
+    return CoordsRotate::apply(x, R, n);
+}
+c10::optional<Tensor> center_apply(Tensor x, Tensor n) {
+    if (!native_fn::plain({&x, &n})) return c10::nullopt;
+    return Coords2Center::apply(x, n);
+}
+
 // Timing loop for bench.py: sets of [coords, out, T, R, center, num_atoms],
 // rotated per launch.  Returns the average HIP-event ms of one launch of
 // translate, rotate, centre and centre-backward, each run `reps` times.
@@ -291,6 +410,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("CoordsRotateGPU_backward_checked", &rotate_backward_checked, "Status bits of the backward", nogil);
     m.def("Coords2CenterGPU_forward_checked", &center_forward_checked, "Status bits of the forward", nogil);
     m.def("Coords2CenterGPU_backward_checked", &center_backward_checked, "Status bits of the backward", nogil);
+    m.def("CoordsTranslate_apply", &translate_apply, "a plain differentiable call, or None", nogil);
+    m.def("CoordsRotate_apply", &rotate_apply, "a plain differentiable call, or None", nogil);
+    m.def("Coords2Center_apply", &center_apply, "a plain differentiable call, or None", nogil);
     m.def("bench", &bench, "average event ms of translate, rotate, centre, centre-backward");
     register_a2c(m);
     register_pdb(m);
