@@ -76,7 +76,8 @@ enum tpl_a2b_error {
  * by a decoupled look-back.  When a chain has at most 4 chunks and every
  * chain's workgroup fits on the device at once, one workgroup takes a whole
  * chain instead (a wave per chunk, the chunks meeting in LDS; the sync words
- * go unused).  The backward chunk is also the checkpoint stride: the forward
+ * go unused).  In the forward, other batches of at most 4096 chains of 3 to 8
+ * chunks are packed into workgroups in the same way.  The backward chunk is also the checkpoint stride: the forward
  * saves the FP64 frame at every backward-chunk boundary, so forward and
  * backward of one step must use the same config. */
 typedef struct tpl_a2b_config {

@@ -284,7 +284,8 @@ class Angles2BackboneStep:
     A step reads ``angles``, ``angles_length`` and ``grad_coords`` from their
     memory at every replay, so a loop updates them in place between replays;
     it writes ``coords`` and ``grad_angles``.  A replay under a capture is
-    captured.  The chunk sizes are the tuned ones for these inputs, or
+    captured.  The chunk sizes are the tuned ones for these inputs (the
+    backward's for both directions where the step has kernels of its own), or
     ``config`` (forward, backward residues per lane).
 
     Replays do not check for NaN or out-of-range lengths (the checks of the
@@ -302,8 +303,15 @@ class Angles2BackboneStep:
         if angles.dtype not in (torch.float32, torch.float64) or angles_length.dtype != torch.int32:
             raise RuntimeError("Angles2BackboneStep: angles must be float32 or float64, angles_length int32")
         B, _, L = angles.shape
-        cfg = tuple(config) if config is not None else _tuning.config_for(angles, angles_length)
         dev, dt = angles.device, angles.dtype
+        if config is not None:
+            cfg = tuple(config)
+        else:
+            cfg = _tuning.config_for(angles, angles_length)
+            own = (cfg[1], cfg[1])
+            with torch.cuda.device(dev):
+                if ext.step_fits(dt == torch.float64, B, L, list(own)):
+                    cfg = own
         self.angles = angles
         self.angles_length = angles_length
         self.config = cfg

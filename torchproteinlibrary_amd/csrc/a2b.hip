@@ -32,8 +32,9 @@
 //     walks its atoms once more for the gradients.
 // Chain kernels (a2b_fwd_chain / a2b_bwd_chain): the same chunk steps with
 // one workgroup per chain of at most 4 chunks, the chunks meeting in LDS
-// instead of through the look-back; used when every chain's workgroup is
-// resident at once.
+// instead of through the look-back, used when every chain's workgroup is
+// resident at once; the forward also packs chains of up to 8 chunks into
+// workgroups by their number of chunks.
 // Plain kernels (a2b_fwd_plain / a2b_bwd_plain) restate the reference GPU
 // algorithm without the O(L^2) derivative tensor: they are the baseline.
 #include <hip/hip_runtime.h>
@@ -992,34 +993,182 @@ __global__ void __launch_bounds__(64) a2b_fwd_chunk(ChunkArgs a) {
     fwd_slot<T, R>(a, slot_at(a, C, st, j), s_x, s_tab, tab);
 }
 
+// ------------------------------------------------------------ chain kernels
+// BINS: every workgroup reads all lengths, at most 16 to a thread.
+constexpr int bins_max_batch(int waves) { return std::min(4096, 16 * 64 * waves); }
+__device__ __forceinline__ int chunks_of(int n, int C) { return (n + C - 1) / C; }
+
+// Share f of F of the zeros of dst[0, count), by one wave.
+template <typename T>
+__device__ __forceinline__ void store_zeros(T* dst, int count, int f, int F, int lane) {
+    constexpr int V = 16 / (int)sizeof(T);
+    const int mis = (int)((reinterpret_cast<uintptr_t>(dst) / sizeof(T)) % V);
+    const int head = min((V - mis) % V, count);
+    const int nvec = (count - head) / V;
+    const int tail0 = head + nvec * V;
+    const u32x4 z = {0u, 0u, 0u, 0u};
+    for (int k = 64 * f + lane; k < nvec; k += 64 * F) __builtin_nontemporal_store(z, reinterpret_cast<u32x4*>(dst + head) + k);
+    if (f == 0) {
+        if (lane < head) dst[lane] = (T)0;
+        if (tail0 + lane < count) dst[tail0 + lane] = (T)0;
+    }
+}
+
+__device__ __forceinline__ int wave_scan_int(int v) {
+    v += __builtin_amdgcn_update_dpp(0, v, kRowShr1, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, kRowShr2, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, kRowShr4, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, kRowShr8, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, kRowBcast15, 0xa, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, kRowBcast31, 0xc, 0xf, false);
+    return v;
+}
+
+// BINS: a chain of nreal chunks takes a slot of nreal waves rounded up to a
+// power of two, and the workgroups of W waves take W / slot chains of one slot
+// size each, the longest chains first; with mixed lengths nearly every wave has
+// a chunk (B=1024 of lengths 30..1000, C = 256, W = 4: 455 workgroups with work
+// instead of 1024).  Each workgroup finds its chains from the lengths.
+//
+// The chains of this workgroup: s_chain[q], q < W / size, or -1; returns the
+// slot size (0: the workgroup has none).  Slot sizes are 2^k, k < 4; counts of
+// the four travel packed, 16 bits each, two to an int.
+template <int R, int W>
+__device__ __forceinline__ int find_chains(const ChunkArgs& a, int* s_chain, int (*s_count)[2], int& nwg) {
+    constexpr int C = 64 * R, NT = 64 * W;
+    const int tid = (int)threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int per = (a.B + NT - 1) / NT, b0 = tid * per;  // per <= 16
+    uint32_t logs = 0;  // of the thread's chains: log2 of the slot size, 2 bits each
+    int c[2] = {0, 0};
+    for (int e0 = 0; e0 < per; e0 += 4) {
+        int raw[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) raw[e] = e0 + e < per && b0 + e0 + e < a.B ? a.lengths[b0 + e0 + e] : -1;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int n = min(max(raw[e], 0), a.L);
+            const int k = (n > C) + (n > 2 * C) + (n > 4 * C);
+            if (e0 + e < per && b0 + e0 + e < a.B) {
+                logs |= (uint32_t)k << (2 * (e0 + e));
+                c[k >> 1] += 1 << (16 * (k & 1));
+            }
+        }
+    }
+    const int i0 = wave_scan_int(c[0]), i1 = wave_scan_int(c[1]);
+    if (lane == 63) {
+        s_count[wave][0] = i0;
+        s_count[wave][1] = i1;
+    }
+    if (tid < W) s_chain[tid] = -1;
+    __syncthreads();
+    int before[2] = {i0 - c[0], i1 - c[1]}, total[2] = {0, 0};
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            if (w < wave) before[h] += s_count[w][h];
+            total[h] += s_count[w][h];
+        }
+    }
+    int g = (int)blockIdx.x, size = 0, mine = -1;
+    nwg = 0;
+#pragma unroll
+    for (int k = 3; k >= 0; --k) {
+        const int n = (total[k >> 1] >> (16 * (k & 1))) & 0xffff, per_wg = W >> k;
+        const int wgs = per_wg > 0 ? (n + per_wg - 1) / per_wg : 0;
+        nwg += wgs;
+        if (size == 0) {
+            if (g < wgs) {
+                size = 1 << k;
+                mine = k;
+            } else {
+                g -= wgs;
+            }
+        }
+    }
+    if (size > 0) {
+        const int per_wg = W / size, r0 = g * per_wg;
+        int r = (before[mine >> 1] >> (16 * (mine & 1))) & 0xffff;
+        for (int e = 0; e < per && r < r0 + per_wg; ++e)
+            if (b0 + e < a.B && (int)(logs >> (2 * e) & 3u) == mine) {
+                if (r >= r0) s_chain[r - r0] = b0 + e;
+                ++r;
+            }
+    }
+    __syncthreads();
+    return size;
+}
+
+// This wave's place: chunk c of chain b (< 0: none), whose chunks are on waves
+// first .. first + size - 1 of the workgroup; nwg workgroups have work (BINS).
+// size = 0: the workgroup has none.  Without BINS workgroup b takes chain b,
+// its slots rotated as the workgroups come round to a CU (8 XCDs of 32 CUs).
+struct Place {
+    int b, c, first, size, nwg;
+};
+template <int R, int W, bool BINS>
+__device__ __forceinline__ Place place_wave(const ChunkArgs& a, int wave, int* s_chain, int (*s_count)[2]) {
+    Place p{};
+    if constexpr (BINS) {
+        p.size = find_chains<R, W>(a, s_chain, s_count, p.nwg);
+        if (p.size == 0) return p;
+        p.b = __builtin_amdgcn_readfirstlane(s_chain[wave / p.size]);
+        p.first = wave / p.size * p.size;
+        p.c = wave - p.first;
+    } else {
+        p.b = (int)blockIdx.x;
+        p.size = W;
+        p.c = (int)((uint32_t)(wave + (p.b >> 3) + (p.b >> 8)) % W);
+    }
+    return p;
+}
+
+// Calls zeros(chain, f, F) so that share f of F of each chain's padding is this
+// wave's: in BINS the chains go over all waves that have work, quarter by
+// quarter (the workgroups of the short chains would have nearly all of it).
+template <int W, bool BINS, typename Zeros>
+__device__ __forceinline__ void spread_zeros(const ChunkArgs& a, const Place& p, int wave, Zeros zeros) {
+    if constexpr (BINS) {
+        for (int u = (int)blockIdx.x * W + wave; u < 4 * a.B; u += p.nwg * W) zeros(u >> 2, u & 3, 4);
+    } else {
+        zeros(p.b, p.c, W);
+    }
+}
+__device__ __forceinline__ int chain_length(const ChunkArgs& a, int b) {
+    const int raw = a.lengths[b];
+    return raw < 0 ? 0 : (raw > a.L ? a.L : raw);
+}
+
 // ------------------------------------------------------------ forward chain
 // Chains of at most kChainMax chunks (L <= kChainMax * C) can skip the
 // look-back: one workgroup per chain, one wave per chunk slot, and the
 // chunks' aggregates meet in LDS across one barrier.  No tickets, records or
 // done counters, and each wave finds its chunk from the workgroup index.
-// Wave w takes slot (w + b) mod W, so that a chain's first chunk, the only
-// one every chain has, does not always fall on the same wave (and SIMD).
-// Otherwise as fwd_slot: pass 1, DPP scan, E = (earlier chunks' aggregates
-// in order) * (lane prefix), checkpoints, pass 2, stores; the slot right
-// past the chain writes its zeros.
-constexpr int kChainMax = 4;
+// The slots rotate over the waves, so that a chain's first chunk, the only one
+// every chain has, does not always fall on the same wave (and SIMD).  Otherwise
+// as fwd_slot: pass 1, DPP scan, E = (earlier chunks' aggregates in order) *
+// (lane prefix), checkpoints, pass 2, stores.  Figures at launch_chain.
+constexpr int kChainMax = 4, kBinsMax = 8;
 
-template <typename T, int R, int W>
+template <typename T, int R, int W, bool BINS>
 __global__ void __launch_bounds__(64 * W) a2b_fwd_chain(ChunkArgs a) {
     constexpr int C = 64 * R;
     constexpr int E9 = 9 * R;
     extern __shared__ __align__(16) unsigned char s_dyn[];
     __shared__ double s_tab[128];
     __shared__ double s_agg[W][kF];
-    const int wave = (int)(threadIdx.x >> 6), lane = (int)(threadIdx.x & 63);
-    const int b = (int)blockIdx.x, L = a.L;
-    const int raw = a.lengths[b];
-    const int n = raw < 0 ? 0 : (raw > L ? L : raw);
-    const int nreal = (n + C - 1) / C;
-    const int c = (wave + (b >> 3) + (b >> 8)) % W;  // this wave's chunk slot
-    const bool real = c < nreal;
-    if (raw != n && threadIdx.x == 0) report_bits(a.rep, TPL_A2B_STATUS_LENGTH);
+    __shared__ int s_chain[BINS ? W : 1], s_count[BINS ? W : 1][2];
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = (int)(threadIdx.x & 63);
     for (int i = (int)threadIdx.x; i < 128; i += 64 * W) s_tab[i] = kTabCS[i];
+    const Place pl = place_wave<R, W, BINS>(a, wave, s_chain, s_count);
+    if (BINS && pl.size == 0) return;
+    const int c = pl.c, L = a.L;
+    const bool some = !BINS || pl.b >= 0;
+    const int b = some ? pl.b : 0;
+    const int n = some ? chain_length(a, b) : 0;
+    const int nreal = (n + C - 1) / C;
+    const bool real = c < nreal;
+    if (some && c == 0 && lane == 0 && a.lengths[b] != n) report_bits(a.rep, TPL_A2B_STATUS_LENGTH);
     T* s_x = reinterpret_cast<T*>(s_dyn) + (size_t)wave * 9 * C;
     T* s_l = s_x + lane * E9;
     T* xrow = static_cast<T*>(a.coords) + (size_t)b * 9 * L;
@@ -1029,7 +1178,7 @@ __global__ void __launch_bounds__(64 * W) a2b_fwd_chain(ChunkArgs a) {
     const int cnt = min(max(n - rl, 0), R);
     T ang[3][R];
     if (real) lane_load_rows<T, R>(arow + rl, L, cnt, L - rl, ang);
-    __syncthreads();  // s_tab
+    if (!BINS) __syncthreads();  // s_tab (find_chains ends with a barrier)
 
     // Pass 1 and the wave's scan.
     double E[kF];
@@ -1058,29 +1207,29 @@ __global__ void __launch_bounds__(64 * W) a2b_fwd_chain(ChunkArgs a) {
         for (int e = 0; e < kF; ++e) agg[e] = read_lane(E[e], 63);
         if (lane == 0) {
 #pragma unroll
-            for (int e = 0; e < kF; ++e) s_agg[c][e] = agg[e];
+            for (int e = 0; e < kF; ++e) s_agg[pl.first + c][e] = agg[e];
         }
         wave_shift_frames(E);
     }
+    // The zeros past the chains' chunks: nothing is loaded from here on, so the
+    // stores drain behind the rest.
+    spread_zeros<W, BINS>(a, pl, wave, [&](int zb, int f, int F) {
+        const int p = min(chunks_of(chain_length(a, zb), C) * C, L);
+        store_zeros<T>(static_cast<T*>(a.coords) + (size_t)9 * zb * L + (size_t)9 * p, 9 * (L - p), f, F, lane);
+    });
     __syncthreads();  // the aggregates
     if (real && c > 0) {
         double P[kF], Q[kF];
 #pragma unroll
-        for (int e = 0; e < kF; ++e) P[e] = s_agg[0][e];
+        for (int e = 0; e < kF; ++e) P[e] = s_agg[pl.first][e];
         for (int j = 1; j < c; ++j) {
-            frame_rmul_to(P, s_agg[j], Q);
+            frame_rmul_to(P, s_agg[pl.first + j], Q);
 #pragma unroll
             for (int e = 0; e < kF; ++e) P[e] = Q[e];
         }
         frame_lmul(P, E);
     }
-    if (!real) {
-        if (c == nreal) {  // the first slot past the chain writes all its zeros
-            const int f0 = 9 * c * C;
-            wave_store_run<T>(xrow + f0, 9 * L - f0, 0, s_x, lane);
-        }
-        return;
-    }
+    if (!real) return;
 
     // Checkpoint at a backward-chunk boundary inside the chain.
     if (a.ckpt && rl > 0 && rl < n && (rl & (a.K - 1)) == 0) {
@@ -1375,8 +1524,7 @@ __global__ void __launch_bounds__(64) a2b_bwd_chunk(ChunkArgs a) {
 }
 
 // ----------------------------------------------------------- backward chain
-// The backward of chains of at most kChainMax chunks: one workgroup per
-// chain, one wave per chunk slot (slot (w + b) mod W, as in the forward), and
+// The backward of such chains: the places of the forward, and
 // each chunk's sum over its atoms meets the others in LDS across one barrier:
 // chunk c adds the sums of chunks c+1 .. nreal-1, in that order.  Otherwise
 // as bwd_slot.
@@ -1386,15 +1534,14 @@ __global__ void __launch_bounds__(64 * W) a2b_bwd_chain(ChunkArgs a) {
     extern __shared__ double s_dynd[];  // [W][6R][64]: each wave's (cos, sin)
     __shared__ double s_tab[128];
     __shared__ double s_tot[W][6];
-    const int wave = (int)(threadIdx.x >> 6), lane = (int)(threadIdx.x & 63);
-    const int b = (int)blockIdx.x, L = a.L;
-    const int raw = a.lengths[b];
-    const int n = raw < 0 ? 0 : (raw > L ? L : raw);
-    const int nreal = (n + C - 1) / C;
-    const int c = (wave + (b >> 3) + (b >> 8)) % W;  // this wave's chunk slot
-    const bool real = c < nreal;
-    if (raw != n && threadIdx.x == 0) report_bits(a.rep, TPL_A2B_STATUS_LENGTH);
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = (int)(threadIdx.x & 63);
     for (int i = (int)threadIdx.x; i < 128; i += 64 * W) s_tab[i] = kTabCS[i];
+    const Place pl = place_wave<R, W, false>(a, wave, nullptr, nullptr);
+    const int b = pl.b, c = pl.c, L = a.L;
+    const int n = chain_length(a, b);
+    const int nreal = (n + C - 1) / C;
+    const bool real = c < nreal;
+    if (c == 0 && lane == 0 && a.lengths[b] != n) report_bits(a.rep, TPL_A2B_STATUS_LENGTH);
     double* s_cs = s_dynd + (size_t)wave * 6 * R * 64;
     T* grow = static_cast<T*>(a.grad_angles) + (size_t)b * 3 * L;
     const T* arow = static_cast<const T*>(a.angles) + (size_t)b * 3 * L;
@@ -1486,15 +1633,14 @@ __global__ void __launch_bounds__(64 * W) a2b_bwd_chain(ChunkArgs a) {
             for (int e = 0; e < 6; ++e) s_tot[c][e] = tot[e];
         }
     }
-    __syncthreads();  // the chunks' sums
-    if (!real) {
-        if (c == nreal) {  // the first slot past the chain writes all its zeros
+    spread_zeros<W, false>(a, pl, wave, [&](int zb, int f, int F) {
+        const int p = min(chunks_of(chain_length(a, zb), C) * C, L);
 #pragma unroll
-            for (int k = 0; k < 3; ++k)
-                wave_store_run<T>(grow + (size_t)k * L + c * C, L - c * C, 0, static_cast<const T*>(nullptr), lane);
-        }
-        return;
-    }
+        for (int k = 0; k < 3; ++k)
+            store_zeros<T>(static_cast<T*>(a.grad_angles) + ((size_t)3 * zb + k) * L + p, L - p, f, F, lane);
+    });
+    __syncthreads();  // the chunks' sums
+    if (!real) return;
     for (int j = c + 1; j < nreal; ++j) {
 #pragma unroll
         for (int e = 0; e < 6; ++e) S[e] += s_tot[j][e];
@@ -1569,13 +1715,6 @@ __global__ void __launch_bounds__(64 * W) a2b_bwd_chain(ChunkArgs a) {
 // W waves' worth of chunks; what its chunks of one chain need of each other
 // meets in LDS, the frames across one barrier and the sums across a second.
 //
-// BINS: a chain of nreal chunks takes a slot of nreal waves rounded up to a
-// power of two, and the workgroups take W / slot chains of one slot size each,
-// the longest chains first; with mixed lengths nearly every wave has a chunk
-// (B=1024 of lengths 30..1000, W = 4: 455 workgroups of work instead of 1024).
-// Each workgroup finds its chains from the lengths.  Without BINS workgroup b
-// takes chain b (fewer chains than fit on the GPU).
-//
 // A lane's LDS: its (cos, sin) pairs element-major as in the backward, and, in
 // the same memory as they are used up, its coordinates value-major at a stride
 // of 65 values (so that neither the lanes' writes nor the transposing reads
@@ -1604,7 +1743,6 @@ constexpr int step_wave_doubles() {
     return step_lead_doubles<T, R>() + 6 * R * 64;
 }
 constexpr int kStepStride = 65;
-constexpr int kStepMaxBatch = 4096;  // BINS: every workgroup reads all lengths
 
 // The wave's chunk run dst[0, count) from its value-major coordinates: elements
 // at or past nsrc are 0.  Element p is value p % N of lane p / N.
@@ -1637,103 +1775,6 @@ __device__ __forceinline__ void store_transposed(T* dst, int count, int nsrc, co
     }
     if (tail0 + lane < count) dst[tail0 + lane] = value(tail0 + lane);
 }
-
-// Share f of F of the zeros of dst[0, count), by one wave.
-template <typename T>
-__device__ __forceinline__ void store_zeros(T* dst, int count, int f, int F, int lane) {
-    constexpr int V = 16 / (int)sizeof(T);
-    const int mis = (int)((reinterpret_cast<uintptr_t>(dst) / sizeof(T)) % V);
-    const int head = min((V - mis) % V, count);
-    const int nvec = (count - head) / V;
-    const int tail0 = head + nvec * V;
-    const u32x4 z = {0u, 0u, 0u, 0u};
-    for (int k = 64 * f + lane; k < nvec; k += 64 * F) __builtin_nontemporal_store(z, reinterpret_cast<u32x4*>(dst + head) + k);
-    if (f == 0) {
-        if (lane < head) dst[lane] = (T)0;
-        if (tail0 + lane < count) dst[tail0 + lane] = (T)0;
-    }
-}
-
-__device__ __forceinline__ int wave_scan_int(int v) {
-    v += __builtin_amdgcn_update_dpp(0, v, kRowShr1, 0xf, 0xf, false);
-    v += __builtin_amdgcn_update_dpp(0, v, kRowShr2, 0xf, 0xf, false);
-    v += __builtin_amdgcn_update_dpp(0, v, kRowShr4, 0xf, 0xf, false);
-    v += __builtin_amdgcn_update_dpp(0, v, kRowShr8, 0xf, 0xf, false);
-    v += __builtin_amdgcn_update_dpp(0, v, kRowBcast15, 0xa, 0xf, false);
-    v += __builtin_amdgcn_update_dpp(0, v, kRowBcast31, 0xc, 0xf, false);
-    return v;
-}
-
-// The chains of this workgroup: s_chain[q], q < W / size, or -1; returns the
-// slot size (0: the workgroup has none).  Slot sizes are 2^k, k < 4; counts of
-// the four travel packed, 16 bits each, two to an int.
-template <int R, int W>
-__device__ __forceinline__ int find_chains(const ChunkArgs& a, int* s_chain, int (*s_count)[2], int& nwg) {
-    constexpr int C = 64 * R, NT = 64 * W;
-    const int tid = (int)threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const int per = (a.B + NT - 1) / NT, b0 = tid * per;  // per <= 16
-    uint32_t logs = 0;  // of the thread's chains: log2 of the slot size, 2 bits each
-    int c[2] = {0, 0};
-    for (int e0 = 0; e0 < per; e0 += 4) {
-        int raw[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) raw[e] = e0 + e < per && b0 + e0 + e < a.B ? a.lengths[b0 + e0 + e] : -1;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int n = min(max(raw[e], 0), a.L);
-            const int k = (n > C) + (n > 2 * C) + (n > 4 * C);
-            if (e0 + e < per && b0 + e0 + e < a.B) {
-                logs |= (uint32_t)k << (2 * (e0 + e));
-                c[k >> 1] += 1 << (16 * (k & 1));
-            }
-        }
-    }
-    const int i0 = wave_scan_int(c[0]), i1 = wave_scan_int(c[1]);
-    if (lane == 63) {
-        s_count[wave][0] = i0;
-        s_count[wave][1] = i1;
-    }
-    if (tid < W) s_chain[tid] = -1;
-    __syncthreads();
-    int before[2] = {i0 - c[0], i1 - c[1]}, total[2] = {0, 0};
-#pragma unroll
-    for (int w = 0; w < W; ++w) {
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            if (w < wave) before[h] += s_count[w][h];
-            total[h] += s_count[w][h];
-        }
-    }
-    int g = (int)blockIdx.x, size = 0, mine = -1;
-    nwg = 0;
-#pragma unroll
-    for (int k = 3; k >= 0; --k) {
-        const int n = (total[k >> 1] >> (16 * (k & 1))) & 0xffff, per_wg = W >> k;
-        const int wgs = per_wg > 0 ? (n + per_wg - 1) / per_wg : 0;
-        nwg += wgs;
-        if (size == 0) {
-            if (g < wgs) {
-                size = 1 << k;
-                mine = k;
-            } else {
-                g -= wgs;
-            }
-        }
-    }
-    if (size > 0) {
-        const int per_wg = W / size, r0 = g * per_wg;
-        int r = (before[mine >> 1] >> (16 * (mine & 1))) & 0xffff;
-        for (int e = 0; e < per && r < r0 + per_wg; ++e)
-            if (b0 + e < a.B && (int)(logs >> (2 * e) & 3u) == mine) {
-                if (r >= r0) s_chain[r - r0] = b0 + e;
-                ++r;
-            }
-    }
-    __syncthreads();
-    return size;
-}
-
-__device__ __forceinline__ int chunks_of(int n, int C) { return (n + C - 1) / C; }
 
 // Long chains (WALK): one wave per chunk, W chunks of a chain to a workgroup,
 // in two kernels.  a2b_step_sums takes each chunk's frame and its sums (M, F)
@@ -1920,28 +1961,15 @@ __global__ void __launch_bounds__(64 * W) a2b_step(ChunkArgs a) {
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = (int)(threadIdx.x & 63);
     const int L = a.L;
     for (int i = (int)threadIdx.x; i < 128; i += 64 * W) s_tab[i] = kTabCS[i];
-    int nwg = 0;
-    int b, c, size, first = 0;  // the chain, this wave's chunk of it, its slot: waves first .. first + size - 1
+    Place pl{};
     if constexpr (MODE == WALK) {
-        size = 1;
-        walk_slot<W>(a, wave, b, c);
-    } else if constexpr (MODE == BINS) {
-        size = find_chains<R, W>(a, s_chain, s_count, nwg);
-        if (size == 0) return;
-        b = __builtin_amdgcn_readfirstlane(s_chain[wave / size]);
-        first = wave / size * size;
-        c = wave - first;
+        walk_slot<W>(a, wave, pl.b, pl.c);
     } else {
-        b = (int)blockIdx.x;
-        size = W;
-        // rotated as the workgroups come round to a CU (8 XCDs of 32 CUs)
-        c = (int)((uint32_t)(wave + (b >> 3) + (b >> 8)) % W);
+        pl = place_wave<R, W, MODE == BINS>(a, wave, s_chain, s_count);
+        if (MODE == BINS && pl.size == 0) return;
     }
-    int n = 0;
-    if (b >= 0) {
-        const int raw = a.lengths[b];
-        n = raw < 0 ? 0 : (raw > L ? L : raw);
-    }
+    const int b = pl.b, c = pl.c, first = pl.first;
+    const int n = b >= 0 ? chain_length(a, b) : 0;
     const int nreal = (n + C - 1) / C;
     const bool real = b >= 0 && c < nreal;
     double* s_wave = s_dynd + (size_t)wave * step_wave_doubles<T, R>();
@@ -2028,19 +2056,14 @@ __global__ void __launch_bounds__(64 * W) a2b_step(ChunkArgs a) {
     }
     // The zeros past the chains' chunks: nothing is loaded from here on, so the
     // stores drain behind the rest.
-    const auto zeros = [&](int zb, int f, int F) {
-        const int raw = a.lengths[zb];
-        const int p = min(chunks_of(raw < 0 ? 0 : (raw > L ? L : raw), C) * C, L);
-        store_zeros<T>(static_cast<T*>(a.coords) + (size_t)9 * zb * L + (size_t)9 * p, 9 * (L - p), f, F, lane);
+    if constexpr (MODE != WALK)
+        spread_zeros<W, MODE == BINS>(a, pl, wave, [&](int zb, int f, int F) {
+            const int p = min(chunks_of(chain_length(a, zb), C) * C, L);
+            store_zeros<T>(static_cast<T*>(a.coords) + (size_t)9 * zb * L + (size_t)9 * p, 9 * (L - p), f, F, lane);
 #pragma unroll
-        for (int k = 0; k < 3; ++k)
-            store_zeros<T>(static_cast<T*>(a.grad_angles) + ((size_t)3 * zb + k) * L + p, L - p, f, F, lane);
-    };
-    if constexpr (MODE == BINS) {
-        for (int u = (int)blockIdx.x * W + wave; u < 4 * a.B; u += nwg * W) zeros(u >> 2, u & 3, 4);
-    } else if constexpr (MODE == CHAIN) {
-        zeros(b, c, W);
-    }
+            for (int k = 0; k < 3; ++k)
+                store_zeros<T>(static_cast<T*>(a.grad_angles) + ((size_t)3 * zb + k) * L + p, L - p, f, F, lane);
+        });
     if (MODE != WALK) __syncthreads();  // the aggregates
     if (real) {
         if constexpr (MODE == WALK) {
@@ -2383,32 +2406,34 @@ KernelFn fwd_kernel<double>(int r) {
 // kChainMaxLds (W waves' staging), so that with the static LDS (sincos table,
 // aggregates: under 1.5 KB) a workgroup stays within 64 KB.  The largest
 // chain staging in use is 54 KB (FP32 forward with 8 residues per lane and 3
-// slots, or FP64 with 4 and 3).
-constexpr size_t kChainMaxLds = 56u << 10;
+// slots, or FP64 with 4 and 3).  Packed (BINS): W = 4 or 8 waves, at most
+// kBinsMaxLds, of which one workgroup fits on a CU.
+constexpr size_t kChainMaxLds = 56u << 10, kBinsMaxLds = 150u << 10;
 template <typename T, int R>
-KernelFn fwd_chain_w(int w) {
+KernelFn fwd_chain_w(int w, bool bins) {
+    if (bins) return w == 4 ? a2b_fwd_chain<T, R, 4, true> : a2b_fwd_chain<T, R, 8, true>;
     switch (w) {
-        case 1: return a2b_fwd_chain<T, R, 1>;
-        case 2: return a2b_fwd_chain<T, R, 2>;
-        case 3: return a2b_fwd_chain<T, R, 3>;
-        default: return a2b_fwd_chain<T, R, 4>;
+        case 1: return a2b_fwd_chain<T, R, 1, false>;
+        case 2: return a2b_fwd_chain<T, R, 2, false>;
+        case 3: return a2b_fwd_chain<T, R, 3, false>;
+        default: return a2b_fwd_chain<T, R, 4, false>;
     }
 }
 template <typename T>
-KernelFn fwd_chain_kernel(int r, int w) {
+KernelFn fwd_chain_kernel(int r, int w, bool bins) {
     switch (r) {
-        case 1: return fwd_chain_w<T, 1>(w);
-        case 2: return fwd_chain_w<T, 2>(w);
-        case 4: return fwd_chain_w<T, 4>(w);
-        default: return fwd_chain_w<T, 8>(w);
+        case 1: return fwd_chain_w<T, 1>(w, bins);
+        case 2: return fwd_chain_w<T, 2>(w, bins);
+        case 4: return fwd_chain_w<T, 4>(w, bins);
+        default: return fwd_chain_w<T, 8>(w, bins);
     }
 }
 template <>
-KernelFn fwd_chain_kernel<double>(int r, int w) {
+KernelFn fwd_chain_kernel<double>(int r, int w, bool bins) {
     switch (r) {
-        case 1: return fwd_chain_w<double, 1>(w);
-        case 2: return fwd_chain_w<double, 2>(w);
-        default: return fwd_chain_w<double, 4>(w);
+        case 1: return fwd_chain_w<double, 1>(w, bins);
+        case 2: return fwd_chain_w<double, 2>(w, bins);
+        default: return fwd_chain_w<double, 4>(w, bins);
     }
 }
 template <typename T, int R>
@@ -2526,33 +2551,6 @@ int resident_workgroups(KernelFn k, int threads, size_t lds) {
     return cache[key] = per_cu * cus;
 }
 
-// The chain kernels take chains of at most kChainMax chunks whose waves'
-// staging (lds each) fits, one workgroup of a.nc waves per chain, and only
-// when every chain's workgroup is resident from the start.  Otherwise the
-// chunk kernels, whose one-wave workgroups put the work first: at B=1024 of
-// lengths 30-1000 with 4 residues per lane the backward's chain workgroups
-// (218 VGPRs, two per CU) ran in two rounds behind waves with nothing to do,
-// 16.3 -> 21.2 us; where they all fit at once they win (steps of fwd+bwd:
-// 256 x 700 residues 24.6 -> 17.0 us, 512 x 50-500 22.7 -> 17.3 us, 32 x 200
-// 14.9 -> 10.9 us, each at the best config of either form).
-bool chain_fits(KernelFn k, const ChunkArgs& a, size_t lds) {
-    if (a.nc > kChainMax || (size_t)a.nc * lds > kChainMaxLds) return false;
-    return a.B <= resident_workgroups(k, 64 * a.nc, a.nc * lds);
-}
-int launch_chain(KernelFn k, const ChunkArgs& a, size_t lds, hipStream_t stream) {
-    hipLaunchKernelGGL(k, dim3((unsigned)a.B), dim3(64 * a.nc), a.nc * lds, stream, a);
-    return hipGetLastError() == hipSuccess ? TPL_A2B_OK : TPL_A2B_ERR_LAUNCH;
-}
-
-// The step's kernels for a shape with R residues per lane.
-struct StepForm {
-    KernelFn kernel, sums;  // sums: WALK
-    int waves;
-    size_t lds;
-    unsigned grid;
-    size_t rec_bytes;  // WALK: the records
-};
-
 // Dynamic LDS beyond 64 KB has to be allowed per kernel and device, once.
 bool allow_lds(KernelFn k, size_t bytes) {
     static std::mutex mu;
@@ -2567,6 +2565,50 @@ bool allow_lds(KernelFn k, size_t bytes) {
     allowed.insert({dev, p});
     return true;
 }
+
+// Launches the chain kernel of chains of a.nc <= kBinsMax chunks (kernel(waves,
+// bins) gives it, lds the staging of one wave), or returns false.  Chains of at
+// most kChainMax chunks take a workgroup of a.nc waves each, if every workgroup
+// is resident from the start.  In the forward the rest are packed (BINS), if
+// they have more than 2 chunks and the batch is not too large for every
+// workgroup to read its lengths.  Otherwise the chunk kernels, whose one-wave
+// workgroups put the work first.
+//
+// Steps of forward and backward in us, float32, with 4 residues per lane:
+//   chain kernels instead of chunk kernels, all resident, each at its best:
+//     256 x 700 residues 24.6 -> 17.0, 512 x 50..500 22.7 -> 17.0,
+//     32 x 200 14.9 -> 9.9;
+//   forward BINS instead of the chunk kernel (the backward fixed):
+//     400 x 1900 71.1 -> 63.6, 400 x 1300 53.7 -> 49.8, 800 x 500..1000
+//     55.2 -> 54.8, 1024 x 30..1000 54.3 -> 53.8 (2 per lane: 61.4 -> 53.2);
+//     with 2 chunks, 1500 x 500, 55.4 -> 56 or worse;
+//   backward BINS: 1024 x 30..1000 30 -> 29.5, but 800 x 500..1000 38.1 -> 42.2:
+//     of its 224 VGPR workgroups two fit on a CU, and a second round of them
+//     starts late.  So the backward has none.
+template <typename Kernel>
+bool launch_chain(Kernel kernel, const ChunkArgs& a, size_t lds, hipStream_t stream, int& rc) {
+    if (a.nc > kBinsMax) return false;
+    for (const bool bins : {false, true}) {
+        if (!bins && a.nc > kChainMax) continue;
+        const int waves = !bins ? a.nc : a.nc <= 4 ? 4 : 8;
+        const KernelFn k = kernel(waves, bins);
+        if (!k || waves * lds > (bins ? kBinsMaxLds : kChainMaxLds) || !allow_lds(k, waves * lds)) continue;
+        if (bins ? a.nc <= 2 || a.B > bins_max_batch(waves) : a.B > resident_workgroups(k, 64 * waves, waves * lds)) continue;
+        hipLaunchKernelGGL(k, dim3((unsigned)a.B), dim3(64 * waves), waves * lds, stream, a);
+        rc = hipGetLastError() == hipSuccess ? TPL_A2B_OK : TPL_A2B_ERR_LAUNCH;
+        return true;
+    }
+    return false;
+}
+
+// The step's kernels for a shape with R residues per lane.
+struct StepForm {
+    KernelFn kernel, sums;  // sums: WALK
+    int waves;
+    size_t lds;
+    unsigned grid;
+    size_t rec_bytes;  // WALK: the records
+};
 
 template <typename T, int R>
 void step_kernel(StepForm& s, StepMode mode) {
@@ -2613,7 +2655,7 @@ bool step_form(int dtype, int B, int L, const tpl_a2b_config* cfg, StepForm& s) 
     if (R == 1 && nc > 4) return false;
     if (!pick(CHAIN)) return false;
     if (B <= resident_workgroups(s.kernel, 64 * s.waves, s.lds)) return true;
-    return B <= kStepMaxBatch && pick(BINS);
+    return B <= bins_max_batch(s.waves) && pick(BINS);
 }
 
 // The two directions, reporting as `rep` says.
@@ -2636,10 +2678,10 @@ int forward_on(int dtype, const void* angles, void* coords, const int32_t* lengt
     bind_sync(a, sync, sync_layout(batch, angles_stride, cfg).fwd);
     const bool f32 = dtype == TPL_A2B_F32;
     const size_t lds = (size_t)9 * 64 * R * (f32 ? 4 : 8);
-    if (a.nc <= kChainMax) {
-        const KernelFn kc = f32 ? fwd_chain_kernel<float>(R, a.nc) : fwd_chain_kernel<double>(R, a.nc);
-        if (chain_fits(kc, a, lds)) return launch_chain(kc, a, lds, static_cast<hipStream_t>(stream));
-    }
+    const auto kernel = [&](int w, bool bins) {
+        return f32 ? fwd_chain_kernel<float>(R, w, bins) : fwd_chain_kernel<double>(R, w, bins);
+    };
+    if (launch_chain(kernel, a, lds, static_cast<hipStream_t>(stream), rc)) return rc;
     return launch(f32 ? fwd_kernel<float>(R) : fwd_kernel<double>(R), a, lds,
                   static_cast<hipStream_t>(stream));
 }
@@ -2666,10 +2708,10 @@ int backward_on(int dtype, void* grad_angles, const void* grad_coords, const voi
     bind_sync(a, sync, sync_layout(batch, angles_stride, cfg).bwd);
     const bool f32 = dtype == TPL_A2B_F32;
     const size_t lds = (size_t)6 * R * 64 * sizeof(double);
-    if (a.nc <= kChainMax) {
-        const KernelFn kc = f32 ? bwd_chain_kernel<float>(R, a.nc) : bwd_chain_kernel<double>(R, a.nc);
-        if (chain_fits(kc, a, lds)) return launch_chain(kc, a, lds, static_cast<hipStream_t>(stream));
-    }
+    const auto kernel = [&](int w, bool bins) -> KernelFn {
+        return bins ? nullptr : f32 ? bwd_chain_kernel<float>(R, w) : bwd_chain_kernel<double>(R, w);
+    };
+    if (launch_chain(kernel, a, lds, static_cast<hipStream_t>(stream), rc)) return rc;
     return launch(f32 ? bwd_kernel<float>(R) : bwd_kernel<double>(R), a, lds,
                   static_cast<hipStream_t>(stream));
 }
@@ -2815,10 +2857,10 @@ int tpl_a2b_forward_noalloc(int dtype, const void* angles, void* coords, const i
     const size_t lds = (size_t)9 * 64 * R * (f32 ? 4 : 8);
     // Chains of at most kChainMax chunks need no look-back words (the same
     // kernel as tpl_a2b_forward's).
-    if (a.nc <= kChainMax) {
-        const KernelFn kc = f32 ? fwd_chain_kernel<float>(R, a.nc) : fwd_chain_kernel<double>(R, a.nc);
-        if (chain_fits(kc, a, lds)) return launch_chain(kc, a, lds, static_cast<hipStream_t>(stream));
-    }
+    const auto kernel = [&](int w, bool bins) {
+        return f32 ? fwd_chain_kernel<float>(R, w, bins) : fwd_chain_kernel<double>(R, w, bins);
+    };
+    if (launch_chain(kernel, a, lds, static_cast<hipStream_t>(stream), rc)) return rc;
     void* base = scratch_address();
     if (!base) return TPL_A2B_ERR_HIP;
     // Tickets, done counters and records must start at zero.  Every call

@@ -627,6 +627,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
                             torch::Tensor, torch::Tensor, std::vector<int64_t>>(),
              "one fwd+bwd step on fixed buffers")
         .def("run", &Step::run, "launch the step on the current stream");
+    m.def("step_fits", [](bool f64, int64_t B, int64_t L, std::vector<int64_t> config) {
+        const tpl_a2b_config cfg = to_config(config);
+        size_t bytes = 0;
+        return tplx_a2b_step_fits(f64 ? TPL_A2B_F64 : TPL_A2B_F32, (int)B, (int)L, &cfg, &bytes) != 0;
+    }, "whether a step of this shape and config has kernels of its own");
     m.doc() = "Angles2Backbone for MI355X: tensor glue over the tpl_a2b C ABI";
     m.def("Angles2BackboneGPU_forward", &forward, "Angles2Backbone gpu forward (chunk scan)");
     m.def("Angles2BackboneGPU_backward", &backward, "Angles2Backbone gpu backward (O(L) adjoint)");
