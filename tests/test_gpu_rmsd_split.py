@@ -1,0 +1,63 @@
+"""Few large structures, several workgroups each, against the same structures
+in a batch of 65, which take one workgroup each: sizes at the edges of the rule
+(8192 atoms, 64 structures), counts at the edges of a workgroup's share, strides
+of every alignment."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("B,A", [(1, 8191), (1, 8192), (3, 8193), (2, 20002), (64, 8195), (40, 13000), (1, 66001)])
+def test_split_matches_one_workgroup(dtype, B, A):
+    from torchproteinlibrary_amd.RMSD import Coords2RMSD
+    rng = np.random.default_rng(B * 7 + A)
+    counts = [A, A - 1, 1024, 1025, 0, 1, 2, 1023, 4, 8191]
+    n = torch.tensor([min(counts[k % len(counts)], A) for k in range(B)], dtype=torch.int32).cuda()
+    step = rng.standard_normal((B, A, 3))
+    x = np.cumsum(1.5 * step / np.linalg.norm(step, axis=2, keepdims=True), axis=1) + 50.0
+    q, _ = np.linalg.qr(rng.standard_normal((3, 3)))
+    y = x @ q + 2.0 * rng.standard_normal((B, A, 3)) - 20.0
+    x, y = (torch.from_numpy(v.reshape(B, 3 * A)).to(dtype).cuda() for v in (x, y))
+    rep = -(-65 // B)
+    got, want = [], []
+    for k, out in ((1, got), (rep, want)):
+        xx = x.repeat(k, 1).requires_grad_(True)
+        layer = Coords2RMSD()
+        r = layer(xx, y.repeat(k, 1), n.repeat(k))
+        g, = torch.autograd.grad(r.sum(), xx)
+        out += [r.detach()[:B], layer.UT[:B], g[:B]]
+    # r^2 n = R2 - 2 lambda: both sums in another order, each within some units
+    # of 2^-53 of R2 <= n d^2, d the largest distance of two atoms; U turns by
+    # as much as the sums change against the spread of the structure.
+    ref = torch.isfinite(want[0]) & (n > 3)
+    assert torch.equal(torch.isfinite(got[0]), torch.isfinite(want[0]))
+    for b in torch.nonzero(ref).flatten().tolist():
+        k = int(n[b])
+        c = x[b, :3 * k].double().view(-1, 3)
+        c = c - c.mean(0)
+        r2 = 4 * (c ** 2).sum().item()
+        rmsd = want[0][b].double().item()
+        tol = 256 * 2.0 ** -53 * r2 / (k * rmsd) + 2 * torch.finfo(dtype).eps * rmsd
+        assert abs(got[0][b].double().item() - rmsd) <= tol, (b, k)
+        spread = torch.linalg.svdvals(c)[1].item() ** 2
+        turn = 256 * 2.0 ** -53 * r2 / spread + 2 * torch.finfo(dtype).eps
+        assert (got[1][b] - want[1][b]).abs().max().double().item() <= turn, (b, k)
+        far = c.norm(dim=1).max().item()
+        tol = (turn * far + 2 * torch.finfo(dtype).eps * (far + 100)) / (k * rmsd) * 4
+        assert (got[2][b] - want[2][b]).abs().max().double().item() <= tol, (b, k)
+        assert not got[2][b, 3 * k:].any()
+
+
+def test_split_errors():
+    from torchproteinlibrary_amd.RMSD import Coords2RMSD
+    x = torch.randn(2, 3 * 9000, device="cuda")
+    y = torch.randn(2, 3 * 9000, device="cuda")
+    n = torch.tensor([9000, 9000], dtype=torch.int32, device="cuda")
+    with pytest.raises(ValueError, match="num_atoms"):
+        Coords2RMSD()(x, y, n + 1)
+    x[1, 3 * 8999] = float("nan")
+    with pytest.raises(Exception, match="forward Nan"):
+        Coords2RMSD()(x, y, n)

@@ -1,5 +1,6 @@
 // Coords2RMSD for MI355X (gfx950): minimal RMSD over rigid rotations and its
-// gradient, each direction one kernel launch.  The C ABI is include/tpl_rmsd.h.
+// gradient, each direction one kernel launch (the forward two for few large
+// structures).  The C ABI is include/tpl_rmsd.h.
 //
 // The layer follows the reference's method (quaternion eigenproblem of the
 // centred correlation matrix; coords2rmsd_interface.cpp:12-49,52-111,
@@ -7,7 +8,8 @@
 //   forward, one workgroup per structure:
 //     1. FP64 moments of the atoms relative to the structure's first atom
 //        (sum x, sum y, sum x y^T, sum |x|^2, sum |y|^2), four atoms per
-//        thread and pass, summed over the workgroup in two levels through LDS;
+//        thread and pass, summed over the workgroup in two levels through LDS
+//        (few large structures: over several workgroups, in two launches);
 //     2. lane 0 centres them, builds the symmetric 4x4 matrix F of the
 //        centred correlation R (the reference's element layout,
 //        coords2rmsd_interface.cpp:153-158), takes its largest eigenpair
@@ -39,28 +41,25 @@ constexpr int kState = 16;           // doubles per structure: cx[3] cy[3] U[9] 
 constexpr int kMoments = 17;         // sx[3] sy[3] sxy[9] sxx syy
 
 // Atoms a0 .. a0+3 of one structure (xyz interleaved) as 12 values: three
-// 16-byte loads per 4 floats (six for doubles) when the run is aligned and
-// whole, else element loads; atoms at or past `lim` read as 0.
+// 16-byte loads per 4 floats (six for doubles) when the run is whole, else
+// element loads; atoms at or past `lim` read as 0.  The loads need the
+// alignment of the values only, so a stride of any size has them: float32, 300
+// structures of 3000..6001 atoms at a stride of 6001, forward 20.7 -> 12.3 us
+// against 16-byte loads where the structure is 16-byte aligned.
 template <typename T>
-__device__ __forceinline__ void load4(const T* p, int a0, int lim, bool vec, double v[12]) {
-    if (vec && a0 + 4 <= lim) {
+__device__ __forceinline__ void load4(const T* p, int a0, int lim, T t[12]) {
+    typedef uint32_t Vec __attribute__((ext_vector_type(4), aligned(4)));
+    if (a0 + 4 <= lim) {
         constexpr int E = 16 / (int)sizeof(T);  // elements per 16-byte load
-        T t[12];
 #pragma unroll
         for (int k = 0; k < 12; k += E) {
-            const uint4 u = *reinterpret_cast<const uint4*>(p + 3 * (size_t)a0 + k);
+            const Vec u = *reinterpret_cast<const Vec*>(p + 3 * (size_t)a0 + k);
             __builtin_memcpy(t + k, &u, 16);
         }
-#pragma unroll
-        for (int k = 0; k < 12; ++k) v[k] = (double)t[k];
     } else {
 #pragma unroll
-        for (int k = 0; k < 12; ++k) v[k] = (a0 + k / 3 < lim) ? (double)p[3 * (size_t)a0 + k] : 0.0;
+        for (int k = 0; k < 12; ++k) t[k] = (a0 + k / 3 < lim) ? p[3 * (size_t)a0 + k] : (T)0;
     }
-}
-
-__device__ __forceinline__ bool aligned16(const void* p) {
-    return (reinterpret_cast<uintptr_t>(p) & 15) == 0;
 }
 
 __device__ __forceinline__ int clamp_count(int n, int A, const Report& rep, bool report_it) {
@@ -71,64 +70,16 @@ __device__ __forceinline__ int clamp_count(int n, int A, const Report& rep, bool
     return n;
 }
 
-template <typename T>
-__global__ void __launch_bounds__(kThreads) rmsd_fwd(const T* __restrict__ x, const T* __restrict__ y,
-                                                     const int32_t* __restrict__ num_atoms,
-                                                     T* rmsd_out, T* ut_out, double* state,
-                                                     Report rep, int A) {
-    // Moment sums over the workgroup: every thread's 17 partial sums (laid
-    // out [moment][thread]), then kParts partial sums per moment, then the
-    // totals.  A cross-lane butterfly over 17 doubles measured 5 us per
-    // workgroup, bound by the LDS crossbar at 16 waves per CU; this takes
-    // three barriers and plain LDS reads.
+// Sums of the threads' moments over the workgroup, in tot (LDS): every thread's
+// 17 partial sums (laid out [moment][thread]), then kParts partial sums per
+// moment, then the totals.  A cross-lane butterfly over 17 doubles measured
+// 5 us per workgroup, bound by the LDS crossbar at 16 waves per CU; this takes
+// plain LDS reads and three barriers.
+__device__ __forceinline__ void workgroup_sums(const double m[kMoments], double* tot) {
     constexpr int kParts = kThreads / kMoments;  // 15 threads per moment in the middle level
     __shared__ double s_m[kMoments * kThreads];
     __shared__ double s_p[kMoments * kParts];
-    __shared__ double s_tot[kMoments];
-    const int b = blockIdx.x, tid = threadIdx.x;
-    const int n = clamp_count(num_atoms[b], A, rep, tid == 0);
-    const T* xb = x + (size_t)b * 3 * A;
-    const T* yb = y + (size_t)b * 3 * A;
-    double x0[3] = {0.0, 0.0, 0.0}, y0[3] = {0.0, 0.0, 0.0};
-    if (n > 0) {
-#pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            x0[c] = (double)xb[c];
-            y0[c] = (double)yb[c];
-        }
-    }
-    double m[kMoments];
-#pragma unroll
-    for (int e = 0; e < kMoments; ++e) m[e] = 0.0;
-    // Four consecutive atoms per thread and pass: one 48-byte run of each
-    // structure per lane, loaded in 16-byte pieces.
-    const bool vec = aligned16(xb) && aligned16(yb);
-    for (int a0 = 4 * tid; a0 < n; a0 += 4 * kThreads) {
-        double xv[12], yv[12];
-        load4(xb, a0, n, vec, xv);
-        load4(yb, a0, n, vec, yv);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const bool in = a0 + j < n;
-            double dx[3], dy[3];
-#pragma unroll
-            for (int c = 0; c < 3; ++c) {
-                dx[c] = in ? xv[3 * j + c] - x0[c] : 0.0;
-                dy[c] = in ? yv[3 * j + c] - y0[c] : 0.0;
-            }
-#pragma unroll
-            for (int c = 0; c < 3; ++c) {
-                m[c] += dx[c];
-                m[3 + c] += dy[c];
-                m[15] += dx[c] * dx[c];
-                m[16] += dy[c] * dy[c];
-            }
-#pragma unroll
-            for (int r = 0; r < 3; ++r)
-#pragma unroll
-                for (int c = 0; c < 3; ++c) m[6 + 3 * r + c] += dx[r] * dy[c];
-        }
-    }
+    const int tid = threadIdx.x;
 #pragma unroll
     for (int e = 0; e < kMoments; ++e) s_m[e * kThreads + tid] = m[e];
     __syncthreads();
@@ -143,12 +94,56 @@ __global__ void __launch_bounds__(kThreads) rmsd_fwd(const T* __restrict__ x, co
         double acc = 0.0;
 #pragma unroll
         for (int part = 0; part < kParts; ++part) acc += s_p[tid * kParts + part];
-        s_tot[tid] = acc;
+        tot[tid] = acc;
     }
     __syncthreads();
-    if (tid != 0) return;
+}
+
+// Thread's moments of atoms first, first + step, .. (runs of four) below n,
+// relative to x0 and y0.
+template <typename T>
+__device__ __forceinline__ void add_moments(const T* xb, const T* yb, int first, int step, int n,
+                                            const double x0[3], const double y0[3], double m[kMoments]) {
+    for (int a0 = first; a0 < n; a0 += step) {
+        T xv[12], yv[12];
+        load4(xb, a0, n, xv);
+        load4(yb, a0, n, yv);
 #pragma unroll
-    for (int e = 0; e < kMoments; ++e) m[e] = s_tot[e];
+        for (int j = 0; j < 4; ++j) {
+            const bool in = a0 + j < n;
+            double dx[3], dy[3];
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                dx[c] = in ? (double)xv[3 * j + c] - x0[c] : 0.0;
+                dy[c] = in ? (double)yv[3 * j + c] - y0[c] : 0.0;
+            }
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                m[c] += dx[c];
+                m[3 + c] += dy[c];
+                m[15] += dx[c] * dx[c];
+                m[16] += dy[c] * dy[c];
+            }
+#pragma unroll
+            for (int r = 0; r < 3; ++r)
+#pragma unroll
+                for (int c = 0; c < 3; ++c) m[6 + 3 * r + c] += dx[r] * dy[c];
+        }
+    }
+}
+template <typename T>
+__device__ __forceinline__ void first_atoms(const T* xb, const T* yb, int n, double x0[3], double y0[3]) {
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        x0[c] = n > 0 ? (double)xb[c] : 0.0;
+        y0[c] = n > 0 ? (double)yb[c] : 0.0;
+    }
+}
+
+// One lane: the result of structure b from its moments.
+template <typename T>
+__device__ __forceinline__ void finish(const double m[kMoments], const double x0[3], const double y0[3], int n, int b,
+                                       T* rmsd_out, T* ut_out, double* state, const Report& rep) {
     const double nd = (double)n;
     double mx[3], my[3];
 #pragma unroll
@@ -192,6 +187,69 @@ __global__ void __launch_bounds__(kThreads) rmsd_fwd(const T* __restrict__ x, co
         s[15] = rmsd;
     }
     if (rmsd != rmsd) report_bits(rep, TPL_RMSD_STATUS_NAN);
+}
+
+template <typename T>
+__global__ void __launch_bounds__(kThreads) rmsd_fwd(const T* __restrict__ x, const T* __restrict__ y,
+                                                     const int32_t* __restrict__ num_atoms, T* rmsd_out, T* ut_out,
+                                                     double* state, Report rep, int A) {
+    __shared__ double s_tot[kMoments];
+    const int b = blockIdx.x, tid = threadIdx.x;
+    const int n = clamp_count(num_atoms[b], A, rep, tid == 0);
+    const T* xb = x + (size_t)b * 3 * A;
+    const T* yb = y + (size_t)b * 3 * A;
+    double x0[3], y0[3], m[kMoments] = {};
+    first_atoms(xb, yb, n, x0, y0);
+    add_moments(xb, yb, 4 * tid, 4 * kThreads, n, x0, y0, m);
+    workgroup_sums(m, s_tot);
+    if (tid != 0) return;
+#pragma unroll
+    for (int e = 0; e < kMoments; ++e) m[e] = s_tot[e];
+    finish(m, x0, y0, n, b, rmsd_out, ut_out, state, rep);
+}
+
+// Few large structures: S workgroups per structure, whose sums go to part
+// [B][kMoments][S], and a wave per structure that adds them up.  One workgroup
+// alone is bound by the latency of its passes (20 of 1024 atoms at 20000):
+// 8 structures of up to 20000 atoms, float64, 14.8 -> 8.3 us; one, float32,
+// 16.0 -> 7.7.
+template <typename T>
+__global__ void __launch_bounds__(kThreads) rmsd_part(const T* __restrict__ x, const T* __restrict__ y,
+                                                      const int32_t* __restrict__ num_atoms, double* part, int A,
+                                                      int S) {
+    __shared__ double s_tot[kMoments];
+    const int b = (int)blockIdx.x / S, s = (int)blockIdx.x - b * S, tid = threadIdx.x;
+    const int n = clamp_count(num_atoms[b], A, Report{nullptr, nullptr}, false);
+    const T* xb = x + (size_t)b * 3 * A;
+    const T* yb = y + (size_t)b * 3 * A;
+    double x0[3], y0[3], m[kMoments] = {};
+    first_atoms(xb, yb, n, x0, y0);
+    add_moments(xb, yb, 4 * (s * kThreads + tid), 4 * kThreads * S, n, x0, y0, m);
+    workgroup_sums(m, s_tot);
+    if (tid < kMoments) part[((size_t)b * kMoments + tid) * S + s] = s_tot[tid];
+}
+template <typename T>
+__global__ void __launch_bounds__(64) rmsd_join(const T* __restrict__ x, const T* __restrict__ y,
+                                                const int32_t* __restrict__ num_atoms,
+                                                const double* __restrict__ part, T* rmsd_out, T* ut_out,
+                                                double* state, Report rep, int A, int S) {
+    __shared__ double s_tot[kMoments];
+    const int b = blockIdx.x, lane = threadIdx.x;
+    const int n = clamp_count(num_atoms[b], A, rep, lane == 0);
+    double x0[3], y0[3], m[kMoments];
+    first_atoms(x + (size_t)b * 3 * A, y + (size_t)b * 3 * A, n, x0, y0);
+    if (lane < kMoments) {
+        const double* p = part + ((size_t)b * kMoments + lane) * S;
+        double v = 0.0;
+#pragma unroll 8
+        for (int s = 0; s < S; ++s) v += p[s];
+        s_tot[lane] = v;
+    }
+    __syncthreads();
+    if (lane != 0) return;
+#pragma unroll
+    for (int e = 0; e < kMoments; ++e) m[e] = s_tot[e];
+    finish(m, x0, y0, n, b, rmsd_out, ut_out, state, rep);
 }
 
 // One thread per atom slot; the grid covers nblk blocks per structure.
@@ -243,27 +301,44 @@ int check(int dtype, int B, int A) {
     return TPL_RMSD_OK;
 }
 
+// Workgroups per structure in the split forward, 1 where it does not pay: every
+// workgroup has a full pass of 1024 atoms and no more of them run than the GPU
+// holds at two per CU; fewer than 8 passes cost less than the second launch (64
+// structures of 5000 atoms take 7.5 us in one launch).
+int split_of(int B, int A) {
+    if (B <= 0 || B > 64) return 1;
+    const int s = std::min({64, A / (4 * kThreads), 512 / B});
+    return s >= 8 ? s : 1;
+}
+
+template <typename T>
+void launch_forward(const void* input, const void* target, const int32_t* num_atoms, void* rmsd, void* ut,
+                    void* state, double* part, const Report& rep, int B, int A, hipStream_t s) {
+    const T *x = static_cast<const T*>(input), *y = static_cast<const T*>(target);
+    T *r = static_cast<T*>(rmsd), *u = static_cast<T*>(ut);
+    double* st = static_cast<double*>(state);
+    const int S = split_of(B, A);
+    if (S > 1 && part) {
+        hipLaunchKernelGGL(rmsd_part<T>, dim3(B * S), dim3(kThreads), 0, s, x, y, num_atoms, part, A, S);
+        hipLaunchKernelGGL(rmsd_join<T>, dim3(B), dim3(64), 0, s, x, y, num_atoms, part, r, u, st, rep, A, S);
+    } else {
+        hipLaunchKernelGGL(rmsd_fwd<T>, dim3(B), dim3(kThreads), 0, s, x, y, num_atoms, r, u, st, rep, A);
+    }
+}
+
 // The two directions, reporting as `rep` says.
-int forward_on(int dtype, const void* input, const void* target, const int32_t* num_atoms,
-                     void* rmsd, void* ut, void* state, const Report& rep, int batch,
-                     int atoms_stride, tpl_rmsd_stream_t stream) {
+int forward_on(int dtype, const void* input, const void* target, const int32_t* num_atoms, void* rmsd, void* ut,
+               void* state, void* workspace, const Report& rep, int batch, int atoms_stride,
+               tpl_rmsd_stream_t stream) {
     const int rc = check(dtype, batch, atoms_stride);
     if (rc != TPL_RMSD_OK) return rc;
     if (batch == 0) return TPL_RMSD_OK;
     if (!num_atoms || !rmsd || !ut || (atoms_stride > 0 && (!input || !target)))
         return TPL_RMSD_ERR_ARG;
     if (state && (reinterpret_cast<uintptr_t>(state) & 255)) return TPL_RMSD_ERR_ARG;
-    hipStream_t s = static_cast<hipStream_t>(stream);
-    if (dtype == TPL_RMSD_F32)
-        hipLaunchKernelGGL(rmsd_fwd<float>, dim3(batch), dim3(kThreads), 0, s,
-                           static_cast<const float*>(input), static_cast<const float*>(target),
-                           num_atoms, static_cast<float*>(rmsd), static_cast<float*>(ut),
-                           static_cast<double*>(state), rep, atoms_stride);
-    else
-        hipLaunchKernelGGL(rmsd_fwd<double>, dim3(batch), dim3(kThreads), 0, s,
-                           static_cast<const double*>(input), static_cast<const double*>(target),
-                           num_atoms, static_cast<double*>(rmsd), static_cast<double*>(ut),
-                           static_cast<double*>(state), rep, atoms_stride);
+    (dtype == TPL_RMSD_F32 ? launch_forward<float> : launch_forward<double>)(
+        input, target, num_atoms, rmsd, ut, state, static_cast<double*>(workspace), rep, batch, atoms_stride,
+        static_cast<hipStream_t>(stream));
     return hipGetLastError() == hipSuccess ? TPL_RMSD_OK : TPL_RMSD_ERR_LAUNCH;
 }
 
@@ -314,7 +389,7 @@ size_t tpl_rmsd_state_bytes(int batch) {
 int tpl_rmsd_forward(int dtype, const void* input, const void* target, const int32_t* num_atoms,
                      void* rmsd, void* ut, void* state, uint32_t* status, int batch,
                      int atoms_stride, tpl_rmsd_stream_t stream) {
-    return forward_on(dtype, input, target, num_atoms, rmsd, ut, state, Report{status, nullptr}, batch,
+    return forward_on(dtype, input, target, num_atoms, rmsd, ut, state, nullptr, Report{status, nullptr}, batch,
                       atoms_stride, stream);
 }
 
@@ -325,10 +400,15 @@ int tpl_rmsd_backward(int dtype, void* grad_input, const void* grad_rmsd, const 
                        batch, atoms_stride, stream);
 }
 
+size_t tplx_rmsd_workspace_bytes(int batch, int atoms_stride) {
+    const int S = split_of(batch, atoms_stride);
+    return S > 1 ? (size_t)batch * kMoments * S * sizeof(double) : 0;
+}
+
 int tplx_rmsd_forward(int dtype, const void* input, const void* target, const int32_t* num_atoms, void* rmsd,
-                      void* ut, void* state, uint32_t* flags, int batch, int atoms_stride,
+                      void* ut, void* state, void* workspace, uint32_t* flags, int batch, int atoms_stride,
                       tpl_rmsd_stream_t stream) {
-    return forward_on(dtype, input, target, num_atoms, rmsd, ut, state, Report{nullptr, flags}, batch,
+    return forward_on(dtype, input, target, num_atoms, rmsd, ut, state, workspace, Report{nullptr, flags}, batch,
                       atoms_stride, stream);
 }
 

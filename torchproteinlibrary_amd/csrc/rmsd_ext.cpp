@@ -83,6 +83,13 @@ hipStream_t stream_of(const torch::Tensor& t) {
     return c10::hip::getCurrentHIPStream(t.device().index()).stream();
 }
 
+// The forward's workspace (undefined where it needs none), from torch's allocator.
+torch::Tensor workspace_for(const torch::Tensor& input, int B, int A) {
+    const size_t need = tplx_rmsd_workspace_bytes(B, A);
+    return need ? torch::empty({(int64_t)need}, input.options().dtype(torch::kByte)) : torch::Tensor();
+}
+void* ptr(const torch::Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
+
 // Coords2RMSDGPU_forward (reference coords2rmsd_interface.cpp:52-57):
 // (centered_coords_src, centered_coords_dst, output, num_atoms, UT) plus the
 // forward->backward state (None: no backward follows) and an optional status.
@@ -127,10 +134,11 @@ int64_t forward_checked(torch::Tensor input, torch::Tensor target, torch::Tensor
     c10::DeviceGuard guard(input.device());
     void* st = (state.has_value() && state->defined()) ? state_ptr(*state, B, input) : nullptr;
     hipStream_t s = stream_of(input);
+    const torch::Tensor ws = workspace_for(input, B, A);
     return host_flags::run(s, [&, B = B, A = A](uint32_t* flags) {
         check_rc(tplx_rmsd_forward(dtype_code(input), input.data_ptr(), target.data_ptr(),
-                                   num_atoms.data_ptr<int32_t>(), output.data_ptr(), UT.data_ptr(), st, flags, B,
-                                   A, s),
+                                   num_atoms.data_ptr<int32_t>(), output.data_ptr(), UT.data_ptr(), st, ptr(ws),
+                                   flags, B, A, s),
                  "Coords2RMSDGPU_forward");
     });
 }
@@ -166,9 +174,11 @@ struct Coords2RMSD : torch::autograd::Function<Coords2RMSD> {
         if (needs)
             state = torch::empty({std::max<int64_t>(1, (int64_t)tpl_rmsd_state_bytes(B))},
                                  x.options().dtype(torch::kByte));
+        const torch::Tensor ws = workspace_for(x, B, A);
         const uint32_t bits = native_fn::run(s, [&, B = B, A = A](uint32_t* flags) {
             check_rc(tplx_rmsd_forward(dt, x.data_ptr(), y.data_ptr(), n.data_ptr<int32_t>(), rmsd.data_ptr(),
-                                       UT.data_ptr(), needs ? state_ptr(state, B, x) : nullptr, flags, B, A, s),
+                                       UT.data_ptr(), needs ? state_ptr(state, B, x) : nullptr, ptr(ws), flags, B, A,
+                                       s),
                      "Coords2RMSDGPU_forward");
         });
         if (bits) native_fn::python(kLayer, "_raise_on_bits", bits, "forward");
@@ -231,8 +241,10 @@ std::tuple<double, double, double> bench(std::vector<std::vector<torch::Tensor>>
     }
     c10::DeviceGuard guard(sets[0][0].device());
     hipStream_t stream = stream_of(sets[0][0]);
+    const torch::Tensor ws = workspace_for(sets[0][0], ss[0].B, ss[0].A);
+    for (const Set& q : ss) TORCH_CHECK(q.B == ss[0].B && q.A == ss[0].A, "bench: sets differ in shape");
     auto fwd = [&](const Set& q) {
-        check_rc(tpl_rmsd_forward(q.dt, q.x, q.y, q.n, q.r, q.ut, q.st, nullptr, q.B, q.A, stream),
+        check_rc(tplx_rmsd_forward(q.dt, q.x, q.y, q.n, q.r, q.ut, q.st, ptr(ws), nullptr, q.B, q.A, stream),
                  "tpl_rmsd_forward");
     };
     auto bwd = [&](const Set& q) {

@@ -6,8 +6,11 @@
 #include "tpl_rmsd.h"
 
 extern "C" {
+// The forward's workspace (its contents do not matter; null: none), with which
+// few large structures take several workgroups each.
+size_t tplx_rmsd_workspace_bytes(int batch, int atoms_stride);
 int tplx_rmsd_forward(int dtype, const void* input, const void* target, const int32_t* num_atoms, void* rmsd,
-                      void* ut, void* state, uint32_t* flags, int batch, int atoms_stride,
+                      void* ut, void* state, void* workspace, uint32_t* flags, int batch, int atoms_stride,
                       tpl_rmsd_stream_t stream);
 int tplx_rmsd_backward(int dtype, void* grad_input, const void* grad_rmsd, const void* input, const void* target,
                        const int32_t* num_atoms, const void* state, uint32_t* flags, int batch, int atoms_stride,
