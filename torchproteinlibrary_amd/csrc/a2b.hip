@@ -258,32 +258,55 @@ __device__ __forceinline__ uint32_t atomic_inc(uint32_t* p) {
 // ------------------------------------------------------------------ lane I/O
 // A lane moves a run of N consecutive elements of T between global memory
 // and registers.  Elements at or past `cnt` read as 0 and are not written.  A
-// run that is whole (cnt >= N) and U-byte aligned moves in U-byte accesses;
-// U = the widest of 16/8/4 bytes dividing the run, fixed per kernel, and every
-// lane of one row shares the alignment, so the branch is uniform there.
-// (Runs here are whole multiples of 2 bytes.)
+// whole run moves in 16-byte accesses and a remainder of 8 and 4 bytes, at any
+// alignment that its elements have (4 bytes are enough for each of them), so
+// that row strides of any length have them.  Against runs that were moved
+// element by element where they were not aligned to the widest power of two in
+// their length, us a step of forward and backward:
+//   64 chains at a stride of 16381, one step of two kernels: 56.9 -> 47.5
+//   1024 chains at 1001, float32, (2,4): 31.6 -> 29.9; at 1000: 29.6 -> 29.2
+//   512 chains at 500, float32, (2,2): 17.2 -> 16.3 (2 residues are 18 floats,
+//   which went in 8-byte accesses)
 template <int U>
 struct Unit;
-template <>
-struct Unit<2> {
-    using type = uint16_t;
-};
 template <>
 struct Unit<4> {
     using type = uint32_t;
 };
 template <>
 struct Unit<8> {
-    using type = uint2;
+    typedef uint32_t type __attribute__((ext_vector_type(2), aligned(4)));
 };
 template <>
 struct Unit<16> {
-    using type = uint4;
+    typedef uint32_t type __attribute__((ext_vector_type(4), aligned(4)));
 };
+
+// Bytes at .. B - 1 of a run of B.
+template <int B, int AT = 0>
+__device__ __forceinline__ void load_bytes(const char* p, char* v) {
+    if constexpr (AT < B) {
+        constexpr int U = B - AT >= 16 ? 16 : B - AT >= 8 ? 8 : 4;
+        const auto u = *reinterpret_cast<const typename Unit<U>::type*>(p + AT);
+        __builtin_memcpy(v + AT, &u, U);
+        load_bytes<B, AT + U>(p, v);
+    }
+}
+// Nontemporal (streaming): the outputs are never read back by the kernel that
+// writes them.
+template <int B, int AT = 0>
+__device__ __forceinline__ void store_bytes(char* p, const char* v) {
+    if constexpr (AT < B) {
+        constexpr int U = B - AT >= 16 ? 16 : B - AT >= 8 ? 8 : 4;
+        typename Unit<U>::type u;
+        __builtin_memcpy(&u, v + AT, U);
+        __builtin_nontemporal_store(u, reinterpret_cast<typename Unit<U>::type*>(p + AT));
+        store_bytes<B, AT + U>(p, v);
+    }
+}
 template <typename T, int N>
-constexpr int unit_bytes() {
-    constexpr int b = N * (int)sizeof(T);
-    return b % 16 == 0 ? 16 : (b % 8 == 0 ? 8 : (b % 4 == 0 ? 4 : 2));
+__device__ __forceinline__ void load_run(const T* p, T (&v)[N]) {
+    load_bytes<N * (int)sizeof(T)>(reinterpret_cast<const char*>(p), reinterpret_cast<char*>(v));
 }
 
 // avail: elements at p that may be read (the run's room in its row); the
@@ -291,14 +314,9 @@ constexpr int unit_bytes() {
 // zeroed with selects, so a lane that ends its chain takes no branch.
 template <typename T, int N>
 __device__ __forceinline__ void lane_load(const T* p, int cnt, T (&v)[N], int avail = -1) {
-    constexpr int U = unit_bytes<T, N>();
-    using V = typename Unit<U>::type;
     if (avail < 0) avail = cnt;
-    if (avail >= N && (reinterpret_cast<uintptr_t>(p) % U) == 0) {
-        V w[N * sizeof(T) / U];
-#pragma unroll
-        for (int i = 0; i < (int)(N * sizeof(T) / U); ++i) w[i] = reinterpret_cast<const V*>(p)[i];
-        __builtin_memcpy(v, w, sizeof(v));
+    if (avail >= N) {
+        load_run(p, v);
 #pragma unroll
         for (int i = 0; i < N; ++i) v[i] = i < cnt ? v[i] : (T)0;
     } else {
@@ -307,57 +325,17 @@ __device__ __forceinline__ void lane_load(const T* p, int cnt, T (&v)[N], int av
     }
 }
 
-// Two runs of the same shape (e.g. coordinates and their gradients) under
-// one alignment test, so their loads are in flight together.
-template <typename T, int N>
-__device__ __forceinline__ void lane_load2(const T* p, const T* q, int cnt, int avail, T (&v)[N],
-                                           T (&w)[N]) {
-    constexpr int U = unit_bytes<T, N>();
-    using V = typename Unit<U>::type;
-    const bool vec = avail >= N && ((reinterpret_cast<uintptr_t>(p) | reinterpret_cast<uintptr_t>(q)) % U) == 0;
-    if (vec) {
-        V a[N * sizeof(T) / U], c[N * sizeof(T) / U];
-#pragma unroll
-        for (int i = 0; i < (int)(N * sizeof(T) / U); ++i) {
-            a[i] = reinterpret_cast<const V*>(p)[i];
-            c[i] = reinterpret_cast<const V*>(q)[i];
-        }
-        __builtin_memcpy(v, a, sizeof(v));
-        __builtin_memcpy(w, c, sizeof(w));
-#pragma unroll
-        for (int i = 0; i < N; ++i) {
-            v[i] = i < cnt ? v[i] : (T)0;
-            w[i] = i < cnt ? w[i] : (T)0;
-        }
-    } else {
-#pragma unroll
-        for (int i = 0; i < N; ++i) {
-            v[i] = i < cnt ? p[i] : (T)0;
-            w[i] = i < cnt ? q[i] : (T)0;
-        }
-    }
-}
-
 // The lane's R angles of the three rows (stride L elements) under one
-// alignment test, so the three loads are in flight together.
+// test, so the three loads are in flight together.
 template <typename T, int R>
 __device__ __forceinline__ void lane_load_rows(const T* p, int L, int cnt, int avail, T (&v)[3][R]) {
-    constexpr int U = unit_bytes<T, R>();
-    using V = typename Unit<U>::type;
-    const bool vec = avail >= R && (reinterpret_cast<uintptr_t>(p) % U) == 0 &&
-                     ((size_t)L * sizeof(T)) % U == 0;
-    if (vec) {
-        V a[3][R * sizeof(T) / U];
+    if (avail >= R) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) load_run(p + (size_t)k * L, v[k]);
 #pragma unroll
         for (int k = 0; k < 3; ++k)
 #pragma unroll
-            for (int i = 0; i < (int)(R * sizeof(T) / U); ++i) a[k][i] = reinterpret_cast<const V*>(p + (size_t)k * L)[i];
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            __builtin_memcpy(v[k], a[k], sizeof(v[k]));
-#pragma unroll
             for (int i = 0; i < R; ++i) v[k][i] = i < cnt ? v[k][i] : (T)0;
-        }
     } else {
 #pragma unroll
         for (int k = 0; k < 3; ++k)
@@ -366,38 +344,10 @@ __device__ __forceinline__ void lane_load_rows(const T* p, int L, int cnt, int a
     }
 }
 
-// Vector types of 4, 8 and 16 bytes that __builtin_nontemporal_store takes.
-template <int U>
-struct StreamUnit;
-template <>
-struct StreamUnit<2> {
-    using type = uint16_t;
-};
-template <>
-struct StreamUnit<4> {
-    using type = uint32_t;
-};
-template <>
-struct StreamUnit<8> {
-    typedef unsigned int type __attribute__((ext_vector_type(2)));
-};
-template <>
-struct StreamUnit<16> {
-    typedef unsigned int type __attribute__((ext_vector_type(4)));
-};
-
-// Whole aligned runs go out as nontemporal (streaming) stores: the outputs
-// are never read back by the kernel that writes them.
 template <typename T, int N>
 __device__ __forceinline__ void lane_store(T* p, int cnt, const T (&v)[N]) {
-    constexpr int U = unit_bytes<T, N>();
-    using V = typename StreamUnit<U>::type;
-    if (cnt >= N && (reinterpret_cast<uintptr_t>(p) % U) == 0) {
-        V w[N * sizeof(T) / U];
-        __builtin_memcpy(w, v, sizeof(v));
-#pragma unroll
-        for (int i = 0; i < (int)(N * sizeof(T) / U); ++i)
-            __builtin_nontemporal_store(w[i], reinterpret_cast<V*>(p) + i);
+    if (cnt >= N) {
+        store_bytes<N * (int)sizeof(T)>(reinterpret_cast<char*>(p), reinterpret_cast<const char*>(v));
     } else {
 #pragma unroll
         for (int i = 0; i < N; ++i)
