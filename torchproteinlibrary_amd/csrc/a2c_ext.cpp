@@ -225,12 +225,14 @@ struct Angles2Coords : torch::autograd::Function<Angles2Coords> {
         ctx->saved_data["length"] = angles.size(2);
         ctx->saved_data["order"] = order;
         ctx->mark_non_differentiable({res_names, atom_names});
+        ctx->set_materialize_grads(false);  // the names' would be filled with zeros for nothing
         return {coords, res_names, atom_names};
     }
     static variable_list backward(AutogradContext* ctx, variable_list grads) {
         const auto saved = ctx->get_saved_variables();
         return native_fn::backward(grads, [&]() -> variable_list {
-            const Tensor &seqs = saved[0], &coords = saved[1], g = grads[0].contiguous();
+            const Tensor &seqs = saved[0], &coords = saved[1];
+            const Tensor g = grads[0].defined() ? grads[0].contiguous() : torch::zeros_like(coords);
             c10::DeviceGuard guard(coords.device());
             const hipStream_t s = stream_of(coords);
             Tensor out = torch::empty({coords.size(0), 8, ctx->saved_data["length"].toInt()}, coords.options());

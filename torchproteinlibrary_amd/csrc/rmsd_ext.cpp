@@ -183,6 +183,7 @@ struct Coords2RMSD : torch::autograd::Function<Coords2RMSD> {
         });
         if (bits) native_fn::python(kLayer, "_raise_on_bits", bits, "forward");
         ctx->mark_non_differentiable({UT});
+        ctx->set_materialize_grads(false);  // UT's would be filled with zeros for nothing
         if (needs) ctx->save_for_backward({x, y, n, state});
         return {rmsd, UT};
     }
@@ -193,7 +194,8 @@ struct Coords2RMSD : torch::autograd::Function<Coords2RMSD> {
             auto [B, A] = check_inputs(x, y, n);
             c10::DeviceGuard guard(x.device());
             const hipStream_t s = stream_of(x);
-            const torch::Tensor g = native_fn::like_dtype(grads[0], x);
+            const torch::Tensor g =
+                grads[0].defined() ? native_fn::like_dtype(grads[0], x) : torch::zeros({B}, x.options());
             check_like(g, x, {B}, "gradRMSD");
             torch::Tensor gx = torch::empty_like(x);
             const uint32_t bits = native_fn::run(s, [&, B = B, A = A](uint32_t* flags) {
