@@ -2437,15 +2437,28 @@ const char* tpl_a2c_strerror(int code) {
 }
 
 int tpl_a2c_num_atoms(const char* sequence) {
-    static const Residue res[kTypes] = A2C_RESIDUES;
+    // Atoms by letter, -1 outside the 20 (32 sequences of 350 letters: 78 -> 7
+    // us against looking up each letter's residue).
+    struct Counts {
+        int8_t of[256];
+    };
+    static const Counts counts = [] {
+        static const Residue res[kTypes] = A2C_RESIDUES;
+        Counts c;
+        for (int k = 0; k < 256; ++k) {
+            const int t = residue_type((uint8_t)k);
+            c.of[k] = (int8_t)(t < 0 ? -1 : res[t].natoms);
+        }
+        return c;
+    }();
     if (!sequence) return -1;
-    int n = 0;
+    int n = 0, bad = 0;
     for (const char* p = sequence; *p; ++p) {
-        const int t = residue_type((uint8_t)*p);
-        if (t < 0) return -1;
-        n += res[t].natoms;
+        const int k = counts.of[(uint8_t)*p];
+        bad |= k;  // negative once a letter is
+        n += k;
     }
-    return n;
+    return bad < 0 ? -1 : n;
 }
 
 int tpl_a2c_forward_ordered(const int32_t* order, int dtype, const uint8_t* sequences, int seq_stride,
