@@ -1,6 +1,6 @@
 """Few large structures, several workgroups each, against the same structures
 in a batch of 65, which take one workgroup each: sizes at the edges of the rule
-(8192 atoms, 64 structures), counts at the edges of a workgroup's share, strides
+(10240 atoms, 32 structures), counts at the edges of a workgroup's share, strides
 of every alignment."""
 import numpy as np
 import pytest
@@ -10,7 +10,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
-@pytest.mark.parametrize("B,A", [(1, 8191), (1, 8192), (3, 8193), (2, 20002), (64, 8195), (40, 13000), (1, 66001)])
+@pytest.mark.parametrize("B,A", [(1, 8191), (1, 8192), (3, 8193), (2, 20002), (64, 8195), (40, 13000), (1, 66001),
+                                 (1, 10239), (1, 10240), (3, 10241), (32, 10243), (33, 10243), (32, 17000)])
 def test_split_matches_one_workgroup(dtype, B, A):
     from torchproteinlibrary_amd.RMSD import Coords2RMSD
     rng = np.random.default_rng(B * 7 + A)
@@ -53,11 +54,39 @@ def test_split_matches_one_workgroup(dtype, B, A):
 
 def test_split_errors():
     from torchproteinlibrary_amd.RMSD import Coords2RMSD
-    x = torch.randn(2, 3 * 9000, device="cuda")
-    y = torch.randn(2, 3 * 9000, device="cuda")
-    n = torch.tensor([9000, 9000], dtype=torch.int32, device="cuda")
+    x = torch.randn(2, 3 * 12000, device="cuda")
+    y = torch.randn(2, 3 * 12000, device="cuda")
+    n = torch.tensor([12000, 12000], dtype=torch.int32, device="cuda")
     with pytest.raises(ValueError, match="num_atoms"):
         Coords2RMSD()(x, y, n + 1)
-    x[1, 3 * 8999] = float("nan")
+    x[1, 3 * 11999] = float("nan")
     with pytest.raises(Exception, match="forward Nan"):
         Coords2RMSD()(x, y, n)
+
+
+@pytest.mark.parametrize("B,A", [(1, 10240), (8, 12001), (32, 10300), (2, 66001)])
+def test_split_accuracy(B, A):
+    """rmsd in float64 against the residuals of the layer's own rotation, summed
+    in extended precision (the rotation's rounding counts in second order)."""
+    from torchproteinlibrary_amd.RMSD import Coords2RMSD
+    rng = np.random.default_rng(A)
+    n = rng.integers(A // 2, A + 1, B)
+    x, y = np.zeros((B, A, 3)), np.zeros((B, A, 3))
+    for b, k in enumerate(n):
+        step = rng.standard_normal((k, 3))
+        x[b, :k] = np.cumsum(1.5 * step / np.linalg.norm(step, axis=1, keepdims=True), axis=0) + 30.0
+        q, _ = np.linalg.qr(rng.standard_normal((3, 3)))
+        q *= np.sign(np.linalg.det(q))
+        y[b, :k] = x[b, :k] @ q + 2.0 * rng.standard_normal((k, 3)) - 20.0
+    layer = Coords2RMSD()
+    r = layer(*(torch.from_numpy(v.reshape(B, 3 * A)).cuda() for v in (x, y)),
+              torch.from_numpy(n.astype(np.int32)).cuda()).cpu().numpy()
+    ut = layer.UT.cpu().numpy().astype(np.longdouble)
+    for b, k in enumerate(n):
+        xb, yb = (v[b, :k].astype(np.longdouble) for v in (x, y))
+        off = (xb - xb.mean(0)) - (yb - yb.mean(0)) @ ut[b].T
+        dev = (off ** 2).sum() + np.longdouble(1e-10)
+        # At most 30 roundings on an atom's way into the sums that keep both
+        # parts, a third of 2^-53 each on average, over at least 120 of them.
+        moments = ((xb - xb[0]) ** 2).sum() + ((yb - yb[0]) ** 2).sum()
+        assert abs(r[b] - np.sqrt(dev / k)) <= 2.0 ** -53 * moments / (2 * np.sqrt(dev * k)) + 1e-15 * r[b], (b, k)

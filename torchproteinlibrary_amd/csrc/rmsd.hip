@@ -74,8 +74,9 @@ __device__ __forceinline__ int clamp_count(int n, int A, const Report& rep, bool
 // 17 partial sums (laid out [moment][thread]), then kParts partial sums per
 // moment, then the totals.  A cross-lane butterfly over 17 doubles measured
 // 5 us per workgroup, bound by the LDS crossbar at 16 waves per CU; this takes
-// plain LDS reads and three barriers.
-__device__ __forceinline__ void workgroup_sums(const double m[kMoments], double* tot) {
+// plain LDS reads and three barriers.  `low` (nullptr: not wanted) takes what
+// the last level rounds off: the levels before it add up few and small terms.
+__device__ __forceinline__ void workgroup_sums(const double m[kMoments], double* tot, double* low) {
     constexpr int kParts = kThreads / kMoments;  // 15 threads per moment in the middle level
     __shared__ double s_m[kMoments * kThreads];
     __shared__ double s_p[kMoments * kParts];
@@ -91,10 +92,15 @@ __device__ __forceinline__ void workgroup_sums(const double m[kMoments], double*
     }
     __syncthreads();
     if (tid < kMoments) {
-        double acc = 0.0;
+        double acc = 0.0, off = 0.0;
 #pragma unroll
-        for (int part = 0; part < kParts; ++part) acc += s_p[tid * kParts + part];
+        for (int part = 0; part < kParts; ++part) {
+            const rmsd_math::Two t = rmsd_math::two_sum(acc, s_p[tid * kParts + part]);
+            acc = t.h;
+            off += t.l;
+        }
         tot[tid] = acc;
+        if (low) low[tid] = off;
     }
     __syncthreads();
 }
@@ -140,6 +146,38 @@ __device__ __forceinline__ void first_atoms(const T* xb, const T* yb, int n, dou
     }
 }
 
+// One lane: the result of structure b, whose means are x0 + mx and y0 + my.
+template <typename T>
+__device__ __forceinline__ void store_result(double rmsd, const double U[9], const double x0[3], const double y0[3],
+                                             const double mx[3], const double my[3], int b, T* rmsd_out, T* ut_out,
+                                             double* state, const Report& rep) {
+    rmsd_out[b] = (T)rmsd;
+#pragma unroll
+    for (int j = 0; j < 3; ++j)
+#pragma unroll
+        for (int k = 0; k < 3; ++k) ut_out[9 * b + 3 * j + k] = (T)U[3 * k + j];
+    if (state) {
+        double* s = state + (size_t)b * kState;
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            s[c] = x0[c] + mx[c];
+            s[3 + c] = y0[c] + my[c];
+        }
+#pragma unroll
+        for (int k = 0; k < 9; ++k) s[6 + k] = U[k];
+        s[15] = rmsd;
+    }
+    if (rmsd != rmsd) report_bits(rep, TPL_RMSD_STATUS_NAN);
+}
+
+// r2 - 2|lambda| is >= 0 in exact arithmetic; for (nearly) identical
+// structures its FP64 rounding (~1e-16 r2) can make it negative, which
+// the reference's formula turns into NaN.  Clamped at 0 here; a NaN (from
+// NaN coordinates) stays NaN and is reported.
+__device__ __forceinline__ double rmsd_of(double dev, double nd) {
+    return sqrt(((dev < 0.0 ? 0.0 : dev) + kEpsLimit) / nd);
+}
+
 // One lane: the result of structure b from its moments.
 template <typename T>
 __device__ __forceinline__ void finish(const double m[kMoments], const double x0[3], const double y0[3], int n, int b,
@@ -162,31 +200,9 @@ __device__ __forceinline__ void finish(const double m[kMoments], const double x0
     double F[16], U[9];
     rmsd_math::f_matrix(R, F);
     const rmsd_math::Eigenpair eig = rmsd_math::max_eigenpair(F, 0.5 * r2);
-    const double lam = eig.lam;
     rmsd_math::u_from_q(eig, U);
-    // r2 - 2|lambda| is >= 0 in exact arithmetic; for (nearly) identical
-    // structures its FP64 rounding (~1e-16 r2) can make it negative, which
-    // the reference's formula turns into NaN.  Clamped at 0 here; a NaN (from
-    // NaN coordinates) stays NaN and is reported.
-    const double dev = r2 - 2.0 * fabs(lam);
-    const double rmsd = sqrt(((dev < 0.0 ? 0.0 : dev) + kEpsLimit) / nd);
-    rmsd_out[b] = (T)rmsd;
-#pragma unroll
-    for (int j = 0; j < 3; ++j)
-#pragma unroll
-        for (int k = 0; k < 3; ++k) ut_out[9 * b + 3 * j + k] = (T)U[3 * k + j];
-    if (state) {
-        double* s = state + (size_t)b * kState;
-#pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            s[c] = x0[c] + mx[c];
-            s[3 + c] = y0[c] + my[c];
-        }
-#pragma unroll
-        for (int k = 0; k < 9; ++k) s[6 + k] = U[k];
-        s[15] = rmsd;
-    }
-    if (rmsd != rmsd) report_bits(rep, TPL_RMSD_STATUS_NAN);
+    const double rmsd = rmsd_of(r2 - 2.0 * fabs(eig.lam), nd);
+    store_result(rmsd, U, x0, y0, mx, my, b, rmsd_out, ut_out, state, rep);
 }
 
 template <typename T>
@@ -201,7 +217,7 @@ __global__ void __launch_bounds__(kThreads) rmsd_fwd(const T* __restrict__ x, co
     double x0[3], y0[3], m[kMoments] = {};
     first_atoms(xb, yb, n, x0, y0);
     add_moments(xb, yb, 4 * tid, 4 * kThreads, n, x0, y0, m);
-    workgroup_sums(m, s_tot);
+    workgroup_sums(m, s_tot, nullptr);
     if (tid != 0) return;
 #pragma unroll
     for (int e = 0; e < kMoments; ++e) m[e] = s_tot[e];
@@ -209,15 +225,22 @@ __global__ void __launch_bounds__(kThreads) rmsd_fwd(const T* __restrict__ x, co
 }
 
 // Few large structures: S workgroups per structure, whose sums go to part
-// [B][kMoments][S], and a wave per structure that adds them up.  One workgroup
-// alone is bound by the latency of its passes (20 of 1024 atoms at 20000):
-// 8 structures of up to 20000 atoms, float64, 14.8 -> 8.3 us; one, float32,
-// 16.0 -> 7.7.
+// [B][kMoments][2][S] with what they round off, and a workgroup per structure that
+// adds them up.  One workgroup alone is bound by the latency of its passes (20
+// of 1024 atoms at 20000), us, back to back: 8 structures of 20000 atoms, float64,
+// 16.4 -> 11.4; one, float32, 15.6 -> 9.6.  The second launch is bound by the
+// eigen-solve of one lane and takes most of that.
+// In float64 the last levels of the sums, the centring and r2 - 2 lambda keep
+// both parts of each number: in another order than one workgroup's the plain
+// sums round as much, but not the same way, and r2 is hundreds of times what
+// remains of it.  rmsd of 8 structures of 9000..12001 atoms, 16 draws, off by
+// (root mean square, relative): one workgroup 1.6e-13, plain split 1.5e-13,
+// this 1.2e-14.
 template <typename T>
 __global__ void __launch_bounds__(kThreads) rmsd_part(const T* __restrict__ x, const T* __restrict__ y,
                                                       const int32_t* __restrict__ num_atoms, double* part, int A,
                                                       int S) {
-    __shared__ double s_tot[kMoments];
+    __shared__ double s_tot[kMoments], s_low[kMoments];
     const int b = (int)blockIdx.x / S, s = (int)blockIdx.x - b * S, tid = threadIdx.x;
     const int n = clamp_count(num_atoms[b], A, Report{nullptr, nullptr}, false);
     const T* xb = x + (size_t)b * 3 * A;
@@ -225,31 +248,79 @@ __global__ void __launch_bounds__(kThreads) rmsd_part(const T* __restrict__ x, c
     double x0[3], y0[3], m[kMoments] = {};
     first_atoms(xb, yb, n, x0, y0);
     add_moments(xb, yb, 4 * (s * kThreads + tid), 4 * kThreads * S, n, x0, y0, m);
-    workgroup_sums(m, s_tot);
-    if (tid < kMoments) part[((size_t)b * kMoments + tid) * S + s] = s_tot[tid];
+    workgroup_sums(m, s_tot, s_low);
+    if (tid < 2 * kMoments)
+        part[((size_t)b * 2 * kMoments + tid) * S + s] = (tid & 1 ? s_low : s_tot)[tid >> 1];
 }
+__device__ __forceinline__ rmsd_math::Two two_sum_over(rmsd_math::Two v, int width) {
+    for (int d = width / 2; d > 0; d >>= 1)
+        v = rmsd_math::two_add(v, rmsd_math::Two{__shfl_xor(v.h, d), __shfl_xor(v.l, d)});
+    return v;
+}
+constexpr int kJoin = 16;                                      // threads per moment
+constexpr int kJoinThreads = (kMoments * kJoin + 63) / 64 * 64;  // whole waves
 template <typename T>
-__global__ void __launch_bounds__(64) rmsd_join(const T* __restrict__ x, const T* __restrict__ y,
-                                                const int32_t* __restrict__ num_atoms,
-                                                const double* __restrict__ part, T* rmsd_out, T* ut_out,
-                                                double* state, Report rep, int A, int S) {
-    __shared__ double s_tot[kMoments];
+__global__ void __launch_bounds__(kJoinThreads) rmsd_join(const T* __restrict__ x, const T* __restrict__ y,
+                                                          const int32_t* __restrict__ num_atoms,
+                                                          const double* __restrict__ part, T* rmsd_out, T* ut_out,
+                                                          double* state, Report rep, int A, int S) {
+    using rmsd_math::Two;
+    __shared__ Two s_tot[kMoments], s_r[10];
     const int b = blockIdx.x, lane = threadIdx.x;
+    Two v{0.0, 0.0};
+    const int e = lane / kJoin;
+    if (e < kMoments) {
+        const double* p = part + ((size_t)b * kMoments + e) * 2 * S;
+        for (int s = lane % kJoin; s < S; s += kJoin) {
+            const Two t = rmsd_math::two_sum(v.h, p[s]);
+            v = Two{t.h, v.l + (t.l + p[S + s])};
+        }
+    }
+    v = two_sum_over(v, kJoin);
+    if (e < kMoments && lane % kJoin == 0) s_tot[e] = v;
+    __syncthreads();
+    if (lane >= 64) return;
     const int n = clamp_count(num_atoms[b], A, rep, lane == 0);
+    const double nd = (double)n;
     double x0[3], y0[3], m[kMoments];
     first_atoms(x + (size_t)b * 3 * A, y + (size_t)b * 3 * A, n, x0, y0);
-    if (lane < kMoments) {
-        const double* p = part + ((size_t)b * kMoments + lane) * S;
-        double v = 0.0;
-#pragma unroll 8
-        for (int s = 0; s < S; ++s) v += p[s];
-        s_tot[lane] = v;
-    }
-    __syncthreads();
-    if (lane != 0) return;
 #pragma unroll
-    for (int e = 0; e < kMoments; ++e) m[e] = s_tot[e];
-    finish(m, x0, y0, n, b, rmsd_out, ut_out, state, rep);
+    for (int k = 0; k < kMoments; ++k) m[k] = s_tot[k].h;
+    if constexpr (sizeof(T) == 4) {  // the rounding to float is far larger
+        if (lane == 0) finish(m, x0, y0, n, b, rmsd_out, ut_out, state, rep);
+        return;
+    }
+    // R by lanes 0-8, |x|^2 and |y|^2 centred by lanes 16-23, each sum less
+    // what centring takes off.
+    if (lane < 9 || (lane >= 16 && lane < 24)) {
+        const int k = lane - 18;
+        const int r = lane < 9 ? lane / 3 : k, c = lane < 9 ? 3 + lane % 3 : k;
+        v = lane < 9 ? s_tot[6 + lane] : k < 0 ? s_tot[lane - 1] : Two{0.0, 0.0};
+        if ((lane < 9 || k >= 0) && n > 0) v = rmsd_math::two_sub(v, rmsd_math::two_mul_div(s_tot[r], s_tot[c], nd));
+    } else {
+        v = Two{0.0, 0.0};
+    }
+    if (lane < 9) s_r[lane] = v;
+    v = two_sum_over(v, 8);
+    if (lane == 16) s_r[9] = v;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");  // one wave is left
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    const Two f = rmsd_math::deviation_factor(s_r, s_r[9], lane < 10 ? lane : 0);
+    double R[9], F[16], U[9], mx[3], my[3];
+#pragma unroll
+    for (int k = 0; k < 9; ++k) R[k] = s_r[k].h;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        mx[c] = n > 0 ? m[c] / nd : 0.0;
+        my[c] = n > 0 ? m[3 + c] / nd : 0.0;
+    }
+    rmsd_math::f_matrix(R, F);
+    const rmsd_math::Eigenpair eig = rmsd_math::max_eigenpair(F, 0.5 * s_r[9].h);
+    v = two_sum_over(lane < 10 ? rmsd_math::deviation_term(f, eig, lane) : Two{0.0, 0.0}, 16);
+    if (lane != 0) return;
+    rmsd_math::u_from_q(eig, U);
+    store_result(rmsd_of(v.h, nd), U, x0, y0, mx, my, b, rmsd_out, ut_out, state, rep);
 }
 
 // One thread per atom slot; the grid covers nblk blocks per structure.
@@ -303,12 +374,14 @@ int check(int dtype, int B, int A) {
 
 // Workgroups per structure in the split forward, 1 where it does not pay: every
 // workgroup has a full pass of 1024 atoms and no more of them run than the GPU
-// holds at two per CU; fewer than 8 passes cost less than the second launch (64
-// structures of 5000 atoms take 7.5 us in one launch).
+// holds at two per CU.  The second launch costs as much as 8 passes, and 64
+// structures fill the GPU by themselves; one launch -> split, float64, us:
+// 8 structures of 8192 atoms 10.4 -> 10.8, of 12001 12.7 -> 11.6, 32 of 12001
+// 12.9 -> 12.1, 64 of 12001 15.8 -> 16.7.
 int split_of(int B, int A) {
-    if (B <= 0 || B > 64) return 1;
+    if (B <= 0 || B > 32) return 1;
     const int s = std::min({64, A / (4 * kThreads), 512 / B});
-    return s >= 8 ? s : 1;
+    return s >= 10 ? s : 1;
 }
 
 template <typename T>
@@ -320,7 +393,7 @@ void launch_forward(const void* input, const void* target, const int32_t* num_at
     const int S = split_of(B, A);
     if (S > 1 && part) {
         hipLaunchKernelGGL(rmsd_part<T>, dim3(B * S), dim3(kThreads), 0, s, x, y, num_atoms, part, A, S);
-        hipLaunchKernelGGL(rmsd_join<T>, dim3(B), dim3(64), 0, s, x, y, num_atoms, part, r, u, st, rep, A, S);
+        hipLaunchKernelGGL(rmsd_join<T>, dim3(B), dim3(kJoinThreads), 0, s, x, y, num_atoms, part, r, u, st, rep, A, S);
     } else {
         hipLaunchKernelGGL(rmsd_fwd<T>, dim3(B), dim3(kThreads), 0, s, x, y, num_atoms, r, u, st, rep, A);
     }
@@ -402,7 +475,7 @@ int tpl_rmsd_backward(int dtype, void* grad_input, const void* grad_rmsd, const 
 
 size_t tplx_rmsd_workspace_bytes(int batch, int atoms_stride) {
     const int S = split_of(batch, atoms_stride);
-    return S > 1 ? (size_t)batch * kMoments * S * sizeof(double) : 0;
+    return S > 1 ? (size_t)batch * 2 * kMoments * S * sizeof(double) : 0;
 }
 
 int tplx_rmsd_forward(int dtype, const void* input, const void* target, const int32_t* num_atoms, void* rmsd,

@@ -31,9 +31,11 @@
 #if defined(__HIPCC__)
 #define RMSD_HD __host__ __device__ __forceinline__
 #define RMSD_UNROLL _Pragma("unroll")
+#define RMSD_EXACT _Pragma("clang fp contract(off)")
 #else
 #define RMSD_HD inline
 #define RMSD_UNROLL
+#define RMSD_EXACT
 #endif
 
 namespace rmsd_math {
@@ -168,6 +170,58 @@ RMSD_HD Eigenpair max_eigenpair(const double F[16], double bound) {
     }
     const double inv = 1.0 / sqrt(w0 * w0 + w1 * w1 + w2 * w2 + w3 * w3);
     return Eigenpair{lam, w0 * inv, w1 * inv, w2 * inv, w3 * inv, degenerate};
+}
+
+// An unevaluated sum h + l, |l| <= 2^-53 |h| after two_sum (T. J. Dekker,
+// Numer. Math. 18 (1971) 224-242).  Contraction is off where it would change
+// what the low part stands for.
+struct Two {
+    double h, l;
+};
+RMSD_HD Two two_sum(double a, double b) {
+    RMSD_EXACT
+    const double s = a + b, t = s - a;
+    return Two{s, (a - (s - t)) + (b - t)};
+}
+RMSD_HD Two two_add(Two a, Two b) {
+    const Two s = two_sum(a.h, b.h);
+    return two_sum(s.h, s.l + (a.l + b.l));
+}
+RMSD_HD Two two_sub(Two a, Two b) { return two_add(a, Two{-b.h, -b.l}); }
+RMSD_HD Two two_mul(Two a, Two b) {
+    RMSD_EXACT
+    const double p = a.h * b.h;
+    return two_sum(p, fma(a.h, b.h, -p) + (a.h * b.l + a.l * b.h));
+}
+// a b / n
+RMSD_HD Two two_mul_div(Two a, Two b, double n) {
+    const Two p = two_mul(a, b);
+    const double q = p.h / n;
+    return two_sum(q, (fma(-q, n, p.h) + p.l) / n);
+}
+
+// r2 - 2 q^T F q, what the rotation of the unit quaternion q leaves of r2, as a
+// sum of ten terms f[k] q_i q_j: an error of q counts in second order only, so
+// this keeps the digits that r2 - 2 lambda of sums rounded to FP64 loses where
+// r2 is many times the result.  The ten f from R and r2, one a call (k: the
+// four squares, then 01 02 03 12 13 23), and the term.
+RMSD_HD Two deviation_factor(const Two* R, Two r2, int k) {
+    const bool square = k < 4;
+    const int a = (int)((0x5211650000ull >> (4 * k)) & 15), b = (int)((0x7633274444ull >> (4 * k)) & 15);
+    // Signs of R[a], R[b] and, in a square, R[8].
+    const double sa = (0x00cu >> k) & 1 ? -1.0 : 1.0, sb = (0x07au >> k) & 1 ? -1.0 : 1.0;
+    const double sc = (0x006u >> k) & 1 ? -1.0 : 1.0;
+    Two f = two_add(Two{sa * R[a].h, sa * R[a].l}, Two{sb * R[b].h, sb * R[b].l});
+    if (square) f = two_add(f, Two{sc * R[8].h, sc * R[8].l});
+    const double w = square ? -2.0 : -4.0;
+    f = Two{w * f.h, w * f.l};
+    return square ? two_add(r2, f) : f;
+}
+RMSD_HD Two deviation_term(Two f, const Eigenpair& e, int k) {
+    const int i = (int)((0x2110003210ull >> (4 * k)) & 15), j = (int)((0x3323213210ull >> (4 * k)) & 15);
+    const double qi = i == 0 ? e.q0 : i == 1 ? e.q1 : i == 2 ? e.q2 : e.q3;
+    const double qj = j == 0 ? e.q0 : j == 1 ? e.q1 : j == 2 ? e.q2 : e.q3;
+    return two_mul(f, two_mul(Two{qi, 0.0}, Two{qj, 0.0}));
 }
 
 }  // namespace rmsd_math
