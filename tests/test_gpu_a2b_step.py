@@ -109,3 +109,40 @@ def test_step_under_capture(B):
         got = step.coords.clone(), step.grad_angles.clone()
         step.replay()
         assert torch.equal(got[0], step.coords) and torch.equal(got[1], step.grad_angles)
+
+
+@pytest.mark.parametrize("dtype,B,L,R", [
+    (torch.float32, 3, 256, 1), (torch.float32, 3, 257, 2), (torch.float32, 3, 513, 4), (torch.float32, 3, 2048, 4),
+    (torch.float32, 3, 2049, 1), (torch.float32, 16, 4096, 1), (torch.float32, 17, 4096, 2),
+    (torch.float32, 3, 4097, 2), (torch.float32, 32, 4200, 4),
+    (torch.float64, 3, 300, 2), (torch.float64, 3, 1024, 2), (torch.float64, 3, 1025, 1), (torch.float64, 20, 4097, 2),
+])
+def test_step_rule(dtype, B, L, R):
+    from torchproteinlibrary_amd import _tuning
+    from torchproteinlibrary_amd.ReducedModel.Angles2Backbone.Angles2Backbone import Angles2BackboneStep
+    lens = _lengths(B, L, "mixed", 64 * R, np.random.default_rng(L))
+    a, ln, g = _case(B, L, lens, dtype, B + L)
+    step = Angles2BackboneStep(a, ln)
+    assert step.config == (R, R)
+    step.grad_coords.copy_(g)
+    step.replay()
+    _check(step, a, ln, g, dtype)
+    # What a caller pins stays first, for the shape or for one mix of lengths.
+    other = (2, 2) if R == 1 else (1, 1)
+    try:
+        for lengths in (ln, None):
+            _tuning.clear()
+            _tuning.set_config(a, other, lengths)
+            assert _tuning.pinned_config(a, ln) == other
+            assert Angles2BackboneStep(a, ln).config == other
+    finally:
+        _tuning.clear()
+    assert _tuning.pinned_config(a, ln) is None
+
+
+def test_step_of_nothing():
+    from torchproteinlibrary_amd.ReducedModel.Angles2Backbone.Angles2Backbone import Angles2BackboneStep
+    for B, L in ((0, 5), (3, 0)):
+        step = Angles2BackboneStep(torch.zeros(B, 3, L, device="cuda"), torch.zeros(B, dtype=torch.int32, device="cuda"))
+        step.replay()
+        assert step.coords.shape == (B, 9 * L) and step.grad_angles.shape == (B, 3, L)

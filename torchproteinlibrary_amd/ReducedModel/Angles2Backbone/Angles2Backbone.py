@@ -268,6 +268,38 @@ class Angles2Backbone(Module):
         return Angles2BackboneGPUFunction.apply(input, angles_length)
 
 
+def _step_residues(dtype, B, L):
+    """Residues per lane of a step, or None where the length mix decides.
+
+    The tuner times the layer's two kernels, and the step's own behave
+    otherwise: up to 8 chunks a chain (4 of 64 residues) are one kernel, more
+    are two, and a wave has both directions' work, so a lane's residues are the
+    length of its chain of operations while the GPU is not full.  Steps, us,
+    by residues per lane (equal lengths, float32 unless marked):
+      one kernel while it can be, with few residues per lane:
+        512 x 100      1:  7.8  2:  9.2    1024 x 20..256  1: 11.8  2: 13.7
+        32 x 700, f64  1: 13.1  2: 10.2    128 x 1030      2: 19.1  4: 13.9
+      but full GPUs go by the mix (800 x 500  2: 20.0  4: 15.8, 1024 x 30..512
+      2: 13.1  4: 16.8; 4000 x 200  1: 66.3  2: 59.2, x 10..200  1: 45.5  2: 48.5);
+      in two kernels, as many waves as there are SIMDs (1024), in chains of at
+      most 64 chunks of 64 (one record per lane to scan):
+        16 x 4000      1: 13.6  2: 15.0  4: 17.9
+        32 x 4000      1: 18.1  2: 15.3  4: 17.9
+        32 x 5000      1: 27.1  2: 20.4  4: 18.4
+        1 x 16384      1: 20.0  2: 17.1  4: 17.5
+    """
+    most = 4 if dtype == torch.float32 else 2
+    if L <= 256:
+        return 1 if B <= 2048 else None
+    if L <= 512:
+        return 2 if most == 2 or B <= 512 else None
+    if L <= 512 * most:
+        return most
+    if L <= 4096 and B * -(-L // 64) <= 1024:
+        return 1
+    return 2 if B * -(-L // 128) <= 1024 else most
+
+
 class Angles2BackboneStep:
     """Angles2Backbone forward and backward for fixed shapes, laid out once
     and replayed.
@@ -284,9 +316,10 @@ class Angles2BackboneStep:
     A step reads ``angles``, ``angles_length`` and ``grad_coords`` from their
     memory at every replay, so a loop updates them in place between replays;
     it writes ``coords`` and ``grad_angles``.  A replay under a capture is
-    captured.  The chunk sizes are the tuned ones for these inputs (the
-    backward's for both directions where the step has kernels of its own), or
-    ``config`` (forward, backward residues per lane).
+    captured.  The chunk sizes are ``config`` (forward, backward residues per
+    lane), those pinned for these inputs, those of a rule on the shape
+    (``_step_residues``), or the tuned ones (the backward's for both
+    directions where the step has kernels of its own).
 
     Replays do not check for NaN or out-of-range lengths (the checks of the
     layer read a status word on the host); lengths must stay within
@@ -307,11 +340,14 @@ class Angles2BackboneStep:
         if config is not None:
             cfg = tuple(config)
         else:
-            cfg = _tuning.config_for(angles, angles_length)
-            own = (cfg[1], cfg[1])
+            cfg = _tuning.pinned_config(angles, angles_length)
+            r = _step_residues(dt, B, L) if cfg is None else cfg[1]
             with torch.cuda.device(dev):
-                if ext.step_fits(dt == torch.float64, B, L, list(own)):
-                    cfg = own
+                if r is None or (cfg is None and not ext.step_fits(dt == torch.float64, B, L, [r, r])):
+                    cfg = _tuning.config_for(angles, angles_length)
+                    r = cfg[1]
+                if ext.step_fits(dt == torch.float64, B, L, [r, r]):
+                    cfg = (r, r)
         self.angles = angles
         self.angles_length = angles_length
         self.config = cfg

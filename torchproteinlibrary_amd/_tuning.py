@@ -17,6 +17,9 @@ tuner ``tpl_a2b_tune`` runs each candidate's forward+backward steps back to
 back, as a training loop does, with the candidates taking turns over a few
 passes, and keeps each one's median.
 
+``Angles2BackboneStep`` asks for these configs only where a rule on its shape
+does not name one (its kernels are not those that are timed here).
+
 Environment: ``TPL_A2B_TUNE=0`` disables tuning (default config always).
 """
 from __future__ import annotations
@@ -30,6 +33,7 @@ from ._native import ext
 
 _lock = threading.Lock()
 _cache: dict = {}
+_pinned: set = set()  # keys of _cache that set_config wrote
 _timings: dict = {}
 _bucket_memo: dict = {}
 _last_bucket: dict = {}
@@ -96,10 +100,22 @@ def set_config(angles_like: torch.Tensor, config, lengths: torch.Tensor | None =
     with _lock:
         shape = _shape_key(angles_like)
         cfg = tuple(int(c) for c in config)
-        if lengths is None:
-            _cache[shape + ("any",)] = cfg
-        else:
-            _cache[shape + (_bucket(angles_like, lengths, True),)] = cfg
+        key = shape + ("any" if lengths is None else _bucket(angles_like, lengths, True),)
+        _cache[key] = cfg
+        _pinned.add(key)
+
+
+def pinned_config(angles: torch.Tensor, lengths: torch.Tensor):
+    """The config that set_config pinned for these inputs, or None."""
+    shape = _shape_key(angles)
+    with _lock:
+        mixes = {key[-1] for key in _pinned if key[:-1] == shape}
+    if not mixes:
+        return None
+    if "any" in mixes:
+        return _cache[shape + ("any",)]
+    bucket = _bucket(angles, lengths, not torch.cuda.is_current_stream_capturing())
+    return _cache[shape + (bucket,)] if bucket in mixes else None
 
 
 def cached_config(angles: torch.Tensor, lengths: torch.Tensor | None = None):
@@ -119,6 +135,7 @@ def timings(angles: torch.Tensor, lengths: torch.Tensor):
 def clear() -> None:
     with _lock:
         _cache.clear()
+        _pinned.clear()
         _timings.clear()
         _bucket_memo.clear()
         _last_bucket.clear()
