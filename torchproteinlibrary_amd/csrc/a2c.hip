@@ -22,11 +22,10 @@
 // 171-184, reduces to this since F x = u cross (x - p)).  u and p follow from
 // the forward's coordinates, so the backward reads those and needs no frames.
 // The subtree of a backbone node is the rest of its residue plus every later
-// residue: a workgroup scan of per-run (sum g, sum x cross g), with runs in
-// reverse thread order so that it is a prefix scan, supplies the downstream
-// part, and each thread walks its residues once more.  For batches that fill the
-// GPU a second backward walks each structure in tiles of consecutive atoms
-// instead (a2c_bwd_tiled), with coalesced loads and each atom read once.
+// residue: again one lane per residue in blocks of 64, whose sums (sum g,
+// sum x cross g) a scan over the lanes and the sums of the later blocks join.
+// Two older backwards stay for callers that pin them: runs of residues per
+// thread (a2c_bwd) and tiles of consecutive atoms (a2c_bwd_tiled).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
