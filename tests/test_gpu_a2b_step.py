@@ -146,3 +146,26 @@ def test_step_of_nothing():
         step = Angles2BackboneStep(torch.zeros(B, 3, L, device="cuda"), torch.zeros(B, dtype=torch.int32, device="cuda"))
         step.replay()
         assert step.coords.shape == (B, 9 * L) and step.grad_angles.shape == (B, 3, L)
+
+
+def test_step_on_another_stream_may_go_while_it_runs():
+    """The memory that only the step holds is not handed out again before a run
+    on another stream than the step's own has ended."""
+    from torchproteinlibrary_amd.ReducedModel.Angles2Backbone.Angles2Backbone import Angles2BackboneStep
+    B, L = 16, 8000
+    a, ln, g = _case(B, L, _lengths(B, L, "mixed", 128, np.random.default_rng(3)), torch.float32, 3)
+    step = Angles2BackboneStep(a, ln)
+    step.grad_coords.copy_(g)
+    step.replay()
+    want = step.coords.clone(), step.grad_angles.clone()
+    coords, grad, grad_coords = step.coords, step.grad_angles, step.grad_coords
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        for _ in range(200):
+            step.replay()
+    del step
+    taken = [torch.full((n,), 255, dtype=torch.uint8, device="cuda") for n in (1 << 18, 1 << 20, 1 << 21, 1 << 22)]
+    side.synchronize()
+    assert torch.equal(coords, want[0]) and torch.equal(grad, want[1])
+    del taken, grad_coords

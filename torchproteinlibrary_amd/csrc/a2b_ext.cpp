@@ -8,6 +8,7 @@
 // Work goes to torch's current HIP stream of the input's device, not the
 // legacy default stream (cBackboneProteinCUDAKernels.cu:166,172,177).
 #include <torch/extension.h>
+#include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <c10/hip/HIPStream.h>
 
 #include <chrono>
@@ -583,6 +584,7 @@ class Step {
         std::tie(B_, L_) = check_inputs(angles, lengths);
         dt_ = dtype_code(angles);
         c10::DeviceGuard guard(angles.device());
+        home_ = c10::hip::getCurrentHIPStream(angles.device().index()).stream();
         check_out(grad_output, angles, {B_, 9 * (int64_t)L_}, "gradOutput");
         check_out(output_coords, angles, {B_, 9 * (int64_t)L_}, "output_coords");
         check_out(grad_input, angles, {B_, 3, L_}, "gradInput");
@@ -596,6 +598,11 @@ class Step {
         const c10::Device dev = angles_.device();
         c10::DeviceGuard guard(dev);
         const hipStream_t s = c10::hip::getCurrentHIPStream(dev.index()).stream();
+        // What only the step holds must outlive its runs on other streams.
+        if (s != home_)
+            for (const torch::Tensor* t : {&records_, &state_, &sync_})
+                if (t->defined())
+                    t->record_stream(at::hip::getCurrentHIPStreamMasqueradingAsCUDA(dev.index()).unwrap());
         const int32_t* len = lengths_.data_ptr<int32_t>();
         int rc;
         if (fused_) {
@@ -616,6 +623,7 @@ class Step {
     tpl_a2b_config cfg_;
     int B_ = 0, L_ = 0, dt_ = 0;
     void *st_ = nullptr, *sy_ = nullptr;
+    hipStream_t home_ = nullptr;  // the stream its memory was allocated on
     bool fused_ = false;
 };
 
