@@ -169,3 +169,15 @@ def test_step_on_another_stream_may_go_while_it_runs():
     side.synchronize()
     assert torch.equal(coords, want[0]) and torch.equal(grad, want[1])
     del taken, grad_coords
+
+
+@pytest.mark.parametrize("B,lo,R", [(600, 500, 2), (768, 500, 2), (769, 500, 4), (1536, 200, 2), (3073, 100, 4)])
+def test_step_rule_counts_waves(B, lo, R):
+    """float32, strides of 257..512 residues: 2 per lane while 3 waves on each of 1024 SIMDs hold all chunks."""
+    from torchproteinlibrary_amd.ReducedModel.Angles2Backbone.Angles2Backbone import Angles2BackboneStep
+    a, ln, g = _case(B, 500, [lo] * B, torch.float32, B)
+    step = Angles2BackboneStep(a, ln)
+    assert step.config == (R, R)
+    step.grad_coords.copy_(g)
+    step.replay()
+    _check(step, a, ln, g, torch.float32)

@@ -268,8 +268,10 @@ class Angles2Backbone(Module):
         return Angles2BackboneGPUFunction.apply(input, angles_length)
 
 
-def _step_residues(dtype, B, L):
-    """Residues per lane of a step, or None where the length mix decides.
+def _step_residues(dtype, B, L, lengths):
+    """Residues per lane of a step, or None where only timing tells.
+    ``lengths()`` gives the lengths on the host, or None where they must not be
+    read; it is called only where the mix decides.
 
     The tuner times the layer's two kernels, and the step's own behave
     otherwise: up to 8 chunks a chain (4 of 64 residues) are one kernel, more
@@ -279,8 +281,10 @@ def _step_residues(dtype, B, L):
       one kernel while it can be, with few residues per lane:
         512 x 100      1:  7.8  2:  9.2    1024 x 20..256  1: 11.8  2: 13.7
         32 x 700, f64  1: 13.1  2: 10.2    128 x 1030      2: 19.1  4: 13.9
-      but full GPUs go by the mix (800 x 500  2: 20.0  4: 15.8, 1024 x 30..512
-      2: 13.1  4: 16.8; 4000 x 200  1: 66.3  2: 59.2, x 10..200  1: 45.5  2: 48.5);
+      but only while all waves of 2 fit, 3 on a SIMD (waves in brackets):
+        1024 x 30..512 [1900]  2: 13.1  4: 16.8    800 x 500  [3200]  2: 20.0  4: 15.8
+        1500 x 30..500 [2700]  2: 16.5  4: 19.5    1500 x 500 [6000]  2: 30.3  4: 26.6
+      and of 1 no line shows (4000 x 200  1: 66.3  2: 59.2, x 10..200  1: 45.5  2: 48.5);
       in two kernels, as many waves as there are SIMDs (1024), in chains of at
       most 64 chunks of 64 (one record per lane to scan):
         16 x 4000      1: 13.6  2: 15.0  4: 17.9
@@ -292,7 +296,10 @@ def _step_residues(dtype, B, L):
     if L <= 256:
         return 1 if B <= 2048 else None
     if L <= 512:
-        return 2 if most == 2 or B <= 512 else None
+        if most == 2 or B <= 512:
+            return 2
+        n = lengths()
+        return None if n is None else 2 if int(((n.clamp(0, L) + 127) // 128).sum()) <= 3072 else 4
     if L <= 512 * most:
         return most
     if L <= 4096 and B * -(-L // 64) <= 1024:
@@ -341,8 +348,9 @@ class Angles2BackboneStep:
             cfg = tuple(config)
         else:
             cfg = _tuning.pinned_config(angles, angles_length)
-            r = _step_residues(dt, B, L) if cfg is None else cfg[1]
             with torch.cuda.device(dev):
+                r = cfg[1] if cfg is not None else _step_residues(
+                    dt, B, L, lambda: None if torch.cuda.is_current_stream_capturing() else angles_length.cpu())
                 if r is None or (cfg is None and not ext.step_fits(dt == torch.float64, B, L, [r, r])):
                     cfg = _tuning.config_for(angles, angles_length)
                     r = cfg[1]
