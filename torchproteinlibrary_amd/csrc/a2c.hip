@@ -591,6 +591,8 @@ template <typename T>
 constexpr int stage_values() {
     return 3 * kStage + 16 / (int)sizeof(T);
 }
+static_assert(stage_values<float>() * sizeof(float) % 16 == 0 && stage_values<double>() * sizeof(double) % 16 == 0,
+              "the waves' stages stand one after another at 16-byte alignment");
 
 // Values [0, count) from the wave's LDS to dst, as 16-byte stores where dst is
 // aligned; s_w[0] holds the value of dst rounded down to 16 bytes, so that both
@@ -1712,16 +1714,20 @@ __device__ __forceinline__ void copy_back_tables(BackTables& tb, int nt) {
 
 // Atoms staged at a time (in float64 a block takes two rounds, so that eight
 // waves fit on a CU), and the values per array: those atoms', two more atoms
-// before them (the C and O of the residue before), and the offset that aligns
-// both sides.
+// before them (the C and O of the residue before), the offset that aligns both
+// sides, and what makes it whole 16-byte blocks: the gradients' array follows
+// the coordinates', and both are written in such blocks.
 template <typename T>
 constexpr int back_stage() {
     return sizeof(T) == 4 ? 576 : 288;
 }
 template <typename T>
 constexpr int back_values() {
-    return 3 * (back_stage<T>() + 2) + 16 / (int)sizeof(T);
+    constexpr int V = 16 / (int)sizeof(T);
+    return (3 * (back_stage<T>() + 2) + V + V - 1) / V * V;
 }
+static_assert(back_values<float>() * sizeof(float) % 16 == 0 && back_values<double>() * sizeof(double) % 16 == 0,
+              "the staged arrays stand one after another at 16-byte alignment");
 
 // A run of values on its way from memory to the wave's LDS: fetch() issues the
 // loads (16 bytes per lane where src is aligned), commit() writes them to LDS,
