@@ -90,3 +90,34 @@ def test_split_accuracy(B, A):
         # parts, a third of 2^-53 each on average, over at least 120 of them.
         moments = ((xb - xb[0]) ** 2).sum() + ((yb - yb[0]) ** 2).sum()
         assert abs(r[b] - np.sqrt(dev / k)) <= 2.0 ** -53 * moments / (2 * np.sqrt(dev * k)) + 1e-15 * r[b], (b, k)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("B,A", [(3, 10240), (2, 12001)])
+def test_split_does_not_depend_on_the_checks(dtype, B, A, monkeypatch):
+    """Native function, Python function and the binding with a status word, with
+    checks and without: the same kernels, so the same bits."""
+    from torchproteinlibrary_amd._native_rmsd import ext
+    from torchproteinlibrary_amd.RMSD.Coords2RMSD.Coords2RMSD import Coords2RMSDFunction
+    python = type("PythonRMSD", (Coords2RMSDFunction,), {})
+    gen = torch.Generator().manual_seed(A)
+    x = torch.randn(B, A, 3, dtype=torch.float64, generator=gen).cumsum(1).reshape(B, 3 * A).to(dtype).cuda()
+    y = (x.cpu().double() + torch.randn(B, 3 * A, dtype=torch.float64, generator=gen)).to(dtype).cuda()
+    n = torch.tensor([A - k for k in range(B)], dtype=torch.int32).cuda()
+    outs = []
+    for checks in ("1", "0"):
+        monkeypatch.setenv("TPL_A2B_CHECKS", checks)
+        for fn in (Coords2RMSDFunction, python):
+            xx = x.clone().requires_grad_(True)
+            r, ut = fn.apply(xx, y, n)
+            outs.append((r.detach(), ut, torch.autograd.grad(r.sum(), xx)[0]))
+    for status in (None, torch.zeros(1, dtype=torch.int32, device="cuda")):
+        r, ut = x.new_empty(B), x.new_empty(B, 3, 3)
+        ext.Coords2RMSDGPU_forward(x, y, r, n, ut, None, status)
+        outs.append((r, ut, outs[0][2]))
+        assert status is None or int(status) == 0
+    for o in outs[1:]:
+        assert all(torch.equal(u, v) for u, v in zip(o, outs[0]))
+    status = torch.zeros(1, dtype=torch.int32, device="cuda")
+    ext.Coords2RMSDGPU_forward(x, y, r, n + 1000, ut, None, status)
+    assert int(status) == 2

@@ -479,9 +479,9 @@ size_t tplx_rmsd_workspace_bytes(int batch, int atoms_stride) {
 }
 
 int tplx_rmsd_forward(int dtype, const void* input, const void* target, const int32_t* num_atoms, void* rmsd,
-                      void* ut, void* state, void* workspace, uint32_t* flags, int batch, int atoms_stride,
-                      tpl_rmsd_stream_t stream) {
-    return forward_on(dtype, input, target, num_atoms, rmsd, ut, state, workspace, Report{nullptr, flags}, batch,
+                      void* ut, void* state, void* workspace, uint32_t* status, uint32_t* flags, int batch,
+                      int atoms_stride, tpl_rmsd_stream_t stream) {
+    return forward_on(dtype, input, target, num_atoms, rmsd, ut, state, workspace, Report{status, flags}, batch,
                       atoms_stride, stream);
 }
 

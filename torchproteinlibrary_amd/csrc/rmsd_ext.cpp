@@ -93,7 +93,8 @@ void* ptr(const torch::Tensor& t) { return t.defined() ? t.data_ptr() : nullptr;
 // Coords2RMSDGPU_forward (reference coords2rmsd_interface.cpp:52-57):
 // (centered_coords_src, centered_coords_dst, output, num_atoms, UT) plus the
 // forward->backward state (None: no backward follows) and an optional status.
-// The inputs need not be centred.
+// The inputs need not be centred.  The workspace as in the checked form, so that
+// the result does not depend on whether a call is checked.
 void forward(torch::Tensor input, torch::Tensor target, torch::Tensor output,
              torch::Tensor num_atoms, torch::Tensor UT, c10::optional<torch::Tensor> state,
              c10::optional<torch::Tensor> status) {
@@ -102,9 +103,10 @@ void forward(torch::Tensor input, torch::Tensor target, torch::Tensor output,
     check_like(UT, input, {B, 3, 3}, "UT");
     c10::DeviceGuard guard(input.device());
     void* st = (state.has_value() && state->defined()) ? state_ptr(*state, B, input) : nullptr;
-    check_rc(tpl_rmsd_forward(dtype_code(input), input.data_ptr(), target.data_ptr(),
-                              num_atoms.data_ptr<int32_t>(), output.data_ptr(), UT.data_ptr(), st,
-                              status_ptr(status, input), B, A, stream_of(input)),
+    const torch::Tensor ws = workspace_for(input, B, A);
+    check_rc(tplx_rmsd_forward(dtype_code(input), input.data_ptr(), target.data_ptr(),
+                               num_atoms.data_ptr<int32_t>(), output.data_ptr(), UT.data_ptr(), st, ptr(ws),
+                               status_ptr(status, input), nullptr, B, A, stream_of(input)),
              "Coords2RMSDGPU_forward");
 }
 
@@ -138,7 +140,7 @@ int64_t forward_checked(torch::Tensor input, torch::Tensor target, torch::Tensor
     return host_flags::run(s, [&, B = B, A = A](uint32_t* flags) {
         check_rc(tplx_rmsd_forward(dtype_code(input), input.data_ptr(), target.data_ptr(),
                                    num_atoms.data_ptr<int32_t>(), output.data_ptr(), UT.data_ptr(), st, ptr(ws),
-                                   flags, B, A, s),
+                                   nullptr, flags, B, A, s),
                  "Coords2RMSDGPU_forward");
     });
 }
@@ -177,8 +179,8 @@ struct Coords2RMSD : torch::autograd::Function<Coords2RMSD> {
         const torch::Tensor ws = workspace_for(x, B, A);
         const uint32_t bits = native_fn::run(s, [&, B = B, A = A](uint32_t* flags) {
             check_rc(tplx_rmsd_forward(dt, x.data_ptr(), y.data_ptr(), n.data_ptr<int32_t>(), rmsd.data_ptr(),
-                                       UT.data_ptr(), needs ? state_ptr(state, B, x) : nullptr, ptr(ws), flags, B, A,
-                                       s),
+                                       UT.data_ptr(), needs ? state_ptr(state, B, x) : nullptr, ptr(ws), nullptr, flags,
+                                       B, A, s),
                      "Coords2RMSDGPU_forward");
         });
         if (bits) native_fn::python(kLayer, "_raise_on_bits", bits, "forward");
@@ -246,7 +248,8 @@ std::tuple<double, double, double> bench(std::vector<std::vector<torch::Tensor>>
     const torch::Tensor ws = workspace_for(sets[0][0], ss[0].B, ss[0].A);
     for (const Set& q : ss) TORCH_CHECK(q.B == ss[0].B && q.A == ss[0].A, "bench: sets differ in shape");
     auto fwd = [&](const Set& q) {
-        check_rc(tplx_rmsd_forward(q.dt, q.x, q.y, q.n, q.r, q.ut, q.st, ptr(ws), nullptr, q.B, q.A, stream),
+        check_rc(tplx_rmsd_forward(q.dt, q.x, q.y, q.n, q.r, q.ut, q.st, ptr(ws), nullptr, nullptr, q.B, q.A,
+                                   stream),
                  "tpl_rmsd_forward");
     };
     auto bwd = [&](const Set& q) {
