@@ -121,3 +121,32 @@ def test_split_does_not_depend_on_the_checks(dtype, B, A, monkeypatch):
     status = torch.zeros(1, dtype=torch.int32, device="cuda")
     ext.Coords2RMSDGPU_forward(x, y, r, n + 1000, ut, None, status)
     assert int(status) == 2
+
+
+# Shapes that split, at the most workgroups a structure gets: 64 from 65536
+# atoms on, 512 / B for 8 < B <= 32, a share per 1024 atoms below; few atoms in a
+# long stride (1, 2 and 3 leave most shares empty, and the rotation of 1 and 2
+# undetermined: their rmsd is compared).
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("B,A", [(8, 12001), (20, 12001), (20, 30000), (9, 57345), (1, 65535), (2, 65536), (3, 65537), (4, 10240)])
+def test_split_shapes_match_one_workgroup(dtype, B, A):
+    from torchproteinlibrary_amd.RMSD import Coords2RMSD
+    gen = torch.Generator().manual_seed(B * 31 + A)
+    counts = ([1, 2, 3, A, A - 1, 1025, 4, 5000] * 4)[:B] if B > 1 else [A]
+    n = torch.tensor(counts, dtype=torch.int32).cuda()
+    step = torch.randn(B, A, 3, dtype=torch.float64, generator=gen)
+    x = (1.5 * step / step.norm(dim=2, keepdim=True)).cumsum(1) + 20.0
+    y = x.flip(2) + 2.0 * torch.randn(B, A, 3, dtype=torch.float64, generator=gen)
+    x, y = (v.reshape(B, 3 * A).to(dtype).cuda() for v in (x, y))
+    got = Coords2RMSD()(x, y, n)
+    rep = -(-33 // B)  # more than 32 structures take one workgroup each
+    want = Coords2RMSD()(x.repeat(rep, 1), y.repeat(rep, 1), n.repeat(rep))[:B]
+    for b, k in enumerate(counts):
+        c, d = (v[b, :3 * k].double().view(-1, 3) for v in (x, y))
+        r2 = float(((c - c[0]) ** 2).sum() + ((d - d[0]) ** 2).sum())
+        rmsd = float(want[b])
+        # r^2 n = R2 - 2 lambda + 1e-10 of sums that round, in either order, to
+        # within 256 units of 2^-53 of r2; r itself is no more than sqrt of that off
+        off = 256 * 2.0 ** -53 * r2
+        tol = min(off / (k * rmsd), (off / k) ** 0.5) + 2 * torch.finfo(dtype).eps * rmsd
+        assert abs(float(got[b]) - rmsd) <= tol, (b, k)
