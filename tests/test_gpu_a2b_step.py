@@ -181,3 +181,31 @@ def test_step_rule_counts_waves(B, lo, R):
     step.grad_coords.copy_(g)
     step.replay()
     _check(step, a, ln, g, torch.float32)
+
+
+@pytest.mark.parametrize("L", [500, 8000])
+def test_step_alone_on_another_stream_may_go_while_it_runs(L):
+    """As above where the caller keeps nothing at all, neither the angles nor the
+    outputs: none of that memory is handed out before the runs have ended."""
+    from torchproteinlibrary_amd.ReducedModel.Angles2Backbone.Angles2Backbone import Angles2BackboneStep
+    B = 16
+    a, ln, g = _case(B, L, [L] * B, torch.float32, 3)
+    step = Angles2BackboneStep(a, ln)
+    step.grad_coords.copy_(g)
+    held = [a, ln, step.grad_coords, step.coords, step.grad_angles, step._state, step._sync]
+    held = [(t.data_ptr(), t.nbytes) for t in held if t.nbytes]
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        busy = torch.empty(1 << 30, dtype=torch.uint8, device="cuda")
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        for _ in range(200):  # some 50 ms before the runs begin
+            busy.fill_(1)
+        for _ in range(20):
+            step.replay()
+    del step, a, ln
+    taken = [torch.empty(size, dtype=torch.uint8, device="cuda") for _, size in held for _ in range(2)]
+    assert not side.query()  # still running: nothing may have been given out
+    for t in taken:
+        assert all(t.data_ptr() + t.nbytes <= p or t.data_ptr() >= p + size for p, size in held)
+    side.synchronize()

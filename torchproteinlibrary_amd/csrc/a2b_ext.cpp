@@ -598,9 +598,11 @@ class Step {
         const c10::Device dev = angles_.device();
         c10::DeviceGuard guard(dev);
         const hipStream_t s = c10::hip::getCurrentHIPStream(dev.index()).stream();
-        // What only the step holds must outlive its runs on other streams.
+        // Whatever the step holds may be held by nobody else by the time it goes,
+        // outputs and inputs too, and must outlive its runs on other streams.
         if (s != home_)
-            for (const torch::Tensor* t : {&records_, &state_, &sync_})
+            for (const torch::Tensor* t :
+                 {&angles_, &lengths_, &grad_output_, &coords_, &grad_input_, &state_, &sync_, &records_})
                 if (t->defined())
                     t->record_stream(at::hip::getCurrentHIPStreamMasqueradingAsCUDA(dev.index()).unwrap());
         const int32_t* len = lengths_.data_ptr<int32_t>();
