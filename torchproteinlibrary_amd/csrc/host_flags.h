@@ -5,7 +5,9 @@
 // process and module.  A call takes a slot, launches, waits for its stream
 // and gives the slot back, so a slot is never written by two calls; a call
 // that finds none free waits for one (they are held only across a launch and
-// its wait, by threads that need no lock of this one's).
+// its wait, by threads that need no lock of this one's).  A call whose launch
+// fails waits too, since it may have put a first kernel on the stream; a slot
+// whose wait fails may still be written and is never given out again.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -38,7 +40,8 @@ class Pool {
             base_ = static_cast<uint32_t*>(m);
             for (int k = 0; k < kSlots; ++k) free_.push_back(k);
         }
-        cv_.wait(lock, [this] { return !free_.empty(); });
+        cv_.wait(lock, [this] { return !free_.empty() || lost_ == kSlots; });
+        if (free_.empty()) throw std::runtime_error("no status flags left: the waits for them failed");
         const int k = free_.back();
         free_.pop_back();
         return base_ + (size_t)k * kWords;
@@ -50,12 +53,20 @@ class Pool {
         }
         cv_.notify_one();
     }
+    void lose() {
+        {
+            std::lock_guard<std::mutex> lock(mu_);
+            ++lost_;
+        }
+        cv_.notify_all();
+    }
 
   private:
     std::mutex mu_;
     std::condition_variable cv_;
     uint32_t* base_ = nullptr;
     std::vector<int> free_;
+    int lost_ = 0;
 };
 
 // Calls launch(flags), which puts kernels on `stream`, waits for the stream
@@ -63,12 +74,24 @@ class Pool {
 template <typename Launch>
 uint32_t run(hipStream_t stream, Launch launch) {
     struct Slot {
+        hipStream_t stream;
         uint32_t* p = Pool::get().take();
-        ~Slot() { Pool::get().give(p); }
-    } slot;
+        bool waited = false;
+        hipError_t wait() {
+            const hipError_t e = hipStreamSynchronize(stream);
+            waited = e == hipSuccess;
+            return e;
+        }
+        ~Slot() {
+            if (waited || wait() == hipSuccess)
+                Pool::get().give(p);
+            else
+                Pool::get().lose();
+        }
+    } slot{stream};
     for (int k = 0; k < kFlags; ++k) __atomic_store_n(slot.p + k, 0u, __ATOMIC_RELEASE);
     launch(slot.p);
-    if (hipStreamSynchronize(stream) != hipSuccess)
+    if (slot.wait() != hipSuccess)
         throw std::runtime_error(std::string("hipStreamSynchronize failed: ") + hipGetErrorString(hipGetLastError()));
     uint32_t bits = 0;
     for (int k = 0; k < kFlags; ++k)
