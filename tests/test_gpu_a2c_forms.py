@@ -244,3 +244,58 @@ def test_layer_raises_where_the_gradient_sum_is_nan(lengths, L):
     g[-1, 3 * (O.num_atoms(seqs[-1]) - 1)] = float("nan")
     with pytest.raises(Exception, match="backward Nan"):
         coords.backward(g)
+
+
+def _through_the_binding(B, L, dtype):
+    """A forward and a backward call on buffers that are there beforehand."""
+    from torchproteinlibrary_amd._native_xform import ext
+    seqs, X = _batch([L] * B, L, B, dtype)
+    A = max(O.num_atoms(s) for s in seqs)
+    S = convertStringList(seqs).to(DEV)
+    coords, g = torch.empty(B, 3 * A, dtype=dtype, device=DEV), torch.randn(B, 3 * A, dtype=dtype, device=DEV)
+    rn, an = (torch.empty(B, A, 4, dtype=torch.uint8, device=DEV) for _ in range(2))
+    ga = torch.empty_like(X)
+
+    def call():
+        assert ext.Angles2Coords_forward_checked(S, X, coords, rn, an) == 0
+        assert ext.Angles2Coords_backward_checked(g, ga, S, coords) == 0
+    return call, (coords, rn, an, ga)
+
+
+@pytest.mark.parametrize("B,L", [(512, 300), (32, 350), (256, 1000), (600, 128)])
+def test_no_workspace_where_none_is_read(B, L):
+    """One workgroup per structure: nothing is allocated beside the outputs."""
+    call, outs = _through_the_binding(B, L, torch.float32)
+    call()
+    want = [t.clone() for t in outs]
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    call()
+    assert torch.cuda.max_memory_allocated() == before
+    assert all(torch.equal(u, v) for u, v in zip(outs, want))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+def test_no_memory_for_the_workspace(dtype):
+    """Where the workspace does not fit, the kernels without one do the call."""
+    B, L = 320, 700
+    call, outs = _through_the_binding(B, L, dtype)
+    call()
+    want = [t.clone() for t in outs]
+    for t in outs:
+        t.fill_(1)
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(DEV).total_memory
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + 4096) / total)
+    try:
+        call()
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    eps = 2.0 ** -23 if dtype == torch.float32 else 0.0
+    scale = float(want[0].abs().max())
+    assert float((outs[0] - want[0]).abs().max()) <= scale * (3 * L * 8 * 2.0 ** -53 + eps)
+    assert torch.equal(outs[1], want[1]) and torch.equal(outs[2], want[2])
+    # the gradients' sums in another order, from coordinates that differ as above
+    scale = want[3].abs().amax(dim=(1, 2), keepdim=True)
+    assert ((outs[3] - want[3]).abs() <= scale * (14 * L * 8 * 2.0 ** -53 + 1e3 * eps)).all()

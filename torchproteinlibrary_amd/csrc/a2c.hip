@@ -2283,6 +2283,17 @@ bool use_groups(int batch, int angles_stride) {
     return batch > cus ? (int64_t)batch * nb >= 3000 : nb > 8 && batch <= cus / 4;
 }
 
+// Whether the group kernels' grids can be counted.
+bool forward_groups_fit(int batch, int angles_stride) {
+    return (int64_t)batch * groups_of(angles_stride) <= INT32_MAX / kGroup;
+}
+// What AUTO takes.  A structure of one block needs no groups, whatever the form.
+int forward_form(int batch, int angles_stride, bool workspace) {
+    const bool groups = workspace && blocks_of(angles_stride) > 1 && forward_groups_fit(batch, angles_stride) &&
+                        use_groups(batch, angles_stride);
+    return groups ? TPLX_A2C_FWD_GROUPS : TPLX_A2C_FWD_FUSED;
+}
+
 template <typename T>
 void launch_forward(int form, hipStream_t s, const uint8_t* sequences, int seq_stride, const T* a, int angles_stride,
                     T* c, uint32_t* rn, uint32_t* an, int atoms_stride, void* workspace, const Report& rep,
@@ -2333,10 +2344,10 @@ int forward_on(int form, const int32_t* order, int dtype, const uint8_t* sequenc
     if (!sequences || (angles_stride > 0 && !angles) || (atoms_stride > 0 && !coords) ||
         (!res_names) != (!atom_names))
         return TPL_A2C_ERR_ARG;
-    const bool groups_fit = workspace && (int64_t)batch * groups_of(angles_stride) <= INT32_MAX / kGroup;
-    if (form == TPLX_A2C_FWD_AUTO)
-        form = groups_fit && use_groups(batch, angles_stride) ? TPLX_A2C_FWD_GROUPS : TPLX_A2C_FWD_FUSED;
-    if (form == TPLX_A2C_FWD_GROUPS && blocks_of(angles_stride) > 1 && !groups_fit) return TPL_A2C_ERR_ARG;
+    if (form == TPLX_A2C_FWD_AUTO) form = forward_form(batch, angles_stride, workspace);
+    if (form == TPLX_A2C_FWD_GROUPS && blocks_of(angles_stride) > 1 &&
+        !(workspace && forward_groups_fit(batch, angles_stride)))
+        return TPL_A2C_ERR_ARG;
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (!tables_ready(s)) return TPL_A2C_ERR_LAUNCH;
     uint32_t* rn = reinterpret_cast<uint32_t*>(res_names);
@@ -2379,6 +2390,15 @@ bool use_back_groups(int batch, int angles_stride) {
     return blocks_of(angles_stride) > 2 && use_groups(batch, angles_stride);
 }
 
+bool backward_groups_fit(int batch, int angles_stride) {
+    return (int64_t)batch * blocks_of(angles_stride) <= INT32_MAX / kBlock;
+}
+int backward_form(int batch, int angles_stride, bool workspace) {
+    const bool groups =
+        workspace && backward_groups_fit(batch, angles_stride) && use_back_groups(batch, angles_stride);
+    return groups ? TPLX_A2C_BWD_GROUPS : TPLX_A2C_BWD_FUSED;
+}
+
 template <typename T>
 int launch_backward(int form, hipStream_t s, const uint8_t* sequences, int seq_stride, const T* x, const T* g,
                     int atoms_stride, T* ga, int angles_stride, void* workspace, const Report& rep,
@@ -2413,10 +2433,9 @@ int backward_on(int form, const int32_t* order, int dtype, const uint8_t* sequen
     if (rc != TPL_A2C_OK) return rc;
     if (batch == 0 || angles_stride == 0) return TPL_A2C_OK;
     if (!sequences || !grad_angles || (atoms_stride > 0 && (!coords || !grad_coords))) return TPL_A2C_ERR_ARG;
-    const bool groups_fit = workspace && (int64_t)batch * blocks_of(angles_stride) <= INT32_MAX / kBlock;
-    if (form == TPLX_A2C_BWD_AUTO)
-        form = groups_fit && use_back_groups(batch, angles_stride) ? TPLX_A2C_BWD_GROUPS : TPLX_A2C_BWD_FUSED;
-    if (form == TPLX_A2C_BWD_GROUPS && !groups_fit) return TPL_A2C_ERR_ARG;
+    if (form == TPLX_A2C_BWD_AUTO) form = backward_form(batch, angles_stride, workspace);
+    if (form == TPLX_A2C_BWD_GROUPS && !(workspace && backward_groups_fit(batch, angles_stride)))
+        return TPL_A2C_ERR_ARG;
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (dtype == TPL_A2C_F32)
         return launch_backward<float>(form, s, sequences, seq_stride, static_cast<const float*>(coords),
@@ -2480,6 +2499,14 @@ int tplx_a2c_forward(int form, const int32_t* order, int dtype, const uint8_t* s
                      tpl_a2c_stream_t stream) {
     return forward_on(form, order, dtype, sequences, seq_stride, angles, angles_stride, coords, res_names,
                       atom_names, atoms_stride, workspace, Report{status, flags}, batch, stream);
+}
+
+int tplx_a2c_forward_form(int batch, int angles_stride, int workspace) {
+    return forward_form(batch, angles_stride, workspace != 0);
+}
+
+int tplx_a2c_backward_form(int batch, int angles_stride, int workspace) {
+    return backward_form(batch, angles_stride, workspace != 0);
 }
 
 size_t tplx_a2c_workspace_bytes(int batch, int angles_stride) {

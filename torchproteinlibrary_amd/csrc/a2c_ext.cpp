@@ -70,11 +70,28 @@ hipStream_t stream_of(const torch::Tensor& t) {
     return c10::hip::getCurrentHIPStream(t.device().index()).stream();
 }
 
-// The forward's workspace (none where it needs none), from torch's allocator.
-torch::Tensor workspace_for(const torch::Tensor& angles) {
-    const size_t need = tplx_a2c_workspace_bytes((int)angles.size(0), (int)angles.size(2));
+// `need` bytes of workspace from torch's allocator, or none if there is no
+// memory for them: the kernels without a workspace do the same.
+torch::Tensor workspace(size_t need, const torch::Tensor& like) {
     if (need == 0) return torch::Tensor();
-    return torch::empty({(int64_t)need}, angles.options().dtype(torch::kByte));
+    try {
+        return torch::empty({(int64_t)need}, like.options().dtype(torch::kByte));
+    } catch (const c10::OutOfMemoryError&) {
+        return torch::Tensor();
+    }
+}
+void* ptr(const torch::Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
+
+// The workspaces of the two directions, where the form that they take reads one.
+torch::Tensor forward_workspace(const torch::Tensor& angles) {
+    const int B = (int)angles.size(0), L = (int)angles.size(2);
+    const bool groups = tplx_a2c_forward_form(B, L, 1) == TPLX_A2C_FWD_GROUPS;
+    return workspace(groups ? tplx_a2c_workspace_bytes(B, L) : 0, angles);
+}
+torch::Tensor backward_workspace(const torch::Tensor& grad_angles) {
+    const int B = (int)grad_angles.size(0), L = (int)grad_angles.size(2);
+    const bool groups = tplx_a2c_backward_form(B, L, 1) == TPLX_A2C_BWD_GROUPS;
+    return workspace(groups ? tplx_a2c_backward_workspace_bytes(B, L) : 0, grad_angles);
 }
 
 void forward_on(const torch::Tensor& sequences, const torch::Tensor& input_angles,
@@ -97,12 +114,11 @@ void forward_on(const torch::Tensor& sequences, const torch::Tensor& input_angle
         TORCH_CHECK(n->device() == input_angles.device(), "names must be on the device of the angles");
     }
     TORCH_CHECK(output_coords.device() == input_angles.device(), "coordinates must be on the device of the angles");
-    const torch::Tensor ws = workspace_for(input_angles);
+    const torch::Tensor ws = forward_workspace(input_angles);
     check_rc(tplx_a2c_forward(TPLX_A2C_FWD_AUTO, order_ptr(order, input_angles), dtype_code(input_angles),
                               sequences.data_ptr<uint8_t>(), (int)sequences.size(1), input_angles.data_ptr(),
                               (int)input_angles.size(2), output_coords.data_ptr(), res_names.data_ptr<uint8_t>(),
-                              atom_names.data_ptr<uint8_t>(), (int)A, ws.defined() ? ws.data_ptr() : nullptr, status,
-                              flags, (int)B, stream),
+                              atom_names.data_ptr<uint8_t>(), (int)A, ptr(ws), status, flags, (int)B, stream),
              "Angles2Coords_forward");
 }
 
@@ -143,13 +159,11 @@ void backward_on(const torch::Tensor& grad_atoms, const torch::Tensor& grad_angl
                 "gradients and coordinates must be on one device");
     const int64_t A = grad_atoms.size(1) / 3;
     TORCH_CHECK(A <= INT32_MAX / 3, "grad_atoms too large");
-    const size_t need = tplx_a2c_backward_workspace_bytes((int)B, (int)grad_angles.size(2));
-    torch::Tensor ws;
-    if (need) ws = torch::empty({(int64_t)need}, grad_angles.options().dtype(torch::kByte));
+    const torch::Tensor ws = backward_workspace(grad_angles);
     check_rc(tplx_a2c_backward(TPLX_A2C_BWD_AUTO, order_ptr(order, grad_angles), dtype_code(grad_angles),
                                sequences.data_ptr<uint8_t>(), (int)sequences.size(1), coords.data_ptr(),
                                grad_atoms.data_ptr(), (int)A, grad_angles.data_ptr(), (int)grad_angles.size(2),
-                               ws.defined() ? ws.data_ptr() : nullptr, status, flags, (int)B, stream),
+                               ptr(ws), status, flags, (int)B, stream),
              "Angles2Coords_backward");
 }
 
@@ -327,24 +341,20 @@ std::tuple<double, double, double> bench(std::vector<std::vector<torch::Tensor>>
     c10::DeviceGuard guard(sets[0][1].device());
     hipStream_t stream = stream_of(sets[0][1]);
     const int dt = dtype_code(sets[0][1]);
-    const torch::Tensor ws = workspace_for(sets[0][1]);
-    const torch::Tensor bws =
-        torch::empty({(int64_t)tplx_a2c_backward_workspace_bytes((int)sets[0][1].size(0), (int)sets[0][1].size(2)) + 16},
-                     sets[0][1].options().dtype(torch::kByte));
+    const torch::Tensor ws = forward_workspace(sets[0][1]), bws = backward_workspace(sets[0][1]);
     for (auto& t : sets) TORCH_CHECK(t[1].sizes() == sets[0][1].sizes(), "bench: sets differ in shape");
     auto fwd = [&](std::vector<torch::Tensor>& t) {
         const int32_t* order = t.size() == 6 ? t[5].data_ptr<int32_t>() : nullptr;
         check_rc(tplx_a2c_forward(TPLX_A2C_FWD_AUTO, order, dt, t[0].data_ptr<uint8_t>(), (int)t[0].size(1),
                                   t[1].data_ptr(), (int)t[1].size(2), t[2].data_ptr(), nullptr, nullptr,
-                                  (int)(t[2].size(1) / 3), ws.defined() ? ws.data_ptr() : nullptr, nullptr, nullptr,
-                                  (int)t[1].size(0), stream),
+                                  (int)(t[2].size(1) / 3), ptr(ws), nullptr, nullptr, (int)t[1].size(0), stream),
                  "forward");
     };
     auto bwd = [&](std::vector<torch::Tensor>& t) {
         const int32_t* order = t.size() == 6 ? t[5].data_ptr<int32_t>() : nullptr;
         check_rc(tplx_a2c_backward(TPLX_A2C_BWD_AUTO, order, dt, t[0].data_ptr<uint8_t>(), (int)t[0].size(1),
                                    t[2].data_ptr(), t[3].data_ptr(), (int)(t[3].size(1) / 3), t[4].data_ptr(),
-                                   (int)t[4].size(2), bws.data_ptr(), nullptr, nullptr, (int)t[1].size(0), stream),
+                                   (int)t[4].size(2), ptr(bws), nullptr, nullptr, (int)t[1].size(0), stream),
                  "backward");
     };
     hipEvent_t e0, e1;

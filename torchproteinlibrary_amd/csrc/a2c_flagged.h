@@ -22,8 +22,12 @@
 #define TPLX_A2C_BWD_GROUPS 2
 
 extern "C" {
-// Bytes of the workspace (16-byte aligned; 0: none is used).  A call writes
-// what it reads there.
+// The form that AUTO takes, with a workspace or without.
+int tplx_a2c_forward_form(int batch, int angles_stride, int workspace);
+int tplx_a2c_backward_form(int batch, int angles_stride, int workspace);
+
+// Bytes of the workspace that the GROUPS form needs (16-byte aligned; 0: none);
+// no other form reads it.  A call writes what it reads there.
 size_t tplx_a2c_workspace_bytes(int batch, int angles_stride);
 
 int tplx_a2c_forward(int form, const int32_t* order, int dtype, const uint8_t* sequences, int seq_stride,
