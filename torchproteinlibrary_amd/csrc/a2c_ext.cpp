@@ -281,12 +281,13 @@ c10::optional<std::tuple<Tensor, Tensor, Tensor>> apply(Tensor angles, Tensor se
 // The sequences of a call as the device wants them: (atom counts, the uint8
 // [batch, longest + 1] tensor of convertStringList on the device, the counts as
 // int32 on the device), copied from pinned memory without a wait; None if
-// a sequence is not a string of the 20 letters, or a capture is open (the
-// copies would read their staging memory again on each replay).
+// a sequence is not a string of the 20 letters, the call is not a plain one (a
+// mode may hand out tensors without memory), or a capture is open (the copies
+// would read their staging memory again on each replay).
 pybind11::object prepare(pybind11::list sequences, torch::Tensor angles) {
     namespace py = pybind11;
     const size_t B = sequences.size();
-    if (B == 0 || !angles.is_cuda()) return py::none();
+    if (B == 0 || !native_fn::plain({&angles})) return py::none();
     c10::DeviceGuard guard(angles.device());
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(stream_of(angles), &capture) != hipSuccess || capture != hipStreamCaptureStatusNone)
