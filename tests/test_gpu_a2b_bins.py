@@ -46,3 +46,34 @@ def test_packed_forward_matches_oracle(dtype, R, chunks, B):
             layer(angles, bad)
     finally:
         _tuning.clear()
+
+
+# One workgroup per chain, 1 to 4 slots: the padding goes over the slots without
+# a chunk, and a chain of one slot has some only if it is empty.
+@pytest.mark.parametrize("dtype,R", [(torch.float32, 1), (torch.float32, 2), (torch.float32, 4), (torch.float64, 2)])
+@pytest.mark.parametrize("slots", [1, 2, 3, 4])
+def test_padding_of_one_workgroup_per_chain(dtype, R, slots):
+    from torchproteinlibrary_amd.ReducedModel import Angles2Backbone
+    C = 64 * R
+    L = slots * C - (slots % 2)
+    lens = torch.tensor([min(v, L) for v in (0, 1, C - 1, C, C + 1, 2 * C, 3 * C + 1, L, 0)], dtype=torch.int32).cuda()
+    angles = torch.rand(9, 3, L, device="cuda", dtype=dtype, generator=torch.Generator("cuda").manual_seed(L)) * 6 - 3
+    g = torch.randn(9, 9 * L, device="cuda", dtype=dtype, generator=torch.Generator("cuda").manual_seed(R))
+    try:
+        _tuning.set_config(angles, (R, R))
+        torch.full((1 << 22,), float("nan"), device="cuda")  # what the outputs' memory may have held
+        a = angles.clone().requires_grad_(True)
+        out = Angles2Backbone()(a, lens)
+        out.backward(g)
+    finally:
+        _tuning.clear()
+    ac = angles.double().cpu().requires_grad_(True)
+    want = Angles2Backbone()(ac, lens.cpu())
+    want.backward(g.double().cpu())
+    eps = torch.finfo(dtype).eps
+    acc = 64 * 3 * L * 2.0 ** -53
+    assert (out.detach().double().cpu() - want.detach()).abs().max() <= 3.8 * L * (2 * eps + acc)
+    scale = ac.grad.abs().amax(dim=(1, 2), keepdim=True)
+    assert ((a.grad.double().cpu() - ac.grad).abs() <= scale * 64 * eps + 3 * L * 3.8 * L * 6 * acc).all()
+    for b, n in enumerate(lens.tolist()):
+        assert not out[b, 9 * n:].any() and not a.grad[b, :, n:].any()

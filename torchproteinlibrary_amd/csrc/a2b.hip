@@ -1076,20 +1076,25 @@ __device__ __forceinline__ Place place_wave(const ChunkArgs& a, int wave, int* s
     return p;
 }
 
-// Calls zeros(chain, f, F) so that share f of F of each chain's padding is this
-// wave's: in BINS the chains go over all waves that have work, quarter by
-// quarter (the workgroups of the short chains would have nearly all of it).
-template <int W, bool BINS, typename Zeros>
-__device__ __forceinline__ void spread_zeros(const ChunkArgs& a, const Place& p, int wave, Zeros zeros) {
-    if constexpr (BINS) {
-        for (int u = (int)blockIdx.x * W + wave; u < 4 * a.B; u += p.nwg * W) zeros(u >> 2, u & 3, 4);
-    } else {
-        zeros(p.b, p.c, W);
-    }
-}
 __device__ __forceinline__ int chain_length(const ChunkArgs& a, int b) {
     const int raw = a.lengths[b];
     return raw < 0 ? 0 : (raw > a.L ? a.L : raw);
+}
+// Calls zeros(chain, its length, f, F) so that share f of F of each chain's
+// padding is this wave's.  In BINS the chains go over all waves that have work,
+// quarter by quarter (the workgroups of the short chains would have nearly all
+// of it).  Otherwise the workgroup's own chain, of length n in nreal chunks, over
+// the waves without a chunk: padding leaves at least one, and on a wave with a
+// chunk the stores' addresses alone take 0.5 us of a 4 us kernel.
+template <int W, bool BINS, typename Zeros>
+__device__ __forceinline__ void spread_zeros(const ChunkArgs& a, const Place& p, int n, int nreal, int wave,
+                                             Zeros zeros) {
+    if constexpr (BINS) {
+        for (int u = (int)blockIdx.x * W + wave; u < 4 * a.B; u += p.nwg * W)
+            zeros(u >> 2, chain_length(a, u >> 2), u & 3, 4);
+    } else if (p.c >= nreal) {
+        zeros(p.b, n, p.c - nreal, W - nreal);
+    }
 }
 
 // ------------------------------------------------------------ forward chain
@@ -1114,8 +1119,12 @@ __global__ void __launch_bounds__(64 * W) a2b_fwd_chain(ChunkArgs a) {
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = (int)(threadIdx.x & 63);
     for (int i = (int)threadIdx.x; i < 128; i += 64 * W) s_tab[i] = kTabCS[i];
     const Place pl = place_wave<R, W, BINS>(a, wave, s_chain, s_count);
-    if (BINS && pl.size == 0) return;
     const int c = pl.c, L = a.L;
+    const auto zeros = [&](int zb, int zn, int f, int F) {
+        const int p = min(chunks_of(zn, C) * C, L);
+        store_zeros<T>(static_cast<T*>(a.coords) + (size_t)9 * zb * L + (size_t)9 * p, 9 * (L - p), f, F, lane);
+    };
+    if (BINS && pl.size == 0) return;
     const bool some = !BINS || pl.b >= 0;
     const int b = some ? pl.b : 0;
     const int n = some ? chain_length(a, b) : 0;
@@ -1166,10 +1175,7 @@ __global__ void __launch_bounds__(64 * W) a2b_fwd_chain(ChunkArgs a) {
     }
     // The zeros past the chains' chunks: nothing is loaded from here on, so the
     // stores drain behind the rest.
-    spread_zeros<W, BINS>(a, pl, wave, [&](int zb, int f, int F) {
-        const int p = min(chunks_of(chain_length(a, zb), C) * C, L);
-        store_zeros<T>(static_cast<T*>(a.coords) + (size_t)9 * zb * L + (size_t)9 * p, 9 * (L - p), f, F, lane);
-    });
+    spread_zeros<W, BINS>(a, pl, n, nreal, wave, zeros);
     __syncthreads();  // the aggregates
     if (real && c > 0) {
         double P[kF], Q[kF];
@@ -1487,14 +1493,24 @@ __global__ void __launch_bounds__(64 * W) a2b_bwd_chain(ChunkArgs a) {
     extern __shared__ double s_dynd[];  // [W][6R][64]: each wave's (cos, sin)
     __shared__ double s_tab[128];
     __shared__ double s_tot[W][6];
-    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = (int)(threadIdx.x & 63);
-    for (int i = (int)threadIdx.x; i < 128; i += 64 * W) s_tab[i] = kTabCS[i];
+    const int wave = (int)(threadIdx.x >> 6), lane = (int)(threadIdx.x & 63);
     const Place pl = place_wave<R, W, false>(a, wave, nullptr, nullptr);
     const int b = pl.b, c = pl.c, L = a.L;
     const int n = chain_length(a, b);
     const int nreal = (n + C - 1) / C;
     const bool real = c < nreal;
     if (c == 0 && lane == 0 && a.lengths[b] != n) report_bits(a.rep, TPL_A2B_STATUS_LENGTH);
+    const auto zeros = [&](int zb, int zn, int f, int F) {
+        const int p = min(chunks_of(zn, C) * C, L);
+#pragma unroll
+        for (int k = 0; k < 3; ++k)
+            store_zeros<T>(static_cast<T*>(a.grad_angles) + ((size_t)3 * zb + k) * L + p, L - p, f, F, lane);
+    };
+    if (W == 1 && !real) {  // only an empty chain has padding here
+        zeros(b, n, 0, 1);
+        return;
+    }
+    for (int i = (int)threadIdx.x; i < 128; i += 64 * W) s_tab[i] = kTabCS[i];
     double* s_cs = s_dynd + (size_t)wave * 6 * R * 64;
     T* grow = static_cast<T*>(a.grad_angles) + (size_t)b * 3 * L;
     const T* arow = static_cast<const T*>(a.angles) + (size_t)b * 3 * L;
@@ -1586,12 +1602,7 @@ __global__ void __launch_bounds__(64 * W) a2b_bwd_chain(ChunkArgs a) {
             for (int e = 0; e < 6; ++e) s_tot[c][e] = tot[e];
         }
     }
-    spread_zeros<W, false>(a, pl, wave, [&](int zb, int f, int F) {
-        const int p = min(chunks_of(chain_length(a, zb), C) * C, L);
-#pragma unroll
-        for (int k = 0; k < 3; ++k)
-            store_zeros<T>(static_cast<T*>(a.grad_angles) + ((size_t)3 * zb + k) * L + p, L - p, f, F, lane);
-    });
+    if (W > 1) spread_zeros<W, false>(a, pl, n, nreal, wave, zeros);
     __syncthreads();  // the chunks' sums
     if (!real) return;
     for (int j = c + 1; j < nreal; ++j) {
@@ -1914,6 +1925,13 @@ __global__ void __launch_bounds__(64 * W) a2b_step(ChunkArgs a) {
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = (int)(threadIdx.x & 63);
     const int L = a.L;
     for (int i = (int)threadIdx.x; i < 128; i += 64 * W) s_tab[i] = kTabCS[i];
+    const auto zeros = [&](int zb, int zn, int f, int F) {
+        const int p = min(chunks_of(zn, C) * C, L);
+        store_zeros<T>(static_cast<T*>(a.coords) + (size_t)9 * zb * L + (size_t)9 * p, 9 * (L - p), f, F, lane);
+#pragma unroll
+        for (int k = 0; k < 3; ++k)
+            store_zeros<T>(static_cast<T*>(a.grad_angles) + ((size_t)3 * zb + k) * L + p, L - p, f, F, lane);
+    };
     Place pl{};
     if constexpr (MODE == WALK) {
         walk_slot<W>(a, wave, pl.b, pl.c);
@@ -2010,13 +2028,7 @@ __global__ void __launch_bounds__(64 * W) a2b_step(ChunkArgs a) {
     // The zeros past the chains' chunks: nothing is loaded from here on, so the
     // stores drain behind the rest.
     if constexpr (MODE != WALK)
-        spread_zeros<W, MODE == BINS>(a, pl, wave, [&](int zb, int f, int F) {
-            const int p = min(chunks_of(chain_length(a, zb), C) * C, L);
-            store_zeros<T>(static_cast<T*>(a.coords) + (size_t)9 * zb * L + (size_t)9 * p, 9 * (L - p), f, F, lane);
-#pragma unroll
-            for (int k = 0; k < 3; ++k)
-                store_zeros<T>(static_cast<T*>(a.grad_angles) + ((size_t)3 * zb + k) * L + p, L - p, f, F, lane);
-        });
+        spread_zeros<W, MODE == BINS>(a, pl, n, nreal, wave, zeros);
     if (MODE != WALK) __syncthreads();  // the aggregates
     if (real) {
         if constexpr (MODE == WALK) {
