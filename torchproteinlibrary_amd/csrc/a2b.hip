@@ -1083,14 +1083,20 @@ __device__ __forceinline__ int chain_length(const ChunkArgs& a, int b) {
 // Calls zeros(chain, its length, f, F) so that share f of F of each chain's
 // padding is this wave's.  In BINS the chains go over all waves that have work,
 // quarter by quarter (the workgroups of the short chains would have nearly all
-// of it).  Otherwise the workgroup's own chain, of length n in nreal chunks, over
-// the waves without a chunk: padding leaves at least one, and on a wave with a
-// chunk the stores' addresses alone take 0.5 us of a 4 us kernel.
+// of it), and over further workgroups up to one per CU where those are few
+// (512 chains of 50..253 at a stride of 2029, float64, forward alone: 23.7 ->
+// 20.5 us, 16 of them 19.0 -> 12.9).  Otherwise the workgroup's own chain, of
+// length n in nreal chunks, over the waves without a chunk: padding leaves at
+// least one, and on a wave with a chunk the stores' addresses alone take 0.5 us
+// of a 4 us kernel.
+constexpr int kZeroWorkgroups = 256;
 template <int W, bool BINS, typename Zeros>
 __device__ __forceinline__ void spread_zeros(const ChunkArgs& a, const Place& p, int n, int nreal, int wave,
                                              Zeros zeros) {
     if constexpr (BINS) {
-        for (int u = (int)blockIdx.x * W + wave; u < 4 * a.B; u += p.nwg * W)
+        const int wgs = max(p.nwg, min(a.B, kZeroWorkgroups));
+        if ((int)blockIdx.x >= wgs) return;
+        for (int u = (int)blockIdx.x * W + wave; u < 4 * a.B; u += wgs * W)
             zeros(u >> 2, chain_length(a, u >> 2), u & 3, 4);
     } else if (p.c >= nreal) {
         zeros(p.b, n, p.c - nreal, W - nreal);
@@ -1124,7 +1130,10 @@ __global__ void __launch_bounds__(64 * W) a2b_fwd_chain(ChunkArgs a) {
         const int p = min(chunks_of(zn, C) * C, L);
         store_zeros<T>(static_cast<T*>(a.coords) + (size_t)9 * zb * L + (size_t)9 * p, 9 * (L - p), f, F, lane);
     };
-    if (BINS && pl.size == 0) return;
+    if (BINS && pl.size == 0) {
+        spread_zeros<W, BINS>(a, pl, 0, 0, wave, zeros);
+        return;
+    }
     const bool some = !BINS || pl.b >= 0;
     const int b = some ? pl.b : 0;
     const int n = some ? chain_length(a, b) : 0;
@@ -1937,7 +1946,10 @@ __global__ void __launch_bounds__(64 * W) a2b_step(ChunkArgs a) {
         walk_slot<W>(a, wave, pl.b, pl.c);
     } else {
         pl = place_wave<R, W, MODE == BINS>(a, wave, s_chain, s_count);
-        if (MODE == BINS && pl.size == 0) return;
+        if (MODE == BINS && pl.size == 0) {
+            spread_zeros<W, true>(a, pl, 0, 0, wave, zeros);
+            return;
+        }
     }
     const int b = pl.b, c = pl.c, first = pl.first;
     const int n = b >= 0 ? chain_length(a, b) : 0;
@@ -2531,34 +2543,54 @@ bool allow_lds(KernelFn k, size_t bytes) {
     return true;
 }
 
-// Launches the chain kernel of chains of a.nc <= kBinsMax chunks (kernel(waves,
-// bins) gives it, lds the staging of one wave), or returns false.  Chains of at
+// Whether packing (BINS) pays in the forward, for chains of nc chunks with R
+// residues per lane, in workgroups with `bytes` of staging of which `resident`
+// fit on the GPU.  Against the chunk kernel, forward alone, by batch (equal lengths /
+// uniform mix; float32 and float64 alike unless said):
+//   3 chunks: 1500 0.95 / 0.97, 3000 1.1 / 1.07, 4096 1.3 / 1.35;
+//   4 chunks: 1500 0.87 / 0.97, 3000 0.95 / 1.0, 4096 1.1 / 1.2;
+//   5 or 6 of a workgroup's 8 waves: 512 0.7 / 0.7, 800 1.1 / 0.83, 3000 1.15 / 1.0;
+//   8 of 8: 512 0.67 / 0.7, 800 0.87 / 0.78, 4096 0.9 / 0.92;
+//   few chains: 1 to 32 with R <= 2 0.95 / 0.97, R = 4 1.04 / 1.05 (64 chains 0.95 / 1.02);
+//   one workgroup per CU (float64 with R = 4, float32 with R = 8): 32 chains
+//     1.2 / 1.25, 128 0.92 / 1.05, 256 0.82 / 0.9, 400 1.02 / 1.06.
+// A batch of short chains in a long stride has work for few workgroups and loses
+// (512 x 50..253 at 2029, float32 with R = 4: 10.4 -> 13.1 us); the host does
+// not know the lengths here.
+bool bins_pay(int R, size_t bytes, int nc, int B, int resident) {
+    if (nc <= 2) return false;
+    if (nc <= 4) return B <= 1024 * (nc - 1);
+    if (bytes > 80u << 10) return B <= resident && 4 * B >= 3 * resident;
+    return B >= (R <= 2 ? 1 : 128) && (nc > 6 || B <= 512);
+}
+
+// Launches the chain kernel of chains of a.nc <= kBinsMax chunks of R residues
+// per lane (kernel(waves, bins) gives it, lds the staging of one wave), or
+// returns false.  Chains of at
 // most kChainMax chunks take a workgroup of a.nc waves each, if every workgroup
-// is resident from the start.  In the forward the rest are packed (BINS), if
-// they have more than 2 chunks and the batch is not too large for every
-// workgroup to read its lengths.  Otherwise the chunk kernels, whose one-wave
-// workgroups put the work first.
+// is resident from the start.  In the forward the rest are packed (BINS) where
+// that pays and the batch is not too large for every workgroup to read its
+// lengths.  Otherwise the chunk kernels, whose one-wave workgroups put the work
+// first.
 //
 // Steps of forward and backward in us, float32, with 4 residues per lane:
 //   chain kernels instead of chunk kernels, all resident, each at its best:
 //     256 x 700 residues 24.6 -> 17.0, 512 x 50..500 22.7 -> 17.0,
 //     32 x 200 14.9 -> 9.9;
-//   forward BINS instead of the chunk kernel (the backward fixed):
-//     400 x 1900 71.1 -> 63.6, 400 x 1300 53.7 -> 49.8, 800 x 500..1000
-//     55.2 -> 54.8, 1024 x 30..1000 54.3 -> 53.8 (2 per lane: 61.4 -> 53.2);
-//     with 2 chunks, 1500 x 500, 55.4 -> 56 or worse;
 //   backward BINS: 1024 x 30..1000 30 -> 29.5, but 800 x 500..1000 38.1 -> 42.2:
 //     of its 224 VGPR workgroups two fit on a CU, and a second round of them
 //     starts late.  So the backward has none.
 template <typename Kernel>
-bool launch_chain(Kernel kernel, const ChunkArgs& a, size_t lds, hipStream_t stream, int& rc) {
+bool launch_chain(Kernel kernel, const ChunkArgs& a, int R, size_t lds, hipStream_t stream, int& rc) {
     if (a.nc > kBinsMax) return false;
     for (const bool bins : {false, true}) {
         if (!bins && a.nc > kChainMax) continue;
         const int waves = !bins ? a.nc : a.nc <= 4 ? 4 : 8;
         const KernelFn k = kernel(waves, bins);
         if (!k || waves * lds > (bins ? kBinsMaxLds : kChainMaxLds) || !allow_lds(k, waves * lds)) continue;
-        if (bins ? a.nc <= 2 || a.B > bins_max_batch(waves) : a.B > resident_workgroups(k, 64 * waves, waves * lds)) continue;
+        const int resident = resident_workgroups(k, 64 * waves, waves * lds);
+        if (bins ? a.B > bins_max_batch(waves) || !bins_pay(R, waves * lds, a.nc, a.B, resident) : a.B > resident)
+            continue;
         hipLaunchKernelGGL(k, dim3((unsigned)a.B), dim3(64 * waves), waves * lds, stream, a);
         rc = hipGetLastError() == hipSuccess ? TPL_A2B_OK : TPL_A2B_ERR_LAUNCH;
         return true;
@@ -2646,7 +2678,7 @@ int forward_on(int dtype, const void* angles, void* coords, const int32_t* lengt
     const auto kernel = [&](int w, bool bins) {
         return f32 ? fwd_chain_kernel<float>(R, w, bins) : fwd_chain_kernel<double>(R, w, bins);
     };
-    if (launch_chain(kernel, a, lds, static_cast<hipStream_t>(stream), rc)) return rc;
+    if (launch_chain(kernel, a, R, lds, static_cast<hipStream_t>(stream), rc)) return rc;
     return launch(f32 ? fwd_kernel<float>(R) : fwd_kernel<double>(R), a, lds,
                   static_cast<hipStream_t>(stream));
 }
@@ -2676,7 +2708,7 @@ int backward_on(int dtype, void* grad_angles, const void* grad_coords, const voi
     const auto kernel = [&](int w, bool bins) -> KernelFn {
         return bins ? nullptr : f32 ? bwd_chain_kernel<float>(R, w) : bwd_chain_kernel<double>(R, w);
     };
-    if (launch_chain(kernel, a, lds, static_cast<hipStream_t>(stream), rc)) return rc;
+    if (launch_chain(kernel, a, R, lds, static_cast<hipStream_t>(stream), rc)) return rc;
     return launch(f32 ? bwd_kernel<float>(R) : bwd_kernel<double>(R), a, lds,
                   static_cast<hipStream_t>(stream));
 }
@@ -2825,7 +2857,7 @@ int tpl_a2b_forward_noalloc(int dtype, const void* angles, void* coords, const i
     const auto kernel = [&](int w, bool bins) {
         return f32 ? fwd_chain_kernel<float>(R, w, bins) : fwd_chain_kernel<double>(R, w, bins);
     };
-    if (launch_chain(kernel, a, lds, static_cast<hipStream_t>(stream), rc)) return rc;
+    if (launch_chain(kernel, a, R, lds, static_cast<hipStream_t>(stream), rc)) return rc;
     void* base = scratch_address();
     if (!base) return TPL_A2B_ERR_HIP;
     // Tickets, done counters and records must start at zero.  Every call
