@@ -209,3 +209,21 @@ def test_step_alone_on_another_stream_may_go_while_it_runs(L):
     for t in taken:
         assert all(t.data_ptr() + t.nbytes <= p or t.data_ptr() >= p + size for p, size in held)
     side.synchronize()
+
+
+@pytest.mark.parametrize("dtype,R,L,B", [
+    (torch.float32, 1, 64, 768), (torch.float64, 1, 33, 768), (torch.float32, 2, 128, 1536), (torch.float32, 1, 128, 1536),
+    (torch.float64, 1, 65, 1536), (torch.float32, 2, 256, 1536), (torch.float64, 2, 129, 3072), (torch.float32, 1, 129, 1280),
+    (torch.float32, 1, 256, 1280), (torch.float64, 1, 256, 3072)])
+def test_step_kernel_of_few_chunks_up_to_a_batch(dtype, R, L, B):
+    """Up to B chains of few chunks the step's own kernel, beyond them the layer's two."""
+    from torchproteinlibrary_amd._native import ext
+    from torchproteinlibrary_amd.ReducedModel.Angles2Backbone.Angles2Backbone import Angles2BackboneStep
+    f64 = dtype == torch.float64
+    assert ext.step_fits(f64, B, L, [R, R]) and not ext.step_fits(f64, B + 1, L, [R, R])
+    for batch in (B, B + 1):
+        a, ln, g = _case(batch, L, _lengths(batch, L, "mixed", 64 * R, np.random.default_rng(L)), dtype, batch)
+        step = Angles2BackboneStep(a, ln, config=(R, R))
+        step.grad_coords.copy_(g)
+        step.replay()
+        _check(step, a, ln, g, dtype)

@@ -2629,6 +2629,22 @@ void step_kernel(StepForm& s, StepMode mode) {
 // barriers, 13.3 us for B = 512, L = 500 against 10.5 with two residues per
 // lane.  Longer chains of up to kWalkMaxChunks chunks: WALK.  The rest (false)
 // goes through the forward and the backward kernel.
+//
+// With few chunks a chain, of few residues per lane, a workgroup of 4 waves has
+// little work, and of large batches every one reads all lengths: the step's kernel
+// against the layer's two at their best, by batch (equal lengths / log-uniform):
+//   1 chunk:  R = 1 1024 1.1 / 1.1, 2048 1.27 / 1.27, 4000 2.4 / 2.4; R = 2 1536 0.94 / 0.95,
+//             2048 1.2 / 1.2
+//   2 chunks: R = 1 1536 0.96 / 0.87, 2048 1.3 / 1.15; R = 2 float32 1536 0.89 / 0.77, 2048
+//             1.19 / 1.07, float64 3000 0.76 / 0.9, 4000 0.93 / 1.11
+//   3, 4:     R = 1 float32 1024 0.9 / 0.78, 1536 1.17 / 0.73, 2048 1.47 / 0.98, float64
+//             3000 0.9 / 0.77, 4000 1.05 / 1.05; R = 2 4000 1.03 / 0.91, float64 0.78 / 0.8
+int step_max_batch(bool f64, int R, int nc) {
+    if (R > 2 || nc > 4) return INT32_MAX;
+    if (nc == 1) return 768 * R;
+    if (nc == 2) return f64 && R == 2 ? 3072 : 1536;
+    return R == 2 ? INT32_MAX : f64 ? 3072 : 1280;
+}
 bool step_form(int dtype, int B, int L, const tpl_a2b_config* cfg, StepForm& s) {
     const int R = cfg->bwd_res_per_lane;
     const int nc = chunks(L, 64 * R);
@@ -2649,7 +2665,7 @@ bool step_form(int dtype, int B, int L, const tpl_a2b_config* cfg, StepForm& s) 
         return true;
     }
     if (dtype == TPL_A2B_F32 && cfg->fwd_res_per_lane != R) return false;
-    if (R == 1 && nc > 4) return false;
+    if ((R == 1 && nc > 4) || B > step_max_batch(dtype == TPL_A2B_F64, R, nc)) return false;
     if (!pick(CHAIN)) return false;
     if (B <= resident_workgroups(s.kernel, 64 * s.waves, s.lds)) return true;
     return B <= bins_max_batch(s.waves) && pick(BINS);
