@@ -299,3 +299,78 @@ def test_no_memory_for_the_workspace(dtype):
     # the gradients' sums in another order, from coordinates that differ as above
     scale = want[3].abs().amax(dim=(1, 2), keepdim=True)
     assert ((outs[3] - want[3]).abs() <= scale * (14 * L * 8 * 2.0 ** -53 + 1e3 * eps)).all()
+
+
+RUNS, TILES = 3, 4
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("shape", range(len(SHAPES)))
+def test_run_and_tile_forms_agree(shape, dtype):
+    """A run of residues per thread, and tiles, against a wave per block."""
+    lengths, L = SHAPES[shape]
+    seqs, X = _batch(lengths, L, 300 + shape, dtype)
+    natoms = [O.num_atoms(s) for s in seqs]
+    A = max(natoms) + (5, 2, 0, 3, 1, 4, 7)[shape]
+    print(f"a2c run and tile forms: {len(lengths)} structures, stride {L}, {dtype}", flush=True)
+    a, b = (_forward(f, seqs, X, A, offset=shape % 3) for f in (FUSED, RUNS))
+    assert a[3] == b[3] == 0
+    assert float((a[0] - b[0]).abs().max()) <= _tolerance(X, float(a[0].abs().max()))
+    assert torch.equal(a[1], b[1]) and torch.equal(a[2], b[2])
+    g = torch.randn(a[0].shape, dtype=dtype, device=DEV, generator=torch.Generator(DEV).manual_seed(shape))
+    coords = a[0].clone()  # at the start of a buffer of its own
+    outs = [_backward(f, seqs, coords, g, L) for f in (FUSED, RUNS) + ((TILES,) if L <= 2048 else ())]
+    tol = 14 * L * 2.0 ** -53 * 8 + (2.0 ** -23 if dtype == torch.float32 else 0.0)
+    scale = outs[0][0].abs().amax(dim=(1, 2), keepdim=True)
+    for ga, st in outs:
+        assert st == 0 and ((ga - outs[0][0]).abs() <= tol * scale).all()
+        for k in range(len(lengths)):
+            assert not ga[k, :, lengths[k]:].any()
+
+
+@pytest.mark.parametrize("L", [40, 200, 700])
+def test_run_and_tile_forms_flag_alike(L):
+    good = "ACDEFGHIKLMNPQRSTVWY" * (L // 20)
+    A = O.num_atoms(good)
+    _, X = _batch([L] * 4, L, 3, torch.float32)
+    g = torch.randn(4, 3 * A, device=DEV)
+    for bad, bit in ((good[:-1] + "X", 1), (good + "G", 2), ("W" * L, 4)):
+        seqs = [good, bad, "G" * L, good[:30]]
+        c, rn, an, st = _forward(RUNS, seqs, X, A)
+        assert st == bit and not c[1].any() and not rn[1].any() and not an[1].any()
+        assert c[0].any() and c[2].any() and c[3].any()
+        for form in (RUNS, TILES):
+            ga, st = _backward(form, seqs, c, g, L)
+            assert st == bit and not ga[1].any() and ga[0].any() and ga[2].any()
+    seqs = [good, good[:70], "G" * L, good[:30]]
+    turn = torch.tensor([2, 0, 3, 1], dtype=torch.int32, device=DEV)
+    beyond = torch.tensor([2, 0, 4, 1], dtype=torch.int32, device=DEV)
+    plain = _forward(RUNS, seqs, X, A)
+    for k in range(3):
+        assert torch.equal(_forward(RUNS, seqs, X, A, turn)[k], plain[k])
+    c, _, _, st = _forward(RUNS, seqs, X, A, beyond)
+    assert st == 8 and bool((c[3] == 7.0).all()) and torch.equal(c[:3], plain[0][:3])
+    for form in (RUNS, TILES):
+        ga = _backward(form, seqs, plain[0], g, L)[0]
+        assert torch.equal(_backward(form, seqs, plain[0], g, L, turn)[0], ga)
+        gb, st = _backward(form, seqs, plain[0], g, L, beyond)
+        assert st == 8 and bool((gb[3] == 7.0).all()) and torch.equal(gb[:3], ga[:3])
+
+
+# Shapes that the layer takes by runs (forward; backward in float64) and tiles (backward).
+@pytest.mark.parametrize("B,L,dtype", [(512, 200, torch.float32), (400, 300, torch.float32), (64, 200, torch.float64)])
+def test_layer_raises_from_every_form(B, L, dtype):
+    from torchproteinlibrary_amd.FullAtomModel import Angles2Coords
+    seqs, X = _batch([L] * B, L, 5, dtype)
+    Y = X.clone()
+    Y[-1, 1, L // 2] = float("nan")
+    with pytest.raises(Exception, match="forward Nan"):
+        Angles2Coords()(Y, seqs)
+    Y = X.clone()
+    Y[0, 7, :] = 1e9  # large, finite: no error
+    Angles2Coords()(Y, seqs)
+    coords = Angles2Coords()(X.requires_grad_(True), seqs)[0]
+    g = torch.zeros_like(coords)
+    g[-1, 3 * (O.num_atoms(seqs[-1]) - 1)] = float("nan")
+    with pytest.raises(Exception, match="backward Nan"):
+        coords.backward(g)

@@ -24,8 +24,9 @@
 // The subtree of a backbone node is the rest of its residue plus every later
 // residue: again one lane per residue in blocks of 64, whose sums (sum g,
 // sum x cross g) a scan over the lanes and the sums of the later blocks join.
-// Two older backwards stay for callers that pin them: runs of residues per
-// thread (a2c_bwd) and tiles of consecutive atoms (a2c_bwd_tiled).
+// For some batches a run of residues per thread (a2c_fwd_runs) is the better form
+// (forward_form).  Two older backwards stay for callers that pin them: runs of
+// residues per thread (a2c_bwd) and tiles of consecutive atoms (a2c_bwd_tiled).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -291,18 +292,6 @@ struct SideRows {
     }
 };
 
-// The structure this workgroup builds: order[blockIdx.x], or blockIdx.x
-// without an order.  An index outside the batch is reported
-// (TPL_A2C_STATUS_ORDER) and the workgroup does nothing (-1).
-__device__ __forceinline__ int structure_of(const int* order, uint32_t* status) {
-    if (!order) return (int)blockIdx.x;
-    const int b = __builtin_amdgcn_readfirstlane(order[blockIdx.x]);
-    if (b >= 0 && b < (int)gridDim.x) return b;
-    if (threadIdx.x == 0 && status)
-        __hip_atomic_fetch_or(status, TPL_A2C_STATUS_ORDER, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    return -1;
-}
-
 // A thread's run of residues [r0, r1) of a structure of L, its first atom and
 // the structure's atoms.
 struct Run {
@@ -326,8 +315,7 @@ struct Run {
 //   * a2c_fwd_single where a structure is one block (angles_stride <= 64): the
 //     wave scans its 64 steps;
 //   * a2c_fwd_fused: one workgroup per structure, whose waves' scans meet in
-//     LDS.  It needs no workspace and one launch, and serves calls without a
-//     workspace and small batches.
+//     LDS.  It needs no workspace and one launch, and serves small batches.
 // Waves whose residues would lie past the structure write its padding's zeros.
 // Against one workgroup of 256 or 512 threads per structure whose threads
 // walked runs of up to four residues and wrote their atoms and names one by one
@@ -1084,6 +1072,222 @@ __global__ void __launch_bounds__(64 * MAXW) __attribute__((amdgpu_waves_per_eu(
     }
 }
 
+// ---- forward: a run of residues per thread ----
+// One workgroup of 256 or 512 threads per structure, a thread multiplying out
+// the steps of up to four consecutive residues and walking them; a workgroup
+// scan joins the threads.  Each thread writes its own atoms, so this is the
+// better form only where little is written or there is little else to wait for
+// (forward_form).
+
+// The 8 angles of residue i, loaded together at the top of the residue so
+// that their latencies overlap (one global-load latency per residue walk
+// instead of one per transform).
+template <typename T>
+struct ResAngles {
+    T v[8];
+    __device__ __forceinline__ void load(const T* ang, int stride, int i) {
+#pragma unroll
+        for (int r = 0; r < 8; ++r) v[r] = ang[(size_t)r * stride + i];
+    }
+};
+
+// The residue step S_i applied to m: m <- m T_CA(phi) T_C(psi) T_N(omega).
+template <typename T>
+__device__ __forceinline__ void residue_step(double m[12], const Tables& tb, const T* ang, int stride, int i) {
+    const double phi = (double)ang[i], psi = (double)ang[(size_t)stride + i], omega = (double)ang[(size_t)2 * stride + i];
+    double s, c;
+    sincos_tab(phi, tb.tab, &s, &c);
+    step(m, tb.bb[0][0], tb.bb[0][1], c, s, geo::R_N_CA);
+    sincos_tab(psi, tb.tab, &s, &c);
+    step(m, tb.bb[1][0], tb.bb[1][1], c, s, geo::R_CA_C);
+    sincos_tab(omega, tb.tab, &s, &c);
+    step(m, tb.bb[2][0], tb.bb[2][1], c, s, geo::R_C_N);
+}
+
+// Per structure: the sequence length (first 0 byte), the residues' validity,
+// this thread's run [r0, r1), and the workgroup scans giving the N frame of
+// residue r0 (frame) and its first atom (atom0); nothing is left to build if the
+// structure is flagged.
+template <int NT, typename T>
+__device__ void prepare(const uint8_t* seq, int seq_stride, const T* ang, int ang_stride,
+                        int atoms_stride, const Report& rep, const Tables& tb, double (*s_m)[NT / 64],
+                        int* s_c, int* s_flag, Run& run, double frame[12], ResAngles<T>& av0,
+                        uint8_t& code0) {
+    const int tid = threadIdx.x;
+    if (tid == 0) {
+        s_flag[0] = seq_stride;  // length
+        s_flag[1] = 0;           // status bits
+    }
+    __syncthreads();
+    find_length<NT>(seq, seq_stride, &s_flag[0]);
+    __syncthreads();
+    int L = s_flag[0];
+    if (L > ang_stride) {
+        if (tid == 0) atomicOr(&s_flag[1], (int)TPL_A2C_STATUS_LENGTH);
+        L = 0;
+    }
+    const int chunk = (L + NT - 1) / NT;
+    const int r0 = min(L, tid * chunk), r1 = min(L, r0 + chunk);
+    // The walk's first residue: its angles and letter are loaded now, so
+    // that they arrive while the workgroup scans.
+    if (r0 < r1) {
+        av0.load(ang, ang_stride, r0);
+        code0 = seq[r0];
+    }
+    double P[12];
+    identity(P);
+    int cnt = 0;
+    bool bad = false;
+    for (int i = r0; i < r1; ++i) {
+        const int t = residue_type(seq[i]);
+        if (t < 0) {
+            bad = true;
+            continue;
+        }
+        cnt += tb.res_i[t] & 0xff;
+        residue_step(P, tb, ang, ang_stride, i);
+    }
+    if (bad) atomicOr(&s_flag[1], (int)TPL_A2C_STATUS_SEQ);
+    // Ordered product of the runs' steps and sum of their atom counts over
+    // the workgroup: inclusive within each wave by DPP, then across waves
+    // through LDS (the waves' totals; each wave composes those before it).
+    // frame = product of the earlier runs' steps, atom0 = their atoms.
+    constexpr int NW = NT / 64;
+    const int wv = tid >> 6;
+    int cinc = cnt;
+    if ((tid & ~63) * chunk < L) {  // a wave whose runs are all past the structure holds identities and zeros
+        cinc = wave_scan_int(cnt);
+        wave_scan_frames(P);
+    }
+    if ((tid & 63) == 63) {
+#pragma unroll
+        for (int k = 0; k < 12; ++k) s_m[k][wv] = P[k];
+        s_c[wv] = cinc;
+    }
+    double E[12];
+#pragma unroll
+    for (int k = 0; k < 12; ++k) E[k] = dpp_double<kWaveShr1, 0xf>(P[k], ident12(k));
+    __syncthreads();
+    double W[12];
+    identity(W);
+    int before = 0, total = 0;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+        if (w < wv) {
+            double Tw[12], R2[12];
+#pragma unroll
+            for (int k = 0; k < 12; ++k) Tw[k] = s_m[k][w];
+            compose(W, Tw, R2);
+#pragma unroll
+            for (int k = 0; k < 12; ++k) W[k] = R2[k];
+            before += s_c[w];
+        }
+        total += s_c[w];
+    }
+    compose(W, E, frame);
+    run.atom0 = before + cinc - cnt;
+    run.total = total;
+    if (run.total > atoms_stride && tid == 0) atomicOr(&s_flag[1], (int)TPL_A2C_STATUS_ATOMS);
+    __syncthreads();
+    const int flags = s_flag[1];
+    if (flags && tid == 0) report_bits(rep, (uint32_t)flags);
+    run.L = L;
+    run.r0 = r0;
+    run.r1 = r1;
+    if (flags) run.L = run.r0 = run.r1 = run.total = 0;
+}
+
+// At 256 threads the forward is held to four waves per SIMD (<= 128 VGPRs,
+// a few dwords spilled) so that four workgroups fit on a CU, as LDS allows:
+// 85 -> 71 us at mixed lengths 30-1000, B=1024, against three workgroups.
+template <int NT, typename T>
+__global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT == 256 ? 4 : 1, 8))) a2c_fwd_runs(
+    const uint8_t* __restrict__ seqs, int seq_stride, const T* __restrict__ angles, int ang_stride,
+    T* __restrict__ coords, uint32_t* __restrict__ res_names, uint32_t* __restrict__ atom_names, int atoms_stride,
+    Report rep, const int* __restrict__ order) {
+    __shared__ Tables tb;
+    __shared__ double s_m[12][NT / 64];  // the waves' products
+    __shared__ int s_c[NT / 64];          // the waves' atom counts
+    __shared__ int s_flag[2];
+    const int b = structure_at(order, (int)blockIdx.x, (int)gridDim.x, rep);
+    if (b < 0) return;
+    const uint8_t* seq = seqs + (size_t)b * seq_stride;
+    const T* ang = angles + (size_t)b * 8 * ang_stride;
+    T* out = coords + (size_t)b * 3 * atoms_stride;
+    copy_tables(tb, NT);
+    __syncthreads();
+    Run run;
+    double G[12];
+    ResAngles<T> av;
+    uint8_t code = 0;
+    prepare<NT>(seq, seq_stride, ang, ang_stride, atoms_stride, rep, tb, s_m, s_c, s_flag, run, G, av, code);
+    int a = run.atom0;
+    uint32_t* rn = res_names ? res_names + (size_t)b * atoms_stride : nullptr;
+    uint32_t* an = atom_names ? atom_names + (size_t)b * atoms_stride : nullptr;
+    for (int i = run.r0; i < run.r1; ++i) {
+        if (__builtin_expect(any_wild(av.v), 0)) report_flag(rep, TPLX_A2C_RANGE);
+        // the next residue's angles and letter go out before this one's work
+        ResAngles<T> nav;
+        uint8_t ncode = 0;
+        if (i + 1 < run.r1) {
+            nav.load(ang, ang_stride, i + 1);
+            ncode = seq[i + 1];
+        }
+        const int t = residue_type(code);
+        const int ri = tb.res_i[t];
+        const int natoms = ri & 0xff, nca = (ri >> 8) & 0xff, nside = ri >> 16;
+        const double* loc = tb.loc[t * kMaxAtoms];
+        double x[3];
+        auto put = [&](int slot, const double m[12]) {
+            apply(m, loc + 3 * slot, x);
+            T* o = out + 3 * (size_t)(a + slot);
+            o[0] = (T)x[0];
+            o[1] = (T)x[1];
+            o[2] = (T)x[2];
+        };
+        put(0, G);
+        double s, c, F[12], CA[12];
+#pragma unroll
+        for (int k = 0; k < 12; ++k) CA[k] = G[k];
+        sincos_tab((double)av.v[0], tb.tab, &s, &c);
+        step(CA, tb.bb[0][0], tb.bb[0][1], c, s, geo::R_N_CA);
+        for (int k = 1; k <= nca; ++k) put(k, CA);
+#pragma unroll
+        for (int k = 0; k < 12; ++k) F[k] = CA[k];
+        SideRows<T> rows(av.v);
+        for (int n = 0; n < nside; ++n) {
+            const int q = t * kMaxSide + n;
+            const int si = tb.side_i[q];
+            const int row = (int)(int8_t)(si & 0xff), first = (si >> 8) & 0xff, count = si >> 16;
+            double ca = tb.side[q][2], sa = tb.side[q][3];
+            if (row >= 0) sincos_tab(rows.pop(), tb.tab, &sa, &ca);
+            step(F, tb.side[q][0], tb.side[q][1], ca, sa, tb.side[q][4]);
+            for (int k = first; k < first + count; ++k) put(k, F);
+        }
+        sincos_tab((double)av.v[1], tb.tab, &s, &c);
+        step(CA, tb.bb[1][0], tb.bb[1][1], c, s, geo::R_CA_C);  // CA now holds the C frame
+        put(natoms - 2, CA);
+        put(natoms - 1, CA);
+        if (rn) {
+            for (int k = 0; k < natoms; ++k) {
+                const uint2 names = tb.name[t * kMaxAtoms + k];
+                rn[a + k] = names.x;
+                an[a + k] = names.y;
+            }
+        }
+        sincos_tab((double)av.v[2], tb.tab, &s, &c);
+        step(CA, tb.bb[2][0], tb.bb[2][1], c, s, geo::R_C_N);
+#pragma unroll
+        for (int k = 0; k < 12; ++k) G[k] = CA[k];
+        a += natoms;
+        av = nav;
+        code = ncode;
+    }
+    for (int k = 3 * run.total + threadIdx.x; k < 3 * atoms_stride; k += NT) out[k] = (T)0;
+    if (rn)
+        for (int k = run.total + threadIdx.x; k < atoms_stride; k += NT) rn[k] = an[k] = 0u;
+}
+
 struct Sums {
     double g[3], xg[3];
 };
@@ -1115,7 +1319,7 @@ __device__ __forceinline__ void sums_add(Sums& s, const double x[3], const doubl
 // workgroup after its next barrier).
 template <int NT>
 __device__ void count_run(const uint8_t* seq, int seq_stride, int ang_stride, int atoms_stride,
-                          uint32_t* status, const int* res_i, int* s_c, int* s_flag, Run& run,
+                          const Report& rep, const int* res_i, int* s_c, int* s_flag, Run& run,
                           int* s_ra = nullptr) {
     const int tid = threadIdx.x;
     if (tid == 0) {
@@ -1167,8 +1371,7 @@ __device__ void count_run(const uint8_t* seq, int seq_stride, int ang_stride, in
     if (run.total > atoms_stride && tid == 0) atomicOr(&s_flag[1], (int)TPL_A2C_STATUS_ATOMS);
     __syncthreads();
     const int flags = s_flag[1];
-    if (flags && tid == 0 && status)
-        __hip_atomic_fetch_or(status, (uint32_t)flags, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (flags && tid == 0) report_bits(rep, (uint32_t)flags);
     run.L = L;
     run.r0 = r0;
     run.r1 = r1;
@@ -1226,13 +1429,13 @@ template <int NT, typename T>
 __global__ void __launch_bounds__(NT) a2c_bwd(const uint8_t* __restrict__ seqs, int seq_stride,
                                               const T* __restrict__ coords, const T* __restrict__ grad_coords,
                                               int atoms_stride, T* __restrict__ grad_angles, int ang_stride,
-                                              uint32_t* status, const int* __restrict__ order) {
+                                              Report rep, const int* __restrict__ order) {
     __shared__ int s_res[kTypes];
     __shared__ int s_side[kTypes * kMaxSide];
     __shared__ double s_v[6][NT / 64];  // the waves' sums
     __shared__ int s_c[NT / 64];        // the waves' atom counts
     __shared__ int s_flag[2];
-    const int b = structure_of(order, status), tid = threadIdx.x;
+    const int b = structure_at(order, (int)blockIdx.x, (int)gridDim.x, rep), tid = threadIdx.x;
     if (b < 0) return;
     const uint8_t* seq = seqs + (size_t)b * seq_stride;
     const T* xs = coords + (size_t)b * 3 * atoms_stride;
@@ -1248,7 +1451,7 @@ __global__ void __launch_bounds__(NT) a2c_bwd(const uint8_t* __restrict__ seqs, 
     }
     __syncthreads();
     Run run;
-    count_run<NT>(seq, seq_stride, ang_stride, atoms_stride, status, s_res, s_c, s_flag, run);
+    count_run<NT>(seq, seq_stride, ang_stride, atoms_stride, rep, s_res, s_c, s_flag, run);
     // pass A: this run's (sum g, sum x cross g)
     Sums run_sum;
     sums_zero(run_sum);
@@ -1285,6 +1488,11 @@ __global__ void __launch_bounds__(NT) a2c_bwd(const uint8_t* __restrict__ seqs, 
     }
     // pass B: gradients, residue by residue
     int a = run.atom0;
+    bool range = false;
+    const auto put = [&](size_t at, double v) {
+        ga[at] = (T)v;
+        range |= out_of_range((T)v);
+    };
     for (int i = run.r0; i < run.r1; ++i) {
         const int t = residue_type(seq[i]);
         const int ri = s_res[t];
@@ -1320,7 +1528,7 @@ __global__ void __launch_bounds__(NT) a2c_bwd(const uint8_t* __restrict__ seqs, 
                     load3(xs + 3 * (size_t)(a + pfirst), q);
                 else
                     q[0] = pCA[0], q[1] = pCA[1], q[2] = pCA[2];
-                ga[(size_t)row * ang_stride + i] = (T)bond_torque(p, q, sSide);
+                put((size_t)row * ang_stride + i, bond_torque(p, q, sSide));
             }
         }
 #pragma unroll
@@ -1332,7 +1540,7 @@ __global__ void __launch_bounds__(NT) a2c_bwd(const uint8_t* __restrict__ seqs, 
         if (i > 0) {
             double pCp[3];
             load3(xs + 3 * (size_t)(a - 2), pCp);
-            ga[(size_t)2 * ang_stride + i - 1] = (T)bond_torque(pN, pCp, incl);
+            put((size_t)2 * ang_stride + i - 1, bond_torque(pN, pCp, incl));
         }
         if (i == run.L - 1) ga[(size_t)2 * ang_stride + i] = (T)0;
         // phi binds CA (on N): all but N
@@ -1341,17 +1549,18 @@ __global__ void __launch_bounds__(NT) a2c_bwd(const uint8_t* __restrict__ seqs, 
             s.g[c] = incl.g[c] - sN.g[c];
             s.xg[c] = incl.xg[c] - sN.xg[c];
         }
-        ga[i] = (T)bond_torque(pCA, pN, s);
+        put(i, bond_torque(pCA, pN, s));
         // psi binds C (on CA): the C group and everything after
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
             s.g[c] = sC.g[c] + excl.g[c];
             s.xg[c] = sC.xg[c] + excl.xg[c];
         }
-        ga[(size_t)ang_stride + i] = (T)bond_torque(pC, pCA, s);
+        put((size_t)ang_stride + i, bond_torque(pC, pCA, s));
         incl = excl;
         a += natoms;
     }
+    if (range) report_flag(rep, TPLX_A2C_RANGE);
     // angles past the sequence (and every angle of a flagged structure)
     for (int k = tid; k < 8 * ang_stride; k += NT)
         if (k % ang_stride >= run.L) ga[k] = (T)0;
@@ -1425,7 +1634,7 @@ __global__ void __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_
                                                               const T* __restrict__ coords,
                                                               const T* __restrict__ grad_coords, int atoms_stride,
                                                               T* __restrict__ grad_angles, int ang_stride,
-                                                              uint32_t* status, const int* __restrict__ order) {
+                                                              Report rep, const int* __restrict__ order) {
     constexpr int NT = kTileThreads, NW = NT / 64, K = kTileK;
     __shared__ int s_res[kTypes];                   // natoms | nca << 8 | nside << 16 | bound rows << 24
     __shared__ int s_side[kTypes * kMaxSide];       // row & 0xff | first << 8 | count << 16
@@ -1438,7 +1647,7 @@ __global__ void __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_
     __shared__ double s_v[6][NW];                   // the waves' sums
     __shared__ int s_c[NW];
     __shared__ int s_flag[2];
-    const int b = structure_of(order, status), tid = threadIdx.x;
+    const int b = structure_at(order, (int)blockIdx.x, (int)gridDim.x, rep), tid = threadIdx.x;
     if (b < 0) return;
     const uint8_t* seq = seqs + (size_t)b * seq_stride;
     const T* xs = coords + (size_t)b * 3 * atoms_stride;
@@ -1494,7 +1703,7 @@ __global__ void __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_
     __syncthreads();
     if (tid < kTypes) s_res[tid] |= bound << 24;
     Run run;
-    count_run<NT>(seq, seq_stride, ang_stride, atoms_stride, status, s_res, s_c, s_flag, run, s_ra);
+    count_run<NT>(seq, seq_stride, ang_stride, atoms_stride, rep, s_res, s_c, s_flag, run, s_ra);
     __syncthreads();
     const int L = run.L;
     for (int i = tid; i < L; i += NT) {
@@ -1534,6 +1743,7 @@ __global__ void __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_
     double carry[6];
 #pragma unroll
     for (int c = 0; c < 6; ++c) carry[c] = 0.0;
+    bool range = false;
     T cx[K][3], cg[K][3];
     int lo = 0, hi = 0;
     if (ntiles > 0) {
@@ -1645,7 +1855,9 @@ __global__ void __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_
             for (int c = 0; c < 3; ++c) q[c] = (double)(qi[m] >= 0 ? s_x[buf][3 * qk + c] : qprev[c]);
 #pragma unroll
             for (int c = 0; c < 6; ++c) sm[c] = sub[m] ? suf[m][c] - s_cs[il[m]][c] : suf[m][c];
-            ga[dst[m]] = (T)bond_torque_rsq(p3, q, sm);
+            const T v = (T)bond_torque_rsq(p3, q, sm);
+            range |= out_of_range(v);
+            ga[dst[m]] = v;
         }
         hi = lo;
         lo = nlo;
@@ -1657,6 +1869,7 @@ __global__ void __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_
                 cg[m][c] = ng[m][c];
             }
     }
+    if (range) report_flag(rep, TPLX_A2C_RANGE);
     // angles past the sequence (and every angle of a flagged structure)
     for (int k = tid; k < 8 * ang_stride; k += NT)
         if (k % ang_stride >= L) ga[k] = (T)0;
@@ -1677,11 +1890,11 @@ __global__ void __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_
 //   * a2c_bwd_fused: one workgroup per structure, whose waves' sums meet in
 //     LDS.  One launch, no workspace.
 // Against runs of residues per thread, or atom tiles walked by one workgroup per
-// structure (kept for callers that pin them), us: lengths 30-1000 at B=1024
-// 94 -> 60 (60 -> 60 with the structures ordered by size), in float64 168 -> 95;
-// 256 x 1000 50 -> 36, 1 x 1000 34 -> 18, 32 x 350 17.1 -> 14.2, 1024 x 128
-// 34 -> 17, 1024 x 30 14.3 -> 9.8, one peptide of 21 in float64 12.0 -> 8.3; 512 x
-// 300 26 -> 29.  What bounds it: the LDS that a block's atoms take holds eight
+// structure (which some batches still take: backward_form), us: lengths 30-1000 at
+// B=1024 94 -> 60 (60 -> 60 with the structures ordered by size), in float64 168 ->
+// 95; 256 x 1000 50 -> 33, 1 x 1000 34 -> 17, 32 x 350 16.8 -> 15.1, 1024 x 128
+// 39 -> 15, 1024 x 30 13.6 -> 9.0, one peptide of 21 in float64 11.3 -> 7.8.  What
+// bounds it: the LDS that a block's atoms take holds eight
 // waves on a CU, and those wait on latencies two thirds of their time.
 struct alignas(16) BackTables {
     int res_i[kTypes];              // natoms | nca << 8 | nside << 16
@@ -2268,30 +2481,61 @@ int compute_units() {
     return cus[dev];
 }
 
-// The group kernels (two launches) or one workgroup per structure.  The group
-// kernels share the blocks evenly over the GPU and win where the structures
-// need more than one round of workgroups (fused -> groups, us, float32 with
-// names: lengths 30-1000 at B=1024 85 -> 62, 1024 x 300 55 -> 46, 300 x 600
-// 44 -> 38, 300 x 1000 57 -> 48; not yet 512 x 300 25 -> 35 and 1024 x 128
-// 22 -> 25), and where a structure has more blocks than a workgroup waves (8 x
-// 3000 82 -> 30, 100 x 1400 48 -> 38) or needs sixteen, which hold few
-// registers, while CUs stay idle (1 x 1000 26 -> 22, 64 x 1000 28 -> 27; 256 x
-// 1000 38 -> 42).
-bool use_groups(int batch, int angles_stride) {
-    const int nb = blocks_of(angles_stride), cus = compute_units();
-    if (nb > 16) return true;
-    return batch > cus ? (int64_t)batch * nb >= 3000 : nb > 8 && batch <= cus / 4;
+// The residues that the longest structure is likely to have: callers give the
+// atoms of the largest one as atoms_stride, 8.2 to a residue on average, while
+// the angles' stride may be a longer one that they keep.  For choosing only.
+int likely_residues(int angles_stride, int atoms_stride) {
+    const int n = atoms_stride / 8 > 1 ? atoms_stride / 8 : 1;
+    return n < angles_stride ? n : angles_stride;
+}
+
+// Run forward: 512 threads for structures that may be longer than 256 residues,
+// up to twice as many structures as CUs (B=256 of 1000 residues: 33.7 -> 28.6
+// us; B=512 of 300: 23.8 -> 21.8 us; at B=1024 512 threads measured slower, with
+// fewer workgroups per CU: mixed lengths 30-1000 48.4 -> 55.7 us, 1024 x 270
+// 32.0 -> 39.6 us).
+bool use_large_fwd(int batch, int ang_stride) {
+    return batch <= 512 && ang_stride > kThreadsSmall;
 }
 
 // Whether the group kernels' grids can be counted.
 bool forward_groups_fit(int batch, int angles_stride) {
     return (int64_t)batch * groups_of(angles_stride) <= INT32_MAX / kGroup;
 }
-// What AUTO takes.  A structure of one block needs no groups, whatever the form.
-int forward_form(int batch, int angles_stride, bool workspace) {
-    const bool groups = workspace && blocks_of(angles_stride) > 1 && forward_groups_fit(batch, angles_stride) &&
-                        use_groups(batch, angles_stride);
-    return groups ? TPLX_A2C_FWD_GROUPS : TPLX_A2C_FWD_FUSED;
+// What AUTO takes.  us of the forms (U: lengths uniform; structures x stride):
+//   GROUPS share the blocks evenly over the GPU, and win where the structures need
+//   more than one round of workgroups, or where there are fewer long ones than
+//   CUs.  Without it -> GROUPS, with names, float32: 1024 x 1000 U 90 -> 63, 2048 x 300
+//   U 58 -> 47, 300 x 600 40 -> 36, 4096 x 200 U 74 -> 70, 100 x 1400 41 -> 37, 8 x 3000 65
+//   -> 28, 64 x 1000 28.2 -> 26.5, 4096 x 128 U 62 -> 55; not 1024 x 200 27 -> 37, 512 x 450 30 -> 38, 64 x 600 21.5
+//   -> 24.7, 256 x 1000 35 -> 40; float64: 200 x 800 U 34 -> 30, not 256 x 600 33 -> 40.
+//   FUSED against RUNS: a wave per block wins while every structure has a CU to
+//   itself, and where RUNS would have 512 threads for little more than 256
+//   residues; otherwise a run per thread does, most where no names are written.
+//   RUNS -> FUSED without names / with names, float32: 256 x 300 16.1 -> 13.6 / 18.9 ->
+//   16.2, 256 x 1000 26.6 -> 31.3 / 37.6 -> 34.7, 512 x 300 21.7 -> 20.8 / 25.9 -> 23.8, 1024 x
+//   300 32 -> 46 / 41 -> 53, 1024 x 128 16.9 -> 18.5 / 20.6 -> 22.0, 8 x 3000 56 -> 75 / 65 ->
+//   82; float64: 256 x 300 18.1 -> 17.1 / 21.2 -> 19.5, 256 x 600 28.6 -> 30.4 / 35.9 -> 32.9,
+//   512 x 200 20 -> 23 / 23 -> 26, 512 x 450 40 -> 38 / 46 -> 42, 64 x 1000 26 -> 33 / 32 -> 37.
+//   With names and 14 to 16 blocks many structures win too (1024 x 1000 float32 131 -> 112, U
+//   longest first 89 -> 76; 300 x 1000 50 -> 55).
+// A structure of one block needs no groups, whatever the form.
+bool forward_groups_pay(bool f64, int batch, int nb) {
+    const int cus = compute_units();
+    if (nb > 16) return true;
+    if (batch <= cus) return f64 ? nb > 10 : nb > 13 && batch <= cus / 2;
+    return nb > 8 || (int64_t)batch * nb >= (nb > 4 ? 5000 : 8000);
+}
+int forward_form(bool f64, int batch, int angles_stride, int atoms_stride, bool names, bool workspace) {
+    const int nb = blocks_of(likely_residues(angles_stride, atoms_stride)), cus = compute_units();
+    if (blocks_of(angles_stride) == 1) return TPLX_A2C_FWD_FUSED;
+    if (workspace && forward_groups_fit(batch, angles_stride) && forward_groups_pay(f64, batch, nb))
+        return TPLX_A2C_FWD_GROUPS;
+    const int most = (f64 ? 8 : 13) + (names ? f64 ? 2 : 3 : 0);
+    const bool fused = batch <= cus                ? nb <= most
+                       : names && nb > 13          ? nb <= 16 && batch >= 2 * cus
+                                                   : batch <= 2 * cus && nb >= 5 && nb <= (f64 ? 10 : 7);
+    return fused ? TPLX_A2C_FWD_FUSED : TPLX_A2C_FWD_RUNS;
 }
 
 template <typename T>
@@ -2300,7 +2544,7 @@ void launch_forward(int form, hipStream_t s, const uint8_t* sequences, int seq_s
                     const int32_t* order, int batch) {
     const int nslot = blocks_of(angles_stride), ng = groups_of(angles_stride);
     const dim3 block(64 * kGroupWaves);
-    if (nslot == 1) {
+    if (nslot == 1 && form != TPLX_A2C_FWD_RUNS) {
         hipLaunchKernelGGL((a2c_fwd_single<T>), dim3((batch + kGroupWaves - 1) / kGroupWaves), block, 0, s, sequences,
                            seq_stride, a, angles_stride, c, rn, an, atoms_stride, rep, order, batch);
         return;
@@ -2320,6 +2564,13 @@ void launch_forward(int form, hipStream_t s, const uint8_t* sequences, int seq_s
         hipLaunchKernelGGL((a2c_fwd_walk<T>), dim3(wgs < fill ? wgs : fill), dim3(64 * kWalkWaves), 0, s, sequences,
                            seq_stride, a, angles_stride, lens, rec, frames, c, rn, an, atoms_stride, rep, order,
                            batch, ng);
+        return;
+    }
+    if (form == TPLX_A2C_FWD_RUNS) {
+        const int nt = use_large_fwd(batch, angles_stride) ? kThreadsLarge : kThreadsSmall;
+        const auto kernel = nt == kThreadsLarge ? a2c_fwd_runs<kThreadsLarge, T> : a2c_fwd_runs<kThreadsSmall, T>;
+        hipLaunchKernelGGL(kernel, dim3(batch), dim3(nt), 0, s, sequences, seq_stride, a, angles_stride, c, rn, an,
+                           atoms_stride, rep, order);
         return;
     }
     // One wave per block up to 8, or up to 16 where every structure can have a
@@ -2344,7 +2595,9 @@ int forward_on(int form, const int32_t* order, int dtype, const uint8_t* sequenc
     if (!sequences || (angles_stride > 0 && !angles) || (atoms_stride > 0 && !coords) ||
         (!res_names) != (!atom_names))
         return TPL_A2C_ERR_ARG;
-    if (form == TPLX_A2C_FWD_AUTO) form = forward_form(batch, angles_stride, workspace);
+    if (form == TPLX_A2C_FWD_AUTO)
+        form = forward_form(dtype == TPL_A2C_F64, batch, angles_stride, atoms_stride, res_names != nullptr,
+                            workspace != nullptr);
     if (form == TPLX_A2C_FWD_GROUPS && blocks_of(angles_stride) > 1 &&
         !(workspace && forward_groups_fit(batch, angles_stride)))
         return TPL_A2C_ERR_ARG;
@@ -2381,21 +2634,18 @@ bool allow_lds(const void* kernel, size_t bytes) {
     return true;
 }
 
-// The backward's block kernels where the forward's rule says so, but not for
-// structures of one or two blocks, which one workgroup each handles well however
-// many there are (fused -> blocks, us, float32: lengths 30-1000 at B=1024
-// 80 -> 60, 1024 x 300 53 -> 50, 300 x 600 47 -> 39, 8 x 3000 78 -> 27, 1 x 1000
-// 26 -> 18; not 1024 x 128 17 -> 24, 256 x 1000 36 -> 43, 512 x 300 29 -> 35).
-bool use_back_groups(int batch, int angles_stride) {
-    return blocks_of(angles_stride) > 2 && use_groups(batch, angles_stride);
-}
-
 bool backward_groups_fit(int batch, int angles_stride) {
     return (int64_t)batch * blocks_of(angles_stride) <= INT32_MAX / kBlock;
 }
-int backward_form(int batch, int angles_stride, bool workspace) {
-    const bool groups =
-        workspace && backward_groups_fit(batch, angles_stride) && use_back_groups(batch, angles_stride);
+// The block kernels share the blocks evenly over the GPU; structures of one or two
+// blocks one workgroup each handles well however many there are (fused -> blocks,
+// us, float32: lengths 30-1000 at B=1024 80 -> 60, 1024 x 300 53 -> 50, 300 x 600
+// 47 -> 39, 8 x 3000 78 -> 27, 1 x 1000 26 -> 18; not 1024 x 128 17 -> 24, 256 x
+// 1000 36 -> 43, 512 x 300 29 -> 35).
+int backward_form(bool, int batch, int angles_stride, int, bool workspace) {
+    const int nb = blocks_of(angles_stride), cus = compute_units();
+    const bool pay = nb > 16 || (batch > cus ? (int64_t)batch * nb >= 3000 : nb > 8 && batch <= cus / 4);
+    const bool groups = workspace && nb > 2 && backward_groups_fit(batch, angles_stride) && pay;
     return groups ? TPLX_A2C_BWD_GROUPS : TPLX_A2C_BWD_FUSED;
 }
 
@@ -2405,7 +2655,15 @@ int launch_backward(int form, hipStream_t s, const uint8_t* sequences, int seq_s
                     const int32_t* order, int batch) {
     const int nslot = blocks_of(angles_stride);
     constexpr size_t per_wave = 2 * back_values<T>() * sizeof(T);
-    if (form == TPLX_A2C_BWD_GROUPS) {
+    if (form == TPLX_A2C_BWD_TILES) {
+        hipLaunchKernelGGL((a2c_bwd_tiled<T>), dim3(batch), dim3(kTileThreads), 0, s, sequences, seq_stride, x, g,
+                           atoms_stride, ga, angles_stride, rep, order);
+    } else if (form == TPLX_A2C_BWD_RUNS) {
+        const int nt = use_large_bwd(angles_stride) ? kThreadsLarge : kThreadsSmall;
+        const auto kernel = nt == kThreadsLarge ? a2c_bwd<kThreadsLarge, T> : a2c_bwd<kThreadsSmall, T>;
+        hipLaunchKernelGGL(kernel, dim3(batch), dim3(nt), 0, s, sequences, seq_stride, x, g, atoms_stride, ga,
+                           angles_stride, rep, order);
+    } else if (form == TPLX_A2C_BWD_GROUPS) {
         int* lens = static_cast<int*>(workspace);
         BackRec* rec = reinterpret_cast<BackRec*>(static_cast<char*>(workspace) + lens_bytes(batch));
         const int wgs = (batch * nslot + kWalkWaves - 1) / kWalkWaves, fill = compute_units();
@@ -2431,9 +2689,11 @@ int backward_on(int form, const int32_t* order, int dtype, const uint8_t* sequen
                 void* workspace, const Report& rep, int batch, tpl_a2c_stream_t stream) {
     const int rc = check(dtype, batch, seq_stride, angles_stride, atoms_stride);
     if (rc != TPL_A2C_OK) return rc;
+    if (form == TPLX_A2C_BWD_TILES && angles_stride > kTileMaxRes) return TPL_A2C_ERR_SIZE;
     if (batch == 0 || angles_stride == 0) return TPL_A2C_OK;
     if (!sequences || !grad_angles || (atoms_stride > 0 && (!coords || !grad_coords))) return TPL_A2C_ERR_ARG;
-    if (form == TPLX_A2C_BWD_AUTO) form = backward_form(batch, angles_stride, workspace);
+    if (form == TPLX_A2C_BWD_AUTO)
+        form = backward_form(dtype == TPL_A2C_F64, batch, angles_stride, atoms_stride, workspace != nullptr);
     if (form == TPLX_A2C_BWD_GROUPS && !(workspace && backward_groups_fit(batch, angles_stride)))
         return TPL_A2C_ERR_ARG;
     hipStream_t s = static_cast<hipStream_t>(stream);
@@ -2501,12 +2761,12 @@ int tplx_a2c_forward(int form, const int32_t* order, int dtype, const uint8_t* s
                       atom_names, atoms_stride, workspace, Report{status, flags}, batch, stream);
 }
 
-int tplx_a2c_forward_form(int batch, int angles_stride, int workspace) {
-    return forward_form(batch, angles_stride, workspace != 0);
+int tplx_a2c_forward_form(int dtype, int batch, int angles_stride, int atoms_stride, int names, int workspace) {
+    return forward_form(dtype == TPL_A2C_F64, batch, angles_stride, atoms_stride, names != 0, workspace != 0);
 }
 
-int tplx_a2c_backward_form(int batch, int angles_stride, int workspace) {
-    return backward_form(batch, angles_stride, workspace != 0);
+int tplx_a2c_backward_form(int dtype, int batch, int angles_stride, int atoms_stride, int workspace) {
+    return backward_form(dtype == TPL_A2C_F64, batch, angles_stride, atoms_stride, workspace != 0);
 }
 
 size_t tplx_a2c_workspace_bytes(int batch, int angles_stride) {
@@ -2536,51 +2796,11 @@ int tpl_a2c_forward(int dtype, const uint8_t* sequences, int seq_stride, const v
 int tpl_a2c_backward_form(int form, const int32_t* order, int dtype, const uint8_t* sequences, int seq_stride,
                           const void* coords, const void* grad_coords, int atoms_stride, void* grad_angles,
                           int angles_stride, uint32_t* status, int batch, tpl_a2c_stream_t stream) {
+    static_assert(TPLX_A2C_BWD_AUTO == TPL_A2C_BWD_AUTO, "one name for both");
     if (form != TPL_A2C_BWD_AUTO && form != TPL_A2C_BWD_RUNS && form != TPL_A2C_BWD_TILES) return TPL_A2C_ERR_ARG;
-    if (form == TPL_A2C_BWD_AUTO)
-        return backward_on(TPLX_A2C_BWD_AUTO, order, dtype, sequences, seq_stride, coords, grad_coords, atoms_stride,
-                           grad_angles, angles_stride, nullptr, Report{status, nullptr}, batch, stream);
-    const int rc = check(dtype, batch, seq_stride, angles_stride, atoms_stride);
-    if (rc != TPL_A2C_OK) return rc;
-    if (form == TPL_A2C_BWD_TILES && angles_stride > kTileMaxRes) return TPL_A2C_ERR_SIZE;
-    if (batch == 0 || angles_stride == 0) return TPL_A2C_OK;
-    if (!sequences || !grad_angles || (atoms_stride > 0 && (!coords || !grad_coords)))
-        return TPL_A2C_ERR_ARG;
-    hipStream_t s = static_cast<hipStream_t>(stream);
-    if (form == TPL_A2C_BWD_TILES) {
-        if (dtype == TPL_A2C_F32)
-            hipLaunchKernelGGL((a2c_bwd_tiled<float>), dim3(batch), dim3(kTileThreads), 0, s, sequences,
-                               seq_stride, static_cast<const float*>(coords),
-                               static_cast<const float*>(grad_coords), atoms_stride,
-                               static_cast<float*>(grad_angles), angles_stride, status, order);
-        else
-            hipLaunchKernelGGL((a2c_bwd_tiled<double>), dim3(batch), dim3(kTileThreads), 0, s, sequences,
-                               seq_stride, static_cast<const double*>(coords),
-                               static_cast<const double*>(grad_coords), atoms_stride,
-                               static_cast<double*>(grad_angles), angles_stride, status, order);
-        return hipGetLastError() == hipSuccess ? TPL_A2C_OK : TPL_A2C_ERR_LAUNCH;
-    }
-    const bool large = use_large_bwd(angles_stride);
-    if (dtype == TPL_A2C_F32) {
-        const float *x = static_cast<const float*>(coords), *g = static_cast<const float*>(grad_coords);
-        float* ga = static_cast<float*>(grad_angles);
-        if (large)
-            hipLaunchKernelGGL((a2c_bwd<kThreadsLarge, float>), dim3(batch), dim3(kThreadsLarge), 0, s,
-                               sequences, seq_stride, x, g, atoms_stride, ga, angles_stride, status, order);
-        else
-            hipLaunchKernelGGL((a2c_bwd<kThreadsSmall, float>), dim3(batch), dim3(kThreadsSmall), 0, s,
-                               sequences, seq_stride, x, g, atoms_stride, ga, angles_stride, status, order);
-    } else {
-        const double *x = static_cast<const double*>(coords), *g = static_cast<const double*>(grad_coords);
-        double* ga = static_cast<double*>(grad_angles);
-        if (large)
-            hipLaunchKernelGGL((a2c_bwd<kThreadsLarge, double>), dim3(batch), dim3(kThreadsLarge), 0, s,
-                               sequences, seq_stride, x, g, atoms_stride, ga, angles_stride, status, order);
-        else
-            hipLaunchKernelGGL((a2c_bwd<kThreadsSmall, double>), dim3(batch), dim3(kThreadsSmall), 0, s,
-                               sequences, seq_stride, x, g, atoms_stride, ga, angles_stride, status, order);
-    }
-    return hipGetLastError() == hipSuccess ? TPL_A2C_OK : TPL_A2C_ERR_LAUNCH;
+    form = form == TPL_A2C_BWD_RUNS ? TPLX_A2C_BWD_RUNS : form == TPL_A2C_BWD_TILES ? TPLX_A2C_BWD_TILES : form;
+    return backward_on(form, order, dtype, sequences, seq_stride, coords, grad_coords, atoms_stride, grad_angles,
+                       angles_stride, nullptr, Report{status, nullptr}, batch, stream);
 }
 
 int tpl_a2c_backward(int dtype, const uint8_t* sequences, int seq_stride, const void* coords,

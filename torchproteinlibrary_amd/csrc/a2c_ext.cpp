@@ -83,14 +83,16 @@ torch::Tensor workspace(size_t need, const torch::Tensor& like) {
 void* ptr(const torch::Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
 
 // The workspaces of the two directions, where the form that they take reads one.
-torch::Tensor forward_workspace(const torch::Tensor& angles) {
+torch::Tensor forward_workspace(const torch::Tensor& angles, int64_t atoms_stride, bool names) {
     const int B = (int)angles.size(0), L = (int)angles.size(2);
-    const bool groups = tplx_a2c_forward_form(B, L, 1) == TPLX_A2C_FWD_GROUPS;
+    const bool groups =
+        tplx_a2c_forward_form(dtype_code(angles), B, L, (int)atoms_stride, names, 1) == TPLX_A2C_FWD_GROUPS;
     return workspace(groups ? tplx_a2c_workspace_bytes(B, L) : 0, angles);
 }
-torch::Tensor backward_workspace(const torch::Tensor& grad_angles) {
+torch::Tensor backward_workspace(const torch::Tensor& grad_angles, int64_t atoms_stride) {
     const int B = (int)grad_angles.size(0), L = (int)grad_angles.size(2);
-    const bool groups = tplx_a2c_backward_form(B, L, 1) == TPLX_A2C_BWD_GROUPS;
+    const bool groups =
+        tplx_a2c_backward_form(dtype_code(grad_angles), B, L, (int)atoms_stride, 1) == TPLX_A2C_BWD_GROUPS;
     return workspace(groups ? tplx_a2c_backward_workspace_bytes(B, L) : 0, grad_angles);
 }
 
@@ -114,7 +116,7 @@ void forward_on(const torch::Tensor& sequences, const torch::Tensor& input_angle
         TORCH_CHECK(n->device() == input_angles.device(), "names must be on the device of the angles");
     }
     TORCH_CHECK(output_coords.device() == input_angles.device(), "coordinates must be on the device of the angles");
-    const torch::Tensor ws = forward_workspace(input_angles);
+    const torch::Tensor ws = forward_workspace(input_angles, A, true);
     check_rc(tplx_a2c_forward(TPLX_A2C_FWD_AUTO, order_ptr(order, input_angles), dtype_code(input_angles),
                               sequences.data_ptr<uint8_t>(), (int)sequences.size(1), input_angles.data_ptr(),
                               (int)input_angles.size(2), output_coords.data_ptr(), res_names.data_ptr<uint8_t>(),
@@ -159,7 +161,7 @@ void backward_on(const torch::Tensor& grad_atoms, const torch::Tensor& grad_angl
                 "gradients and coordinates must be on one device");
     const int64_t A = grad_atoms.size(1) / 3;
     TORCH_CHECK(A <= INT32_MAX / 3, "grad_atoms too large");
-    const torch::Tensor ws = backward_workspace(grad_angles);
+    const torch::Tensor ws = backward_workspace(grad_angles, A);
     check_rc(tplx_a2c_backward(TPLX_A2C_BWD_AUTO, order_ptr(order, grad_angles), dtype_code(grad_angles),
                                sequences.data_ptr<uint8_t>(), (int)sequences.size(1), coords.data_ptr(),
                                grad_atoms.data_ptr(), (int)A, grad_angles.data_ptr(), (int)grad_angles.size(2),
@@ -342,7 +344,8 @@ std::tuple<double, double, double> bench(std::vector<std::vector<torch::Tensor>>
     c10::DeviceGuard guard(sets[0][1].device());
     hipStream_t stream = stream_of(sets[0][1]);
     const int dt = dtype_code(sets[0][1]);
-    const torch::Tensor ws = forward_workspace(sets[0][1]), bws = backward_workspace(sets[0][1]);
+    const torch::Tensor ws = forward_workspace(sets[0][1], sets[0][2].size(1) / 3, false),
+                        bws = backward_workspace(sets[0][1], sets[0][2].size(1) / 3);
     for (auto& t : sets) TORCH_CHECK(t[1].sizes() == sets[0][1].sizes(), "bench: sets differ in shape");
     auto fwd = [&](std::vector<torch::Tensor>& t) {
         const int32_t* order = t.size() == 6 ? t[5].data_ptr<int32_t>() : nullptr;
