@@ -24,9 +24,9 @@
 // The subtree of a backbone node is the rest of its residue plus every later
 // residue: again one lane per residue in blocks of 64, whose sums (sum g,
 // sum x cross g) a scan over the lanes and the sums of the later blocks join.
-// For some batches a run of residues per thread (a2c_fwd_runs) is the better form
-// (forward_form).  Two older backwards stay for callers that pin them: runs of
-// residues per thread (a2c_bwd) and tiles of consecutive atoms (a2c_bwd_tiled).
+// For some batches a run of residues per thread (a2c_fwd_runs, a2c_bwd) or tiles
+// of consecutive atoms (a2c_bwd_tiled) are the better form (forward_form,
+// backward_form).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -2637,16 +2637,38 @@ bool allow_lds(const void* kernel, size_t bytes) {
 bool backward_groups_fit(int batch, int angles_stride) {
     return (int64_t)batch * blocks_of(angles_stride) <= INT32_MAX / kBlock;
 }
-// The block kernels share the blocks evenly over the GPU; structures of one or two
-// blocks one workgroup each handles well however many there are (fused -> blocks,
-// us, float32: lengths 30-1000 at B=1024 80 -> 60, 1024 x 300 53 -> 50, 300 x 600
-// 47 -> 39, 8 x 3000 78 -> 27, 1 x 1000 26 -> 18; not 1024 x 128 17 -> 24, 256 x
-// 1000 36 -> 43, 512 x 300 29 -> 35).
-int backward_form(bool, int batch, int angles_stride, int, bool workspace) {
+// What AUTO takes.  us of the forms (U: lengths uniform):
+//   GROUPS as in the forward, from 5 blocks on; FUSED -> GROUPS, float32: 1024 x 1000 U 91 ->
+//   77, 2048 x 300 U 85 -> 52, 700 x 300 40 -> 37, 64 x 600 23 -> 21, 8 x 3000 70 -> 25; not
+//   1024 x 200 27 -> 40, 256 x 1000 33 -> 41, 512 x 450 34 -> 39.
+//   FUSED otherwise, but for
+//   - TILES in float32, whose workgroup of one structure has two on a CU: with 5 to 7
+//     blocks beyond a structure per CU, with 5 to 10 up to two (FUSED -> TILES: 400 x 300 26.5 ->
+//     24.5, 1024 x 300 52 -> 48, 512 x 600 48 -> 45, 1500 x 400 U longest first 67 -> 59; not
+//     260 x 450 27 -> 30, 2048 x 500 U 98 -> 109);
+//   - RUNS in float64, where a block's atoms are staged in two rounds, for up to a
+//     structure of 256 residues per CU (FUSED -> RUNS: 128 x 64 15.4 -> 13.1, 128 x 128 15.9
+//     -> 14.7, 64 x 200 18.0 -> 16.0; not 320 x 200 19.7 -> 29, 256 x 300 20.5 -> 27, 1 x 128
+//     12.9 -> 13.9) and two of 64 (512 x 64 17.1 -> 15.0);
+//   - TILES for short structures in a long stride, whose workgroups of a wave per
+//     block of the stride would be nearly idle (FUSED -> TILES: 500 x 20..100 at 800 22.5
+//     -> 15.0, float64 31.5 -> 22.1; 1024 x 25..125 at 1000 39 -> 32, GROUPS 28).
+int backward_form(bool f64, int batch, int angles_stride, int atoms_stride, bool workspace) {
     const int nb = blocks_of(angles_stride), cus = compute_units();
-    const bool pay = nb > 16 || (batch > cus ? (int64_t)batch * nb >= 3000 : nb > 8 && batch <= cus / 4);
-    const bool groups = workspace && nb > 2 && backward_groups_fit(batch, angles_stride) && pay;
-    return groups ? TPLX_A2C_BWD_GROUPS : TPLX_A2C_BWD_FUSED;
+    const bool tiles_fit = angles_stride <= kTileMaxRes, two_each = 2 * batch >= 3 * cus && batch <= 2 * cus;
+    if (4 * likely_residues(angles_stride, atoms_stride) <= angles_stride && batch > cus && tiles_fit &&
+        (!workspace || batch <= 2 * cus))
+        return TPLX_A2C_BWD_TILES;
+    if (workspace && backward_groups_fit(batch, angles_stride) && nb > 4 && !(two_each && nb <= 10)) {
+        if (nb > 16 || (batch <= cus ? nb > 8 && batch <= cus / 2 : (int64_t)batch * nb >= 3000))
+            return TPLX_A2C_BWD_GROUPS;
+    }
+    if (f64) {
+        const bool runs = angles_stride > 36 && nb <= 4 && batch >= 16 && batch <= (nb == 1 ? 2 * cus : cus);
+        return runs ? TPLX_A2C_BWD_RUNS : TPLX_A2C_BWD_FUSED;
+    }
+    const bool tiles = nb >= 5 && (nb <= 7 ? 4 * batch >= 5 * cus : nb <= 10 && two_each);
+    return tiles && tiles_fit ? TPLX_A2C_BWD_TILES : TPLX_A2C_BWD_FUSED;
 }
 
 template <typename T>
