@@ -227,3 +227,26 @@ def test_step_kernel_of_few_chunks_up_to_a_batch(dtype, R, L, B):
         step.grad_coords.copy_(g)
         step.replay()
         _check(step, a, ln, g, dtype)
+
+
+@pytest.mark.parametrize("R", [1, 2])
+@pytest.mark.parametrize("B,L,kind", [(600, 333, "mixed"), (16, 1024, "mixed"), (3, 2049, "equal"), (19, 4100, "mixed"),
+                                      (9, 8400, "long"), (9, 16500, "long")])
+def test_step_gradients_in_float64(R, B, L, kind):
+    """Relative to each chain's largest gradient.  The frame of a residue is a
+    product of 3 n steps, which turns with their roundings (3 n of them, some
+    2^-53 each), and a torque sum of as many terms as the gradient rounds less:
+    8 n 2^-53, 1.5e-11 at the longest; a record or a sum in float32 is 6e-8 off."""
+    from torchproteinlibrary_amd.ReducedModel.Angles2Backbone.Angles2Backbone import Angles2BackboneStep
+    lens = _lengths(B, L, kind, 64 * R, np.random.default_rng(L + R))
+    a, ln, g = _case(B, L, lens, torch.float64, B + L)
+    step = Angles2BackboneStep(a, ln, config=(R, R))
+    step.grad_coords.copy_(g)
+    step.replay()
+    c, ga = _oracle(a, ln, g)
+    n = ln.double().cpu().clamp_min(1)
+    scale = ga.abs().amax(dim=(1, 2))
+    off = (step.grad_angles.cpu() - ga).abs().amax(dim=(1, 2))
+    assert (off <= 8 * n * 2.0 ** -53 * scale).all(), (off / scale / n * 2.0 ** 53).max()
+    reach = c.abs().amax(dim=1)
+    assert ((step.coords.cpu() - c).abs().amax(dim=1) <= 8 * n * 2.0 ** -53 * reach).all()
