@@ -2517,8 +2517,8 @@ bool forward_groups_fit(int batch, int angles_stride) {
 //   300 32 -> 46 / 41 -> 53, 1024 x 128 16.9 -> 18.5 / 20.6 -> 22.0, 8 x 3000 56 -> 75 / 65 ->
 //   82; float64: 256 x 300 18.1 -> 17.1 / 21.2 -> 19.5, 256 x 600 28.6 -> 30.4 / 35.9 -> 32.9,
 //   512 x 200 20 -> 23 / 23 -> 26, 512 x 450 40 -> 38 / 46 -> 42, 64 x 1000 26 -> 33 / 32 -> 37.
-//   With names and 14 to 16 blocks many structures win too (1024 x 1000 float32 131 -> 112, U
-//   longest first 89 -> 76; 300 x 1000 50 -> 55).
+//   With names and 14 to 16 blocks many structures win too in float32 (1024 x 1000 131 -> 112,
+//   U longest first 89 -> 76; not 300 x 1000 50 -> 55, float64 188 -> 194).
 // A structure of one block needs no groups, whatever the form.
 bool forward_groups_pay(bool f64, int batch, int nb) {
     const int cus = compute_units();
@@ -2533,7 +2533,7 @@ int forward_form(bool f64, int batch, int angles_stride, int atoms_stride, bool 
         return TPLX_A2C_FWD_GROUPS;
     const int most = (f64 ? 8 : 13) + (names ? f64 ? 2 : 3 : 0);
     const bool fused = batch <= cus                ? nb <= most
-                       : names && nb > 13          ? nb <= 16 && batch >= 2 * cus
+                       : names && !f64 && nb > 13  ? nb <= 16 && batch >= 2 * cus
                                                    : batch <= 2 * cus && nb >= 5 && nb <= (f64 ? 10 : 7);
     return fused ? TPLX_A2C_FWD_FUSED : TPLX_A2C_FWD_RUNS;
 }
@@ -2575,8 +2575,9 @@ void launch_forward(int form, hipStream_t s, const uint8_t* sequences, int seq_s
     }
     // One wave per block up to 8, or up to 16 where every structure can have a
     // CU; above that the waves go round.  Beyond one structure per CU the
-    // kernel is held to 128 VGPRs, so that two workgroups of 8 waves fit (512 x
-    // 300: 30 -> 25 us).
+    // kernel is held to 128 VGPRs, so that two workgroups of 8 waves fit, and
+    // spills: 100 bytes in float32 (512 x 300: 30 -> 25 us), 152 in float64 (512
+    // x 300 31.7 -> 29.0, 512 x 600 60.8 -> 53.5).
     const bool few = batch <= compute_units();
     const int most = few ? 16 : 8, rounds = (nslot + most - 1) / most, nw = (nslot + rounds - 1) / rounds;
     const auto kernel = nw > 8 ? a2c_fwd_fused<16, 4, T> : few ? a2c_fwd_fused<8, 2, T> : a2c_fwd_fused<8, 4, T>;
