@@ -555,8 +555,10 @@ def a2c_bench(lengths_mixed, steps, warmup, cpu_seconds, with_cpu):
     forward and backward launches over rotating buffer sets (names not
     written).  Random sequences (uniform over the 20 amino acids) and angles
     phi ~ N(-1.1, 0.3), psi ~ N(2.3, 0.4), omega = pi + N(0, 0.05), side-chain
-    angles ~ U(-pi, pi).  The structures go to the GPU in the order the layer
-    uses (``schedule``: the most atoms first when sizes differ)."""
+    angles ~ U(-pi, pi).  The calls have a workspace, as the layer's do, and an
+    order (``schedule``: the most atoms first when sizes differ), which the
+    layer's do not: the shared blocks that mixed sizes run as take 3% less
+    forward and 1% more backward with it (1024 structures of 50..1000)."""
     import numpy as np
     import torch
     from torchproteinlibrary_amd._native_xform import ext as xext

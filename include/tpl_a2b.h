@@ -77,9 +77,10 @@ enum tpl_a2b_error {
  * chain's workgroup fits on the device at once, one workgroup takes a whole
  * chain instead (a wave per chunk, the chunks meeting in LDS; the sync words
  * go unused).  In the forward, other batches of at most 4096 chains of 3 to 8
- * chunks are packed into workgroups in the same way.  The backward chunk is also the checkpoint stride: the forward
- * saves the FP64 frame at every backward-chunk boundary, so forward and
- * backward of one step must use the same config. */
+ * chunks are packed into workgroups in the same way where that is faster.  The
+ * backward chunk is also the checkpoint stride: the forward saves the FP64
+ * frame at every backward-chunk boundary, so forward and backward of one step
+ * must use the same config. */
 typedef struct tpl_a2b_config {
     int32_t fwd_res_per_lane; /* 1, 2, 4 or 8 (TPL_A2B_F64: up to 4) */
     int32_t bwd_res_per_lane; /* 1, 2 or 4 (TPL_A2B_F64: up to 2) */

@@ -274,8 +274,9 @@ def _step_residues(dtype, B, L, lengths):
     read; it is called only where the mix decides.
 
     The tuner times the layer's two kernels, and the step's own behave
-    otherwise: up to 8 chunks a chain (4 of 64 residues) are one kernel, more
-    are two, and a wave has both directions' work, so a lane's residues are the
+    otherwise: up to 8 chunks a chain (4 of 64 residues) are one kernel (1 to 4
+    chunks of few residues per lane only up to a batch; beyond it the layer's
+    two, as tuned), more are two, and a wave has both directions' work, so a lane's residues are the
     length of its chain of operations while the GPU is not full.  Steps, us,
     by residues per lane (equal lengths, float32 unless marked):
       one kernel while it can be, with few residues per lane:
@@ -316,8 +317,9 @@ class Angles2BackboneStep:
     (``grad_coords`` -> ``grad_angles``) on the current stream, with nothing
     allocated, no host synchronisation and one launch per step, or two: chains
     of at most 8 chunks run in one kernel when both directions have the same
-    chunk size (in float64 always), chains of up to 256 chunks in two, other
-    shapes in the layer's two.  In the step's own kernels the coordinates are
+    chunk size (in float64 always) and, with few short chunks, the batch is not
+    too large for it, chains of up to 256 chunks in two, other shapes in the
+    layer's two.  In the step's own kernels the coordinates are
     those the gradients are computed from, rounded once from float64; they can
     differ from the layer's in the last digits.
     A step reads ``angles``, ``angles_length`` and ``grad_coords`` from their
